@@ -199,7 +199,7 @@ struct Rep {
     unsigned long long* perm_cnt;  // [2 + 2N] attempts, accepts, perm_attempt[N], perm_accept[N]
     double perm_log_eps;            // log of the table cutoff epsilon
     double perm_eps;                // the cutoff epsilon
-    double* perm_t;                 // [2][N][N] PermBisectTable's table (old path, new path)
+    double* perm_t;                 // [N][N] PermBisectTable's table (old path, then new path) past its LDS
     int tab_k;                      // PermBisectTable's n_perm_part (0: not configured)
     int tab_balance;                // its final check: 0 the reference's, 1 detailed balance
     int perm_n_level;               // bisection level of the permuting move

@@ -64,12 +64,12 @@ int noalloc_scratch_ptr(int device, void** out) {
     return SPIMC_OK;
 }
 
-constexpr int kRhoKpt = 8;        // k-vectors per thread in k_rho (default; SPIMC_RHO_KPT 2, 4, 8, 16)
+constexpr int kRhoKpt = 8;              // k-vectors per thread in k_rho (default; SPIMC_RHO_KPT 2, 4, 8, 16)
 constexpr int kRhoKptMin = 2;     // smallest chunking: bounds the number of k chunks
 constexpr int kNumCUs = 256;      // MI355X compute units (for workgroups-per-replica choices)
 // fewest waves for which the pair-once adjoint beats the per-particle one
 constexpr long long kAdjPairsMinWaves = 4096;
-// PermBisectTable: particles of a replica (two N x N tables) and cycle-list entries
+// PermBisectTable: particles of a replica (an N x N table) and cycle-list entries
 constexpr int kTabMaxN = 1024;
 constexpr double kTabMaxEntries = 268435456.;
 constexpr int kBuildKpt = 2;
@@ -269,7 +269,7 @@ struct RepHost {
     int n_chunks = 1;
     char* perm_arena = nullptr;    // perm, iperm
     char* perm_scratch = nullptr;  // the permuting move's chain arrays and counters
-    double* perm_t = nullptr;      // PermBisectTable's two N x N tables
+    double* perm_t = nullptr;      // PermBisectTable's N x N table
 };
 
 // Replicas with identical constant tables (k-set, Ewald coefficients, pair and
@@ -415,6 +415,7 @@ struct spimc_ctx {
     void (*adj_pairs_fn)(const Rep*, unsigned int, int, int) = nullptr;
     int adj_pairs_env = -1;
     bool perm_table = false;  // the running permuting stage is PermBisectTable's
+    int tab_n = 0;            // largest replica whose cycle table fits in the table proposal's LDS
     bool adj_pairs_ok = false;  // its tables and slots fit in LDS
     int groups_wanted = 1;
     bool fork = false;  // rho_k beside the pair kernel on a second stream per group
@@ -1295,11 +1296,16 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
     hipStream_t st = G.stream;
     int rc;
     const bool tuned = c->lds_doubles_max > 0;
-    const size_t shmem = (size_t)c->max_N * (sizeof(double) + sizeof(int));
-    if ((rc = launch(c, SPIMC_KERNEL_PROPOSE, c->perm_table ? k_propose_perm<true> : k_propose_perm<false>, R,
-                     kPermBlock, shmem, st, reps, R, (int)tuned,
-                     c->perm_stage)))
-        return rc;
+    if (c->perm_table) {
+        const size_t shmem = tab_lds_head(c->max_N) + (size_t)c->tab_n * c->tab_n * sizeof(double);
+        rc = launch(c, SPIMC_KERNEL_PROPOSE, k_propose_perm<true>, R, kTabBlock, shmem, st, reps, R, (int)tuned,
+                    c->perm_stage, c->max_N, c->tab_n);
+    } else {
+        const size_t shmem = (size_t)c->max_N * (sizeof(double) + sizeof(int));
+        rc = launch(c, SPIMC_KERNEL_PROPOSE, k_propose_perm<false>, R, kPermBlock, shmem, st, reps, R, (int)tuned,
+                    c->perm_stage, c->max_N, 0);
+    }
+    if (rc) return rc;
     const bool fork = c->any_long && G.side;
     hipStream_t rst = fork ? G.side : st;
     if (fork) {
@@ -1544,6 +1550,23 @@ int ensure_perm(spimc_ctx* c, bool scratch) {
     c->perm_on = true;
     drop_graphs(c);
     return upload_reps(c);
+}
+
+// The LDS of the table proposal: what its static arrays, the rows and the
+// binomials leave of the CU's 160 KB holds the cycle table of replicas of up to
+// tab_n particles (about 125); larger ones keep theirs in global memory.
+int set_tab_lds(spimc_ctx* c) {
+    if (c->tab_n) return SPIMC_OK;
+    hipFuncAttributes at{};
+    HIPCHK(hipFuncGetAttributes(&at, (const void*)k_propose_perm<true>));
+    const size_t used = at.sharedSizeBytes + tab_lds_head(c->max_N), cap = 160 * 1024;
+    int n = 1;
+    for (const auto& h : c->reps)
+        if (used + (size_t)h.dev.N * h.dev.N * sizeof(double) <= cap) n = std::max(n, h.dev.N);
+    HIPCHK(hipFuncSetAttribute((const void*)k_propose_perm<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)(cap - at.sharedSizeBytes)));
+    c->tab_n = n;
+    return SPIMC_OK;
 }
 
 int finish_stage(spimc_ctx* c, const std::vector<unsigned int>& cnt, uint32_t mx, uint8_t* accepted);
@@ -2525,7 +2548,7 @@ int spimc_perm_table_configure(spimc_ctx* c, uint32_t r, uint32_t n_perm_part, u
     if (entries > (double)kTabMaxEntries)
         return fail(SPIMC_ERR_UNSUPPORTED, "the permutation table's cycle list exceeds 2^28 entries");
     HIPCHK(hipDeviceSynchronize());
-    if (!h.perm_t) HIPCHK(hipMalloc((void**)&h.perm_t, 2 * (size_t)N * N * sizeof(double)));
+    if (!h.perm_t) HIPCHK(hipMalloc((void**)&h.perm_t, (size_t)N * N * sizeof(double)));
     h.dev.perm_t = h.perm_t;
     h.dev.tab_k = (int)n_perm_part;
     h.dev.tab_balance = (int)balance;
@@ -2539,6 +2562,7 @@ int spimc_perm_table_stage(spimc_ctx* c, const uint32_t* n_attempts, uint32_t n_
             return fail(SPIMC_ERR_STATE, "spimc_perm_table_configure was not called for a replica with attempts");
     int rc = ensure_perm(c, true);
     if (rc) return rc;
+    if ((rc = set_tab_lds(c))) return rc;
     c->perm_table = true;
     rc = run_stage(c, 3, n_attempts, n_uniform, accepted, false);
     c->perm_table = false;

@@ -37,6 +37,13 @@ __device__ __forceinline__ double chain_new(const Rep& R, int b0, int nb, int n,
     return R.ch_new[((size_t)i * (nb - 1) + t - 1) * 3 + d];
 }
 
+// bytes of the table proposal's dynamic LDS before its table: the walk's row and
+// visited map, and the binomials, of the largest replica
+__host__ __device__ inline size_t tab_lds_head(int max_n) {
+    return ((size_t)max_n * (sizeof(double) + sizeof(int)) + (size_t)7 * (max_n + 1) * sizeof(unsigned int) + 15) &
+           ~(size_t)15;
+}
+
 constexpr int kPermStage = 256;  // beads of a proposal bisected on LDS by one wavefront
 
 // Orders the LDS traffic of one wavefront (the compiler may not move loads or
@@ -106,99 +113,122 @@ __device__ __forceinline__ int perm_level_step(const Rep& R, Prop* pr, int level
 // GenCombPermK are not in the reference tree; both lists are taken here in
 // lexicographic order (permutations of 0..k-1; subsets by their sorted
 // members), as in the oracle.  An entry is never stored: thread t of the
-// proposal's workgroup walks entries [E t / 256, E (t + 1) / 256) of the list.
+// proposal's workgroup owns the subsets [C t / BS, C (t + 1) / BS), C = N over k,
+// of every type.
+//
+// What bounds it is the latency of the table reads along a thread's subsets,
+// with one workgroup per replica.  So the table sits in LDS where it fits, a
+// subset's k^2 table values are read once and every type's weight formed from
+// them (k <= 4: the types are unrolled), the entry is found from the types'
+// totals and then the threads' sums of one type, and only the thread that owns
+// it walks its few entries again.  N = 32, k = 3 (29760 entries), 16 replicas:
+// the proposal took 578 us with the table in global memory, an entry at a time
+// on 256 threads, and the list walked four times; 55 us so.
 // ---------------------------------------------------------------------------
 constexpr int kTabMaxK = 6;
+constexpr int kTabBlock = 512;   // threads of the table proposal (1024 spill registers: 65 us against 55)
+constexpr int kTabTypes = 720;   // kTabMaxK!
 
-__device__ __forceinline__ long long tab_binom(int n, int r) {
-    if (r < 0 || r > n) return 0;
-    long long v = 1;
-    for (int i = 1; i <= r; ++i) v = v * (n - r + i) / i;
-    return v;
-}
-// element j of a k-array held in registers (no dynamic register indexing)
-__device__ __forceinline__ int tab_pick(const int (&a)[kTabMaxK], int j) {
+constexpr int tab_fact(int k) { return k < 2 ? 1 : k * tab_fact(k - 1); }
+template <int K>
+inline constexpr int kTabFact = tab_fact(K);
+
+// element j of an array held in registers (no dynamic register indexing)
+template <int K>
+__device__ __forceinline__ int tab_pick(const int (&a)[K], int j) {
     int v = a[0];
 #pragma unroll
-    for (int i = 1; i < kTabMaxK; ++i) v = j == i ? a[i] : v;
+    for (int i = 1; i < K; ++i) v = j == i ? a[i] : v;
     return v;
 }
-// the rank-th k-subset of 0..n-1 in lexicographic order
-__device__ __forceinline__ void tab_subset(long long rank, int n, int k, int (&s)[kTabMaxK]) {
-    int x = 0;
-#pragma unroll
-    for (int i = 0; i < kTabMaxK; ++i) {
-        if (i < k) {
-            for (;;) {
-                const long long c = tab_binom(n - x - 1, k - i - 1);
-                if (rank < c) break;
-                rank -= c;
-                ++x;
-            }
-            s[i] = x++;
-        } else {
-            s[i] = 0;
-        }
+// binom[q (N + 1) + m] = m over q for q <= k, m <= N (below 2^32: the cycle list
+// holds at most 2^28 entries), by the workgroup.  The quotients are exact: each
+// is a whole number below 2^53.
+__device__ __forceinline__ void tab_binom(unsigned int* binom, int N, int k, int tid, int nthr) {
+    for (int t = tid; t < (k + 1) * (N + 1); t += nthr) {
+        const int q = t / (N + 1), m = t % (N + 1);
+        double v = q <= m ? 1. : 0.;
+        for (int i = 1; i <= q && q <= m; ++i) v = v * (double)(m - q + i) / (double)i;
+        binom[t] = (unsigned int)v;
     }
 }
-// the next k-subset in lexicographic order; false after the last
-__device__ __forceinline__ bool tab_next_subset(int n, int k, int (&s)[kTabMaxK]) {
-    int top = -1;  // the last position below its maximum n - k + i
+// the rank-th K-subset of 0..N-1 in lexicographic order: element i is the
+// largest x with C(N - lo, q) - C(N - x, q) <= rank, q = K - i, lo the first
+// candidate (those are the subsets whose element i lies in [lo, x))
+template <int K>
+__device__ __forceinline__ void tab_subset(unsigned int rank, const unsigned int* binom, int N, int (&s)[K]) {
+    int lo = 0;
 #pragma unroll
-    for (int i = 0; i < kTabMaxK; ++i)
-        if (i < k && s[i] != n - k + i) top = i;
-    if (top < 0) return false;
+    for (int i = 0; i < K; ++i) {
+        const unsigned int* c = binom + (K - i) * (N + 1);
+        const unsigned int all = c[N - lo];
+        int a = lo, b = N - (K - i) + 1;  // the element is in [a, b)
+        while (b - a > 1) {
+            const int x = (a + b) >> 1;
+            if (all - c[N - x] <= rank)
+                a = x;
+            else
+                b = x;
+        }
+        rank -= all - c[N - a];
+        s[i] = a;
+        lo = a + 1;
+    }
+}
+// the next K-subset in lexicographic order (the last one stays)
+template <int K>
+__device__ __forceinline__ void tab_next_subset(int N, int (&s)[K]) {
+    int top = -1;  // the last position below its maximum N - K + i
 #pragma unroll
-    for (int i = 0; i < kTabMaxK; ++i) {
+    for (int i = 0; i < K; ++i)
+        if (s[i] != N - K + i) top = i;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
         if (i == top) s[i] += 1;
-        if (i > top && i < k) s[i] = s[i - 1] + 1;
+        if (i > 0 && top >= 0 && i > top) s[i] = s[i > 0 ? i - 1 : 0] + 1;
     }
-    return true;
 }
-// the rank-th permutation of 0..k-1 in lexicographic order
-__device__ __forceinline__ void tab_perm(int rank, int k, int (&p)[kTabMaxK]) {
-    int fact = 1;
-    for (int i = 2; i < k; ++i) fact *= i;  // (k - 1)!
+// the rank-th permutation of 0..K-1 in lexicographic order
+template <int K>
+__host__ __device__ constexpr void tab_perm(int rank, int (&p)[K]) {
+    int fact = kTabFact<K - 1>;
     unsigned used = 0;
-#pragma unroll
-    for (int i = 0; i < kTabMaxK; ++i) {
-        if (i < k) {
-            const int d = rank / fact;
-            rank -= d * fact;
-            if (k - 1 - i > 0) fact /= (k - 1 - i);
-            int c = 0, seen = -1;
-            for (int v = 0; v < k; ++v)
-                if (!((used >> v) & 1u) && ++seen == d) {
-                    c = v;
-                    break;
-                }
-            p[i] = c;
-            used |= 1u << c;
-        } else {
-            p[i] = i;
-        }
+    for (int i = 0; i < K; ++i) {
+        const int d = rank / fact;
+        rank -= d * fact;
+        if (K - 1 - i > 0) fact /= (K - 1 - i);
+        int c = 0, seen = -1;
+        for (int v = 0; v < K; ++v)
+            if (!((used >> v) & 1u) && ++seen == d) c = v;
+        p[i] = c;
+        used |= 1u << c;
     }
 }
+template <int K>
+struct TabTypes {
+    int p[kTabFact<K>][K];
+    constexpr TabTypes() : p() {
+        for (int t = 0; t < kTabFact<K>; ++t) tab_perm<K>(t, p[t]);
+    }
+};
 // ConstructPermTable's weight of entry (subset s, type p): the product of
 // t(part(i), part(perm(i))) in order (perm_bisect_table_class.h:18-20)
-__device__ __forceinline__ double tab_weight(const double* __restrict__ t, int N, int k, const int (&s)[kTabMaxK],
-                                             const int (&p)[kTabMaxK]) {
+template <int K>
+__device__ __forceinline__ double tab_weight(const double* t, int N, const int (&s)[K], const int (&p)[K]) {
     double w = 1.;
 #pragma unroll
-    for (int i = 0; i < kTabMaxK; ++i)
-        if (i < k) w *= t[(size_t)s[i] * N + tab_pick(s, p[i])];
+    for (int i = 0; i < K; ++i) w *= t[(size_t)s[i] * N + tab_pick<K>(s, p[i])];
     return w;
 }
 // UpdatePermTable (perm_bisect_table_class.h:31-51) into t: the path ends n links
 // after slice b0; pi (LDS, or null for the identity) maps particle j to the
 // particle whose old end j's chain now reaches.
-__device__ __forceinline__ void tab_build(const Rep& R, int b0, int nb, const int* pi, double* __restrict__ t,
-                                          int tid) {
+__device__ __forceinline__ void tab_build(const Rep& R, int b0, int nb, const int* pi, double* t, int tid, int nthr) {
 #pragma clang fp contract(off)
     const int N = R.N, e_end = (b0 + nb) % R.M;
     const bool end_wrapped = b0 + nb >= R.M;
     const double i4ltn = 1. / (4. * R.lambda * R.tau) / nb;
-    for (int idx = tid; idx < N * N; idx += kPermBlock) {
+    for (int idx = tid; idx < N * N; idx += nthr) {
         const int i = idx / N, j = idx % N;
         const int ei = pi ? pi[i] : i, ej = pi ? pi[j] : j;
         const int li = end_wrapped ? label_after_wrap(R, ei) : ei, lj = end_wrapped ? label_after_wrap(R, ej) : ej;
@@ -214,81 +244,217 @@ __device__ __forceinline__ void tab_build(const Rep& R, int b0, int nb, const in
         t[idx] = e > R.perm_log_eps ? exp(e) : 0.;
     }
 }
-// One pass of the workgroup over the cycle list of table t: returns the
-// running total of the weights above epsilon (each thread sums its entries in
-// order, the thread sums are added in thread order: the association differs
-// from the reference's single running sum in the last bits).  With select, also
-// the first entry whose running total exceeds x and the last entry above
-// epsilon (-1 if none) in *sel, *last.  sh: kPermBlock doubles of LDS.
-__device__ __forceinline__ double tab_pass(const Rep& R, const double* __restrict__ t, int tid, bool select, double x,
-                                           double* sh, long long* shl, long long* sel, long long* last) {
-    const int N = R.N, k = R.tab_k;
-    const long long n_comb = tab_binom(N, k);
-    long long fk = 1;
-    for (int i = 2; i <= k; ++i) fk *= i;
-    const long long E = n_comb * fk;
-    const long long lo = E * tid / kPermBlock, hi = E * (tid + 1) / kPermBlock;
-    const double eps = R.perm_eps;
-    int s[kTabMaxK], p[kTabMaxK];
-    auto walk = [&](double run, bool pick, long long* found, long long* lastp) {
-        if (lo >= hi) return run;
-        int type = (int)(lo / n_comb);
-        tab_perm(type, k, p);
-        tab_subset(lo % n_comb, N, k, s);
-        for (long long e = lo; e < hi; ++e) {
-            const double w = tab_weight(t, N, k, s, p);
-            if (w > eps) {
-                run += w;
-                if (pick) {
-                    *lastp = e;
-                    if (*found < 0 && run > x) *found = e;
+
+// LDS of the table proposal's sums
+struct TabLds {
+    double tot[kTabTypes];                  // total of every type
+    double part[kTabBlock / kWave][24];     // wavefronts' sums
+    double base[kTabBlock / kWave];
+    int owner, any;
+    int type, comb;  // the selected entry: its type, the rank of its subset
+};
+
+// The totals of every type's weights above epsilon into S.tot; returns their sum
+// in type order.  The sums associate differently from the reference's single
+// running sum (last-bit differences): a thread's subsets in order, the lanes of
+// a wavefront by its reduction, the wavefronts in order.
+template <int K>
+__device__ __forceinline__ double tab_totals(const double* t, int N, double eps, const int (&s0)[K], int cnt, TabLds& S,
+                                             int tid) {
+    constexpr int F = kTabFact<K>, G = F < 24 ? F : 24, W = kTabBlock / kWave;
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+    for (int f0 = 0; f0 < F; f0 += G) {
+        double sum[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) sum[g] = 0.;
+        int s[K];
+        if constexpr (K <= 4) {
+            constexpr TabTypes<K> types;
+#pragma unroll
+            for (int i = 0; i < K; ++i) s[i] = s0[i];
+            for (int e = 0; e < cnt; ++e) {
+                double v[K][K];
+#pragma unroll
+                for (int i = 0; i < K; ++i)
+#pragma unroll
+                    for (int j = 0; j < K; ++j) v[i][j] = t[(size_t)s[i] * N + s[j]];
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    double x = 1.;
+#pragma unroll
+                    for (int i = 0; i < K; ++i) x *= v[i][types.p[g][i]];
+                    sum[g] += x > eps ? x : 0.;
                 }
+                tab_next_subset<K>(N, s);
             }
-            if (!tab_next_subset(N, k, s)) {
-                ++type;
-                if (type < (int)fk) {
-                    tab_perm(type, k, p);
-                    tab_subset(0, N, k, s);
+        } else {
+            // 120 and 720 types: a walk of the subsets per type
+#pragma unroll 1
+            for (int g = 0; g < G; ++g) {
+                int p[K];
+                tab_perm<K>(f0 + g, p);
+#pragma unroll
+                for (int i = 0; i < K; ++i) s[i] = s0[i];
+                double a = 0.;
+                for (int e = 0; e < cnt; ++e) {
+                    const double x = tab_weight<K>(t, N, s, p);
+                    a += x > eps ? x : 0.;
+                    tab_next_subset<K>(N, s);
                 }
+                a = wave_sum(a);
+                if (lane == 0) S.part[w][g] = a;
             }
         }
-        return run;
-    };
-    sh[tid] = walk(0., false, nullptr, nullptr);
-    __syncthreads();
+        if constexpr (K <= 4) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const double a = wave_sum(sum[g]);
+                if (lane == 0) S.part[w][g] = a;
+            }
+        }
+        __syncthreads();
+        if (tid < G) {
+            double a = 0.;
+            for (int i = 0; i < W; ++i) a += S.part[i][tid];
+            S.tot[f0 + tid] = a;
+        }
+        __syncthreads();
+    }
+    double tot = 0.;
+    for (int f = 0; f < F; ++f) tot += S.tot[f];
+    return tot;
+}
+
+// SelectCycle (perm_bisect_table_class.h:105-119): the first entry whose running
+// total exceeds x, from the types' totals in S.tot, into S.type and S.comb; if x
+// is at or past the total, the last entry above epsilon with last set, else (or
+// with none) false.
+template <int K>
+__device__ __forceinline__ bool tab_select(const double* t, int N, double eps, const int (&s0)[K],
+                                                unsigned int first, int cnt, double x, bool last,
+                                                TabLds& S, int tid) {
+    constexpr int F = kTabFact<K>;
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+    int type = -1, filled = -1;
+    double run = 0.;
+    for (int f = 0; f < F && type < 0; ++f) {
+        const double v = S.tot[f];
+        if (v > 0.) filled = f;
+        if (run + v > x)
+            type = f;
+        else
+            run += v;
+    }
+    const bool past = type < 0;
+    if (past) {
+        if (!last || filled < 0) return false;
+        type = filled;
+    }
+    int p[K], s[K];
+    tab_perm<K>(type, p);
+#pragma unroll
+    for (int i = 0; i < K; ++i) s[i] = s0[i];
+    double mine = 0.;
+    for (int e = 0; e < cnt; ++e) {
+        const double v = tab_weight<K>(t, N, s, p);
+        mine += v > eps ? v : 0.;
+        tab_next_subset<K>(N, s);
+    }
+    double incl = mine;
+    for (int o = 1; o < kWave; o <<= 1) {
+        const double v = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += v;
+    }
+    if (lane == kWave - 1) S.base[w] = incl;
     if (tid == 0) {
-        double acc = 0.;
-        for (int i = 0; i < kPermBlock; ++i) {
-            const double v = sh[i];
-            sh[i] = acc;  // exclusive
-            acc += v;
-        }
-        shl[0] = __double_as_longlong(acc);
+        S.owner = kTabBlock;
+        S.any = -1;
+        S.type = type;
+        S.comb = -1;
     }
     __syncthreads();
-    const double total = __longlong_as_double(shl[0]);
-    if (select) {
-        long long f = -1, l = -1;
-        walk(sh[tid], true, &f, &l);
-        __syncthreads();
-        shl[1 + tid] = f;
-        shl[1 + kPermBlock + tid] = l;
-        __syncthreads();
-        if (tid == 0) {
-            long long fb = -1, lb = -1;
-            for (int i = 0; i < kPermBlock; ++i) {
-                if (fb < 0 && shl[1 + i] >= 0) fb = shl[1 + i];
-                if (shl[1 + kPermBlock + i] >= 0) lb = shl[1 + kPermBlock + i];
+    double pre = run;
+    for (int i = 0; i < w; ++i) pre += S.base[i];
+    if (!past && pre + incl > x) atomicMin(&S.owner, tid);
+    if (mine > 0.) atomicMax(&S.any, tid);
+    __syncthreads();
+    // x fell between the type's total and its threads' sums (rounding): the
+    // type's last entry
+    const int owner = S.owner < kTabBlock ? S.owner : S.any;
+    if (tid == owner) {
+        double r = pre + (incl - mine);
+        int found = -1, end = -1;
+#pragma unroll
+        for (int i = 0; i < K; ++i) s[i] = s0[i];
+        for (int e = 0; e < cnt; ++e) {
+            const double v = tab_weight<K>(t, N, s, p);
+            if (v > eps) {
+                r += v;
+                end = (int)first + e;
+                if (found < 0 && !past && r > x) found = end;
             }
-            shl[1] = fb;
-            shl[2] = lb;
+            tab_next_subset<K>(N, s);
         }
-        __syncthreads();
-        *sel = shl[1];
-        *last = shl[2];
-        __syncthreads();
+        S.comb = found >= 0 ? found : end;
     }
-    return total;
+    __syncthreads();
+    return S.comb >= 0;
+}
+
+// The table of the old path, its total, the selection, and the table and total of
+// the new path (ConstructPermTable, SelectCycle: perm_bisect_table_class.h:10-28,
+// 105-119, 216-225), on the whole workgroup.  t: N x N doubles (LDS, or the
+// replica's buffer).  draw(tot0) returns x for the selection; out: the selected
+// subset and type, its weight, and the two totals (false: nothing selected).
+struct TabChoice {
+    int part[kTabMaxK], type[kTabMaxK];
+    double weight, tot0, tot1;
+};
+template <int K, class Draw>
+__device__ __forceinline__ bool tab_choose(const Rep& R, int b0, int nb, double* t, const unsigned int* binom, int* map,
+                                           TabLds& S, TabChoice& out, int tid, bool last, Draw draw) {
+    const int N = R.N;
+    const double eps = R.perm_eps;
+    const unsigned int n_comb = binom[K * (N + 1) + N];
+    const unsigned int lo = (unsigned int)((unsigned long long)n_comb * (unsigned int)tid / kTabBlock);
+    const unsigned int hi = (unsigned int)((unsigned long long)n_comb * (unsigned int)(tid + 1) / kTabBlock);
+    int s0[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) s0[i] = i;
+    if (lo < hi) tab_subset<K>(lo, binom, N, s0);
+    tab_build(R, b0, nb, nullptr, t, tid, kTabBlock);
+    __syncthreads();
+    const double tot0 = tab_totals<K>(t, N, eps, s0, (int)(hi - lo), S, tid);
+    const double x = draw(tot0);
+    if (!tab_select<K>(t, N, eps, s0, lo, (int)(hi - lo), x, last, S, tid)) return false;
+    int sb[K], tp[K];
+    tab_perm<K>(S.type, tp);
+    tab_subset<K>((unsigned int)S.comb, binom, N, sb);
+    const double weight = tab_weight<K>(t, N, sb, tp);
+    double tot1 = tot0;
+    if (K < N) {
+        // the new path's ends: chain part(i) reaches the old end of part(type(i))
+        for (int j = tid; j < N; j += kTabBlock) map[j] = j;
+        __syncthreads();  // also: every thread has read the old path's table
+        if (tid == 0)
+#pragma unroll
+            for (int i = 0; i < K; ++i) map[sb[i]] = tab_pick<K>(sb, tp[i]);
+        __syncthreads();
+        tab_build(R, b0, nb, map, t, tid, kTabBlock);
+        __syncthreads();
+        tot1 = tab_totals<K>(t, N, eps, s0, (int)(hi - lo), S, tid);
+    }
+    if (tid == 0) {
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            out.part[i] = sb[i];
+            out.type[i] = tp[i];
+        }
+        out.weight = weight;
+        out.tot0 = tot0;
+        out.tot1 = tot1;
+    }
+    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -309,9 +475,12 @@ __device__ __forceinline__ double tab_pass(const Rep& R, const double* __restric
 // TABLE: PermBisectTable::Attempt (perm_bisect_table_class.h:122-228) instead:
 // bead0, the table's selection uniform, then the same bisection; the final
 // table check after level 0 is k_decide's (Prop::tab_*).
+// tab_n: largest replica whose N x N table fits behind the row in dynamic LDS
 template <bool TABLE>
-__global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restrict__ reps, int n_reps, int tuned,
-                                                             int stage_max) {
+__global__ __launch_bounds__(TABLE ? kTabBlock : kPermBlock) void k_propose_perm(const Rep* __restrict__ reps, int n_reps,
+                                                                                 int tuned, int stage_max, int max_n,
+                                                                                 int tab_n) {
+    constexpr int BS = TABLE ? kTabBlock : kPermBlock;
     const int r = blockIdx.x;
     if (r >= n_reps) return;
     const Rep& R = reps[r];
@@ -319,7 +488,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
     extern __shared__ double lds[];
     double* t_row = lds;
     int* vis = reinterpret_cast<int*>(lds + R.N);
-    __shared__ double red[kPermBlock / kWave];
+    __shared__ double red[BS / kWave];
     __shared__ int s_i[8];
     __shared__ double s_w[2];
     __shared__ unsigned long long s_seq;
@@ -348,7 +517,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
     // device draw counters: 0 bead0 and p0; 1 + step the walk; N + 3 + level the
     // level uniforms; N + 3 + n_level + g / 2 the normals
     const uint32_t c_lev = (uint32_t)N + 3u, c_norm = c_lev + (uint32_t)n_lev;
-    for (int i = tid; i < N; i += kPermBlock) vis[i] = -1;
+    for (int i = tid; i < N; i += BS) vis[i] = -1;
     if (tid == 0) {
         int bad = 0, b0, p0;
         long long cur = 0;
@@ -382,65 +551,53 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
     int p = p0, n = 0, stop = 0;  // stop: 1 closed, 2 walk stopped, 3 error
     __shared__ int s_tp[kTabMaxK];  // the table entry's permutation type
     if constexpr (TABLE) {
-        // ---- the table of the old path, its running total, the selection
-        // (ConstructPermTable, SelectCycle: perm_bisect_table_class.h:10-28,105-119)
-        // and the table of the new path (:216-225) ----
-        __shared__ double sh[kPermBlock];
-        __shared__ long long shl[1 + 2 * kPermBlock];
+        __shared__ TabLds S;
+        __shared__ TabChoice ch;
         const int k = R.tab_k;
-        double* t0 = R.perm_t;
-        double* t1 = R.perm_t + (size_t)N * N;
-        tab_build(R, b0, nb, nullptr, t0, tid);
+        // behind the row and the visited map of the largest replica: the binomials, the table
+        unsigned int* binom = reinterpret_cast<unsigned int*>(reinterpret_cast<int*>(lds + max_n) + max_n);
+        double* t_lds = lds + (tab_lds_head(max_n) / sizeof(double));
+        tab_binom(binom, N, k, tid, BS);
         __syncthreads();
-        long long sel = -1, last = -1;
-        const double tot0 = tab_pass(R, t0, tid, false, 0., sh, shl, &sel, &last);
-        if (tid == 0) {
-            int bad = s_i[3];
-            long long cur = s_cur;
-            const double u = tape ? tape_get(R, cur++, &bad) : rng.unif(1u, 0);
-            s_w[1] = tot0 * u;  // UnifRand(0, perm_tot_0)
-            s_i[3] = bad;
-            s_cur = cur;
-        }
-        __syncthreads();
-        tab_pass(R, t0, tid, true, s_w[1], sh, shl, &sel, &last);
+        auto draw = [&](double tot0) {
+            if (tid == 0) {
+                int bad = s_i[3];
+                long long cur = s_cur;
+                const double u = tape ? tape_get(R, cur++, &bad) : rng.unif(1u, 0);
+                s_w[1] = tot0 * u;  // UnifRand(0, perm_tot_0)
+                s_i[3] = bad;
+                s_cur = cur;
+            }
+            __syncthreads();
+            return s_w[1];
+        };
         // x at or past the total (rounding): the last entry free-running, an error on a tape
-        if (sel < 0 && !tape) sel = last;
-        if (sel < 0) {
+        auto choose = [&](double* t) {
+            switch (k) {
+                case 1: return tab_choose<1>(R, b0, nb, t, binom, vis, S, ch, tid, !tape, draw);
+                case 2: return tab_choose<2>(R, b0, nb, t, binom, vis, S, ch, tid, !tape, draw);
+                case 3: return tab_choose<3>(R, b0, nb, t, binom, vis, S, ch, tid, !tape, draw);
+                case 4: return tab_choose<4>(R, b0, nb, t, binom, vis, S, ch, tid, !tape, draw);
+                case 5: return tab_choose<5>(R, b0, nb, t, binom, vis, S, ch, tid, !tape, draw);
+                default: return tab_choose<6>(R, b0, nb, t, binom, vis, S, ch, tid, !tape, draw);
+            }
+        };
+        if (!(N <= tab_n ? choose(t_lds) : choose(R.perm_t))) {
             stop = 3;
         } else {
             stop = 1;
             n = k;
-            const long long n_comb = tab_binom(N, k);
-            int sb[kTabMaxK], tp[kTabMaxK];
-            tab_perm((int)(sel / n_comb), k, tp);
-            tab_subset(sel % n_comb, N, k, sb);
             if (tid == 0) {
                 for (int i = 0; i < k; ++i) {
-                    R.ch_lbl[i] = tab_pick(sb, i);
-                    s_tp[i] = tab_pick(tp, i);
+                    R.ch_lbl[i] = ch.part[i];
+                    s_tp[i] = ch.type[i];
                 }
-                s_w[0] = tab_weight(t0, N, k, sb, tp);
-            }
-            // the new path's ends: chain part(i) reaches the old end of part(type(i))
-            for (int j = tid; j < N; j += kPermBlock) vis[j] = j;
-            __syncthreads();
-            if (tid == 0)
-                for (int i = 0; i < k; ++i) vis[tab_pick(sb, i)] = tab_pick(sb, tab_pick(tp, i));
-            __syncthreads();
-            double tot1 = tot0;
-            if (k < N) {
-                tab_build(R, b0, nb, vis, t1, tid);
-                __syncthreads();
-                tot1 = tab_pass(R, t1, tid, false, 0., sh, shl, &sel, &last);
-            }
-            if (tid == 0) {
+                s_w[0] = ch.weight;
                 pr->tab_on = k < N;
-                pr->tab_ratio = R.tab_balance ? tot0 / (tot1 * s_w[0]) : tot0 / tot1;
+                pr->tab_ratio = R.tab_balance ? ch.tot0 / (ch.tot1 * ch.weight) : ch.tot0 / ch.tot1;
                 pr->u_tab = tape ? 0. : rng.unif(2u, 0);
             }
-            __syncthreads();
-            for (int j = tid; j < N; j += kPermBlock) vis[j] = -1;
+            for (int j = tid; j < N; j += BS) vis[j] = -1;
         }
         __syncthreads();
     }
@@ -454,7 +611,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
 #pragma clang fp contract(off)
             double a[3];
             for (int d = 0; d < 3; ++d) a[d] = pos_at(R, d, b0, p);
-            for (int j = tid; j < N; j += kPermBlock) {
+            for (int j = tid; j < N; j += BS) {
                 const int lj = end_wrapped ? label_after_wrap(R, j) : j;
                 double dd[3];
                 for (int d = 0; d < 3; ++d) dd[d] = minimg(a[d] - pos_at(R, d, e_end, lj), R.L, R.iL);
@@ -548,7 +705,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
     int bad = s_i[3];
     // the visited map becomes the chain map before the wrap; chain labels after
     // it; the chain-end map of NEW mode and the first chain of each of its cycles
-    for (int i = tid; i < n; i += kPermBlock) {
+    for (int i = tid; i < n; i += BS) {
         const int l = R.ch_lbl[i];
         R.mv_pre[l] = i;
         const int l2 = label_after_wrap(R, l);
@@ -579,7 +736,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
             pr->tape_next = cur;
         }
         __syncthreads();
-        for (int i = tid; i < n; i += kPermBlock) {
+        for (int i = tid; i < n; i += BS) {
             R.mv_pre[R.ch_lbl[i]] = -1;
             R.mv_post[R.ch_lbl2[i]] = -1;
         }
@@ -614,7 +771,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
     __shared__ double st_z[kPermStage * 3 + 1], st_u[kMaxLevel];
     const int per = (nb + 1) * 3;
     if (fast) {
-        for (int idx = tid; idx < n * per; idx += kPermBlock) {
+        for (int idx = tid; idx < n * per; idx += BS) {
             const int i = idx / per, t = (idx % per) / 3, d = idx % 3;
             const double x = chain_old(R, b0, t, i, d);
             st_old[idx] = x;
@@ -623,17 +780,17 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
         }
         if (!tape) {
             const int n_norm = 3 * n * (nb - 1);  // at least the open chains' count
-            for (int q = tid; 2 * q < n_norm; q += kPermBlock) {
+            for (int q = tid; 2 * q < n_norm; q += BS) {
                 double z0, z1;
                 rng.normal2(c_norm + (uint32_t)q, &z0, &z1);
                 st_z[2 * q] = z0;
                 st_z[2 * q + 1] = z1;
             }
-            for (int l = tid; l < n_lev; l += kPermBlock) st_u[l] = rng.unif(c_lev + (uint32_t)l, 0);
+            for (int l = tid; l < n_lev; l += BS) st_u[l] = rng.unif(c_lev + (uint32_t)l, 0);
         }
     } else {
         // NEW positions start as the old ones
-        for (int idx = tid; idx < n * nm; idx += kPermBlock) {
+        for (int idx = tid; idx < n * nm; idx += BS) {
             const int i = idx / nm, t = idx % nm + 1;
             for (int d = 0; d < 3; ++d) R.ch_new[(size_t)idx * 3 + d] = chain_old(R, b0, t, i, d);
         }
@@ -730,7 +887,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
         }
         __syncthreads();
         if (s_i[6]) {
-            for (int i = tid; i < n; i += kPermBlock) {
+            for (int i = tid; i < n; i += BS) {
                 R.mv_pre[R.ch_lbl[i]] = -1;
                 R.mv_post[R.ch_lbl2[i]] = -1;
             }
@@ -747,7 +904,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
             const double sigma = sqrt(R.lambda * level_tau);
             const double i4lt_b = 1. / (4. * R.lambda * (0.5 * R.tau * (double)skip));
             double lspo = 0., lspn = 0.;
-            for (int it = tid; it < n_open * nmid; it += kPermBlock) {
+            for (int it = tid; it < n_open * nmid; it += BS) {
 #pragma clang fp contract(off)
                 const int i = vis[it / nmid], k = it % nmid;
                 const int a = 2 * k * skip, b = a + skip, c = a + 2 * skip;
@@ -781,7 +938,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
             const int nlinks = nb >> level;
             const double i4lt_k = 1. / (4. * R.lambda * level_tau);
             double ko = 0., kn = 0.;
-            for (int it = tid; it < n * nlinks; it += kPermBlock) {
+            for (int it = tid; it < n * nlinks; it += BS) {
                 const int i = it / nlinks, a = (it % nlinks) * skip, b = a + skip;
                 const bool ring = nb == M;
                 double dd[3];
@@ -796,10 +953,10 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
                     kn += free_neg_log(&R.kin[level], R.kin_images, i4lt_k, dd);
                 }
             }
-            lspo = block_sum<kPermBlock>(lspo, red);
-            lspn = block_sum<kPermBlock>(lspn, red);
-            ko = block_sum<kPermBlock>(ko, red);
-            kn = block_sum<kPermBlock>(kn, red);
+            lspo = block_sum<BS>(lspo, red);
+            lspn = block_sum<BS>(lspn, red);
+            ko = block_sum<BS>(ko, red);
+            kn = block_sum<BS>(kn, red);
             bad = __syncthreads_or(bad);  // a tape overrun in any thread's draws
             cur += 3 * n_open * nmid;
             g_base += 3u * (uint32_t)(n_open * nmid);
@@ -813,7 +970,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
             cur += 1;
             __syncthreads();
             if (s_i[6]) {
-                for (int i = tid; i < n; i += kPermBlock) {
+                for (int i = tid; i < n; i += BS) {
                     R.mv_pre[R.ch_lbl[i]] = -1;
                     R.mv_post[R.ch_lbl2[i]] = -1;
                 }
@@ -831,9 +988,9 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
     const bool single = n == 1 && (!R.use_long_range || (R.ritems_bis && nm * R.n_chunks <= R.n_ritems_bis));
     if (single) {
         const int l1 = R.ch_lbl[0], l2 = R.ch_lbl2[0];
-        for (int idx = tid; idx < nm * 3; idx += kPermBlock) R.prop_new[idx] = R.ch_new[idx];
+        for (int idx = tid; idx < nm * 3; idx += BS) R.prop_new[idx] = R.ch_new[idx];
         if (R.use_long_range)
-            for (int t = tid; t < 6 * nm; t += kPermBlock) {
+            for (int t = tid; t < 6 * nm; t += BS) {
                 const int m = t / 6;
                 double xo[3], xn[3];
                 for (int d = 0; d < 3; ++d) {
@@ -860,7 +1017,7 @@ __global__ __launch_bounds__(kPermBlock) void k_propose_perm(const Rep* __restri
         }
         if (tid < kWave) rho_items_write(R, 0, 0, 0, 0, tid);
         if (R.use_long_range)
-            for (int m = tid; m < nm; m += kPermBlock) moved_row(R, m, (b0 + 1 + m) % M);
+            for (int m = tid; m < nm; m += BS) moved_row(R, m, (b0 + 1 + m) % M);
     }
 }
 
