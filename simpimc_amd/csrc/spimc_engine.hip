@@ -251,6 +251,10 @@ struct RepHost {
     std::vector<int> kidx;
     std::vector<int4> k_runs;  // runs of consecutive n2 at fixed (n0, n1), ordered by (n0, n1)
     std::vector<int> k_order;  // k index of each k-vector in run order
+    std::vector<int4> cols;    // columns (n0, n1) and their entries (Rep::cols, Rep::col_k)
+    std::vector<int2> col_k;
+    int col_max = 0;           // largest |n2| + 1
+    bool col_twice = false;    // a k-vector listed twice
     std::vector<double> kmag, coef_s, coef_b, coef_v;
     SplHost v_r, v_long_r, u, du, u_long_r, du_long_r;
     Spl2Host u2, du2;
@@ -411,9 +415,15 @@ struct spimc_ctx {
     int pair_variant = 3;  // 0 Bare, 1 David order 2, 2 David other order, 3 mixed
     void (*adj_lds_fn)(const Rep*, unsigned int, int) = nullptr;
     // the pair-once adjoint (two launches), used when its link ranges give the
-    // GPU enough waves; SPIMC_ADJ_PAIRS = 0 / 1 forces the choice
+    // GPU enough waves; SPIMC_ADJ_PAIRS forces the per-particle kernel (0), this one
+    // (1) or a workgroup per link (2)
     void (*adj_pairs_fn)(const Rep*, unsigned int, int, int) = nullptr;
     int adj_pairs_env = -1;
+    // the pair-once adjoint with a workgroup per link, for few replicas, and its
+    // shares (grown to the largest call)
+    void (*adj_links_fn)(const Rep*, int, int, int, double*) = nullptr;
+    double* d_adj_part = nullptr;
+    size_t adj_part_cap = 0;
     bool perm_table = false;  // the running permuting stage is PermBisectTable's
     int tab_n = 0;            // largest replica whose cycle table fits in the table proposal's LDS
     bool adj_pairs_ok = false;  // its tables and slots fit in LDS
@@ -432,6 +442,12 @@ struct spimc_ctx {
     int lds_adj_max = 0, lds_whole_max = 0;
     // dynamic LDS bytes of the run-ordered long-range adjoint (0: the per-particle table kernel)
     size_t adj_runs_lds = 0;
+    // the unrolled long-range adjoint (0: not for these k-vectors): registers for
+    // |n2| + 1 of col_max, weights per slice, and its weight buffer (grown to the
+    // largest call)
+    int col_max = 0, col_stride = 0;
+    double4* d_col_w = nullptr;
+    size_t col_w_cap = 0;
     // timing: per-launch dispatch events (every kernel) and device clocks (pair, rho_k)
     bool timing = false, clock = false;
     double clock_hz = 0.;
@@ -673,6 +689,8 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         std::sort(idx.begin(), idx.end(), [&](int a, int b) { return key(a) < key(b); });
         h.k_runs.clear();
         h.k_order.clear();
+        h.cols.clear();
+        h.col_k.clear();
         auto emit = [&](int n0, int n1, const std::vector<int>& ks, const std::vector<int>& n2s, int lo, int hi) {
             // ks[lo..hi] have consecutive n2s; split at 0 into an ascending and a descending run
             int z = lo;
@@ -701,6 +719,17 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
                 emit(n0, n1, ks, n2s, (int)lo, (int)hi);
                 lo = hi + 1;
             }
+            // the same column for the unrolled long-range adjoint
+            int top = 0;
+            for (int n2 : n2s) top = std::max(top, std::abs(n2));
+            const int at = (int)h.col_k.size();
+            const int len = (top + kAdjColPad) / kAdjColPad * kAdjColPad;
+            h.cols.push_back(make_int4((n0 + 128) | (n1 + 128) << 8, len, at, 0));
+            h.col_k.resize(at + len, make_int2(-1, -1));
+            for (size_t i = 0; i < ks.size(); ++i)
+                (n2s[i] >= 0 ? h.col_k[at + n2s[i]].x : h.col_k[at - n2s[i]].y) = ks[i];
+            h.col_max = std::max(h.col_max, top + 1);
+            h.col_twice = h.col_twice || std::adjacent_find(n2s.begin(), n2s.end()) != n2s.end();
             a = e;
         }
     }
@@ -787,6 +816,8 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
             R.coef_v = cv.take<double>(std::max(nk, 1));
             R.k_runs = cv.take<int4>(std::max<size_t>(h.k_runs.size(), 1));
             R.k_order = cv.take<int>(std::max(nk, 1));
+            R.cols = cv.take<int4>(std::max<size_t>(h.cols.size(), 1));
+            R.col_k = cv.take<int2>(std::max<size_t>(h.col_k.size(), 1));
             if (h.v_r.n) R.v_r = carve_spline(cv, h.v_r);
             if (h.v_long_r.n) R.v_long_r = carve_spline(cv, h.v_long_r);
             if (h.u.n) R.u = carve_spline(cv, h.u);
@@ -848,6 +879,8 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
     R.n_links_max = M;
     R.n_chunks = h.n_chunks;
     R.n_runs = (int)h.k_runs.size();
+    R.n_cols = (int)h.cols.size();
+    R.n_col_k = (int)h.col_k.size();
     R.rho_kpt = c->rho_kpt;
     R.index = r;
     R.L = L;
@@ -923,6 +956,8 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         R.coef_v = O.coef_v;
         R.k_runs = O.k_runs;
         R.k_order = O.k_order;
+        R.cols = O.cols;
+        R.col_k = O.col_k;
         R.v_r = O.v_r;
         R.v_long_r = O.v_long_r;
         R.u = O.u;
@@ -959,6 +994,8 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         HIPCHK(hipMemcpy((void*)R.coef_v, h.coef_v.data(), nk * sizeof(double), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy((void*)R.k_runs, h.k_runs.data(), h.k_runs.size() * sizeof(int4), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy((void*)R.k_order, h.k_order.data(), nk * sizeof(int), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy((void*)R.cols, h.cols.data(), h.cols.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy((void*)R.col_k, h.col_k.data(), h.col_k.size() * sizeof(int2), hipMemcpyHostToDevice));
     }
     int rc;
     if ((rc = upload_spline(R.v_r, h.v_r)) || (rc = upload_spline(R.v_long_r, h.v_long_r)) ||
@@ -1709,6 +1746,36 @@ int est_pair_whole(spimc_ctx* c, Rep* base, int nrep, int which) {
 int est_finalize(spimc_ctx* c, Rep* base, int nrep, int what, int acc) {
     return launch(c, SPIMC_KERNEL_ESTIMATORS, k_finalize, (nrep + 63) / 64, 64, 0, c->stream, base, nrep, what, acc);
 }
+// The long-range adjoint by columns: the slices' weights, then the particles, as
+// many replicas at a time as keep the weights within kColBytes.
+constexpr size_t kColBytes = 512u << 20;
+int est_long_cols(spimc_ctx* c, Rep* base, int nrep, int out_est, int compat) {
+    const size_t per = (size_t)c->max_M * c->col_stride;
+    const int step = (int)std::max<size_t>(1, std::min<size_t>(nrep, kColBytes / sizeof(double4) / per));
+    if (per * step > c->col_w_cap) {
+        HIPCHK(hipStreamSynchronize(c->stream));
+        if (c->d_col_w) (void)hipFree(c->d_col_w);
+        c->d_col_w = nullptr;
+        c->col_w_cap = 0;
+        HIPCHK(hipMalloc((void**)&c->d_col_w, per * step * sizeof(double4)));
+        c->col_w_cap = per * step;
+    }
+    auto fn = c->col_max <= 8 ? k_adjoint_cols<8> : c->col_max <= 12 ? k_adjoint_cols<12> : k_adjoint_cols<kAdjColMax>;
+    for (int r = 0; r < nrep; r += step) {
+        const int n = std::min(step, nrep - r), tiles = (c->max_N + 63) / 64;
+        // segments: enough wavefronts for three per SIMD
+        const long long waves = (long long)tiles * c->max_M * n;
+        const int seg = (int)std::max<long long>(1, std::min<long long>(8, 12 * kNumCUs / std::max<long long>(1, waves)));
+        const int tpb = seg > 1 ? 1 : std::min(4, tiles);
+        int rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_weights, dim3(c->max_M, n), 256, 0, c->stream, base + r,
+                        c->max_M, c->col_stride, c->d_col_w);
+        if (!rc)
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, fn, dim3((tiles + tpb - 1) / tpb, c->max_M, n), 64 * seg * tpb, 0, c->stream,
+                        base + r, seg, c->max_M, c->col_stride, (const double4*)c->d_col_w, out_est, compat);
+        if (rc) return rc;
+    }
+    return SPIMC_OK;
+}
 int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, int out_est) {
     dim3 g((c->max_N + 63) / 64, c->max_M, nrep);
     int rc;
@@ -1726,20 +1793,40 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
         // workgroups per replica: enough to fill the GPU when the replicas are few
         const int bpr = std::max(1, std::min(c->max_M, (2 * kNumCUs + nrep - 1) / nrep));
         // pair-once kernel: at most max_M / 2 link ranges of 16 waves' worth per
-        // replica; chosen when they give at least kAdjPairsMinWaves waves
+        // replica; chosen when they give at least kAdjPairsMinWaves waves, else the
+        // workgroup-per-link form
         const int rng_max = std::max(1, c->max_M / 2);
         const int bpr2 = std::max(1, std::min((rng_max + kAdjPairWaves - 1) / kAdjPairWaves,
                                               (int)((kAdjPairsMinWaves + kAdjPairWaves * nrep - 1) / (kAdjPairWaves * nrep))));
         const long long waves2 = (long long)nrep * std::min(kAdjPairWaves * bpr2, rng_max);
-        const bool pairs = c->adj_pairs_ok &&
-                           (c->adj_pairs_env >= 0 ? c->adj_pairs_env != 0 : waves2 >= kAdjPairsMinWaves);
-        if (pairs) {
-            const size_t shmem2 = shmem + (size_t)kAdjPairWaves * kAdjSlotDoubles * sizeof(double);
+        const int form = !c->adj_pairs_ok ? 0 : c->adj_pairs_env >= 0 ? c->adj_pairs_env : waves2 >= kAdjPairsMinWaves ? 1 : 2;
+        const size_t shmem2 = shmem + (size_t)kAdjPairWaves * kAdjSlotDoubles * sizeof(double);
+        if (form == 1) {
             rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_pairs_fn, dim3(nrep, bpr2), kAdjLdsBlock, shmem2, c->stream,
                         base, terms, out_est, 0);
             if (!rc)
                 rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_pairs_fn, dim3(nrep, bpr2), kAdjLdsBlock, shmem2, c->stream,
                             base, terms, out_est, 1);
+        } else if (form == 2) {
+            // workgroups per link: as many as give every CU one, at most one per tile pair
+            const int tiles = (c->max_N + 63) / 64;
+            const int h = std::max(1, std::min(tiles * (tiles + 1) / 2, kNumCUs / std::max(1, c->max_M * nrep)));
+            const size_t need = (size_t)nrep * h * c->max_M * 6 * c->max_N;
+            if (need > c->adj_part_cap) {
+                HIPCHK(hipStreamSynchronize(c->stream));
+                if (c->d_adj_part) (void)hipFree(c->d_adj_part);
+                c->d_adj_part = nullptr;
+                c->adj_part_cap = 0;
+                HIPCHK(hipMalloc((void**)&c->d_adj_part, need * sizeof(double)));
+                c->adj_part_cap = need;
+            }
+            rc = SPIMC_OK;
+            if (terms & SPIMC_GRAD_PAIR_SHORT)
+                rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_links_fn, dim3(c->max_M * h, nrep), kAdjLdsBlock, shmem2,
+                            c->stream, base, h, c->max_M, c->max_N, c->d_adj_part);
+            if (!rc)
+                rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_gather, dim3(c->max_M, nrep), 256, 0, c->stream, base,
+                            terms, out_est, h, c->max_M, c->max_N, (const double*)c->d_adj_part);
         } else {
             rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_lds_fn, dim3(nrep, bpr), kAdjLdsBlock, shmem, c->stream, base,
                         terms, out_est);
@@ -1748,13 +1835,14 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
         rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_local, g, 64, 0, c->stream, base, terms, out_est);
     }
     if (rc || !(terms & SPIMC_GRAD_PAIR_LONG) || !c->any_long) return rc;
+    if (c->col_max > 0) return est_long_cols(c, base, nrep, out_est, compat);
     if (c->adj_runs_lds > 0) {
         dim3 gr(c->max_M, nrep);
         return launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_long_runs, gr, kAdjRunBlock, c->adj_runs_lds, c->stream, base,
                       out_est, compat);
     }
     int mx = 0;
-    for (auto& h : c->reps) mx = std::max(mx, h.dev.max_idx);
+    for (int r = 0; r < nrep; ++r) mx = std::max(mx, c->reps[(base - c->d_reps) + r].dev.max_idx);
     if (mx > kAdjMaxIdx) return fail(SPIMC_ERR_UNSUPPORTED, "adjoint long range supports |n| <= 40");
     const size_t shmem = (size_t)64 * 3 * (mx + 1) * sizeof(double2) + kAdjTile * (sizeof(double2) + sizeof(int) + sizeof(double));
     return launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_long, g, 64, shmem, c->stream, base, out_est, compat);
@@ -1987,7 +2075,9 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
                                                         : vi == 2 ? k_adjoint_local_lds<2, 0> : k_adjoint_local_lds<0, 0>;
         c->adj_pairs_fn = vi == 0 ? k_adjoint_pairs_lds<1, 0> : vi == 1 ? k_adjoint_pairs_lds<2, 2>
                                                             : vi == 2 ? k_adjoint_pairs_lds<2, 0> : k_adjoint_pairs_lds<0, 0>;
-        if (const char* fa = std::getenv("SPIMC_ADJ_PAIRS")) c->adj_pairs_env = std::atoi(fa) != 0;
+        c->adj_links_fn = vi == 0 ? k_adjoint_links<1, 0> : vi == 1 ? k_adjoint_links<2, 2>
+                                                      : vi == 2 ? k_adjoint_links<2, 0> : k_adjoint_links<0, 0>;
+        if (const char* fa = std::getenv("SPIMC_ADJ_PAIRS")) c->adj_pairs_env = std::max(0, std::min(2, std::atoi(fa)));
         if (c->lds_adj_max > 0 &&
             hipFuncSetAttribute((const void*)c->adj_lds_fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 c->lds_adj_max * (int)sizeof(double)) != hipSuccess)
@@ -1997,6 +2087,8 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             const size_t b2 = ((size_t)c->lds_adj_max + (size_t)kAdjPairWaves * kAdjSlotDoubles) * sizeof(double);
             c->adj_pairs_ok = c->lds_adj_max > 0 && b2 <= kPairLdsMaxBytes &&
                               hipFuncSetAttribute((const void*)c->adj_pairs_fn,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)b2) == hipSuccess &&
+                              hipFuncSetAttribute((const void*)c->adj_links_fn,
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)b2) == hipSuccess;
         }
         bool whole = c->lds_doubles_max > 0;
@@ -2009,7 +2101,14 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
         for (auto& h : c->reps)
             if (h.dev.use_long_range)
                 c->adj_runs_lds = std::max(c->adj_runs_lds, (size_t)h.dev.nk * sizeof(double2) + (size_t)h.dev.n_runs * sizeof(int4));
+        // every replica's columns fit the unrolled form (SPIMC_ADJ_RUNS = 0 or 1 asks for the others)
         const char* fr = std::getenv("SPIMC_ADJ_RUNS");
+        for (auto& h : c->reps)
+            if (h.dev.use_long_range && !fr) {
+                c->col_max = std::max(c->col_max, h.col_twice ? kAdjColMax + 1 : h.col_max);
+                c->col_stride = std::max(c->col_stride, (int)h.col_k.size());
+            }
+        if (c->col_max > kAdjColMax) c->col_max = 0;
         if (c->adj_runs_lds > kPairLdsMaxBytes || (fr && std::atoi(fr) == 0)) c->adj_runs_lds = 0;
         if (c->adj_runs_lds > 0 &&
             hipFuncSetAttribute((const void*)k_adjoint_long_runs, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2027,7 +2126,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
                 n_replicas, c->lds_doubles_max ? "k_pair_lds" : "k_pair",
                 c->lds_doubles_max, c->pair_block,
                 "k_rho_loop",
-                c->rho_kpt, c->rho_bpc, c->adj_runs_lds ? "k_adjoint_long_runs" : "k_adjoint_long",
+                c->rho_kpt, c->rho_bpc, c->col_max ? "k_adjoint_cols" : c->adj_runs_lds ? "k_adjoint_long_runs" : "k_adjoint_long",
                 c->lds_adj_max ? "k_adjoint_local_lds" : "k_adjoint_local", c->lds_whole_max ? "k_pair_whole_lds" : "k_pair_whole");
     int rc = upload_reps(c);
     if (rc) return bail(rc);
@@ -2075,7 +2174,7 @@ int spimc_ctx_destroy(spimc_ctx* c) {
         if (h.perm_t) (void)hipFree(h.perm_t);
     }
     for (void* p : {(void*)c->d_reps, (void*)c->d_counts, (void*)c->d_work, (void*)c->d_gr_rmax, (void*)c->d_error,
-                    (void*)c->d_tmp, (void*)c->d_items_tmp})
+                    (void*)c->d_tmp, (void*)c->d_items_tmp, (void*)c->d_adj_part, (void*)c->d_col_w})
         if (p) (void)hipFree(p);
     for (auto& t : c->pending) {
         (void)hipEventDestroy(t.a);
@@ -2406,30 +2505,9 @@ int spimc_action_gradient(spimc_ctx* c, uint32_t r, uint32_t terms, int compat, 
         return fail(SPIMC_ERR_ARG, "compat gradient covers the pair action only");
     const Rep& R = c->reps[r].dev;
     Rep* base = c->d_reps + r;
-    dim3 g((R.N + 63) / 64, R.M, 1);
-    // Long range.  Adjoint: d/dr of sum_k coef_s |rho_k|^2 per slice.  Compat:
-    // IlkkaPairAction::CalcGradientULong (ilkka_pair_action_class.h:231-249),
-    // sum_k u_long_k k Im(conj(rho_k) e^{i k.r}) -- half the adjoint term -- added
-    // once per particle pair (pair_action_class.h:331-334), i.e. (N - 1) times;
-    // zero for the Bare and David actions (pair_action_class.h:158-165).
-    const bool long_on = (terms & SPIMC_GRAD_PAIR_LONG) && R.use_long_range &&
-                         (!compat || R.pair_type == SPIMC_PAIR_ILKKA);
-    if (compat) {
-        rc = launch(c, SPIMC_KERNEL_ADJOINT, k_grad_compat, g, 64, 0, c->stream, base, 0,
-                    (terms & SPIMC_GRAD_PAIR_SHORT) ? 1 : 0);
-    } else {
-        rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_local, g, 64, 0, c->stream, base, terms, 0);
-    }
-    if (!rc && long_on && c->adj_runs_lds > 0) {
-        rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_long_runs, dim3(R.M, 1), kAdjRunBlock, c->adj_runs_lds,
-                    c->stream, base, 0, compat);
-    } else if (!rc && long_on) {
-        if (R.max_idx > kAdjMaxIdx) return fail(SPIMC_ERR_UNSUPPORTED, "adjoint long range supports |n| <= 40");
-        const size_t shmem = (size_t)64 * 3 * (R.max_idx + 1) * sizeof(double2) +
-                             kAdjTile * (sizeof(double2) + sizeof(int) + sizeof(double));
-        rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_long, g, 64, shmem, c->stream, base, 0, compat);
-    }
-    if (rc || (rc = sync_and_resolve(c))) return rc;
+    // (est_gradient: one replica, the adjoint or the reference's differences)
+    if ((rc = est_gradient(c, base, 1, terms, compat, 0))) return rc;
+    if ((rc = sync_and_resolve(c))) return rc;
     HIPCHK(hipMemcpy(out, R.grad, (size_t)3 * R.M * R.N * sizeof(double), hipMemcpyDeviceToHost));
     if (!compat && terms == SPIMC_GRAD_ALL) c->adjoint_fresh = true;
     return SPIMC_OK;

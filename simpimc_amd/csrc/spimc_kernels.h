@@ -50,6 +50,14 @@ __device__ __forceinline__ T gld(const T* p) {
     return *(const __attribute__((address_space(1))) T*)p;
 }
 
+// Loads of data that no kernel writes while this one runs, at an address all
+// lanes share: scalar loads.  (Through a generic pointer the compiler would
+// take the value for a per-lane one.)
+template <class T>
+__device__ __forceinline__ T uld(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)p;
+}
+
 // Partial sums passed between the workgroups of one launch (k_round): 64-bit
 // atomic stores and loads at agent scope, which the memory model performs at
 // the device's coherence point, so a workgroup on another XCD reads them
@@ -2041,6 +2049,35 @@ __device__ __forceinline__ void adj_kinetic(const Rep& R, int b, int i, double* 
     }
 }
 
+// One pair-link's shares of dS/dr: with r = r_q(b) - r_p(b),
+// dU/dr_p(b) = -(U_r rhat + U_s shat) = -e0, dU/dr_p(b+1) = -(U_r' rphat - U_s shat) = -e1,
+// and q's are e0, e1.  The geometry is link_geom_fast's.
+template <int PT, int NORD>
+__device__ __forceinline__ void adj_pair_eval(const Rep& R, const double* lds, const double* a0, const double* c0,
+                                              const double* a1, const double* c1, double* rv, double* rpv, double* e0,
+                                              double* e1) {
+    double rr = 0., pp = 0., ss = 0.;
+    for (int d = 0; d < 3; ++d) {
+        rv[d] = c0[d] - a0[d];
+        rpv[d] = c1[d] - a1[d];
+        rv[d] -= rint(rv[d] * R.iL) * R.L;
+        rpv[d] += rint((rv[d] - rpv[d]) * R.iL) * R.L;
+        const double sv = rv[d] - rpv[d];
+        rr += rv[d] * rv[d];
+        pp += rpv[d] * rpv[d];
+        ss += sv * sv;
+    }
+    const double r = sqrt_pos(rr), rp = sqrt_pos(pp), sl = sqrt_pos(ss);
+    double ur, urp, us;
+    pair_u_grad_lds<PT, NORD>(R, lds, r, rp, sl, ur, urp, us);
+    const double fr = ur / r, frp = urp / rp, so = (sl > 0.) ? us / sl : 0.;
+    for (int d = 0; d < 3; ++d) {
+        const double sv = rv[d] - rpv[d];
+        e0[d] = fr * rv[d] + so * sv;
+        e1[d] = frp * rpv[d] - so * sv;
+    }
+}
+
 // Adds the short-range pair terms of link (b, b+1) to dS/dr at beads b and b+1,
 // one wave, each pair-link evaluated once for both of its particles.  The
 // particles are taken in tiles of 64.  For a tile pair (I, J >= I), lane l holds
@@ -2076,30 +2113,13 @@ __device__ void adj_link_pairs(const Rep& R, const double* lds, double* slot, do
                     c0[d] = pos_at(R, d, b, q);
                     c1[d] = pos_at(R, d, b1, q);
                 }
-                // the geometry of link_geom_fast, s = r - r' formed again where it is used
-                double rv[3], rpv[3], rr = 0., pp = 0., ss = 0.;
+                double rv[3], rpv[3], e0[3], e1[3];
+                adj_pair_eval<PT, NORD>(R, lds, a0, c0, a1, c1, rv, rpv, e0, e1);
                 for (int d = 0; d < 3; ++d) {
-                    rv[d] = c0[d] - a0[d];
-                    rpv[d] = c1[d] - a1[d];
-                    rv[d] -= rint(rv[d] * R.iL) * R.L;
-                    rpv[d] += rint((rv[d] - rpv[d]) * R.iL) * R.L;
-                    const double sv = rv[d] - rpv[d];
-                    rr += rv[d] * rv[d];
-                    pp += rpv[d] * rpv[d];
-                    ss += sv * sv;
-                }
-                const double r = sqrt_pos(rr), rp = sqrt_pos(pp), sl = sqrt_pos(ss);
-                double ur, urp, us;
-                // r = r_q(b) - r_p(b): dU/dr_p(b) = -(U_r rhat + U_s shat), dU/dr_p(b+1) = -(U_r' rphat - U_s shat)
-                pair_u_grad_lds<PT, NORD>(R, lds, r, rp, sl, ur, urp, us);
-                const double fr = ur / r, frp = urp / rp, so = (sl > 0.) ? us / sl : 0.;
-                for (int d = 0; d < 3; ++d) {
-                    const double sv = rv[d] - rpv[d];
-                    const double e0 = fr * rv[d] + so * sv, e1 = frp * rpv[d] - so * sv;
-                    acc[d] -= e0;
-                    acc[3 + d] -= e1;
-                    slot[d * kWave + ql] += e0;
-                    slot[(3 + d) * kWave + ql] += e1;
+                    acc[d] -= e0[d];
+                    acc[3 + d] -= e1[d];
+                    slot[d * kWave + ql] += e0[d];
+                    slot[(3 + d) * kWave + ql] += e1[d];
                 }
             }
             if (diag) {
@@ -2167,6 +2187,119 @@ __global__ __launch_bounds__(kAdjLdsBlock) void k_adjoint_pairs_lds(const Rep* _
     }
     if (pairs)
         for (int b = b_lo + 1; b < b_hi; ++b) adj_link_pairs<PT, NORD>(R, lds, slot, o, b, lane);
+}
+
+// Analytic adjoint, local terms, for few replicas: each pair-link evaluated once,
+// with a whole workgroup per link (h workgroups when M links alone leave CUs
+// idle).  A range of links per wavefront, as above, needs thousands of links in
+// flight; here the 64 partner rotations of a tile pair (64 x 64 particles) are
+// dealt to the workgroup's 16 wavefronts, so one chain fills the chip.  What
+// bounds it then is the evaluation itself, at LDS-gather latency: N = 256,
+// M = 128, one replica, 75 us, against 563 us for a thread per bead
+// on the LDS tables (twice the evaluations, a quarter of the threads busy) and
+// 1177 us for a thread per bead on the global ones.
+// Each tile pair's sums are added over the wavefronts in order and go to the
+// link's own share of part, [h][M][link's first and second slice][3][particle]
+// (strides: max_M, max_N), which k_adjoint_gather adds up: every sum is formed
+// in a fixed order, with no atomics.
+template <int PT, int NORD>
+__global__ __launch_bounds__(kAdjLdsBlock) void k_adjoint_links(const Rep* __restrict__ reps, int h, int max_M, int max_N,
+                                                                double* __restrict__ part) {
+    extern __shared__ double lds[];
+    const Rep R = reps[blockIdx.y];
+    const int b = blockIdx.x / h, hh = blockIdx.x % h;
+    if (b >= R.M || R.N < 2 || R.pair_type == 0) return;
+    stage_tables(R, lds, false);
+    const int M = R.M, N = R.N, b1 = b + 1 == M ? 0 : b + 1, T = (N + kWave - 1) / kWave;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    double* slots = lds + R.lds_doubles;  // [wavefront][6][64]
+    double* slot = slots + w * kAdjSlotDoubles;
+    double* P = part + (((size_t)blockIdx.y * h + hh) * max_M + b) * 6 * max_N;
+    // thread t < 384 owns component t / 64 of the particles t % 64 + 64 J
+    const bool own = threadIdx.x < kAdjSlotDoubles;
+    double* Pt = P + (size_t)(threadIdx.x >> 6) * max_N + lane;
+    if (own)
+        for (int J = 0; J * kWave + lane < N; ++J) Pt[J * kWave] = 0.;
+    const int n_pairs = T * (T + 1) / 2;
+    const int u_lo = (int)((long long)n_pairs * hh / h), u_hi = (int)((long long)n_pairs * (hh + 1) / h);
+    int I = 0, J = u_lo;  // tile pair u is (I, J >= I), row by row
+    while (J >= T - I) {
+        J -= T - I;
+        ++I;
+    }
+    J += I;
+    for (int u = u_lo; u < u_hi; ++u) {
+        const bool diag = J == I;
+        const int nI = min(kWave, N - I * kWave), nJ = min(kWave, N - J * kWave), p = I * kWave + lane;
+        const bool pv = lane < nI;
+        double a0[3], a1[3], acc[6] = {0., 0., 0., 0., 0., 0.};
+        for (int d = 0; d < 3; ++d) {
+            a0[d] = pv ? pos_at(R, d, b, p) : 0.;
+            a1[d] = pv ? pos_at(R, d, b1, p) : 0.;
+        }
+        for (int k = 0; k < 6; ++k) slot[k * kWave + lane] = 0.;
+        const int s1 = diag ? nI / 2 : kWave - 1;
+        for (int s = (diag ? 1 : 0) + w; s <= s1; s += kAdjPairWaves) {
+            const int ql = diag ? (pv ? (lane + s) % nI : lane) : ((lane + s) & (kWave - 1));
+            const bool act = pv && (diag ? !((nI % 2 == 0) && s == nI / 2 && lane >= nI / 2) : ql < nJ);
+            if (!act) continue;
+            const int q = J * kWave + ql;
+            double c0[3], c1[3];
+            for (int d = 0; d < 3; ++d) {
+                c0[d] = pos_at(R, d, b, q);
+                c1[d] = pos_at(R, d, b1, q);
+            }
+            double rv[3], rpv[3], e0[3], e1[3];
+            adj_pair_eval<PT, NORD>(R, lds, a0, c0, a1, c1, rv, rpv, e0, e1);
+            for (int d = 0; d < 3; ++d) {
+                acc[d] -= e0[d];
+                acc[3 + d] -= e1[d];
+                slot[d * kWave + ql] += e0[d];
+                slot[(3 + d) * kWave + ql] += e1[d];
+            }
+        }
+        __syncthreads();
+        double v = 0.;
+        if (own) {
+            for (int i = 0; i < kAdjPairWaves; ++i) v += slots[i * kAdjSlotDoubles + threadIdx.x];
+            if (lane < nJ) Pt[J * kWave] += v;
+        }
+        __syncthreads();
+        for (int k = 0; k < 6; ++k) slot[k * kWave + lane] = acc[k];
+        __syncthreads();
+        if (own) {
+            v = 0.;
+            for (int i = 0; i < kAdjPairWaves; ++i) v += slots[i * kAdjSlotDoubles + threadIdx.x];
+            if (pv) Pt[I * kWave] += v;
+        }
+        __syncthreads();
+        if (++J == T) J = ++I;
+    }
+}
+
+// dS/dr of every bead from k_adjoint_links's shares: the kinetic term, then the
+// link the bead begins and the one it ends, share by share.
+__global__ __launch_bounds__(256) void k_adjoint_gather(const Rep* __restrict__ reps, unsigned int terms, int out_est,
+                                                        int h, int max_M, int max_N, const double* __restrict__ part) {
+    const Rep& R = reps[blockIdx.y];
+    const int b = blockIdx.x;
+    if (b >= R.M) return;
+    const int bp = b == 0 ? R.M - 1 : b - 1;
+    const bool pairs = (terms & 2u) && R.pair_type != 0 && R.N > 1;
+    for (int p = threadIdx.x; p < R.N; p += 256) {
+        double g[3] = {0., 0., 0.};
+        if (terms & 1u) adj_kinetic(R, b, p, g);
+        if (pairs)
+            for (int hh = 0; hh < h; ++hh) {
+                const double* P = part + ((size_t)blockIdx.y * h + hh) * max_M * 6 * max_N + p;
+                for (int d = 0; d < 3; ++d)
+                    g[d] += P[((size_t)b * 6 + d) * max_N] + P[((size_t)bp * 6 + 3 + d) * max_N];
+            }
+        double* o = (out_est ? R.grad_est : R.grad) + 3 * ((size_t)b * R.N + p);
+        o[0] = g[0];
+        o[1] = g[1];
+        o[2] = g[2];
+    }
 }
 
 // Whole-path pair sums with LDS tables (which 0: CalcdUdBeta, 1: CalcV on plain
@@ -2295,6 +2428,153 @@ __global__ __launch_bounds__(64) void k_adjoint_long(const Rep* __restrict__ rep
         o[0] += f * g[0];
         o[1] += f * g[1];
         o[2] += f * g[2];
+    }
+}
+
+// Long-range adjoint: dS_long/dr_p(b) = -2 s box sum_k c_k n_k Im(conj(rho_k) e^{ik.r}).
+// The k-vectors are grouped in columns (n0, n1) of n2 = -m..m.  With w = c conj(rho)
+// and c_n = e^{i n phi_2}, a column's sums over n >= 0,
+//   A = sum w(n) c_n + w(-n) conj(c_n),   B = sum n (w(n) c_n - w(-n) conj(c_n)),
+// take four real weights per n (k_adjoint_weights writes them, once per slice):
+//   s1 = Re(w+ + w-), s2 = Im(w- - w+), s3 = Re(w+ - w-), s4 = Im(w+ + w-):
+//   A = (s1 cx + s2 cy, s3 cy + s4 cx),   B = n (s3 cx - s4 cy, s1 cy - s2 cx),
+// and the gradient takes Im(E A) n0, Im(E A) n1, Im(E B), E = e^{i (n0 phi_0 + n1 phi_1)}.
+// So both signs of n2 cost eight multiply-adds, all independent, with a
+// particle's c_n and n c_n in registers (NM of them); walking the runs of
+// consecutive n2 (k_adjoint_long_runs, kept for |n2| above 15) is one serial
+// chain of complex products, nine operations a k-vector.  The weights are the
+// same for every lane: they come through the scalar cache, which leaves LDS
+// and the vector memory path free (a broadcast LDS read costs as much as a
+// gather).  A wavefront takes 64 particles of a slice and one of the block's
+// segments of the columns; the segments' sums are added in order.
+// N = 256, M = 128, 1979 k-vectors: one replica 170 us by runs with a thread per
+// particle, 57 us by runs in 16 segments, 47 us so (36 us and the weights' 11);
+// 512 replicas 14.6 ms by runs, 14.1 ms (17 ms with a tile per workgroup: the
+// weights then miss the scalar cache); N = 1024, 4012 k-vectors, 8 replicas
+// 2.9 ms by runs, 1.6 ms.
+constexpr int kAdjColMax = 16;  // |n2| + 1 at most
+constexpr int kAdjColPad = 4;   // a column's entries are padded (k = -1) to whole groups of this
+__global__ __launch_bounds__(256) void k_adjoint_weights(const Rep* __restrict__ reps, int max_M, int stride,
+                                                         double4* __restrict__ wts) {
+    const Rep& R = reps[blockIdx.y];
+    const int b = blockIdx.x;
+    if (b >= R.M || !R.use_long_range || R.pair_type == 0) return;
+    const double2* rb = R.rho + ((size_t)R.sel[b] * R.M + b) * R.nk;
+    double4* o = wts + ((size_t)blockIdx.y * max_M + b) * stride;
+    for (int t = threadIdx.x; t < R.n_col_k; t += 256) {
+        const int2 k = R.col_k[t];  // the k-vectors at n2 and -n2, or -1
+        double2 p = make_double2(0., 0.), m = p;
+        if (k.x >= 0) {
+            const double2 v = rb[k.x];
+            const double c = R.coef_s[k.x];
+            p = make_double2(c * v.x, -c * v.y);
+        }
+        if (k.y >= 0) {
+            const double2 v = rb[k.y];
+            const double c = R.coef_s[k.y];
+            m = make_double2(c * v.x, -c * v.y);
+        }
+        o[t] = make_double4(p.x + m.x, m.y - p.y, p.x - m.x, p.y + m.y);
+    }
+}
+// blockDim.x = 64 n_seg tiles-per-block: n_seg > 1 splits one tile's columns; with
+// one segment up to four tiles of a slice share a workgroup, and so its weights
+// in the scalar cache.
+template <int NM>
+__global__ __launch_bounds__(512) void k_adjoint_cols(const Rep* __restrict__ reps, int n_seg, int max_M, int stride,
+                                                      const double4* __restrict__ wts, int out_est, int compat) {
+    const Rep& R = reps[blockIdx.z];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const int seg = n_seg > 1 ? wave : 0, b = blockIdx.y;
+    const int p0 = (n_seg > 1 ? (int)blockIdx.x : (int)blockIdx.x * (int)(blockDim.x / kWave) + wave) * kWave;
+    if (b >= R.M || p0 >= R.N || !R.use_long_range || R.pair_type == 0) return;
+    __shared__ double sums[512 * 3];
+    const int p = min(p0 + lane, R.N - 1);
+    // the segment's columns, about as many weights each
+    const int4* __restrict__ cols = R.cols;
+    const int n_cols = R.n_cols;
+    auto first = [&](int t) {
+        int lo = 0, hi = n_cols;
+        while (lo < hi) {
+            const int m = (lo + hi) >> 1;
+            if (uld(&cols[m].z) < t)
+                lo = m + 1;
+            else
+                hi = m;
+        }
+        return lo;
+    };
+    const int u_lo = n_seg > 1 ? first(R.n_col_k * seg / n_seg) : 0;
+    const int u_hi = n_seg > 1 ? first(R.n_col_k * (seg + 1) / n_seg) : n_cols;
+    const double4* __restrict__ W = wts + ((size_t)blockIdx.z * max_M + b) * stride;
+    double2 st[3], c[NM], nc[NM];
+    for (int d = 0; d < 3; ++d) {
+        double sn, cs;
+        sincos(pos_at(R, d, b, p) * R.box, &sn, &cs);
+        st[d] = make_double2(cs, sn);
+    }
+    c[0] = make_double2(1., 0.);
+    nc[0] = make_double2(0., 0.);
+#pragma unroll
+    for (int n = 1; n < NM; ++n) {
+        c[n] = cmul(st[2], c[n - 1]);
+        nc[n] = make_double2(n * c[n].x, n * c[n].y);
+    }
+    const double2 cst0 = make_double2(st[0].x, -st[0].y), cst1 = make_double2(st[1].x, -st[1].y);
+    double2 e0 = make_double2(1., 0.), e1 = make_double2(1., 0.);
+    int c0 = 0, c1 = 0;
+    double g0 = 0., g1 = 0., g2 = 0.;
+    for (int u = u_lo; u < u_hi; ++u) {
+        // n0 + 128 | (n1 + 128) << 8, entries (n = 0 .. entries - 1), first entry
+        const int n01 = uld(&cols[u].x), len = uld(&cols[u].y);
+        const int n0 = (n01 & 255) - 128, n1 = (n01 >> 8) - 128;
+        for (; c0 < n0; ++c0) e0 = cmul(e0, st[0]);
+        for (; c0 > n0; --c0) e0 = cmul(e0, cst0);
+        for (; c1 < n1; ++c1) e1 = cmul(e1, st[1]);
+        for (; c1 > n1; --c1) e1 = cmul(e1, cst1);
+        const double* w = reinterpret_cast<const double*>(W + uld(&cols[u].z));
+        double ax = 0., ay = 0., bx = 0., by = 0.;
+#pragma unroll
+        for (int q = 0; q < NM; q += kAdjColPad) {
+            if (q < len) {  // (a break would keep the loop from unrolling: c and nc would go to scratch)
+                double s[kAdjColPad][4];
+#pragma unroll
+                for (int i = 0; i < 4 * kAdjColPad; ++i) s[i / 4][i % 4] = uld(w + 4 * q + i);
+#pragma unroll
+                for (int i = 0; i < kAdjColPad; ++i) {
+                    const int n = q + i;
+                    ax = fma(s[i][1], c[n].y, fma(s[i][0], c[n].x, ax));
+                    ay = fma(s[i][3], c[n].x, fma(s[i][2], c[n].y, ay));
+                    if (n > 0) {
+                        bx = fma(-s[i][3], nc[n].y, fma(s[i][2], nc[n].x, bx));
+                        by = fma(-s[i][1], nc[n].x, fma(s[i][0], nc[n].y, by));
+                    }
+                }
+            }
+        }
+        const double2 e = cmul(e0, e1);
+        const double ia = fma(e.x, ay, e.y * ax);
+        g0 = fma((double)n0, ia, g0);
+        g1 = fma((double)n1, ia, g1);
+        g2 = fma(e.x, by, fma(e.y, bx, g2));
+    }
+    const double f = -2. * long_grad_scale(R, compat) * R.long_scale * R.box;
+    double* o = (out_est ? R.grad_est : R.grad) + 3 * ((size_t)b * R.N + p0);
+    if (n_seg > 1) {
+        double* mine = sums + threadIdx.x * 3;
+        mine[0] = g0;
+        mine[1] = g1;
+        mine[2] = g2;
+        __syncthreads();
+        for (int t = threadIdx.x; t < 3 * kWave && p0 + t / 3 < R.N; t += blockDim.x) {
+            double g = 0.;
+            for (int i = 0; i < n_seg; ++i) g += sums[i * 3 * kWave + t];
+            o[t] += f * g;
+        }
+    } else if (p0 + lane < R.N) {
+        o[3 * lane] += f * g0;
+        o[3 * lane + 1] += f * g1;
+        o[3 * lane + 2] += f * g2;
     }
 }
 
