@@ -66,6 +66,7 @@ int noalloc_scratch_ptr(int device, void** out) {
 
 constexpr int kRhoKpt = 8;              // k-vectors per thread in k_rho (default; SPIMC_RHO_KPT 2, 4, 8, 16)
 constexpr int kRhoKptMin = 2;     // smallest chunking: bounds the number of k chunks
+constexpr int kPairBlocks[4] = {256, 512, 768, 1024};  // workgroup sizes of the LDS pair kernel
 constexpr int kNumCUs = 256;      // MI355X compute units (for workgroups-per-replica choices)
 // fewest waves for which the pair-once adjoint beats the per-particle one
 constexpr long long kAdjPairsMinWaves = 4096;
@@ -378,7 +379,9 @@ struct Group {
     // one-launch bisection rounds: pair workgroups per replica, rho_k items per
     // workgroup, the rho_k workgroups' items (first, count, group-local replica),
     // and the replicas' arrival counters (zero between rounds)
+    int round_qpw[2] = {256, 256};  // partners per wavefront of a link
     int round_bpr[2] = {1, 1}, round_ipb[2] = {1, 1}, n_rgrp[2] = {0, 0};  // per move
+    double rho_bytes[2] = {0., 0.};  // rho_k read and written by a round, per move
     int4* d_rgrp[2] = {nullptr, nullptr};
     unsigned int* d_arrive = nullptr;
 };
@@ -409,9 +412,13 @@ struct spimc_ctx {
     bool adjoint_fresh = false;
     // LDS bytes/8 of the largest pair table when every replica's tables stage through LDS, else 0
     int lds_doubles_max = 0;
-    // the LDS pair kernel specialised for the replicas' pair type (mixed types: generic)
-    void (*pair_lds_fn)(const Rep*, int, int, unsigned long long*) = nullptr;
+    // the LDS pair kernel specialised for the replicas' pair type (mixed types:
+    // generic), per workgroup size (kPairBlocks)
+    void (*pair_lds_fn[4])(const Rep*, int, int, unsigned long long*) = {nullptr, nullptr, nullptr, nullptr};
     int pair_block = kPairLdsBlock;
+    // launch shapes chosen per stage by rule (fork_now, pair_block_now,
+    // one_launch_now) until an environment variable or spimc_autotune sets them
+    bool auto_fork = true, auto_block = true, auto_one = true;
     int pair_variant = 3;  // 0 Bare, 1 David order 2, 2 David other order, 3 mixed
     void (*adj_lds_fn)(const Rep*, unsigned int, int) = nullptr;
     // the pair-once adjoint (two launches), used when its link ranges give the
@@ -475,7 +482,7 @@ struct spimc_ctx {
     // a round in one launch (k_round: pair links, rho_k items, then the replica's
     // decision and next proposal by its last workgroup), for small batches
     bool one_launch = false;
-    void (*round_fn[2])(const Rep*, int, int, const RhoItem*, const int4*, int, unsigned int*) = {nullptr, nullptr};
+    void (*round_fn[2])(const Rep*, int, int, int, const RhoItem*, const int4*, int, unsigned int*) = {nullptr, nullptr};
     int one_moves = 1;  // one-launch rounds for bisection (1), or for both moves (2)
     std::string noalloc_error;  // why the address lookup failed, if it did
 };
@@ -1056,6 +1063,7 @@ int build_work_lists(spimc_ctx* c, Group& G) {
         HIPCHK(hipMemset(d, 0, n * sizeof(RhoItem)));
     }
     int ob = 0, od = 0;
+    G.rho_bytes[0] = G.rho_bytes[1] = 0.;
     for (int r = G.r0; r < G.r0 + G.n; ++r) {
         Rep& R = c->reps[r].dev;
         if (!R.use_long_range) continue;
@@ -1066,6 +1074,8 @@ int build_work_lists(spimc_ctx* c, Group& G) {
         R.n_ritems_dis = nd;
         ob += nb;
         od += nd;
+        G.rho_bytes[0] += 32. * R.nk * ((1 << R.n_level) - 1);
+        G.rho_bytes[1] += 32. * R.nk * R.M;
     }
     if (c->round_fn[0] && c->lds_doubles_max > 0) {
         // one-launch rounds, per move: pair workgroups per replica (fewer links
@@ -1073,20 +1083,27 @@ int build_work_lists(spimc_ctx* c, Group& G) {
         // partners), and as many rho_k items per workgroup as keep the launch
         // within what the GPU holds at once (a deciding workgroup would otherwise
         // hold a slot that later workgroups wait for)
-        const int waves = kRoundBlock / 64;
+        constexpr int waves = kRoundBlock / 64;
         int max_N = 1;
         for (int r = G.r0; r < G.r0 + G.n; ++r) max_N = std::max(max_N, c->reps[r].dev.N);
-        const int lpb = waves / std::min(waves, (max_N + 255) / 256);
         for (int mv = 0; mv < 2; ++mv) {
             const int links = mv == 0 ? G.max_bis_links : G.max_M, n_items = mv == 0 ? ob : od;
-            G.round_bpr[mv] = std::max(1, std::min((links + lpb - 1) / lpb, (2 * kNumCUs + G.n - 1) / G.n));
             int occ = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)c->round_fn[mv], kRoundBlock,
                                                              (size_t)c->lds_doubles_max * sizeof(double)) != hipSuccess)
                 occ = 1;
+            const int cap = std::max(1, occ) * kNumCUs;
+            // a link's partners over as many wavefronts as still let every rho_k item
+            // have a workgroup of its own (N = 256, M = 128, one
+            // replica: 22 us a bisection round with 64 partners each, 26 us with 256)
+            for (int qpw : {64, 128, 256}) {
+                const int lpb = waves / pair_split<waves>(max_N, qpw);
+                G.round_qpw[mv] = qpw;
+                G.round_bpr[mv] = std::max(1, std::min((links + lpb - 1) / lpb, (2 * kNumCUs + G.n - 1) / G.n));
+                if (G.n * G.round_bpr[mv] + n_items <= cap) break;
+            }
             // at least half of what the GPU holds goes to rho_k workgroups, also
             // when the pair workgroups alone would fill it
-            const int cap = std::max(1, occ) * kNumCUs;
             const int room = std::max(cap / 2, cap - G.n * G.round_bpr[mv]);
             G.round_ipb[mv] = std::max(1, (n_items + room - 1) / room);
             if (const char* f = std::getenv("SPIMC_ROUND_IPB")) G.round_ipb[mv] = std::max(1, std::atoi(f));
@@ -1173,24 +1190,65 @@ int ensure_tmp(spimc_ctx* c, size_t n_doubles, size_t n_items) {
     return SPIMC_OK;
 }
 
-// One round of a move stage for every replica.
-// Selects the LDS pair kernel of workgroup size bs (256, 512, 768 or 1024).
-int set_pair_block(spimc_ctx* c, int bs) {
+// The LDS pair kernels of every workgroup size for the context's pair type.
+int set_pair_fns(spimc_ctx* c) {
     using PairFn = void (*)(const Rep*, int, int, unsigned long long*);
     const PairFn fns[4][4] = {
         {k_pair_lds<1, 0, 256>, k_pair_lds<2, 2, 256>, k_pair_lds<2, 0, 256>, k_pair_lds<0, 0, 256>},
         {k_pair_lds<1, 0, 512>, k_pair_lds<2, 2, 512>, k_pair_lds<2, 0, 512>, k_pair_lds<0, 0, 512>},
         {k_pair_lds<1, 0, 768>, k_pair_lds<2, 2, 768>, k_pair_lds<2, 0, 768>, k_pair_lds<0, 0, 768>},
         {k_pair_lds<1, 0, 1024>, k_pair_lds<2, 2, 1024>, k_pair_lds<2, 0, 1024>, k_pair_lds<0, 0, 1024>}};
-    const int bi = bs == 256 ? 0 : bs == 512 ? 1 : bs == 768 ? 2 : bs == 1024 ? 3 : -1;
-    if (bi < 0) return fail(SPIMC_ERR_ARG, "pair workgroup size must be 256, 512, 768 or 1024");
-    c->pair_block = bs;
-    c->pair_lds_fn = fns[bi][c->pair_variant];
-    if (c->lds_doubles_max > 0 &&
-        hipFuncSetAttribute((const void*)c->pair_lds_fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            c->lds_doubles_max * (int)sizeof(double)) != hipSuccess)
-        return fail(SPIMC_ERR_HIP, "pair kernel LDS size");
+    for (int i = 0; i < 4; ++i) {
+        c->pair_lds_fn[i] = fns[i][c->pair_variant];
+        if (c->lds_doubles_max > 0 &&
+            hipFuncSetAttribute((const void*)c->pair_lds_fn[i], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                c->lds_doubles_max * (int)sizeof(double)) != hipSuccess)
+            return fail(SPIMC_ERR_HIP, "pair kernel LDS size");
+    }
     return SPIMC_OK;
+}
+
+// Sets the LDS pair kernel's workgroup size (256, 512, 768 or 1024).
+int set_pair_block(spimc_ctx* c, int bs) {
+    if (std::find(std::begin(kPairBlocks), std::end(kPairBlocks), bs) == std::end(kPairBlocks))
+        return fail(SPIMC_ERR_ARG, "pair workgroup size must be 256, 512, 768 or 1024");
+    c->pair_block = bs;
+    return SPIMC_OK;
+}
+
+// Whether a round's rho_k kernel runs beside its pair kernel.  By rule: from 256 MB
+// of rho_k traffic a round (60 us of it at the copy rate).  The second stream's
+// events cost 12 us a round: N = 256, M = 128, 1979 k-vectors, bisection of 128
+// replicas (121 MB) 69 us beside, 62 us after; displacement of 64 (519 MB) 159 us
+// beside, 176 us after, of 32 (259 MB) 101 and 99; N = 128, M = 64, 257 k-vectors,
+// displacement of 256 replicas (135 MB) 165 us beside, 130 us after.
+constexpr double kForkBytes = 256e6;
+bool fork_now(const spimc_ctx* c, const Group& G, int move) {
+    return c->auto_fork ? G.rho_bytes[move == 1] >= kForkBytes : c->fork;
+}
+
+// Workgroup size of a round's LDS pair kernel, one wavefront a link at a time.  By
+// rule: the smallest whose workgroups still number at most the CUs, so that few
+// replicas spread their links over more of the chip (N = 256, M = 128: bisection
+// of 1 replica 34 us a round with 256 threads, 44 us with 1024; displacement of
+// 16 replicas 63 us with 512, 73 and 72 us with 256 and 1024); beside rho_k 512,
+// which leaves room for its workgroups on every CU.
+int pair_block_now(const spimc_ctx* c, int n_reps, int links, bool beside) {
+    if (!c->auto_block) return c->pair_block;
+    if (beside) return 512;
+    for (int bs : kPairBlocks)
+        if ((long long)n_reps * ((links + bs / 64 - 1) / (bs / 64)) <= kNumCUs) return bs;
+    return kPairLdsBlock;
+}
+
+int launch_pair_lds(spimc_ctx* c, hipStream_t st, Rep* reps, int n_reps, int links, bool beside, unsigned long long* kt) {
+    const int bs = pair_block_now(c, n_reps, links, beside), waves = bs / 64;
+    // workgroups per replica: one when the replicas fill the GPU, more (up to one
+    // per bs / 64 links) when they are few
+    const int bpr = std::max(1, std::min((links + waves - 1) / waves, (2 * kNumCUs + n_reps - 1) / n_reps));
+    const int i = (int)(std::find(std::begin(kPairBlocks), std::end(kPairBlocks), bs) - std::begin(kPairBlocks));
+    return launch(c, SPIMC_KERNEL_PAIR, c->pair_lds_fn[i], n_reps * bpr, bs, (size_t)c->lds_doubles_max * sizeof(double),
+                  st, reps, n_reps, bpr, kt);
 }
 
 // Dynamic LDS of the persistent kernel: the pair tables (rounded to 16 bytes),
@@ -1223,12 +1281,22 @@ bool one_launch_eligible(const spimc_ctx* c) {
     return c->round_fn[0] && c->round_fn[1] && c->lds_doubles_max > 0 && c->fuse_rounds && !c->perm_on &&
            c->rho_kpt == kRhoKpt;
 }
-// Whether a stage of this move runs one-launch rounds: bisection, and with
-// one_moves 2 displacement too; not while the device clocks time the pair and
-// rho_k kernels (k_round has no separate rho_k kernel to time, so those rounds
-// run as three launches).
+// Whether a stage of this move runs one-launch rounds; not while the device clocks
+// or events time the pair and rho_k kernels (k_round has no separate rho_k kernel
+// to time, so those rounds run as three launches).  By rule: where a rho_k
+// workgroup takes at most two items for the launch to fit what the GPU holds at
+// once, four with tables of more than 48 KB (which three launches stage too).  A
+// round then, against three launches: N = 32, M = 32, bisection of 1 replica 16
+// and 23 us, of 128 (two items) 22 and 28, of 256 (four) 50 and 33; N = 256,
+// M = 128 with the 96 KB table, bisection of 16 (two items) 27 and 47 us, of 32
+// (four) 30 and 38, of 64 (eight) 84 and 46; displacement of 4 (four) 39 and 38,
+// of 8 (eight) 82 and 45.
 bool one_launch_now(const spimc_ctx* c, int move) {
-    return c->one_launch && move < c->one_moves && !c->clock && one_launch_eligible(c);
+    if (c->clock || !one_launch_eligible(c)) return false;
+    if (!c->auto_one) return c->one_launch && move < c->one_moves;
+    if (c->timing) return false;
+    const int most = (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024 ? 4 : 2;
+    return move < 2 && c->groups[0].round_ipb[move] <= most;
 }
 
 
@@ -1309,8 +1377,9 @@ int capture_pers_graph(spimc_ctx* c, int move) {
 
 // The rho_k kernel of a round: rho_bpc workgroups per CU looping over the items
 // (0: one workgroup per item).
-int launch_rho(spimc_ctx* c, hipStream_t st, const RhoItem* ri, int nr, unsigned long long* kt) {
-    const int g = c->rho_bpc > 0 ? std::min(nr, c->rho_bpc * kNumCUs) : nr;
+int launch_rho(spimc_ctx* c, hipStream_t st, const RhoItem* ri, int nr, bool beside, unsigned long long* kt) {
+    const int bpc = c->auto_fork ? (beside ? 2 : 0) : c->rho_bpc;
+    const int g = bpc > 0 ? std::min(nr, bpc * kNumCUs) : nr;
     return launch(c, SPIMC_KERNEL_RHO, c->rho_loop_fn, g, kRhoBlock, 0, st, ri, nr, kt);
 }
 
@@ -1350,7 +1419,7 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
         HIPCHK(hipStreamWaitEvent(G.side, G.ev_fork, 0));
     }
     if (c->any_long) {
-        if (G.n_ritem_bis && (rc = launch_rho(c, rst, G.d_ritem_bis, G.n_ritem_bis, nullptr))) return rc;
+        if (G.n_ritem_bis && (rc = launch_rho(c, rst, G.d_ritem_bis, G.n_ritem_bis, c->fork, nullptr))) return rc;
         int max_chunks = 1, max_slots = 1;
         for (int r = G.r0; r < G.r0 + G.n; ++r) {
             max_chunks = std::max(max_chunks, c->reps[r].dev.n_chunks);
@@ -1368,14 +1437,9 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
     }
     if (fork) HIPCHK(hipEventRecord(G.ev_join, G.side));
     if (tuned) {
-        const size_t lds = (size_t)c->lds_doubles_max * sizeof(double);
         int max_links = 1;
         for (int r = G.r0; r < G.r0 + G.n; ++r) max_links = std::max(max_links, 1 << c->reps[r].dev.perm_n_level);
-        const int waves = c->pair_block / 64;
-        const int bpr = std::max(1, std::min((max_links + waves - 1) / waves, (2 * kNumCUs + R - 1) / R));
-        if ((rc = launch(c, SPIMC_KERNEL_PAIR, c->pair_lds_fn, R * bpr, c->pair_block, lds, st, reps, R, bpr,
-                         (unsigned long long*)nullptr)))
-            return rc;
+        if ((rc = launch_pair_lds(c, st, reps, R, max_links, c->fork, nullptr))) return rc;
     }
     // as many workgroups as a full grid: a listed item each, the others return at once
     if ((rc = launch(c, SPIMC_KERNEL_PAIR, k_pair_multi_list, R * kPairMultiBpr, kPairMultiBlock, 0, st, reps,
@@ -1394,7 +1458,7 @@ int launch_one_round(spimc_ctx* c, const Group& G, int move) {
     const int R = G.n;
     const size_t shmem = (size_t)c->lds_doubles_max * sizeof(double);
     return launch(c, SPIMC_KERNEL_PAIR, c->round_fn[move], R * G.round_bpr[move] + G.n_rgrp[move], kRoundBlock, shmem,
-                  G.stream, c->d_reps + G.r0, R, G.round_bpr[move],
+                  G.stream, c->d_reps + G.r0, R, G.round_bpr[move], G.round_qpw[move],
                   (const RhoItem*)(move == 0 ? G.d_ritem_bis : G.d_ritem_dis), (const int4*)G.d_rgrp[move],
                   G.round_ipb[move], G.d_arrive);
 }
@@ -1426,29 +1490,20 @@ int launch_round(spimc_ctx* c, const Group& G, int move) {
     const int np = move == 0 ? G.n_pair_bis : G.n_pair_dis;
     const RhoItem* ri = move == 0 ? G.d_ritem_bis : G.d_ritem_dis;
     const int nr = move == 0 ? G.n_ritem_bis : G.n_ritem_dis;
-    if (c->fork && c->lds_doubles_max > 0 && np && G.side && nr) {
+    const int links = move == 0 ? G.max_bis_links : G.max_M;
+    if (fork_now(c, G, move) && c->lds_doubles_max > 0 && np && G.side && nr) {
         // fork: rho_k on the side stream beside the pair kernel, joined before the decision
         HIPCHK(hipEventRecord(G.ev_fork, st));
         HIPCHK(hipStreamWaitEvent(G.side, G.ev_fork, 0));
-        if ((rc = launch_rho(c, G.side, ri, nr, kt))) return rc;
+        if ((rc = launch_rho(c, G.side, ri, nr, true, kt))) return rc;
         HIPCHK(hipEventRecord(G.ev_join, G.side));
-        const size_t shmem = (size_t)c->lds_doubles_max * sizeof(double);
-        const int waves = c->pair_block / 64, max_links = move == 0 ? G.max_bis_links : G.max_M;
-        const int bpr = std::max(1, std::min((max_links + waves - 1) / waves, (2 * kNumCUs + R - 1) / R));
-        rc = launch(c, SPIMC_KERNEL_PAIR, c->pair_lds_fn, R * bpr, c->pair_block, shmem, st, reps, R, bpr, kt);
-        if (rc) return rc;
+        if ((rc = launch_pair_lds(c, st, reps, R, links, true, kt))) return rc;
         if (multi && (rc = launch_pair_multi(c, G, st))) return rc;
         HIPCHK(hipStreamWaitEvent(st, G.ev_join, 0));
     } else if (c->lds_doubles_max > 0 && np) {
-        const size_t shmem = (size_t)c->lds_doubles_max * sizeof(double);
-        // workgroups per replica: one when the replicas fill the GPU, more (up to one
-        // per BS/64 links) when they are few
-        const int waves = c->pair_block / 64, max_links = move == 0 ? G.max_bis_links : G.max_M;
-        const int bpr = std::max(1, std::min((max_links + waves - 1) / waves, (2 * kNumCUs + R - 1) / R));
-        rc = launch(c, SPIMC_KERNEL_PAIR, c->pair_lds_fn, R * bpr, c->pair_block, shmem, st, reps, R, bpr, kt);
-        if (rc) return rc;
+        if ((rc = launch_pair_lds(c, st, reps, R, links, false, kt))) return rc;
         if (multi && (rc = launch_pair_multi(c, G, st))) return rc;
-        if (nr) rc = launch_rho(c, st, ri, nr, kt);
+        if (nr) rc = launch_rho(c, st, ri, nr, false, kt);
         if (rc) return rc;
     } else {
         if (np) {
@@ -1458,7 +1513,7 @@ int launch_round(spimc_ctx* c, const Group& G, int move) {
         }
         if (multi && (rc = launch_pair_multi(c, G, st))) return rc;
         if (nr) {
-            if ((rc = launch_rho(c, st, ri, nr, kt))) return rc;
+            if ((rc = launch_rho(c, st, ri, nr, false, kt))) return rc;
         }
     }
     if (c->fuse_rounds) return SPIMC_OK;  // decided by the next round's first launch or the stage's end
@@ -1966,11 +2021,18 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
     // SPIMC_STREAMS (replica groups), SPIMC_FORK and SPIMC_RHO_BPC override.
     c->groups_wanted = 1;
     if (const char* f = std::getenv("SPIMC_STREAMS")) c->groups_wanted = std::max(1, std::atoi(f));
+    if (c->groups_wanted > 1) c->auto_fork = c->auto_block = c->auto_one = false;
     c->fork = n_replicas >= 64;
-    if (const char* f = std::getenv("SPIMC_FORK")) c->fork = std::atoi(f) != 0;
+    if (const char* f = std::getenv("SPIMC_FORK")) {
+        c->fork = std::atoi(f) != 0;
+        c->auto_fork = false;
+    }
     if (const char* f = std::getenv("SPIMC_PERM_STAGE")) c->perm_stage = std::max(0, std::min(kPermStage, std::atoi(f)));
     c->rho_bpc = c->fork ? 2 : c->groups_wanted > 1 ? 3 : 0;
-    if (const char* f = std::getenv("SPIMC_RHO_BPC")) c->rho_bpc = std::max(0, std::atoi(f));
+    if (const char* f = std::getenv("SPIMC_RHO_BPC")) {
+        c->rho_bpc = std::max(0, std::atoi(f));
+        c->auto_fork = false;
+    }
     {
         using RhoFn = void (*)(const Rep*, const uint2*, int, int, unsigned long long*);
         const RhoFn fns[2][4] = {{k_rho<2, false>, k_rho<4, false>, k_rho<8, false>, k_rho<16, false>},
@@ -2035,15 +2097,18 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
         int bs = (c->groups_wanted > 1 || c->fork) ? 512 : kPairLdsBlock;
         if (const char* fb = std::getenv("SPIMC_PAIR_BLOCK")) {
             const int v = std::atoi(fb);
-            if (v == 256 || v == 512 || v == 768 || v == 1024) bs = v;
+            if (v == 256 || v == 512 || v == 768 || v == 1024) {
+                bs = v;
+                c->auto_block = false;
+            }
         }
         const int vi = pt == SPIMC_PAIR_BARE ? 0 : pt == SPIMC_PAIR_DAVID ? (nord == 2 ? 1 : 2) : 3;
         c->pair_variant = vi;
-        if (set_pair_block(c, bs) != SPIMC_OK) c->lds_doubles_max = 0;
+        if (set_pair_fns(c) != SPIMC_OK || set_pair_block(c, bs) != SPIMC_OK) c->lds_doubles_max = 0;
         {
             // one-launch rounds (SPIMC_ONE_LAUNCH or spimc_autotune): the pair type's
             // instantiation with the default rho_k chunking
-            using RoundFn = void (*)(const Rep*, int, int, const RhoItem*, const int4*, int, unsigned int*);
+            using RoundFn = void (*)(const Rep*, int, int, int, const RhoItem*, const int4*, int, unsigned int*);
             const RoundFn rf[2][2][4] = {
                 {{k_round<1, 0, kRhoKpt, false, 0>, k_round<2, 2, kRhoKpt, false, 0>, k_round<2, 0, kRhoKpt, false, 0>,
                   k_round<0, 0, kRhoKpt, false, 0>},
@@ -2060,6 +2125,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
                                             c->lds_doubles_max * (int)sizeof(double)) != hipSuccess)
                         c->round_fn[0] = c->round_fn[1] = nullptr;
             if (const char* fo = std::getenv("SPIMC_ONE_LAUNCH")) {
+                c->auto_one = false;
                 c->one_launch = std::atoi(fo) != 0;
                 c->one_moves = std::atoi(fo) >= 2 ? 2 : 1;
             }
@@ -2135,7 +2201,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
         if ((rc = upload_reps(c))) return bail(rc);  // the replicas now point at their rho_k items
         if (std::getenv("SPIMC_VERBOSE"))
             fprintf(stderr, "spimc: %d replica group(s), rho_k beside the pair kernel on a second stream: %s\n",
-                    (int)c->groups.size(), c->fork ? "yes" : "no");
+                    (int)c->groups.size(), c->auto_fork ? "by rule" : c->fork ? "yes" : "no");
     }
     if ((rc = spimc_obs_configure(c, SPIMC_ENERGY_THERMAL, 0, 1e300, 0., 0., 100))) return bail(rc);
     *out = c;
@@ -2882,6 +2948,8 @@ int spimc_autotune(spimc_ctx* c, uint32_t n_rounds, int32_t* chosen) {
     // the sweep's mix: N M / 2^l bisection attempts per N displace attempts
     const Rep& R0 = c->reps[0].dev;
     const uint32_t n_dis = std::max<uint32_t>(1, (uint32_t)((uint64_t)n_rounds * (1u << R0.n_level) / R0.M));
+    const bool saved_auto[3] = {c->auto_fork, c->auto_block, c->auto_one};
+    c->auto_fork = c->auto_block = c->auto_one = false;
     double best_t = 1e300;
     Shape best = saved;
     int tried = 0;
@@ -2907,6 +2975,9 @@ int spimc_autotune(spimc_ctx* c, uint32_t n_rounds, int32_t* chosen) {
             c->one_moves = saved.one >= 2 ? 2 : 1;
             if (c->lds_doubles_max > 0) (void)set_pair_block(c, saved.bs);
             (void)set_pers_block(c, saved.pers);
+            c->auto_fork = saved_auto[0];
+            c->auto_block = saved_auto[1];
+            c->auto_one = saved_auto[2];
             return rc;
         }
         ++tried;

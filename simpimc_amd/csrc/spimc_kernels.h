@@ -693,7 +693,9 @@ constexpr int kPairLdsBlock = 1024;
 // (COH: as agent-scope atomic stores).
 // One lane's OLD and NEW sums of window link j over the partners q_lo + lane,
 // q_lo + lane + 64, ... below q_hi (q_lo a multiple of 128).
-template <int PT, int NORD>
+// ONE: ranges of at most 64 partners take one each (k_pair_lds has none; the
+// second copy of the evaluation would cost it registers).
+template <int PT, int NORD, bool ONE = false>
 __device__ __forceinline__ void pair_link_range(const Rep& R, const double* lds, const Prop& pr, int j, int q_lo,
                                                 int q_hi, int lane, double& uo, double& un) {
     const int M = R.M, p = pr.p;
@@ -707,7 +709,24 @@ __device__ __forceinline__ void pair_link_range(const Rep& R, const double* lds,
     }
     uo = 0.;
     un = 0.;
-    {
+    if (ONE && q_hi - q_lo <= kWave) {
+        // one partner per lane
+        const int q = q_lo + lane;
+        const bool ok = q < q_hi && q != p;
+        const int qa = q < q_hi ? q : q_lo;
+        double a0[3], a1[3];
+        for (int d = 0; d < 3; ++d) {
+            a0[d] = pos_at(R, d, s0, qa);
+            a1[d] = pos_at(R, d, s1, qa);
+        }
+        double r, rp, s2;
+        link_rr_s2(po0, a0, po1, a1, R.L, R.iL, r, rp, s2);
+        const double uo1 = pair_u_lds_s2<PT, NORD>(R, lds, r, rp, s2);
+        link_rr_s2(pn0, a0, pn1, a1, R.L, R.iL, r, rp, s2);
+        const double un1 = pair_u_lds_s2<PT, NORD>(R, lds, r, rp, s2);
+        uo = ok ? uo1 : 0.;
+        un = ok ? un1 : 0.;
+    } else {
         const int N = q_hi;
         // two partners per lane per step: independent evaluation chains for the scheduler
         for (int q = q_lo + lane; q < N; q += 2 * kWave) {
@@ -753,29 +772,31 @@ __device__ __forceinline__ void pair_links_lds(const Rep& R, const double* lds, 
     }
 }
 
-// Wavefronts per window link of a W-wavefront workgroup: a replica of more
-// than 256 particles splits each link's partners over up to W wavefronts.
+// Wavefronts per window link of a W-wavefront workgroup: a link's partners are
+// split over up to W wavefronts of at least qpw (64, 128 or 256) partners each.
 template <int W>
-__device__ __forceinline__ int pair_split(int N) {
-    return min(W, (N + 4 * kWave - 1) / (4 * kWave));
+__host__ __device__ __forceinline__ int pair_split(int N, int qpw) {
+    const int n = (N + qpw - 1) / qpw;
+    return n < W ? n : W;
 }
 
 // The window links of a proposal on a W-wavefront workgroup (part of bpr for
-// the replica), ns = pair_split<W>(N) wavefronts per link: wavefront w takes
-// link jb + w / ns and partner range w % ns, ranges of q_len partners (a
+// the replica), ns = pair_split<W>(N, qpw) wavefronts per link: wavefront w takes
+// link jb + w / ns and partner range w % ns, ranges of q_len partners (64, or a
 // multiple of 128).  A link's sum adds its ranges' wavefront sums in range
 // order; with ns = 1 it is pair_links_lds's.  Every wavefront of the
 // workgroup calls it (it holds workgroup barriers); wpart: W entries of LDS.
 template <int PT, int NORD, bool COH, int W>
 __device__ __forceinline__ void pair_links_split(const Rep& R, const double* lds, const Prop& pr, int part, int bpr,
-                                                 int w, int lane, double2* wpart) {
-    const int ns = pair_split<W>(R.N), lpb = W / ns;
-    const int q_len = ((R.N + ns - 1) / ns + 2 * kWave - 1) / (2 * kWave) * (2 * kWave);
+                                                 int qpw, int w, int lane, double2* wpart) {
+    const int ns = pair_split<W>(R.N, qpw), lpb = W / ns;
+    const int q_each = (R.N + ns - 1) / ns;
+    const int q_len = q_each <= kWave ? kWave : (q_each + 2 * kWave - 1) / (2 * kWave) * (2 * kWave);
     for (int jb = part * lpb; jb < pr.n_links; jb += bpr * lpb) {
         const int j = jb + w / ns, k = w % ns;
         double uo = 0., un = 0.;
         if (w < lpb * ns && j < pr.n_links) {
-            pair_link_range<PT, NORD>(R, lds, pr, j, k * q_len, min(R.N, (k + 1) * q_len), lane, uo, un);
+            pair_link_range<PT, NORD, true>(R, lds, pr, j, k * q_len, min(R.N, (k + 1) * q_len), lane, uo, un);
             uo = wave_sum(uo);
             un = wave_sum(un);
         }
@@ -1360,7 +1381,7 @@ __global__ __launch_bounds__(kDisBlock) void k_decide_propose_displace(const Rep
 // the next round.
 constexpr int kRoundBlock = kRhoBlock;
 template <int PT, int NORD, int KPT, bool NT, int MOVE>
-__global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ reps, int n_reps, int bpr,
+__global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ reps, int n_reps, int bpr, int qpw,
                                                        const RhoItem* __restrict__ items,
                                                        const int4* __restrict__ rgrp, int ipb,
                                                        unsigned int* __restrict__ arrive) {
@@ -1386,7 +1407,7 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
         }
         const Prop pr = *R.prop;
         constexpr int W = kRoundBlock / kWave;
-        if (pr.status == 1 && !pr.generic && part * (W / pair_split<W>(R.N)) < pr.n_links) {
+        if (pr.status == 1 && !pr.generic && part * (W / pair_split<W>(R.N, qpw)) < pr.n_links) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int t = threadIdx.x + k * kRoundBlock;
@@ -1395,7 +1416,7 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
             // the rest (large tables: 96 KB for David's)
             stage_batched(lds, R.bt_a.c, R.bt_b.c, na, nd, 4 * kRoundBlock, kRoundBlock);
             __syncthreads();
-            pair_links_split<PT, NORD, true, W>(R, lds, pr, part, bpr, w, lane, wpart);
+            pair_links_split<PT, NORD, true, W>(R, lds, pr, part, bpr, qpw, w, lane, wpart);
         }
     } else {
         // a group of up to ipb rho_k items of one replica, one after the other
