@@ -426,6 +426,8 @@ struct spimc_ctx {
     // (1) or a workgroup per link (2)
     void (*adj_pairs_fn)(const Rep*, unsigned int, int, int) = nullptr;
     int adj_pairs_env = -1;
+    // the reference's finite differences on the LDS tables (nullptr: global tables)
+    void (*compat_fn)(const Rep*, int, int, int) = nullptr;
     // the pair-once adjoint with a workgroup per link, for few replicas, and its
     // shares (grown to the largest call)
     void (*adj_links_fn)(const Rep*, int, int, int, double*) = nullptr;
@@ -1835,8 +1837,17 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
     dim3 g((c->max_N + 63) / 64, c->max_M, nrep);
     int rc;
     if (compat) {
-        rc = launch(c, SPIMC_KERNEL_ADJOINT, k_grad_compat, g, 64, 0, c->stream, base, out_est,
-                    (terms & SPIMC_GRAD_PAIR_SHORT) ? 1 : 0);
+        const int short_on = (terms & SPIMC_GRAD_PAIR_SHORT) ? 1 : 0;
+        if (c->compat_fn) {
+            // particles per workgroup: halved until the workgroups number the CUs
+            int np = std::min(c->max_N, kCompatBlock);
+            while (np > 64 && (long long)c->max_M * nrep * ((c->max_N + np - 1) / np) < kNumCUs) np = (np + 1) / 2;
+            const size_t shmem = ((size_t)c->lds_adj_max + (size_t)kCompatBlock * 3) * sizeof(double);
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(c->max_M, (c->max_N + np - 1) / np, nrep), kCompatBlock,
+                        shmem, c->stream, base, out_est, short_on, np);
+        } else {
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, k_grad_compat, g, 64, 0, c->stream, base, out_est, short_on);
+        }
         bool ilkka_long = false;
         for (int r = 0; r < nrep; ++r) {
             const Rep& Rr = c->reps[(base - c->d_reps) + r].dev;
@@ -2148,6 +2159,14 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             hipFuncSetAttribute((const void*)c->adj_lds_fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 c->lds_adj_max * (int)sizeof(double)) != hipSuccess)
             c->lds_adj_max = 0;
+        if (c->lds_adj_max > 0) {
+            c->compat_fn = vi == 0 ? k_grad_compat_lds<1, 0> : vi == 1 ? k_grad_compat_lds<2, 2>
+                                                     : vi == 2 ? k_grad_compat_lds<2, 0> : k_grad_compat_lds<0, 0>;
+            const size_t b3 = ((size_t)c->lds_adj_max + (size_t)kCompatBlock * 3) * sizeof(double);
+            if (b3 > kPairLdsMaxBytes || hipFuncSetAttribute((const void*)c->compat_fn,
+                                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)b3) != hipSuccess)
+                c->compat_fn = nullptr;
+        }
         {
             // the pair-once kernel adds its waves' partner slots to the tables
             const size_t b2 = ((size_t)c->lds_adj_max + (size_t)kAdjPairWaves * kAdjSlotDoubles) * sizeof(double);

@@ -1880,6 +1880,170 @@ __global__ __launch_bounds__(64) void k_grad_compat(const Rep* __restrict__ reps
     o[2] = g[2];
 }
 
+// Loads a replica's link-action tables (du_only: the David du_kj_dbeta table
+// instead) into LDS.
+__device__ __forceinline__ void stage_tables(const Rep& R, double* lds, bool du_only) {
+    if (du_only)
+        stage_batched(lds, R.bt_du.c, R.bt_du.c, R.lds_doubles_du, R.lds_doubles_du, 0, (int)blockDim.x);
+    else
+        stage_batched(lds, R.bt_a.c, R.bt_b.c, R.bt_a.ncoef * R.bt_a.ncomp, R.lds_doubles, 0, (int)blockDim.x);
+    __syncthreads();
+}
+
+// The same for the Bare and David actions with the tables in LDS.  Central
+// differences in bead (b, p) of the links (b, b + 1) and (b, b - 1): the bead's
+// own distance r is the same in both links and r' does not move, so the terms of
+// r alone are evaluated once for the two links and those of r' alone not at all:
+// 6 radial terms per pair for Bare (24 with each link action formed whole), 6
+// radial and 12 off-diagonal ones for David.  Where a shifted component crosses
+// half the box the two sides see different images and r' moves with them; those
+// pairs form the whole difference.  The differences are the reference's up to the
+// rounding of the terms that cancel.
+// blockIdx.x: slice; np particles per workgroup (a tile blockIdx.y of the slice's),
+// whose 1024 / np groups of threads share the partners; the groups' sums are added
+// in order.  Bound by FP64 arithmetic and LDS gathers: N = 77, M = 50, 12 replicas
+// 1243 us with a thread per bead on the global tables, 104 us so.
+constexpr int kCompatBlock = 1024;
+// radial part of the Bare link action / tau at one distance
+__device__ __forceinline__ double bare_radial_lds(const Rep& R, const double* lds, double r) {
+    r = clampd(r, R.r_v_min, R.r_v_max);
+    double v = R.is_coulomb ? 0.5 / r : 0.5 * bt_apply(lds, bt_basis(R.bt_a, r));
+    if (R.use_long_range) {
+        const double* vl = lds + (R.is_coulomb ? 0 : R.bt_a.ncoef);
+        v -= 0.5 * bt_apply(vl, bt_basis(R.bt_b, clampd(r, R.r_l_min, R.r_l_max)));
+    }
+    return v;
+}
+__device__ __forceinline__ double david_radial_lds(const Rep& R, const double* lds, double r) {
+    return 0.5 * bt_apply(lds, bt_basis(R.bt_a, clampd(r, R.g_min, R.g_max)));
+}
+// off-diagonal part of the David link action
+template <int NORD>
+__device__ __forceinline__ double david_off_lds(const Rep& R, const double* lds, double r, double rp, double s2) {
+    const double q = 0.5 * (r + rp), z = r - rp;
+    double u = 0.;
+    if (s2 > 0.0 && q < R.g_max) {
+        const BBasis bq = bt_basis(R.bt_a, q);
+        const double z2 = z * z;
+        double sp[4], zp[4];
+        sp[0] = 1.;
+        zp[0] = 1.;
+#pragma unroll
+        for (int e = 1; e <= (NORD ? NORD : 3); ++e) {
+            sp[e] = sp[e - 1] * s2;
+            zp[e] = zp[e - 1] * z2;
+        }
+        const int n_order = NORD ? NORD : R.n_order;
+#pragma unroll
+        for (int k = 1; k <= (NORD ? NORD : 3); ++k) {
+            if (k > n_order) break;
+#pragma unroll
+            for (int j = 0; j <= k; ++j)
+                u += bt_apply(lds + (size_t)(k * (k + 1) / 2 + j) * R.bt_a.ncoef, bq) * zp[j] * sp[k - j];
+        }
+    }
+    return u;
+}
+template <int PT, int NORD>
+__global__ __launch_bounds__(kCompatBlock) void k_grad_compat_lds(const Rep* __restrict__ reps, int out_est, int short_on,
+                                                                  int np) {
+    extern __shared__ double lds[];
+    const Rep R = reps[blockIdx.z];
+    const int b = blockIdx.x, p0 = blockIdx.y * np, N = R.N, M = R.M;
+    if (b >= M || p0 >= N) return;
+    const bool on = short_on && R.pair_type != 0 && N > 1;
+    if (on) stage_tables(R, lds, false);
+    double* sums = lds + R.lds_doubles;  // [group][np][3]
+    const int n = min(np, N - p0), n_grp = kCompatBlock / n;
+    const int grp = threadIdx.x / n, lp = threadIdx.x % n, p = p0 + lp;
+    const bool bare = PT == 1 || (PT == 0 && R.pair_type == 1);
+    const double eps = 1.e-4;
+    double g[3] = {0., 0., 0.};
+    if (on && grp < n_grp) {
+        const int bj = b + 1 == M ? 0 : b + 1, bk = b == 0 ? M - 1 : b - 1;
+        const int q_lo = (int)((long long)N * grp / n_grp), q_hi = (int)((long long)N * (grp + 1) / n_grp);
+        double r0[3], pj[3], pk[3];
+        for (int d = 0; d < 3; ++d) {
+            r0[d] = pos_at(R, d, b, p);
+            pj[d] = pos_at(R, d, bj, p);
+            pk[d] = pos_at(R, d, bk, p);
+        }
+        for (int q = q_lo; q < q_hi; ++q) {
+            if (q == p) continue;
+            // r with each component unshifted and shifted by -+eps, and the image each took
+            double rv[3], rs[3][2], vj[3], vk[3];
+            bool wrap[3];
+            double x2[3];
+            for (int d = 0; d < 3; ++d) {
+                const double qb = pos_at(R, d, b, q), x = qb - r0[d];
+                const double i0 = rint(x * R.iL);
+                rv[d] = x - i0 * R.L;
+                const double xp = qb - (r0[d] + eps), xm = qb - (r0[d] - eps);
+                const double ip = rint(xp * R.iL), im = rint(xm * R.iL);
+                rs[d][0] = xp - ip * R.L;
+                rs[d][1] = xm - im * R.L;
+                x2[d] = rv[d] * rv[d];
+                vj[d] = pos_at(R, d, bj, q) - pj[d];
+                vk[d] = pos_at(R, d, bk, q) - pk[d];
+                // does either side of the difference see another image of r or r'?
+                wrap[d] = ip != im || rint((rs[d][0] - vj[d]) * R.iL) != rint((rs[d][1] - vj[d]) * R.iL) ||
+                          rint((rs[d][0] - vk[d]) * R.iL) != rint((rs[d][1] - vk[d]) * R.iL);
+                vj[d] += rint((rv[d] - vj[d]) * R.iL) * R.L;
+                vk[d] += rint((rv[d] - vk[d]) * R.iL) * R.L;
+            }
+            const double rj = sqrt_pos(vj[0] * vj[0] + vj[1] * vj[1] + vj[2] * vj[2]);
+            const double rk = sqrt_pos(vk[0] * vk[0] + vk[1] * vk[1] + vk[2] * vk[2]);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                double diff = 0.;
+#pragma unroll
+                for (int sg = 0; sg < 2; ++sg) {
+                    const double x = rs[d][sg];
+                    double r2 = x * x;
+                    for (int e = 0; e < 3; ++e)
+                        if (e != d) r2 += x2[e];
+                    const double r = sqrt_pos(r2);
+                    double f = 2. * (bare ? bare_radial_lds(R, lds, r) : david_radial_lds(R, lds, r));
+                    for (int lk = 0; lk < 2; ++lk) {
+                        const double* v = lk ? vk : vj;
+                        double rp = lk ? rk : rj, y = v[d];
+                        if (wrap[d]) {
+                            // r' follows this side's image
+                            y += rint((x - y) * R.iL) * R.L;
+                            double t = y * y;
+                            for (int e = 0; e < 3; ++e)
+                                if (e != d) t += v[e] * v[e];
+                            rp = sqrt_pos(t);
+                            f += bare ? bare_radial_lds(R, lds, rp) : david_radial_lds(R, lds, rp);
+                        }
+                        if (!bare) {
+                            double s2 = (x - y) * (x - y);
+                            for (int e = 0; e < 3; ++e)
+                                if (e != d) {
+                                    const double sv = rv[e] - v[e];
+                                    s2 += sv * sv;
+                                }
+                            f += david_off_lds<NORD>(R, lds, r, rp, s2);
+                        }
+                    }
+                    diff += sg ? -f : f;
+                }
+                g[d] += diff;
+            }
+        }
+        const double c = (bare ? R.tau : 1.) / (2. * eps);
+        for (int d = 0; d < 3; ++d) sums[((size_t)grp * n + lp) * 3 + d] = c * g[d];
+    }
+    __syncthreads();
+    double* o = (out_est ? R.grad_est : R.grad) + 3 * ((size_t)b * N + p0);
+    for (int t = threadIdx.x; t < 3 * n; t += kCompatBlock) {
+        double v = 0.;
+        if (on)
+            for (int i = 0; i < n_grp; ++i) v += sums[(size_t)i * 3 * n + t];
+        o[t] = v;
+    }
+}
+
 // Analytic adjoint, local terms: kinetic links (b-1,b), (b,b+1) and short-range
 // pair links of every other particle.  Writes (overwrites) grad.
 __global__ __launch_bounds__(64) void k_adjoint_local(const Rep* __restrict__ reps, unsigned int terms, int out_est) {
@@ -1939,16 +2103,6 @@ __global__ __launch_bounds__(64) void k_adjoint_local(const Rep* __restrict__ re
     o[0] = g[0];
     o[1] = g[1];
     o[2] = g[2];
-}
-
-// Loads a replica's link-action tables (du_only: the David du_kj_dbeta table
-// instead) into LDS.
-__device__ __forceinline__ void stage_tables(const Rep& R, double* lds, bool du_only) {
-    if (du_only)
-        stage_batched(lds, R.bt_du.c, R.bt_du.c, R.lds_doubles_du, R.lds_doubles_du, 0, (int)blockDim.x);
-    else
-        stage_batched(lds, R.bt_a.c, R.bt_b.c, R.bt_a.ncoef * R.bt_a.ncomp, R.lds_doubles, 0, (int)blockDim.x);
-    __syncthreads();
 }
 
 // Analytic adjoint, local terms with LDS tables: one 1024-thread workgroup per
