@@ -244,6 +244,7 @@ BTabHost make_btab(const double* x, int n, const std::vector<const double*>& ys)
 }
 
 constexpr size_t kPairLdsMaxBytes = 150 * 1024;
+constexpr size_t kStageBytes = 256 * 1024;  // staging area of small reads (larger ones are plain copies)
 
 struct RepHost {
     spimc_system_desc d{};
@@ -395,7 +396,12 @@ struct spimc_ctx {
     hipEvent_t stage_ready = nullptr;
     uint2* d_items_tmp = nullptr;
     size_t items_tmp_cap = 0;
-    unsigned int* d_counts = nullptr;
+    // pinned host memory, also addressed by kernels: the replay-error flag, the
+    // stage's attempt counts (one per replica) and the staging area of small reads
+    char* pin = nullptr;
+    volatile unsigned int* h_error = nullptr;
+    unsigned int* counts = nullptr;
+    unsigned char* stage = nullptr;
     double* d_tmp = nullptr;  // interface partials + result
     size_t tmp_cap = 0;
     bool any_long = false;
@@ -467,7 +473,6 @@ struct spimc_ctx {
     uint64_t t_n[SPIMC_KERNEL_COUNT] = {0};
     double t_bytes[SPIMC_KERNEL_COUNT] = {0};
     unsigned long long* d_work = nullptr;
-    unsigned int* d_error = nullptr;
     unsigned long long work_seen[WORK_COUNT] = {0, 0};
     // a replica's path may be permuted: rounds also launch the label-general pair kernel
     bool perm_on = false;
@@ -527,6 +532,24 @@ int launch(spimc_ctx* c, int kernel, void (*k)(P...), dim3 grid, dim3 block, siz
     if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) return fail(SPIMC_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
     if (ea && eb) c->pending.push_back({kernel, ea, eb});
+    return SPIMC_OK;
+}
+
+// Reads n_a and n_b 8-byte words from two device arrays (one kernel into the
+// staging area; plain copies when they exceed it).  Ordered after the stream's work.
+int read_words(spimc_ctx* c, const void* a, int n_a, void* out_a, const void* b, int n_b, void* out_b) {
+    using u64 = unsigned long long;
+    if (((size_t)n_a + n_b) * sizeof(u64) > kStageBytes) {
+        HIPCHK(hipStreamSynchronize(c->stream));
+        if (n_a) HIPCHK(hipMemcpy(out_a, a, n_a * sizeof(u64), hipMemcpyDeviceToHost));
+        if (n_b) HIPCHK(hipMemcpy(out_b, b, n_b * sizeof(u64), hipMemcpyDeviceToHost));
+        return SPIMC_OK;
+    }
+    k_pack<<<(n_a + n_b + 255) / 256, 256, 0, c->stream>>>((u64*)c->stage, (const u64*)a, n_a, (const u64*)b, n_b);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(c->stream));
+    if (n_a) std::memcpy(out_a, c->stage, n_a * sizeof(u64));
+    if (n_b) std::memcpy(out_b, c->stage + n_a * sizeof(u64), n_b * sizeof(u64));
     return SPIMC_OK;
 }
 
@@ -1351,7 +1374,7 @@ void drop_graphs(spimc_ctx* c) {
 // set (k_stage_begin reads them from d_counts).
 int launch_pers_stage(spimc_ctx* c, int move) {
     const int R = (int)c->reps.size();
-    int rc = launch(c, SPIMC_KERNEL_DECIDE, k_stage_begin, (R + 63) / 64, 64, 0, c->stream, c->d_reps, R, c->d_counts);
+    int rc = launch(c, SPIMC_KERNEL_DECIDE, k_stage_begin, (R + 63) / 64, 64, 0, c->stream, c->d_reps, R, (const unsigned int*)c->counts);
     if (rc) return rc;
     return launch(c, SPIMC_KERNEL_PROPOSE, c->pers_fn, R, c->pers_block, pers_shmem(c), c->stream, c->d_reps, R, move,
                   c->lds_doubles_max > 0 ? 1 : 0, (int)pers_tables(c));
@@ -1681,7 +1704,7 @@ int run_stage(spimc_ctx* c, int move, const uint32_t* counts, uint32_t n_uniform
         // the whole stage in one launch (from a captured graph with use_graph)
         const bool pgraph = use_graph && !c->timing;
         if (pgraph && (rc = capture_pers_graph(c, move))) return rc;
-        HIPCHK(hipMemcpyAsync(c->d_counts, cnt.data(), R * sizeof(unsigned int), hipMemcpyHostToDevice, c->stream));
+        std::copy(cnt.begin(), cnt.end(), c->counts);
         if (pgraph)
             HIPCHK(hipGraphLaunch(c->pers_graph[move], c->stream));
         else if ((rc = launch_pers_stage(c, move)))
@@ -1692,8 +1715,8 @@ int run_stage(spimc_ctx* c, int move, const uint32_t* counts, uint32_t n_uniform
     if (graph)
         for (auto& G : c->groups)
             if ((rc = capture_round_graph(c, G, move))) return rc;
-    HIPCHK(hipMemcpyAsync(c->d_counts, cnt.data(), R * sizeof(unsigned int), hipMemcpyHostToDevice, c->stream));
-    rc = launch(c, SPIMC_KERNEL_DECIDE, k_stage_begin, (R + 63) / 64, 64, 0, c->stream, c->d_reps, R, c->d_counts);
+    std::copy(cnt.begin(), cnt.end(), c->counts);  // (the last stage's kernels have finished)
+    rc = launch(c, SPIMC_KERNEL_DECIDE, k_stage_begin, (R + 63) / 64, 64, 0, c->stream, c->d_reps, R, (const unsigned int*)c->counts);
     if (rc) return rc;
     const int n_groups = (int)c->groups.size();
     std::vector<uint32_t> gmx(n_groups, 0);
@@ -1744,10 +1767,8 @@ int finish_stage(spimc_ctx* c, const std::vector<unsigned int>& cnt, uint32_t mx
     if ((rc = sync_and_resolve(c))) return rc;
     c->adjoint_fresh = false;
     // replay errors: one context-wide flag, then the replica that raised it
-    unsigned int any = 0;
-    HIPCHK(hipMemcpy(&any, c->d_error, sizeof any, hipMemcpyDeviceToHost));
-    if (any) {
-        HIPCHK(hipMemset(c->d_error, 0, sizeof any));
+    if (*c->h_error) {
+        *c->h_error = 0;
         for (int r = 0; r < R; ++r) {
             Counters k;
             HIPCHK(hipMemcpy(&k, c->reps[r].dev.cnt, sizeof(Counters), hipMemcpyDeviceToHost));
@@ -1761,9 +1782,15 @@ int finish_stage(spimc_ctx* c, const std::vector<unsigned int>& cnt, uint32_t mx
         }
     }
     for (int r = 0; r < R; ++r) c->reps[r].stage_attempts = cnt[r];
-    if (accepted)
+    if (accepted && (size_t)R * mx <= kStageBytes) {
+        k_pack_accepted<<<R, 256, 0, c->stream>>>(c->d_reps, c->counts, mx, c->stage);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (int r = 0; r < R; ++r) std::memcpy(accepted + (size_t)r * mx, c->stage + (size_t)r * mx, cnt[r]);
+    } else if (accepted) {
         for (int r = 0; r < R; ++r)
             HIPCHK(hipMemcpy(accepted + (size_t)r * mx, c->reps[r].accepted, cnt[r], hipMemcpyDeviceToHost));
+    }
     return SPIMC_OK;
 }
 
@@ -2069,8 +2096,15 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
         c->max_nk = std::max(c->max_nk, R.nk);
     }
     if (hipMalloc((void**)&c->d_reps, n_replicas * sizeof(Rep)) != hipSuccess) return bail(fail(SPIMC_ERR_NOMEM, "rep table"));
-    if (hipMalloc((void**)&c->d_counts, n_replicas * sizeof(unsigned int)) != hipSuccess)
-        return bail(fail(SPIMC_ERR_NOMEM, "counts"));
+    {
+        const size_t b_cnt = ((size_t)n_replicas * sizeof(unsigned int) + 255) & ~(size_t)255;
+        if (hipHostMalloc((void**)&c->pin, 256 + b_cnt + kStageBytes, hipHostMallocDefault) != hipSuccess)
+            return bail(fail(SPIMC_ERR_NOMEM, "pinned host memory"));
+        c->h_error = reinterpret_cast<volatile unsigned int*>(c->pin);
+        *c->h_error = 0;
+        c->counts = reinterpret_cast<unsigned int*>(c->pin + 256);
+        c->stage = reinterpret_cast<unsigned char*>(c->pin + 256 + b_cnt);
+    }
     if (hipMalloc((void**)&c->d_work, WORK_COUNT * sizeof(unsigned long long)) != hipSuccess)
         return bail(fail(SPIMC_ERR_NOMEM, "work counters"));
     if (hipMemset(c->d_work, 0, WORK_COUNT * sizeof(unsigned long long)) != hipSuccess)
@@ -2084,10 +2118,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
     }
     if (hipMalloc((void**)&c->d_gr_rmax, n_replicas * sizeof(double)) != hipSuccess)
         return bail(fail(SPIMC_ERR_NOMEM, "g(r) table"));
-    if (hipMalloc((void**)&c->d_error, sizeof(unsigned int)) != hipSuccess ||
-        hipMemset(c->d_error, 0, sizeof(unsigned int)) != hipSuccess)
-        return bail(fail(SPIMC_ERR_NOMEM, "error flag"));
-    for (auto& h : c->reps) h.dev.ctx_error = c->d_error;
+    for (auto& h : c->reps) h.dev.ctx_error = const_cast<unsigned int*>(c->h_error);
     {
         bool all = true;
         for (auto& h : c->reps) {
@@ -2258,9 +2289,10 @@ int spimc_ctx_destroy(spimc_ctx* c) {
         if (h.perm_scratch) (void)hipFree(h.perm_scratch);
         if (h.perm_t) (void)hipFree(h.perm_t);
     }
-    for (void* p : {(void*)c->d_reps, (void*)c->d_counts, (void*)c->d_work, (void*)c->d_gr_rmax, (void*)c->d_error,
+    for (void* p : {(void*)c->d_reps, (void*)c->d_work, (void*)c->d_gr_rmax,
                     (void*)c->d_tmp, (void*)c->d_items_tmp, (void*)c->d_adj_part, (void*)c->d_col_w})
         if (p) (void)hipFree(p);
+    if (c->pin) (void)hipHostFree(c->pin);
     for (auto& t : c->pending) {
         (void)hipEventDestroy(t.a);
         (void)hipEventDestroy(t.b);
@@ -2304,12 +2336,13 @@ int spimc_rho_k_download(spimc_ctx* c, uint32_t r, double* rho) {
     if (!rho) return fail(SPIMC_ERR_ARG, "null output");
     const Rep& R = c->reps[r].dev;
     if (!R.use_long_range) return fail(SPIMC_ERR_STATE, "replica has no long-range action");
+    // the committed rows lie in two buffers: gathered on the device, then one copy
+    // (a copy a row took 1.2 ms for 128 rows)
+    if ((rc = ensure_tmp(c, (size_t)2 * R.M * R.nk, 0))) return rc;
+    k_gather_rho<<<R.M, 256, 0, c->stream>>>(c->d_reps, (int)r, reinterpret_cast<double2*>(c->d_tmp));
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
-    std::vector<unsigned char> sel(R.M);
-    HIPCHK(hipMemcpy(sel.data(), R.sel, R.M, hipMemcpyDeviceToHost));
-    for (int b = 0; b < R.M; ++b)
-        HIPCHK(hipMemcpy(rho + (size_t)2 * b * R.nk, R.rho + ((size_t)sel[b] * R.M + b) * R.nk,
-                         (size_t)R.nk * sizeof(double2), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(rho, c->d_tmp, (size_t)R.M * R.nk * sizeof(double2), hipMemcpyDeviceToHost));
     return SPIMC_OK;
 }
 
@@ -2775,23 +2808,19 @@ int spimc_perm_counters(spimc_ctx* c, uint32_t r, uint64_t* out) {
     if (!out) return fail(SPIMC_ERR_ARG, "null argument");
     const Rep& R = c->reps[r].dev;
     const size_t n = 2 + 2 * (size_t)R.N;
-    HIPCHK(hipDeviceSynchronize());
     if (!R.perm_cnt) {
         for (size_t i = 0; i < n; ++i) out[i] = 0;
         return SPIMC_OK;
     }
-    std::vector<unsigned long long> v(n);
-    HIPCHK(hipMemcpy(v.data(), R.perm_cnt, n * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < n; ++i) out[i] = v[i];
-    return SPIMC_OK;
+    return read_words(c, R.perm_cnt, (int)n, out, nullptr, 0, nullptr);
 }
 
 int spimc_move_counters(spimc_ctx* c, uint32_t r, uint64_t* out) {
     int rc = check_rep(c, r);
     if (rc) return rc;
     Counters k;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(&k, c->reps[r].dev.cnt, sizeof k, hipMemcpyDeviceToHost));
+    static_assert(sizeof(Counters) % 8 == 0, "read in 8-byte words");
+    if ((rc = read_words(c, c->reps[r].dev.cnt, sizeof k / 8, &k, nullptr, 0, nullptr))) return rc;
     out[0] = k.bis_att;
     out[1] = k.bis_acc;
     out[2] = k.dis_att;
@@ -2857,22 +2886,9 @@ int spimc_obs_configure(spimc_ctx* c, int energy_estimator, uint32_t virial_wind
 
 int spimc_obs_reset(spimc_ctx* c, uint32_t which) {
     if (!c) return fail(SPIMC_ERR_ARG, "null context");
+    k_obs_reset<<<(unsigned)c->reps.size(), 256, 0, c->stream>>>(c->d_reps, which, c->gr_n_r);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
-    for (auto& h : c->reps) {
-        const Rep& R = h.dev;
-        if (which & SPIMC_OBS_ENERGY) {
-            HIPCHK(hipMemset(R.e_acc, 0, 2 * sizeof(double)));
-            HIPCHK(hipMemset(R.n_measure, 0, sizeof(unsigned long long)));
-        }
-        if (which & SPIMC_OBS_SK) {
-            HIPCHK(hipMemset(R.sk_acc, 0, std::max(R.nk, 1) * sizeof(double)));
-            HIPCHK(hipMemset(R.n_measure + 1, 0, sizeof(unsigned long long)));
-        }
-        if (which & SPIMC_OBS_GR) {
-            HIPCHK(hipMemset(R.gr_cnt, 0, c->gr_n_r * sizeof(unsigned long long)));
-            HIPCHK(hipMemset(R.n_measure + 2, 0, sizeof(unsigned long long)));
-        }
-    }
     return SPIMC_OK;
 }
 
@@ -2889,24 +2905,22 @@ int spimc_obs_read(spimc_ctx* c, uint32_t r, uint32_t which, double* out, uint64
     if (rc) return rc;
     if (!out || !n_measure) return fail(SPIMC_ERR_ARG, "null output");
     const Rep& R = c->reps[r].dev;
-    HIPCHK(hipStreamSynchronize(c->stream));
     unsigned long long nm[3];
-    HIPCHK(hipMemcpy(nm, R.n_measure, sizeof nm, hipMemcpyDeviceToHost));
     if (which == SPIMC_OBS_ENERGY) {
-        HIPCHK(hipMemcpy(out, R.e_acc, 2 * sizeof(double), hipMemcpyDeviceToHost));
-        *n_measure = nm[0];
+        rc = read_words(c, R.n_measure, 3, nm, R.e_acc, 2, out);
+        if (!rc) *n_measure = nm[0];
     } else if (which == SPIMC_OBS_SK) {
-        if (R.nk) HIPCHK(hipMemcpy(out, R.sk_acc, R.nk * sizeof(double), hipMemcpyDeviceToHost));
-        *n_measure = nm[1];
+        rc = read_words(c, R.n_measure, 3, nm, R.sk_acc, R.nk, out);
+        if (!rc) *n_measure = nm[1];
     } else if (which == SPIMC_OBS_GR) {
         std::vector<unsigned long long> v(c->gr_n_r);
-        HIPCHK(hipMemcpy(v.data(), R.gr_cnt, v.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < v.size(); ++i) out[i] = (double)v[i];
-        *n_measure = nm[2];
+        rc = read_words(c, R.n_measure, 3, nm, R.gr_cnt, (int)v.size(), v.data());
+        for (size_t i = 0; i < v.size() && !rc; ++i) out[i] = (double)v[i];
+        if (!rc) *n_measure = nm[2];
     } else {
         return fail(SPIMC_ERR_ARG, "read one observable at a time");
     }
-    return SPIMC_OK;
+    return rc;
 }
 
 // ---- batched sweep ------------------------------------------------------------

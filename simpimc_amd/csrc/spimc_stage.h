@@ -658,7 +658,7 @@ __device__ __forceinline__ void stage_body(const Rep& R, int move, bool tables, 
         if (TAPE) *R.tape_cursor = st.cursor;
         if (st.error) {
             c->error = 1;
-            atomicOr(R.ctx_error, 1u);
+            ctx_error_set(R);
         }
         R.prop->status = 0;
     }
