@@ -153,7 +153,7 @@ struct Rep {
     BTab bt_a, bt_b;
     BTab bt_du;            // David du_kj_dbeta components 0..n_val (estimators)
     int lds_doubles;       // doubles of LDS the pair kernel stages (0: tables stay in global memory)
-    int lds_doubles_du;    // doubles of LDS the beta-derivative estimator stages (0: global)
+    int lds_doubles_du;    // doubles of LDS the whole-path pair sums stage of it (0: global)
     int pad4;
     // kinetic and sampling image splines (n_images > 0 only)
     Spl kin[kMaxKinSplines];
@@ -577,41 +577,6 @@ __device__ __forceinline__ double pair_u_lds(const Rep& R, const double* lds, do
         }
     }
     return u;
-}
-
-// dU/dbeta of a link (CalcdUdBeta) from LDS tables: Bare uses the pair tables
-// [v_r][v_long_r]; David uses du_kj_dbeta components 0..n_val at `ldu`.
-__device__ __forceinline__ double pair_du_dbeta_lds(const Rep& R, const double* lds, const double* ldu, double r0,
-                                                    double r1, double s) {
-    if (R.pair_type == 1) return pair_u_lds(R, lds, r0, r1, s) / R.tau;
-    const BTab& T = R.bt_du;
-    const double q = 0.5 * (r0 + r1), z = r0 - r1;
-    clamp2(R.g_min, R.g_max, r0, r1);
-    const BBasis b0 = bt_basis(T, r0), b1 = bt_basis(T, r1);
-    const double v = 0.5 * (bt_apply(ldu, b0) + bt_apply(ldu, b1));
-    double du = 0.5 * (bt_apply(ldu + T.ncoef, b0) + bt_apply(ldu + T.ncoef, b1));
-    du += v;
-    if (s > 0.0 && q < R.g_max) {
-        const BBasis bq = bt_basis(T, q);
-        double z_2 = z * z, s_2 = s * s, i_s_2 = 1. / s_2, s_2_k = s_2;
-        for (int k = 1; k <= R.n_order; ++k) {
-            double z_2_j = 1., cur_s = s_2_k;
-            for (int j = 0; j <= k; ++j) {
-                du += bt_apply(ldu + (size_t)(k * (k + 1) / 2 + j + 1) * T.ncoef, bq) * z_2_j * cur_s;
-                z_2_j *= z_2;
-                cur_s *= i_s_2;
-            }
-            s_2_k *= s_2;
-        }
-    }
-    return du;
-}
-
-// CalcV from LDS tables (Bare: [v_r][v_long_r]; David: component 0 of du).
-__device__ __forceinline__ double pair_v_lds(const Rep& R, const double* lds, const double* ldu, double r0, double r1) {
-    if (R.pair_type == 1) return pair_u_lds(R, lds, r0, r1, 0.) / R.tau;
-    clamp2(R.g_min, R.g_max, r0, r1);
-    return 0.5 * (bt_apply(ldu, bt_basis(R.bt_du, r0)) + bt_apply(ldu, bt_basis(R.bt_du, r1)));
 }
 
 // dU/dr, dU/dr', dU/ds of the level-0 link action from LDS tables.

@@ -455,6 +455,9 @@ struct spimc_ctx {
     // LDS doubles of the adjoint kernel (pair tables) and of the whole-path
     // estimator kernel (Bare: pair tables, David: du table); 0 = global tables
     int lds_adj_max = 0, lds_whole_max = 0;
+    void (*whole_fn)(const Rep*, int, int, int, double*) = nullptr;
+    double* d_whole = nullptr;  // its partial sums
+    double* d_vir = nullptr;    // partial sums of the kinetic virial, per 64 particles
     // dynamic LDS bytes of the run-ordered long-range adjoint (0: the per-particle table kernel)
     size_t adj_runs_lds = 0;
     // the unrolled long-range adjoint (0: not for these k-vectors): registers for
@@ -971,8 +974,10 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
                           (s.pair_type == SPIMC_PAIR_BARE && (s.bare_is_coulomb || h.bt_a.knots) && (!lr || h.bt_b.knots));
         R.lds_doubles = (have && nd * sizeof(double) <= kPairLdsMaxBytes) ? (int)std::max<size_t>(nd, 1) : 0;
         R.lds_doubles_du = 0;
-        if (s.pair_type == SPIMC_PAIR_DAVID && h.bt_du.knots && h.bt_du.c.size() * sizeof(double) <= kPairLdsMaxBytes)
-            R.lds_doubles_du = (int)h.bt_du.c.size();
+        // (components 0 and 1 are staged as one)
+        const size_t nd_du = h.bt_du.c.size() - (h.bt_du.knots ? h.bt_du.knots + 2 : 0);
+        if (s.pair_type == SPIMC_PAIR_DAVID && h.bt_du.knots && nd_du * sizeof(double) <= kPairLdsMaxBytes)
+            R.lds_doubles_du = (int)nd_du;
     }
     R.tape = nullptr;
     R.tape_len = 0;
@@ -1810,25 +1815,45 @@ int est_kin_dbeta(spimc_ctx* c, Rep* base, int nrep) {
     dim3 g(c->max_M, nrep);
     return launch(c, SPIMC_KERNEL_ESTIMATORS, k_kin_dbeta, g, 256, 0, c->stream, base, kSlotKin);
 }
+// Workgroups of the whole-path pair sums per replica: W that give every CU one,
+// as S slice ranges of about eight slices (a range's first slice is evaluated for
+// it alone) and Q parts of the pairs, or shorter ranges where the pairs are too
+// few for Q (a workgroup's threads take a pair each).
+void whole_split(const spimc_ctx* c, int nrep, int& S, int& Q) {
+    const int W = std::max(1, kNumCUs / nrep);
+    const long long pairs = (long long)c->max_N * (c->max_N / 2);
+    const int q_max = (int)std::max<long long>(1, std::min<long long>(W, pairs / kWholeBlock));
+    S = std::max(std::min(W, (c->max_M + 7) / 8), std::min(c->max_M, W / q_max));
+    Q = std::max(1, std::min(q_max, W / S));
+}
 int est_pair_whole(spimc_ctx* c, Rep* base, int nrep, int which) {
     int rc;
     if (c->lds_whole_max > 0) {
         const size_t shmem = (size_t)c->lds_whole_max * sizeof(double);
-        // workgroups per replica, each over every spb-th slice: enough to fill the
-        // GPU when the replicas are few
-        const int spb = std::max(1, std::min(c->max_M, (2 * kNumCUs + nrep - 1) / nrep));
-        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_pair_whole_lds, dim3(nrep, spb), kAdjLdsBlock, shmem, c->stream, base,
-                    which, kSlotPair);
+        int S, Q;
+        whole_split(c, nrep, S, Q);
+        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, c->whole_fn, dim3(nrep, S * Q), kWholeBlock, shmem, c->stream, base, which, S,
+                    Q, c->d_whole);
     } else {
         dim3 g(c->max_M, nrep);
         rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_pair_whole, g, 256, 0, c->stream, base, which, kSlotPair);
     }
     if (rc || !c->any_long) return rc;
-    dim3 g2((c->max_nk + 255) / 256, nrep);
-    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_long_whole, g2, 256, 0, c->stream, base, which);
+    dim3 g2((c->max_nk + 63) / 64, nrep);
+    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_long_whole, g2, kSumBlock, 0, c->stream, base, which);
+}
+int est_kin_virial(spimc_ctx* c, Rep* base, int nrep, int W) {
+    const int tiles = (c->max_N + 63) / 64;
+    int rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_kin_virial, dim3(tiles, nrep), kVirBlock, 0, c->stream, base, W, c->d_vir);
+    if (rc) return rc;
+    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_kin_virial_sum, nrep, 64, 0, c->stream, base, W, tiles, kSlotVirial,
+                  (const double*)c->d_vir);
 }
 int est_finalize(spimc_ctx* c, Rep* base, int nrep, int what, int acc) {
-    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_finalize, (nrep + 63) / 64, 64, 0, c->stream, base, nrep, what, acc);
+    int S = 0, Q = 0;
+    if (c->lds_whole_max > 0) whole_split(c, nrep, S, Q);
+    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_finalize, nrep, 256, 0, c->stream, base, what, acc,
+                  c->lds_whole_max > 0 ? (const double*)c->d_whole : (const double*)nullptr, S * Q);
 }
 // The long-range adjoint by columns: the slices' weights, then the particles, as
 // many replicas at a time as keep the weights within kColBytes.
@@ -1950,7 +1975,7 @@ int energy_accumulate(spimc_ctx* c, Rep* base, int nrep) {
         return SPIMC_OK;
     }
     const int W = (int)c->virial_window;
-    rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_kin_virial, nrep, 256, 0, c->stream, base, W, kSlotVirial);
+    rc = est_kin_virial(c, base, nrep, W);
     if (rc) return rc;
     int from_sweep = 0;
     if (c->energy_estimator == SPIMC_ENERGY_VIRIAL_COMPAT) {
@@ -1976,16 +2001,17 @@ int obs_accumulate_all(spimc_ctx* c, uint32_t which) {
     if (which & SPIMC_OBS_ENERGY)
         if ((rc = energy_accumulate(c, c->d_reps, R))) return rc;
     if ((which & SPIMC_OBS_SK) && c->any_long) {
-        dim3 g((c->max_nk + 255) / 256, R);
+        dim3 g((c->max_nk + 63) / 64, R);
         const double kc = c->sk_k_cut;
-        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_sk, g, 256, 0, c->stream, c->d_reps, kc);
+        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_sk, g, kSumBlock, 0, c->stream, c->d_reps, kc);
         if (rc) return rc;
     }
     if (which & SPIMC_OBS_GR) {
         dim3 g(c->max_M, R);
         const double rmin = c->gr_r_min;
         const int nr = (int)c->gr_n_r;
-        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_gr, g, 256, 0, c->stream, c->d_reps, rmin, 0., nr, c->d_gr_rmax);
+        const int bs = (long long)c->max_M * R < 4 * kNumCUs ? 1024 : 256;
+        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_gr, g, bs, 0, c->stream, c->d_reps, rmin, 0., nr, c->d_gr_rmax);
         if (rc) return rc;
     }
     return SPIMC_OK;
@@ -2116,6 +2142,8 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             return bail(fail(SPIMC_ERR_HIP, "wall clock rate"));
         c->clock_hz = 1e3 * khz;
     }
+    if (hipMalloc((void**)&c->d_vir, (size_t)n_replicas * ((c->max_N + 63) / 64) * sizeof(double)) != hipSuccess)
+        return bail(fail(SPIMC_ERR_NOMEM, "virial partial sums"));
     if (hipMalloc((void**)&c->d_gr_rmax, n_replicas * sizeof(double)) != hipSuccess)
         return bail(fail(SPIMC_ERR_NOMEM, "g(r) table"));
     for (auto& h : c->reps) h.dev.ctx_error = const_cast<unsigned int*>(c->h_error);
@@ -2230,8 +2258,12 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             hipFuncSetAttribute((const void*)k_adjoint_long_runs, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)c->adj_runs_lds) != hipSuccess)
             c->adj_runs_lds = 0;
+        c->whole_fn = vi == 0 ? k_pair_whole_lds<1, 0> : vi == 1 ? k_pair_whole_lds<2, 2>
+                                                   : vi == 2 ? k_pair_whole_lds<2, 0> : k_pair_whole_lds<0, 0>;
+        if (hipMalloc((void**)&c->d_whole, ((size_t)n_replicas + kNumCUs) * sizeof(double)) != hipSuccess)
+            return bail(fail(SPIMC_ERR_NOMEM, "whole-path partial sums"));
         if (c->lds_whole_max > 0 &&
-            hipFuncSetAttribute((const void*)k_pair_whole_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+            hipFuncSetAttribute((const void*)c->whole_fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 c->lds_whole_max * (int)sizeof(double)) != hipSuccess)
             c->lds_whole_max = 0;
     }
@@ -2290,7 +2322,7 @@ int spimc_ctx_destroy(spimc_ctx* c) {
         if (h.perm_t) (void)hipFree(h.perm_t);
     }
     for (void* p : {(void*)c->d_reps, (void*)c->d_work, (void*)c->d_gr_rmax,
-                    (void*)c->d_tmp, (void*)c->d_items_tmp, (void*)c->d_adj_part, (void*)c->d_col_w})
+                    (void*)c->d_tmp, (void*)c->d_items_tmp, (void*)c->d_adj_part, (void*)c->d_col_w, (void*)c->d_whole, (void*)c->d_vir})
         if (p) (void)hipFree(p);
     if (c->pin) (void)hipHostFree(c->pin);
     for (auto& t : c->pending) {
@@ -2608,7 +2640,7 @@ int spimc_kinetic_virial_energy(spimc_ctx* c, uint32_t r, uint32_t window, doubl
     if (!out) return fail(SPIMC_ERR_ARG, "null output");
     const Rep& R = c->reps[r].dev;
     const int W = window ? (int)window : 0;
-    rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_kin_virial, 1, 256, 0, c->stream, c->d_reps + r, W, kSlotVirial);
+    rc = est_kin_virial(c, c->d_reps + r, 1, W);
     if (rc || (rc = sync_and_resolve(c))) return rc;
     HIPCHK(hipMemcpy(out, R.scratch + kSlotVirial * R.M, sizeof(double), hipMemcpyDeviceToHost));
     return SPIMC_OK;

@@ -29,7 +29,7 @@ enum { WORK_PAIR_LINKS = 0, WORK_RHO_SLICEK = 1, WORK_COUNT = 2 };
 // long-range k-chunk partials, then two results.
 constexpr int kSlotKin = 0, kSlotPair = 1, kSlotCentroid = 2, kSlotVirial = 3;
 __host__ __device__ inline size_t scratch_long(int M) { return (size_t)4 * M; }
-__host__ __device__ inline size_t scratch_res(int M, int nk) { return (size_t)4 * M + (nk + 255) / 256 + 1; }
+__host__ __device__ inline size_t scratch_res(int M, int nk) { return (size_t)4 * M + (nk + kWave - 1) / kWave + 1; }
 __host__ __device__ inline size_t scratch_size(int M, int nk) { return scratch_res(M, nk) + 4; }
 
 // Blocks are dispatched round-robin over the 8 XCDs; this remap hands each XCD
@@ -1785,68 +1785,115 @@ __global__ __launch_bounds__(256) void k_pair_whole(const Rep* __restrict__ reps
     if (threadIdx.x == 0) R.scratch[slot * R.M + b] = t;
 }
 
-// sum_k coef(k) sum_b |rho(b,k)|^2 per k chunk, plus (chunk 0) the k=0 and r=0
-// constants: which 0 CalcdUdBetaLong (coef_b, const_du), 1 CalcVLong (coef_v,
-// const_v)
-__global__ __launch_bounds__(256) void k_long_whole(const Rep* __restrict__ reps, int which) {
-    const Rep& R = reps[blockIdx.y];
-    const int k = (int)(blockIdx.x * 256 + threadIdx.x);
-    if ((int)blockIdx.x * 256 >= R.nk) return;
+// sum_b |rho(b,k)|^2 for the 64 k-vectors of a 1024-thread workgroup (k the lane's;
+// valid on the first wavefront): its 16 wavefronts share the slices, four loads in
+// flight each, and are added in order.  (A thread per k-vector that walked the
+// slices, each load behind its buffer selector, left 8 workgroups for 1979
+// k-vectors: 73 us for M = 128, 5 us so.)
+constexpr int kSumBlock = 1024;
+__device__ __forceinline__ double sum_rho2(const Rep& R, int k, double* sh) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, M = R.M;
+    constexpr int W = kSumBlock / kWave;
     double t = 0.;
-    if (k < R.nk && R.use_long_range) {
-        for (int b = 0; b < R.M; ++b) {
-            const double2 v = R.rho[((size_t)R.sel[b] * R.M + b) * R.nk + k];
-            t += v.x * v.x + v.y * v.y;
+    if (k < R.nk)
+        for (int b = w; b < M; b += 4 * W) {
+            double2 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int s = b + i * W;
+                v[i] = s < M ? ld2<false>(R.rho + ((size_t)R.sel[s] * M + s) * R.nk + k) : make_double2(0., 0.);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t += v[i].x * v[i].x + v[i].y * v[i].y;
         }
-        t *= which ? R.coef_v[k] : R.coef_b[k];
-    }
-    __shared__ double sh[4];
-    t = block_sum<256>(t, sh);
-    if (threadIdx.x == 0) R.scratch[scratch_long(R.M) + blockIdx.x] = t + (blockIdx.x == 0 ? (which ? R.const_v : R.const_du) : 0.);
+    sh[threadIdx.x] = t;
+    __syncthreads();
+    t = 0.;
+    if (w == 0)
+        for (int i = 0; i < W; ++i) t += sh[i * kWave + lane];
+    return t;
 }
 
-// Kinetic::VirialEnergy (kinetic_class.h:48-102), thread per particle
-__global__ __launch_bounds__(256) void k_kin_virial(const Rep* __restrict__ reps, int W_in, int slot) {
-    const Rep& R = reps[blockIdx.x];
-    const int M = R.M;
-    const int W = W_in > 0 ? W_in : M;
-    const double wt = W * R.tau;
-    double tot = 0.;
-    // the walks follow the path: past slice M - 1 a bead is followed by slice 0
-    // of the particle perm[label]
-    for (int p = threadIdx.x; p < R.N; p += 256) {
-        int b_0 = 0, b_1 = 1 % M, b_2 = 2 % M;
-        int l_0 = p, l_1 = next_label(R, 0, p), l_2 = next_label(R, b_1, l_1);
-        double d1[3], dL[3], t[3];
-        for (int d = 0; d < 3; ++d) d1[d] = minimg(pos_at(R, d, b_1, l_1) - pos_at(R, d, b_0, l_0), R.L, R.iL);
-        for (int d = 0; d < 3; ++d) dL[d] = d1[d];
-        for (int sk = 1; sk < W; ++sk) {
-            for (int d = 0; d < 3; ++d) t[d] = minimg(pos_at(R, d, b_2, l_2) - pos_at(R, d, b_1, l_1), R.L, R.iL);
-            for (int d = 0; d < 3; ++d) dL[d] += t[d];
-            b_1 = b_2;
-            l_1 = l_2;
-            l_2 = next_label(R, b_2, l_2);
-            b_2 = (b_2 + 1) % M;
+// sum_k coef(k) sum_b |rho(b,k)|^2 per 64 k-vectors, plus (the first) the k=0 and
+// r=0 constants: which 0 CalcdUdBetaLong (coef_b, const_du), 1 CalcVLong (coef_v,
+// const_v)
+__global__ __launch_bounds__(kSumBlock) void k_long_whole(const Rep* __restrict__ reps, int which) {
+    const Rep& R = reps[blockIdx.y];
+    __shared__ double sh[kSumBlock];
+    const int k = (int)(blockIdx.x * kWave + (threadIdx.x & (kWave - 1)));
+    if ((int)blockIdx.x * kWave >= R.nk || !R.use_long_range) return;
+    double t = sum_rho2(R, k, sh);
+    if (threadIdx.x >= kWave) return;
+    t = k < R.nk ? t * (which ? R.coef_v[k] : R.coef_b[k]) : 0.;
+    t = wave_sum(t);
+    if (threadIdx.x == 0)
+        R.scratch[scratch_long(R.M) + blockIdx.x] = t + (blockIdx.x == 0 ? (which ? R.const_v : R.const_du) : 0.);
+}
+
+// Kinetic::VirialEnergy (kinetic_class.h:48-102): -1 / (4 lambda tau W tau) times
+// the sum over the beads of D . d, d the link leaving the bead and D the W links
+// from it, for 64 particles per workgroup; the walks follow the path: past slice
+// M - 1 a bead is followed by slice 0 of the particle perm[label].  A window of the
+// whole closed path has the same D (its winding) at every bead, and a particle's
+// sum is |D|^2: its links are shared by the workgroup's 16 wavefronts.  Otherwise
+// each wavefront takes a share of the beads, adds the first one's W links and then
+// moves the window.  (A thread per particle took two dependent walks of M slices
+// on one workgroup: 493 us for N = 1024, M = 128, 10 us so.)
+constexpr int kVirBlock = 1024;
+__global__ __launch_bounds__(kVirBlock) void k_kin_virial(const Rep* __restrict__ reps, int W_in, double* __restrict__ part) {
+    const Rep& R = reps[blockIdx.y];
+    const int M = R.M, N = R.N, W = W_in > 0 ? W_in : M;
+    constexpr int G = kVirBlock / kWave;
+    __shared__ double sh[kVirBlock * 3];
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, p = blockIdx.x * kWave + lane;
+    if ((int)blockIdx.x * kWave >= N) return;
+    const bool valid = p < N;
+    // link leaving position c of the walk from (p, 0), 0 <= c < 2 M
+    const int pw = valid ? label_after_wrap(R, p) : 0;
+    auto link = [&](int c, double* t) {
+        const int b = c < M ? c : c - M, l = c < M ? p : pw;
+        const int bn = b + 1 == M ? 0 : b + 1, ln = b + 1 == M ? label_after_wrap(R, l) : l;
+        for (int d = 0; d < 3; ++d) t[d] = minimg(pos_at(R, d, bn, ln) - pos_at(R, d, b, l), R.L, R.iL);
+    };
+    const int lo = (int)((long long)M * w / G), hi = (int)((long long)M * (w + 1) / G);
+    const bool ring = W == M && R.perm == nullptr;
+    double D[3] = {0., 0., 0.}, t[3], tot = 0.;
+    if (valid && ring) {
+        for (int c = lo; c < hi; ++c) {
+            link(c, t);
+            for (int d = 0; d < 3; ++d) D[d] += t[d];
         }
-        tot -= (dL[0] * d1[0] + dL[1] * d1[1] + dL[2] * d1[2]) * R.kin_i4lt / wt;
-        for (int bi = 1; bi < M; ++bi) {
-            for (int d = 0; d < 3; ++d) dL[d] -= d1[d];
-            for (int d = 0; d < 3; ++d) t[d] = minimg(pos_at(R, d, b_2, l_2) - pos_at(R, d, b_1, l_1), R.L, R.iL);
-            for (int d = 0; d < 3; ++d) dL[d] += t[d];
-            l_0 = next_label(R, b_0, l_0);
-            b_0 = (b_0 + 1) % M;
-            const int bn = (b_0 + 1) % M, ln = next_label(R, b_0, l_0);
-            for (int d = 0; d < 3; ++d) d1[d] = minimg(pos_at(R, d, bn, ln) - pos_at(R, d, b_0, l_0), R.L, R.iL);
-            b_1 = b_2;
-            l_1 = l_2;
-            l_2 = next_label(R, b_2, l_2);
-            b_2 = (b_2 + 1) % M;
-            tot -= (dL[0] * d1[0] + dL[1] * d1[1] + dL[2] * d1[2]) * R.kin_i4lt / wt;
+    } else if (valid && lo < hi) {
+        for (int c = lo; c < lo + W; ++c) {
+            link(c, t);
+            for (int d = 0; d < 3; ++d) D[d] += t[d];
+        }
+        for (int c = lo; c < hi; ++c) {
+            double a[3];
+            link(c, a);
+            tot += D[0] * a[0] + D[1] * a[1] + D[2] * a[2];
+            if (c + 1 == hi) break;
+            link(c + W, t);
+            for (int d = 0; d < 3; ++d) D[d] += t[d] - a[d];
         }
     }
-    __shared__ double sh[4];
-    tot = block_sum<256>(tot, sh);
-    if (threadIdx.x == 0) R.scratch[slot * M] = R.kin_dbeta_const / W + tot;
+    for (int d = 0; d < 3; ++d) sh[threadIdx.x * 3 + d] = ring ? D[d] : d == 0 ? tot : 0.;
+    __syncthreads();
+    if (w) return;
+    double v[3] = {0., 0., 0.};
+    for (int i = 0; i < G; ++i)
+        for (int d = 0; d < 3; ++d) v[d] += sh[(i * kWave + lane) * 3 + d];
+    tot = wave_sum(ring ? v[0] * v[0] + v[1] * v[1] + v[2] * v[2] : v[0]);
+    if (lane == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = -tot * R.kin_i4lt / (W * R.tau);
+}
+// its workgroups' sums and the constant into the replica's scratch
+__global__ __launch_bounds__(64) void k_kin_virial_sum(const Rep* __restrict__ reps, int W_in, int n_part, int slot,
+                                                       const double* __restrict__ part) {
+    const Rep& R = reps[blockIdx.x];
+    double t = 0.;
+    for (int i = threadIdx.x; i < (R.N + kWave - 1) / kWave; i += kWave) t += part[(size_t)blockIdx.x * n_part + i];
+    t = wave_sum(t);
+    if (threadIdx.x == 0) R.scratch[slot * R.M] = R.kin_dbeta_const / (W_in > 0 ? W_in : R.M) + t;
 }
 
 // ---------------------------------------------------------------------------
@@ -1932,13 +1979,9 @@ __global__ __launch_bounds__(64) void k_grad_compat(const Rep* __restrict__ reps
     o[2] = g[2];
 }
 
-// Loads a replica's link-action tables (du_only: the David du_kj_dbeta table
-// instead) into LDS.
-__device__ __forceinline__ void stage_tables(const Rep& R, double* lds, bool du_only) {
-    if (du_only)
-        stage_batched(lds, R.bt_du.c, R.bt_du.c, R.lds_doubles_du, R.lds_doubles_du, 0, (int)blockDim.x);
-    else
-        stage_batched(lds, R.bt_a.c, R.bt_b.c, R.bt_a.ncoef * R.bt_a.ncomp, R.lds_doubles, 0, (int)blockDim.x);
+// Loads a replica's link-action tables into LDS.
+__device__ __forceinline__ void stage_tables(const Rep& R, double* lds) {
+    stage_batched(lds, R.bt_a.c, R.bt_b.c, R.bt_a.ncoef * R.bt_a.ncomp, R.lds_doubles, 0, (int)blockDim.x);
     __syncthreads();
 }
 
@@ -2004,7 +2047,7 @@ __global__ __launch_bounds__(kCompatBlock) void k_grad_compat_lds(const Rep* __r
     const int b = blockIdx.x, p0 = blockIdx.y * np, N = R.N, M = R.M;
     if (b >= M || p0 >= N) return;
     const bool on = short_on && R.pair_type != 0 && N > 1;
-    if (on) stage_tables(R, lds, false);
+    if (on) stage_tables(R, lds);
     double* sums = lds + R.lds_doubles;  // [group][np][3]
     const int n = min(np, N - p0), n_grp = kCompatBlock / n;
     const int grp = threadIdx.x / n, lp = threadIdx.x % n, p = p0 + lp;
@@ -2170,7 +2213,7 @@ __global__ __launch_bounds__(kAdjLdsBlock) void k_adjoint_local_lds(const Rep* _
     // gridDim.y workgroups per replica (when replicas are few), each taking a
     // contiguous block of the slice ranges
     const Rep R = reps[blockIdx.x];  // by value: the fields used stay in registers
-    stage_tables(R, lds, false);
+    stage_tables(R, lds);
     const int M = R.M, N = R.N, bpr = gridDim.y;
     const int per_blk = kAdjLdsBlock / N > 0 ? kAdjLdsBlock / N : 1;  // slice ranges per particle in one workgroup
     const int per = min(M, per_blk * bpr);                               // ... over the replica's workgroups
@@ -2388,7 +2431,7 @@ __global__ __launch_bounds__(kAdjLdsBlock) void k_adjoint_pairs_lds(const Rep* _
     const Rep R = reps[blockIdx.x];
     const bool pairs = (terms & 2u) && R.pair_type != 0 && R.N > 1;
     if (phase == 1 && !pairs) return;
-    if (pairs) stage_tables(R, lds, false);
+    if (pairs) stage_tables(R, lds);
     const int M = R.M, N = R.N;
     const int n_rng = max(1, min(kAdjPairWaves * (int)gridDim.y, M / 2));
     const int w = blockIdx.y * kAdjPairWaves + threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
@@ -2436,7 +2479,7 @@ __global__ __launch_bounds__(kAdjLdsBlock) void k_adjoint_links(const Rep* __res
     const Rep R = reps[blockIdx.y];
     const int b = blockIdx.x / h, hh = blockIdx.x % h;
     if (b >= R.M || R.N < 2 || R.pair_type == 0) return;
-    stage_tables(R, lds, false);
+    stage_tables(R, lds);
     const int M = R.M, N = R.N, b1 = b + 1 == M ? 0 : b + 1, T = (N + kWave - 1) / kWave;
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     double* slots = lds + R.lds_doubles;  // [wavefront][6][64]
@@ -2529,67 +2572,141 @@ __global__ __launch_bounds__(256) void k_adjoint_gather(const Rep* __restrict__ 
     }
 }
 
-// Whole-path pair sums with LDS tables (which 0: CalcdUdBeta, 1: CalcV on plain
-// minimum images): gridDim.y 1024-thread workgroups per replica (blockIdx.x),
-// each over every gridDim.y-th slice, per-slice partials.
-__global__ __launch_bounds__(kAdjLdsBlock) void k_pair_whole_lds(const Rep* __restrict__ reps, int which, int slot) {
+// Whole-path pair sums with LDS tables (which 0: CalcdUdBeta over every link, 1:
+// CalcV on plain minimum images), one partial sum per workgroup, S x Q workgroups
+// per replica (blockIdx.y): S contiguous slice ranges, Q parts of the pairs
+// (i, i + d mod N), d = 1..N/2.  A thread walks each of its pairs along its range
+// of slices.  What bounds it is the gathers from the LDS tables (36 doubles a link
+// with every term read), so a link reads fewer: dU/dbeta takes the sum of the
+// potential and the first component as one table (stage_whole), and the radial
+// term at a link's second slice is the next link's first where both see the same
+// image, which leaves 24; on plain minimum images the two are always the same, and
+// a potential is one term per slice.  dU/dbeta and the potential of N = 1024,
+// M = 128, one replica, 862 us together, 2495 us with a workgroup per slice (half
+// the CUs) and every term read; dU/dbeta of 512 replicas of N = 256, M = 128
+// 18.8 ms, 26.5 ms before; of one 51 us, 114 us before.
+constexpr int kWholeBlock = 1024;
+// The tables of the whole-path sums.  Bare: [v_r][v_long_r].  David: which 0 the
+// sum of components 0 and 1 of du_kj_dbeta, then components 2..n_val; which 1
+// component 0.
+__device__ __forceinline__ void stage_whole(const Rep& R, double* lds, int which) {
+    if (R.pair_type != 2) {
+        stage_batched(lds, R.bt_a.c, R.bt_b.c, R.bt_a.ncoef * R.bt_a.ncomp, R.lds_doubles, 0, (int)blockDim.x);
+    } else {
+        const int nc = R.bt_du.ncoef, n = which ? nc : nc * (R.bt_du.ncomp - 1);
+        for (int t = threadIdx.x; t < n; t += (int)blockDim.x)
+            lds[t] = which ? R.bt_du.c[t] : t < nc ? R.bt_du.c[t] + R.bt_du.c[nc + t] : R.bt_du.c[nc + t];
+    }
+    __syncthreads();
+}
+template <int PT, int NORD>
+__global__ __launch_bounds__(kWholeBlock) void k_pair_whole_lds(const Rep* __restrict__ reps, int which, int S, int Q,
+                                                                double* __restrict__ part) {
     extern __shared__ double lds[];
-    const Rep& R = reps[blockIdx.x];
-    // David: the du_kj_dbeta table (potential in component 0); Bare: the pair tables
-    stage_tables(R, lds, R.pair_type == 2);
-    const double* ldu = lds;
-    __shared__ double red[kAdjLdsBlock / kWave];
-    const int N = R.N, M = R.M, half = N / 2;
-    // slices b = blockIdx.y, + gridDim.y, ...: each slice's sum is made by one
-    // workgroup in the same order whatever the number of workgroups
-    for (int b = blockIdx.y; b < M; b += gridDim.y) {
-        const int b1 = (b + 1) % M;
-        double t = 0.;
-        // pairs (i, i + d mod N), d = 1..N/2: thread handles i = tid % N and a slice of d
-        const int per = kAdjLdsBlock / N > 0 ? kAdjLdsBlock / N : 1;
-        for (int unit = threadIdx.x; unit < N * per; unit += kAdjLdsBlock) {
-            const int i = unit % N, part = unit / N;
-            const int d_lo = 1 + (int)((long long)half * part / per), d_hi = 1 + (int)((long long)half * (part + 1) / per);
-            double a0[3], a1[3];
-            for (int d = 0; d < 3; ++d) {
-                a0[d] = pos_at(R, d, b, i);
-                a1[d] = pos_at(R, d, b1, i);
-            }
-            for (int dd = d_lo; dd < d_hi; ++dd) {
-                if ((N % 2 == 0) && dd == half && i >= half) continue;
-                const int j = (i + dd) % N;
-                double c0[3], c1[3];
-                for (int d = 0; d < 3; ++d) {
-                    c0[d] = pos_at(R, d, b, j);
-                    c1[d] = pos_at(R, d, b1, j);
-                }
-                if (which == 0) {
-                    LinkGeom g;
-                    if (i < j)
-                        link_geom_fast(a0, c0, a1, c1, R.L, R.iL, g);
-                    else
-                        link_geom_fast(c0, a0, c1, a1, R.L, R.iL, g);
-                    t += pair_du_dbeta_lds(R, lds, ldu, g.r, g.rp, g.s);
-                } else {
-                    double v0[3], v1[3];
+    const Rep R = reps[blockIdx.x];
+    __shared__ double red[kWholeBlock / kWave];
+    const int s = blockIdx.y / Q, q = blockIdx.y % Q, N = R.N, M = R.M, half = N / 2;
+    const int b_lo = (int)((long long)M * s / S), b_hi = (int)((long long)M * (s + 1) / S);
+    const bool on = R.pair_type != 0 && half > 0 && b_lo < b_hi;
+    double t = 0.;
+    if (on) {
+        stage_whole(R, lds, which);
+        const bool bare = PT == 1 || (PT == 0 && R.pair_type == 1);
+        const BTab& T = R.bt_du;
+        auto radial = [&](double r) {
+            return bare ? bare_radial_lds(R, lds, r) : 0.5 * bt_apply(lds, bt_basis(T, clampd(r, R.g_min, R.g_max)));
+        };
+        const long long n_pairs = (long long)N * half;
+        const long long u_lo = n_pairs * q / Q, u_hi = n_pairs * (q + 1) / Q;
+        for (long long u = u_lo + threadIdx.x; u < u_hi; u += kWholeBlock) {
+            const int dd = 1 + (int)(u / N), i = (int)(u % N);
+            if ((N % 2 == 0) && dd == half && i >= half) continue;
+            const int j = i + dd < N ? i + dd : i + dd - N;
+            double rv[3];
+            for (int d = 0; d < 3; ++d) rv[d] = minimg(pos_at(R, d, b_lo, j) - pos_at(R, d, b_lo, i), R.L, R.iL);
+            double r = sqrt_pos(rv[0] * rv[0] + rv[1] * rv[1] + rv[2] * rv[2]);
+            double f = radial(r);
+            if (which) {
+                // sum over the links of (v(r_b) + v(r_b+1)) / 2 = sum over the slices of v(r_b)
+                t += 2. * f;
+                for (int b = b_lo + 1; b < b_hi; ++b) {
+                    double rr = 0.;
                     for (int d = 0; d < 3; ++d) {
-                        v0[d] = minimg(a0[d] - c0[d], R.L, R.iL);
-                        v1[d] = minimg(a1[d] - c1[d], R.L, R.iL);
+                        const double x = minimg(pos_at(R, d, b, j) - pos_at(R, d, b, i), R.L, R.iL);
+                        rr += x * x;
                     }
-                    t += pair_v_lds(R, lds, ldu, sqrt(v0[0] * v0[0] + v0[1] * v0[1] + v0[2] * v0[2]),
-                                    sqrt(v1[0] * v1[0] + v1[1] * v1[1] + v1[2] * v1[2]));
+                    t += 2. * radial(sqrt_pos(rr));
                 }
+                continue;
+            }
+            // the link's second slice is loaded one link ahead
+            double xi[3], xj[3];
+            int bn = b_lo + 1 == M ? 0 : b_lo + 1;
+            for (int d = 0; d < 3; ++d) {
+                xi[d] = pos_at(R, d, bn, i);
+                xj[d] = pos_at(R, d, bn, j);
+            }
+            for (int b = b_lo; b < b_hi; ++b) {
+                double rp[3], nx[3], dx[3], pp = 0., s2 = 0.;
+                for (int d = 0; d < 3; ++d) dx[d] = xj[d] - xi[d];
+                bn = bn + 1 == M ? 0 : bn + 1;
+                for (int d = 0; d < 3; ++d) {
+                    xi[d] = pos_at(R, d, bn, i);
+                    xj[d] = pos_at(R, d, bn, j);
+                }
+                bool same = true;  // r' is the next link's r
+                for (int d = 0; d < 3; ++d) {
+                    const double x = dx[d];
+                    const double shift = rint((rv[d] - x) * R.iL), home = rint(x * R.iL);
+                    rp[d] = x + shift * R.L;
+                    nx[d] = x - home * R.L;
+                    same = same && shift == -home;
+                    const double sv = rv[d] - rp[d];
+                    pp += rp[d] * rp[d];
+                    s2 += sv * sv;
+                }
+                const double r1 = sqrt_pos(pp), f1 = radial(r1);
+                t += f + f1;
+                if (!bare) {
+                    const double qm = 0.5 * (r + r1), z = r - r1;
+                    if (s2 > 0.0 && qm < R.g_max) {
+                        const BBasis bq = bt_basis(T, qm);
+                        const double z2 = z * z;
+                        double sp[4], zp[4];
+                        sp[0] = 1.;
+                        zp[0] = 1.;
+#pragma unroll
+                        for (int e = 1; e <= (NORD ? NORD : 3); ++e) {
+                            sp[e] = sp[e - 1] * s2;
+                            zp[e] = zp[e - 1] * z2;
+                        }
+                        const int n_order = NORD ? NORD : R.n_order;
+#pragma unroll
+                        for (int k = 1; k <= (NORD ? NORD : 3); ++k) {
+                            if (k > n_order) break;
+#pragma unroll
+                            for (int e = 0; e <= k; ++e)
+                                t += bt_apply(lds + (size_t)(k * (k + 1) / 2 + e) * T.ncoef, bq) * zp[e] * sp[k - e];
+                        }
+                    }
+                }
+                r = r1;
+                f = f1;
+                if (!same) {
+                    r = sqrt_pos(nx[0] * nx[0] + nx[1] * nx[1] + nx[2] * nx[2]);
+                    f = radial(r);
+                }
+                for (int d = 0; d < 3; ++d) rv[d] = nx[d];
             }
         }
-        t = wave_sum(t);
-        if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = t;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double tt = 0.;
-            for (int w = 0; w < kAdjLdsBlock / kWave; ++w) tt += red[w];
-            R.scratch[slot * M + b] = tt;
-        }
-        __syncthreads();
+    }
+    t = wave_sum(t);
+    if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double tt = 0.;
+        for (int w = 0; w < kWholeBlock / kWave; ++w) tt += red[w];
+        part[(size_t)blockIdx.x * S * Q + blockIdx.y] = tt;
     }
 }
 
@@ -2915,32 +3032,35 @@ __global__ __launch_bounds__(256) void k_centroid(const Rep* __restrict__ reps, 
 // Scratch layout per replica: [slot][M] for slots 0..3, then long-range chunk
 // partials, then the two results.
 
-__global__ void k_finalize(const Rep* __restrict__ reps, int n_reps, int what, int acc) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_reps) return;
-    const Rep& R = reps[r];
+// One workgroup per replica; the partials are added lane by lane, then the lanes.
+// pair_part: the pair sums' n_pair partials per replica (nullptr: per slice in the
+// scratch, from the global-table kernel).
+__global__ __launch_bounds__(256) void k_finalize(const Rep* __restrict__ reps, int what, int acc,
+                                                  const double* __restrict__ pair_part, int n_pair) {
+    const Rep& R = reps[blockIdx.x];
     const int M = R.M;
     const double* S = R.scratch;
     double* res = R.scratch + scratch_res(M, R.nk);
-    if (what == 0) {
-        double t = R.kin_dbeta_const;
-        for (int b = 0; b < M; ++b) t += S[kSlotKin * M + b];
-        res[0] = t;
-    } else if (what == 1) {
-        double t = 0.;
-        for (int b = 0; b < M; ++b) t += S[kSlotPair * M + b];
-        if (R.use_long_range && R.pair_type != 0) {
-            const double* lw = R.scratch + scratch_long(M);
-            double l = 0.;
-            for (int c = 0; c < (R.nk + 255) / 256; ++c) l += lw[c];
-            t += l;
-        }
-        res[1] = t;
-    } else if (what == 2) {
-        double c = 0.;
-        for (int b = 0; b < M; ++b) c += S[kSlotCentroid * M + b];
-        res[0] = S[kSlotVirial * M] + c / (2. * R.tau);
+    __shared__ double sh[4];
+    const int slot = what == 0 ? kSlotKin : what == 1 ? kSlotPair : kSlotCentroid;
+    const bool parts = what == 1 && pair_part;
+    const double* v = parts ? pair_part + (size_t)blockIdx.x * n_pair : S + slot * M;
+    const int n = parts ? n_pair : M;
+    double t = 0., l = 0.;
+    for (int b = threadIdx.x; b < n; b += 256) t += v[b];
+    if (what == 1 && R.use_long_range && R.pair_type != 0) {
+        const double* lw = R.scratch + scratch_long(M);
+        for (int c = threadIdx.x; c < (R.nk + kWave - 1) / kWave; c += 256) l += lw[c];
     }
+    t = block_sum<256>(t, sh);
+    l = block_sum<256>(l, sh);
+    if (threadIdx.x) return;
+    if (what == 0)
+        res[0] = R.kin_dbeta_const + t;
+    else if (what == 1)
+        res[1] = t + l;
+    else
+        res[0] = S[kSlotVirial * M] + t / (2. * R.tau);
     if (acc) {
         R.e_acc[0] += res[0];
         R.e_acc[1] += res[1];
@@ -2951,41 +3071,43 @@ __global__ void k_finalize(const Rep* __restrict__ reps, int n_reps, int what, i
 // ---------------------------------------------------------------------------
 // K8: StructureFactor::Accumulate (structure_factor_class.h:15-32)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_sk(const Rep* __restrict__ reps, double k_cut) {
+__global__ __launch_bounds__(kSumBlock) void k_sk(const Rep* __restrict__ reps, double k_cut) {
     const Rep& R = reps[blockIdx.y];
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= R.nk) return;
+    __shared__ double sh[kSumBlock];
+    if ((int)blockIdx.x * kWave >= R.nk) return;
+    const int k = blockIdx.x * kWave + (threadIdx.x & (kWave - 1));
     if (threadIdx.x == 0 && blockIdx.x == 0) R.n_measure[1] += 1;
-    if (!(R.kmag[k] < k_cut)) return;
-    double t = 0.;
-    for (int b = 0; b < R.M; ++b) {
-        const double2 v = R.rho[((size_t)R.sel[b] * R.M + b) * R.nk + k];
-        t += v.x * v.x + v.y * v.y;
-    }
-    R.sk_acc[k] += t;
+    const double t = sum_rho2(R, k, sh);
+    if (threadIdx.x < kWave && k < R.nk && R.kmag[k] < k_cut) R.sk_acc[k] += t;
 }
 
 // ---------------------------------------------------------------------------
 // K9: PairCorrelation::Accumulate (pair_correlation_class.h:15-28) with
 // LinearGrid::ReverseMap (observable_class.h:56-62); LDS histogram per slice.
+// The workgroup's threads share the pairs (i, i + d mod N), i fastest; 1024 of
+// them while the slices alone do not fill the chip (N = 256, M = 128, one replica
+// 54 us with 256 threads, a particle each, 27 us so).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_gr(const Rep* __restrict__ reps, double r_min, double d_ir, int n_r,
+__global__ __launch_bounds__(1024) void k_gr(const Rep* __restrict__ reps, double r_min, double d_ir, int n_r,
                                             const double* __restrict__ r_max_per_rep) {
     const Rep& R = reps[blockIdx.y];
     const int b = blockIdx.x;
     if (b >= R.M) return;
     __shared__ unsigned int hist[kGrBins];
-    for (int i = threadIdx.x; i < n_r; i += 256) hist[i] = 0;
+    const int nthr = blockDim.x;
+    for (int i = threadIdx.x; i < n_r; i += nthr) hist[i] = 0;
     __syncthreads();
     const int N = R.N, half = N / 2;
     double dir = d_ir;
     if (r_max_per_rep) dir = 1. / ((r_max_per_rep[blockIdx.y] - r_min) / (n_r - 1.));
-    for (int i = threadIdx.x; i < N; i += 256) {
+    const int groups = max(1, nthr / N);  // threads per particle
+    for (int u = threadIdx.x; u < N * groups; u += nthr) {
+        const int i = u % N, grp = u / N;
         double a[3];
         for (int d = 0; d < 3; ++d) a[d] = pos_at(R, d, b, i);
-        for (int dd = 1; dd <= half; ++dd) {
+        for (int dd = 1 + grp; dd <= half; dd += groups) {
             if ((N % 2 == 0) && dd == half && i >= half) continue;
-            const int j = (i + dd) % N;
+            const int j = i + dd < N ? i + dd : i + dd - N;
             const int lo = min(i, j), hi = max(i, j);
             double v[3];
             {
@@ -3003,7 +3125,7 @@ __global__ __launch_bounds__(256) void k_gr(const Rep* __restrict__ reps, double
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n_r; i += 256)
+    for (int i = threadIdx.x; i < n_r; i += nthr)
         if (hist[i]) atomicAdd(&R.gr_cnt[i], (unsigned long long)hist[i]);
     if (threadIdx.x == 0 && b == 0) R.n_measure[2] += 1;
 }
