@@ -394,15 +394,15 @@ struct spimc_ctx {
     Rep* d_reps = nullptr;
     std::vector<Group> groups;
     hipEvent_t stage_ready = nullptr;
-    uint2* d_items_tmp = nullptr;
-    size_t items_tmp_cap = 0;
     // pinned host memory, also addressed by kernels: the replay-error flag, the
     // stage's attempt counts (one per replica) and the staging area of small reads
     char* pin = nullptr;
     volatile unsigned int* h_error = nullptr;
     unsigned int* counts = nullptr;
     unsigned char* stage = nullptr;
-    double* d_tmp = nullptr;  // interface partials + result
+    double* d_tmp = nullptr;  // interface partials
+    unsigned int* d_iface = nullptr;  // arrivals of an interface query's workgroups (zero between queries)
+    double* h_result = nullptr;       // its result, in pinned memory
     size_t tmp_cap = 0;
     bool any_long = false;
     int max_M = 0, max_N = 0, max_nk = 0;
@@ -448,7 +448,6 @@ struct spimc_ctx {
     // k_rho variant: k-vectors per thread and non-temporal rho_k traffic
     int rho_kpt = kRhoKpt;
     bool rho_nt = true;  // measured: slightly faster, and keeps the pair tables in L2
-    void (*rho_fn)(const Rep*, const uint2*, int, int, unsigned long long*) = nullptr;
     // looping variant with rho_bpc workgroups per CU (0: one workgroup per item)
     int rho_bpc = 0;
     void (*rho_loop_fn)(const RhoItem*, int, unsigned long long*) = nullptr;
@@ -1204,18 +1203,12 @@ int build_groups(spimc_ctx* c, int n_groups) {
     return SPIMC_OK;
 }
 
-int ensure_tmp(spimc_ctx* c, size_t n_doubles, size_t n_items) {
+int ensure_tmp(spimc_ctx* c, size_t n_doubles) {
     if (n_doubles > c->tmp_cap) {
         if (c->d_tmp) (void)hipFree(c->d_tmp);
         c->d_tmp = nullptr;
         HIPCHK(hipMalloc((void**)&c->d_tmp, n_doubles * sizeof(double)));
         c->tmp_cap = n_doubles;
-    }
-    if (n_items > c->items_tmp_cap) {
-        if (c->d_items_tmp) (void)hipFree(c->d_items_tmp);
-        c->d_items_tmp = nullptr;
-        HIPCHK(hipMalloc((void**)&c->d_items_tmp, n_items * sizeof(uint2)));
-        c->items_tmp_cap = n_items;
     }
     return SPIMC_OK;
 }
@@ -1538,7 +1531,7 @@ int launch_round(spimc_ctx* c, const Group& G, int move) {
     } else {
         if (np) {
             const int g = (np + 3) / 4;
-            rc = launch(c, SPIMC_KERNEL_PAIR, k_pair, g, kPairBlock, 0, st, all, pi, np, 0, kt);
+            rc = launch(c, SPIMC_KERNEL_PAIR, k_pair, g, kPairBlock, 0, st, all, pi, np, kt);
             if (rc) return rc;
         }
         if (multi && (rc = launch_pair_multi(c, G, st))) return rc;
@@ -2098,11 +2091,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
         c->auto_fork = false;
     }
     {
-        using RhoFn = void (*)(const Rep*, const uint2*, int, int, unsigned long long*);
-        const RhoFn fns[2][4] = {{k_rho<2, false>, k_rho<4, false>, k_rho<8, false>, k_rho<16, false>},
-                                 {k_rho<2, true>, k_rho<4, true>, k_rho<8, true>, k_rho<16, true>}};
         const int ki = c->rho_kpt == 2 ? 0 : c->rho_kpt == 4 ? 1 : c->rho_kpt == 8 ? 2 : 3;
-        c->rho_fn = fns[c->rho_nt ? 1 : 0][ki];
         using RhoLoopFn = void (*)(const RhoItem*, int, unsigned long long*);
         const RhoLoopFn lfns[2][4] = {
             {k_rho_loop<2, false>, k_rho_loop<4, false>, k_rho_loop<8, false>, k_rho_loop<16, false>},
@@ -2128,6 +2117,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             return bail(fail(SPIMC_ERR_NOMEM, "pinned host memory"));
         c->h_error = reinterpret_cast<volatile unsigned int*>(c->pin);
         *c->h_error = 0;
+        c->h_result = reinterpret_cast<double*>(c->pin + 128);
         c->counts = reinterpret_cast<unsigned int*>(c->pin + 256);
         c->stage = reinterpret_cast<unsigned char*>(c->pin + 256 + b_cnt);
     }
@@ -2142,6 +2132,9 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             return bail(fail(SPIMC_ERR_HIP, "wall clock rate"));
         c->clock_hz = 1e3 * khz;
     }
+    if (hipMalloc((void**)&c->d_iface, sizeof(unsigned int)) != hipSuccess ||
+        hipMemset(c->d_iface, 0, sizeof(unsigned int)) != hipSuccess)
+        return bail(fail(SPIMC_ERR_NOMEM, "interface counter"));
     if (hipMalloc((void**)&c->d_vir, (size_t)n_replicas * ((c->max_N + 63) / 64) * sizeof(double)) != hipSuccess)
         return bail(fail(SPIMC_ERR_NOMEM, "virial partial sums"));
     if (hipMalloc((void**)&c->d_gr_rmax, n_replicas * sizeof(double)) != hipSuccess)
@@ -2322,7 +2315,7 @@ int spimc_ctx_destroy(spimc_ctx* c) {
         if (h.perm_t) (void)hipFree(h.perm_t);
     }
     for (void* p : {(void*)c->d_reps, (void*)c->d_work, (void*)c->d_gr_rmax,
-                    (void*)c->d_tmp, (void*)c->d_items_tmp, (void*)c->d_adj_part, (void*)c->d_col_w, (void*)c->d_whole, (void*)c->d_vir})
+                    (void*)c->d_tmp, (void*)c->d_iface, (void*)c->d_adj_part, (void*)c->d_col_w, (void*)c->d_whole, (void*)c->d_vir})
         if (p) (void)hipFree(p);
     if (c->pin) (void)hipHostFree(c->pin);
     for (auto& t : c->pending) {
@@ -2370,7 +2363,7 @@ int spimc_rho_k_download(spimc_ctx* c, uint32_t r, double* rho) {
     if (!R.use_long_range) return fail(SPIMC_ERR_STATE, "replica has no long-range action");
     // the committed rows lie in two buffers: gathered on the device, then one copy
     // (a copy a row took 1.2 ms for 128 rows)
-    if ((rc = ensure_tmp(c, (size_t)2 * R.M * R.nk, 0))) return rc;
+    if ((rc = ensure_tmp(c, (size_t)2 * R.M * R.nk))) return rc;
     k_gather_rho<<<R.M, 256, 0, c->stream>>>(c->d_reps, (int)r, reinterpret_cast<double2*>(c->d_tmp));
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -2394,7 +2387,16 @@ int spimc_set_proposal(spimc_ctx* c, uint32_t r, uint32_t particle, uint32_t b_f
     if (particle >= (uint32_t)R.N || n_beads == 0 || n_beads > (uint32_t)R.M || !r_new)
         return fail(SPIMC_ERR_ARG, "bad proposal");
     if (c->prop_set && c->prop_rep != (int)r) return fail(SPIMC_ERR_STATE, "a proposal on another replica is pending");
-    HIPCHK(hipMemcpy(R.prop_new, r_new, (size_t)3 * n_beads * sizeof(double), hipMemcpyHostToDevice));
+    if (n_beads <= (uint32_t)kPropArg) {
+        // as a kernel argument: nothing to wait for, later work on the stream follows it
+        PropBeads v;
+        std::memcpy(v.x, r_new, (size_t)3 * n_beads * sizeof(double));
+        if ((rc = launch(c, SPIMC_KERNEL_PROPOSE, k_set_proposal, 1, 3 * kPropArg, 0, c->stream, c->d_reps, (int)r, (int)n_beads, v)))
+            return rc;
+    } else {
+        HIPCHK(hipMemcpyAsync(R.prop_new, r_new, (size_t)3 * n_beads * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+    }
     c->prop_set = true;
     c->rho_updated = false;
     c->prop_rep = r;
@@ -2404,28 +2406,24 @@ int spimc_set_proposal(spimc_ctx* c, uint32_t r, uint32_t particle, uint32_t b_f
     return SPIMC_OK;
 }
 
-static int write_iface_prop(spimc_ctx* c, uint32_t r, int p, int b0, int n_links) {
+// The record of an interface query on particle p (the pending proposal's beads if it is p's).
+static Prop iface_prop(const spimc_ctx* c, uint32_t r, int p) {
     Prop pr{};
-    pr.status = 0;
     pr.move = 2;
-    pr.p = p;
-    pr.p2 = p;
-    pr.b0 = b0;
-    pr.n_links = n_links;
+    pr.p = pr.p2 = p;
     const bool mine = c->prop_set && c->prop_rep == (int)r && c->prop_p == p;
     pr.first = mine ? c->prop_first : 0;
     pr.count = mine ? c->prop_count : 0;
-    HIPCHK(hipMemcpy(c->reps[r].dev.prop, &pr, sizeof(Prop), hipMemcpyHostToDevice));
-    return SPIMC_OK;
+    return pr;
 }
 
 static int finish_proposal(spimc_ctx* c, uint32_t r, int accept) {
     int rc = check_rep(c, r);
     if (rc) return rc;
     if (!c->prop_set || c->prop_rep != (int)r) return fail(SPIMC_ERR_STATE, "no proposal pending on this replica");
-    if ((rc = write_iface_prop(c, r, c->prop_p, c->prop_first, 0))) return rc;
     const int upd = c->rho_updated ? 1 : 0;
-    rc = launch(c, SPIMC_KERNEL_DECIDE, k_commit, 1, 256, 0, c->stream, c->d_reps, (int)r, accept, upd);
+    rc = launch(c, SPIMC_KERNEL_DECIDE, k_commit, 1, 256, 0, c->stream, c->d_reps, (int)r, iface_prop(c, r, c->prop_p),
+                accept, upd);
     if (rc) return rc;
     c->prop_set = false;
     c->rho_updated = false;
@@ -2439,12 +2437,11 @@ int spimc_reject_proposal(spimc_ctx* c, uint32_t r) { return finish_proposal(c, 
 namespace {
 
 // Device memory of one GetAction query beyond its inputs and outputs: per-slice
-// long-range partials and the result (tmp, doubles) and the pair / rho_k work
-// items (items).  spimc_get_action grows context buffers for them;
-// spimc_get_action_noalloc carves them from the device scratch array.
+// long-range partials.  spimc_get_action grows a context buffer for them;
+// spimc_get_action_noalloc takes them from the device scratch array, whose limits
+// also count the work items it once held.
 struct IfaceScratch {
     double* tmp;
-    uint2* items;
     size_t tmp_cap, items_cap;
 };
 
@@ -2470,10 +2467,9 @@ int get_action_impl(spimc_ctx* c, uint32_t r, int action, int mode, uint32_t b0,
             return fail(SPIMC_ERR_ARG, "query too large for the fixed scratch: n_bead + 8 partials and n_bead * k chunks "
                                        "work items must fit spimc_get_action_noalloc's scratch (SPIMC_NOALLOC_SCRATCH_BYTES)");
     } else {
-        if ((rc = ensure_tmp(c, need_tmp, need_items))) return rc;
-        sc = IfaceScratch{c->d_tmp, c->d_items_tmp, c->tmp_cap, c->items_tmp_cap};
+        if ((rc = ensure_tmp(c, need_tmp))) return rc;
+        sc = IfaceScratch{c->d_tmp, c->tmp_cap, need_items};
     }
-    double* d_out = sc.tmp + R.M;
     if (action == SPIMC_ACTION_KINETIC) {
         if (level >= kMaxKinSplines || (R.kin_images > 0 && level >= c->reps[r].kin.size()))
             return fail(SPIMC_ERR_UNSUPPORTED, "kinetic level out of range");
@@ -2488,49 +2484,25 @@ int get_action_impl(spimc_ctx* c, uint32_t r, int action, int mode, uint32_t b0,
         }
         if (span % skip) return fail(SPIMC_ERR_ARG, "window not a multiple of the level step");
         const int nl = (int)(span / skip);
-        if ((rc = write_iface_prop(c, r, p, (int)b0, 0))) return rc;
-        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_kinetic_window, 1, 64, 0, c->stream, c->d_reps, (int)r, mode, p, (int)b0, nl, (int)level, d_out);
+        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_kinetic_window, 1, 64, 0, c->stream, c->d_reps, (int)r, iface_prop(c, r, p),
+                    mode, p, (int)b0, nl, (int)level, c->h_result);
     } else {
         // PairAction::GetAction: 0 above max_level (= 0), and for is_constant
         if (level > 0 || R.pair_type == SPIMC_PAIR_NONE || R.N == 1) return SPIMC_OK;
         const int nl = (int)(b1 - b0);
-        if ((rc = write_iface_prop(c, r, p, (int)b0, nl))) return rc;
-        if (nl > 0) {
-            // work items (r, link j), written on the device
-            rc = launch(c, SPIMC_KERNEL_PAIR, k_iface_items, (nl + 255) / 256, 256, 0, c->stream, sc.items, (int)r, nl, 0);
-            if (rc) return rc;
-            const int g = (nl + 3) / 4;
-            rc = launch(c, SPIMC_KERNEL_PAIR, k_pair, g, kPairBlock, 0, c->stream, c->d_reps, (const uint2*)sc.items, nl, 1, nullptr);
-            if (rc) return rc;
-        }
-        int n_long = 0;
-        if (R.use_long_range) {
-            const bool mine = c->prop_set && c->prop_rep == (int)r && c->prop_p == p;
-            if (mode == SPIMC_MODE_NEW && mine && !c->rho_updated) {
-                // work items (r, moved bead m << 8 | k chunk), after the pair kernel has read its items
-                const int nri = c->prop_count * R.n_chunks;
-                rc = launch(c, SPIMC_KERNEL_RHO, k_iface_items, (nri + 255) / 256, 256, 0, c->stream, sc.items, (int)r, nri,
-                            R.n_chunks);
-                if (rc) return rc;
-                const int gph = (6 * c->prop_count + 63) / 64;
-                rc = launch(c, SPIMC_KERNEL_RHO, k_phase_proposal, gph, 64, 0, c->stream, c->d_reps, (int)r);
-                if (rc) return rc;
-                rc = launch(c, SPIMC_KERNEL_RHO, c->rho_fn, nri, kRhoBlock, 0, c->stream, c->d_reps, (const uint2*)sc.items, nri, 1, nullptr);
-                if (rc) return rc;
-                c->rho_updated = true;
-            }
-            n_long = (int)((b1 - b0 + skip - 1) / skip);
-            const int upd = (mine && c->rho_updated) ? 1 : 0;
-            if (n_long > 0) {
-                rc = launch(c, SPIMC_KERNEL_RHO, k_long_window, n_long, 256, 0, c->stream, c->d_reps, (int)r, mode, (int)b0, upd, sc.tmp);
-                if (rc) return rc;
-            }
-        }
-        rc = launch(c, SPIMC_KERNEL_PAIR, k_action_sum, 1, 64, 0, c->stream, c->d_reps, (int)r, mode, nl, n_long, (const double*)sc.tmp, d_out);
+        const bool mine = c->prop_set && c->prop_rep == (int)r && c->prop_p == p;
+        // NEW mode with a proposal updates rho_k of its slices once
+        const int n_update = R.use_long_range && mode == SPIMC_MODE_NEW && mine && !c->rho_updated ? c->prop_count : 0;
+        const int n_long = R.use_long_range ? nl : 0;
+        if (nl + n_update == 0) return SPIMC_OK;
+        rc = launch(c, SPIMC_KERNEL_PAIR, k_iface_pair, nl + n_update + n_long, kIfaceBlock, 0, c->stream, c->d_reps, (int)r,
+                    iface_prop(c, r, p), mode, (int)b0, nl, n_update, n_long, (mine && c->rho_updated) ? 1 : 0, sc.tmp,
+                    c->d_iface, c->h_result);
+        if (n_update) c->rho_updated = true;
     }
     if (rc) return rc;
     if ((rc = sync_and_resolve(c))) return rc;
-    HIPCHK(hipMemcpy(out, d_out, sizeof(double), hipMemcpyDeviceToHost));
+    *out = *(volatile double*)c->h_result;
     return SPIMC_OK;
 }
 
@@ -2549,9 +2521,7 @@ int spimc_get_action_noalloc(spimc_ctx* c, uint32_t r, int action, int mode, uin
         return fail(SPIMC_ERR_HIP, "device scratch of this context's device is not available: " + c->noalloc_error);
     // the scratch array: long-range partials and result first, then the work items
     constexpr size_t kTmpBytes = kNoAllocScratchBytes / 4;
-    IfaceScratch sc{reinterpret_cast<double*>(c->noalloc_scratch),
-                    reinterpret_cast<uint2*>(static_cast<char*>(c->noalloc_scratch) + kTmpBytes),
-                    kTmpBytes / sizeof(double), (kNoAllocScratchBytes - kTmpBytes) / sizeof(uint2)};
+    IfaceScratch sc{reinterpret_cast<double*>(c->noalloc_scratch), kTmpBytes / sizeof(double), (kNoAllocScratchBytes - kTmpBytes) / sizeof(uint2)};
     return get_action_impl(c, r, action, mode, b0, b1, parts, n_parts, level, out, &sc);
 }
 
@@ -2590,13 +2560,11 @@ int spimc_get_action_laplacian(spimc_ctx* c, uint32_t r, int action, int mode, u
     }
     // the pair action: 0 above max_level (= 0) and for is_constant
     if (level > 0 || R.pair_type == SPIMC_PAIR_NONE || R.N == 1 || b1 == b0) return SPIMC_OK;
-    if ((rc = write_iface_prop(c, r, p, (int)b0, 0))) return rc;
-    if ((rc = ensure_tmp(c, 1, 0))) return rc;
-    rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_pair_laplacian, 1, kLapBlock, 0, c->stream, c->d_reps, (int)r, mode, (int)b0,
-                (int)b1, p, c->d_tmp);
+    rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_pair_laplacian, 1, kLapBlock, 0, c->stream, c->d_reps, (int)r,
+                iface_prop(c, r, p), mode, (int)b0, (int)b1, p, c->h_result);
     if (rc) return rc;
     if ((rc = sync_and_resolve(c))) return rc;
-    HIPCHK(hipMemcpy(out, c->d_tmp, sizeof(double), hipMemcpyDeviceToHost));
+    *out = *(volatile double*)c->h_result;
     return SPIMC_OK;
 }
 
@@ -2611,9 +2579,9 @@ int spimc_d_action_d_beta(spimc_ctx* c, uint32_t r, int action, double* out) {
     } else {
         if ((rc = est_pair_whole(c, base, 1, 0)) || (rc = est_finalize(c, base, 1, 1, 0))) return rc;
     }
-    if ((rc = sync_and_resolve(c))) return rc;
     double res[2];
-    HIPCHK(hipMemcpy(res, R.scratch + scratch_res(R.M, R.nk), sizeof res, hipMemcpyDeviceToHost));
+    if ((rc = read_words(c, R.scratch + scratch_res(R.M, R.nk), 2, res, nullptr, 0, nullptr))) return rc;
+    if ((rc = sync_and_resolve(c))) return rc;
     *out = action == SPIMC_ACTION_KINETIC ? res[0] : (R.pair_type == SPIMC_PAIR_NONE ? 0. : res[1]);
     return SPIMC_OK;
 }
@@ -2627,9 +2595,9 @@ int spimc_potential(spimc_ctx* c, uint32_t r, int action, double* out) {
     if (action == SPIMC_ACTION_KINETIC || R.pair_type == SPIMC_PAIR_NONE) return SPIMC_OK;
     Rep* base = c->d_reps + r;
     if ((rc = est_pair_whole(c, base, 1, 1)) || (rc = est_finalize(c, base, 1, 1, 0))) return rc;
-    if ((rc = sync_and_resolve(c))) return rc;
     double res[2];
-    HIPCHK(hipMemcpy(res, R.scratch + scratch_res(R.M, R.nk), sizeof res, hipMemcpyDeviceToHost));
+    if ((rc = read_words(c, R.scratch + scratch_res(R.M, R.nk), 2, res, nullptr, 0, nullptr))) return rc;
+    if ((rc = sync_and_resolve(c))) return rc;
     *out = res[1];
     return SPIMC_OK;
 }
@@ -2641,9 +2609,8 @@ int spimc_kinetic_virial_energy(spimc_ctx* c, uint32_t r, uint32_t window, doubl
     const Rep& R = c->reps[r].dev;
     const int W = window ? (int)window : 0;
     rc = est_kin_virial(c, c->d_reps + r, 1, W);
-    if (rc || (rc = sync_and_resolve(c))) return rc;
-    HIPCHK(hipMemcpy(out, R.scratch + kSlotVirial * R.M, sizeof(double), hipMemcpyDeviceToHost));
-    return SPIMC_OK;
+    if (rc || (rc = read_words(c, R.scratch + kSlotVirial * R.M, 1, out, nullptr, 0, nullptr))) return rc;
+    return sync_and_resolve(c);
 }
 
 int spimc_action_gradient(spimc_ctx* c, uint32_t r, uint32_t terms, int compat, double* out) {

@@ -576,35 +576,19 @@ __device__ __forceinline__ void propose_displace_body(const Rep* __restrict__ re
     propose_displace_impl(reps[r], (int)threadIdx.x, BlockSync{}, true);
 }
 
-// Phase tables of an interface proposal's moved beads (before k_rho in interface mode).
-__global__ __launch_bounds__(64) void k_phase_proposal(const Rep* __restrict__ reps, int r) {
-    const Rep& R = reps[r];
-    const Prop pr = *R.prop;
-    for (int t = blockIdx.x * 64 + threadIdx.x; t < 6 * pr.count; t += gridDim.x * 64) {
-        const int m = t / 6, s = (pr.first + m) % R.M;
-        double xo[3], xn[3];
-        for (int d = 0; d < 3; ++d) {
-            xo[d] = pos_at(R, d, s, pr.p);
-            xn[d] = R.prop_new[3 * m + d];
-        }
-        moved_phase_chain(R, m, t % 6, xo, xn);
-        if (t % 6 == 0) moved_row(R, m, s);
-    }
-}
-
 // ---------------------------------------------------------------------------
 // K1: short-range pair action of the moved particle on the window links,
 // OLD and NEW (pair_action_class.h:279-290), one wavefront per (replica, link).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void pair_block(const Rep* __restrict__ reps, const uint2* __restrict__ items, int n_items,
-                                           int interface_mode, int blk) {
+                                           int blk) {
     const int item = blk * (kPairBlock / kWave) + (threadIdx.x >> 6);
     const int lane = threadIdx.x & (kWave - 1);
     if (item >= n_items) return;
     const uint2 it = items[item];
     const Rep& R = reps[it.x];
     const Prop pr = *R.prop;
-    if (!interface_mode && (pr.status != 1 || pr.generic)) return;
+    if (pr.status != 1 || pr.generic) return;
     const int j = (int)it.y;
     if (j >= pr.n_links) return;
     const int M = R.M, N = R.N, p = pr.p;
@@ -869,10 +853,9 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) void k_
 }
 
 __global__ __launch_bounds__(kPairBlock) void k_pair(const Rep* __restrict__ reps, const uint2* __restrict__ items,
-                                                     int n_items, int interface_mode,
-                                                     unsigned long long* __restrict__ kt) {
+                                                     int n_items, unsigned long long* __restrict__ kt) {
     kt_begin(kt, KT_PAIR);
-    pair_block(reps, items, n_items, interface_mode, xcd_remap(blockIdx.x, gridDim.x));
+    pair_block(reps, items, n_items, xcd_remap(blockIdx.x, gridDim.x));
     kt_end(kt, KT_PAIR);
 }
 
@@ -882,80 +865,6 @@ __global__ __launch_bounds__(kPairBlock) void k_pair(const Rep* __restrict__ rep
 // long-range action sums of CalcULong (bare_pair_action_class.h:153-172,
 // david_pair_action_class.h:105-123) for OLD and NEW.
 // ---------------------------------------------------------------------------
-template <int KPT, bool NT = false>
-__device__ __forceinline__ void rho_block(const Rep* __restrict__ reps, const uint2* __restrict__ items, int n_items,
-                                          int interface_mode, int blk) {
-    if (blk >= n_items) return;
-    const uint2 it = items[blk];
-    const Rep& R = reps[it.x];
-    const Prop pr = *R.prop;
-    if (!interface_mode && pr.status != 1) return;
-    const int m = (int)(it.y >> 8), chunk = (int)(it.y & 255);
-    if (m >= pr.count) return;
-    const int M = R.M, nk = R.nk, stride = R.max_idx + 1;
-    const int2 row = R.rho_rows[m];
-    const int s = row.x, cur = row.y;
-    __shared__ double2 tab[2 * 3 * (kMaxIdx + 1)];
-    __shared__ double red[2][kRhoBlock / kWave];
-    // the six phase chains of this moved bead (OLD x3, NEW x3)
-    const double2* src = R.phase + (size_t)m * 6 * stride;
-    for (int t = threadIdx.x; t < 6 * stride; t += kRhoBlock) tab[t] = src[t];
-    const double2* __restrict__ rc = R.rho + ((size_t)cur * M + s) * nk;
-    double2* __restrict__ rn = R.rho + ((size_t)(1 - cur) * M + s) * nk;
-    const int k0 = chunk * kRhoBlock * KPT + threadIdx.x;
-    // issue the rho_k and k-table loads before waiting on the tables
-    double2 rv[KPT];
-    int kp[KPT];
-    double cf[KPT];
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const int k = k0 + i * kRhoBlock;
-        const bool ok = k < nk;
-        rv[i] = ok ? ld2<NT>(rc + k) : make_double2(0., 0.);
-        kp[i] = ok ? gld(R.kidx + k) : (128 | (128 << 8) | (128 << 16));
-        cf[i] = ok ? gld(R.coef_s + k) : 0.;
-    }
-    __syncthreads();
-    double ao = 0., an = 0.;
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const int k = k0 + i * kRhoBlock;
-        const double2 en = phase_k(&tab[3 * stride], stride, kp[i]);
-        const double2 eo = phase_k(tab, stride, kp[i]);
-        double2 nv;
-        nv.x = rv[i].x + (en.x - eo.x);
-        nv.y = rv[i].y + (en.y - eo.y);
-        if (k < nk) st2<NT>(rn + k, nv);
-        ao += cf[i] * (rv[i].x * rv[i].x + rv[i].y * rv[i].y);
-        an += cf[i] * (nv.x * nv.x + nv.y * nv.y);
-    }
-    ao = wave_sum(ao);
-    an = wave_sum(an);
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    if (lane == 0) {
-        red[0][w] = ao;
-        red[1][w] = an;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double to = 0., tn = 0.;
-        for (int i = 0; i < kRhoBlock / kWave; ++i) {
-            to += red[0][i];
-            tn += red[1][i];
-        }
-        R.rho_part[m * R.n_chunks + chunk] = make_double2(to, tn);
-    }
-}
-
-template <int KPT, bool NT>
-__global__ __launch_bounds__(kRhoBlock) void k_rho(const Rep* __restrict__ reps, const uint2* __restrict__ items,
-                                                   int n_items, int interface_mode,
-                                                   unsigned long long* __restrict__ kt) {
-    kt_begin(kt, KT_RHO);
-    rho_block<KPT, NT>(reps, items, n_items, interface_mode, xcd_remap(blockIdx.x, gridDim.x));
-    kt_end(kt, KT_RHO);
-}
-
 // One rho_k work item on a whole kRhoBlock-thread workgroup: its rho_k, k-table
 // and phase-chain loads are all issued before the first wait; the item's
 // (OLD, NEW) sums go to *d.part.  The caller separates items that reuse tab and
@@ -1567,13 +1476,29 @@ __global__ void k_stage_begin(const Rep* __restrict__ reps, int n_reps, const un
 }
 
 // ---------------------------------------------------------------------------
-// Interface kernels (Action::GetAction in a chosen mode)
+// Interface kernels (Action::GetAction in a chosen mode).  A query is a few
+// microseconds of work, so launches, copies and synchronisations are its cost:
+// the proposal's record comes as a kernel argument (NEW beads of up to 64 slices
+// too), a pair query is one launch whose last workgroup adds the terms, and the
+// result goes to pinned host memory.  An attempt of N = 32, M = 32 (proposal, four
+// queries, accept) took 238 us with 10 blocking copies and 14 launches,
+// 81 us so.
 // ---------------------------------------------------------------------------
+constexpr int kPropArg = 64;
+struct PropBeads {
+    double x[3 * kPropArg];
+};
+__global__ __launch_bounds__(3 * kPropArg) void k_set_proposal(const Rep* __restrict__ reps, int r, int n, PropBeads v) {
+    if ((int)threadIdx.x < 3 * n) reps[r].prop_new[threadIdx.x] = v.x[threadIdx.x];
+}
+__device__ __forceinline__ void host_result(double* out, double v) {
+    __hip_atomic_store(out, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Kinetic::GetAction (kinetic_class.h:105-122) for the proposal's particle p.
-__global__ __launch_bounds__(64) void k_kinetic_window(const Rep* __restrict__ reps, int r, int mode, int p, int b0,
-                                                        int n_links, int level, double* __restrict__ out) {
+__global__ __launch_bounds__(64) void k_kinetic_window(const Rep* __restrict__ reps, int r, Prop pr, int mode, int p,
+                                                        int b0, int n_links, int level, double* __restrict__ out) {
     const Rep& R = reps[r];
-    const Prop pr = *R.prop;
     const int skip = 1 << level, M = R.M;
     const double i4lt = 1. / (4. * R.lambda * (R.tau * (double)skip));
     double tot = 0.;
@@ -1593,41 +1518,107 @@ __global__ __launch_bounds__(64) void k_kinetic_window(const Rep* __restrict__ r
         tot += free_neg_log(&R.kin[level], R.kin_images, i4lt, dd);
     }
     tot = wave_sum(tot);
-    if (threadIdx.x == 0) *out = tot;
+    if (threadIdx.x == 0) host_result(out, tot);
 }
 
-// Long-range sum of CalcULong over window slices in a mode; NEW mode reads the
-// spare buffer for slices the proposal moved (after k_rho in interface mode).
-__global__ __launch_bounds__(256) void k_long_window(const Rep* __restrict__ reps, int r, int mode, int b0,
-                                                     int rho_updated, double* __restrict__ part) {
+// PairAction::GetAction (pair_action_class.h:267-302) of particle p at level 0 in
+// one mode.  Workgroups: one per window link (its partners over the threads), then
+// one per slice the proposal moves whose NEW rho_k is not there yet (n_update:
+// Species::UpdateRhoK, species_class.h:406-425, with the slice's CalcULong sum when
+// it lies in the window), then one per other window slice (CalcULong on the
+// committed rho_k, or on the spare row where NEW mode updated it before).  The
+// terms pass between workgroups as agent-scope atomic stores and loads (see
+// k_round); the last one to arrive adds them in link and slice order.
+constexpr int kIfaceBlock = 256;
+__global__ __launch_bounds__(kIfaceBlock) void k_iface_pair(const Rep* __restrict__ reps, int r, Prop pr, int mode, int b0,
+                                                            int n_links, int n_update, int n_long, int rho_updated,
+                                                            double* __restrict__ part, unsigned int* __restrict__ arrive,
+                                                            double* __restrict__ out) {
     const Rep& R = reps[r];
-    const Prop pr = *R.prop;
-    const int w = blockIdx.x, M = R.M;
-    const int s = (b0 + w) % M;
-    int m = s - pr.first;
-    if (m < 0) m += M;
-    const bool moved = mode && rho_updated && (m < pr.count);
-    const int buf = moved ? 1 - R.sel[s] : R.sel[s];
-    const double2* rb = R.rho + ((size_t)buf * M + s) * R.nk;
+    const int M = R.M, N = R.N, p = pr.p, tid = threadIdx.x;
+    __shared__ double sh[kIfaceBlock / kWave];
+    __shared__ double2 tab[6 * (kMaxIdx + 1)];
+    __shared__ int s_last;
+    const int blk = blockIdx.x;
     double t = 0.;
-    for (int k = threadIdx.x; k < R.nk; k += 256) {
-        double2 v = rb[k];
-        t += R.coef_s[k] * (v.x * v.x + v.y * v.y);
+    double* to = nullptr;
+    if (blk < n_links) {
+        const int s0 = (b0 + blk) % M, s1 = s0 + 1 == M ? 0 : s0 + 1;
+        double a0[3], a1[3];
+        for (int d = 0; d < 3; ++d) {
+            a0[d] = mode ? pos_new(R, pr, d, s0) : pos_at(R, d, s0, p);
+            a1[d] = mode ? pos_new(R, pr, d, s1) : pos_at(R, d, s1, p);
+        }
+        for (int q = tid; q < N; q += kIfaceBlock) {
+            if (q == p) continue;
+            double c0[3], c1[3];
+            for (int d = 0; d < 3; ++d) {
+                c0[d] = pos_at(R, d, s0, q);
+                c1[d] = pos_at(R, d, s1, q);
+            }
+            LinkGeom g;
+            link_geom(a0, c0, a1, c1, R.L, R.iL, g);
+            t += pair_u(R, g.r, g.rp, g.s);
+        }
+        to = &R.pair_part[blk].x;
+    } else if (blk < n_links + n_update) {
+        const int m = blk - n_links, s = (pr.first + m) % M, stride = R.max_idx + 1;
+        int w = s - b0 % M;
+        if (w < 0) w += M;
+        const int cur = R.sel[s];
+        const double2* rc = R.rho + ((size_t)cur * M + s) * R.nk;
+        double2* rn = R.rho + ((size_t)(1 - cur) * M + s) * R.nk;
+        if (tid < 6) {
+            const int d = tid % 3;
+            phase_chain((tid >= 3 ? R.prop_new[3 * m + d] : pos_at(R, d, s, p)) * R.box, R.max_idx, tab + tid * stride);
+        }
+        __syncthreads();
+        for (int k = tid; k < R.nk; k += kIfaceBlock) {
+            const double2 v = ld2<false>(rc + k);
+            const int kp = gld(R.kidx + k);
+            const double2 en = phase_k(&tab[3 * stride], stride, kp), eo = phase_k(tab, stride, kp);
+            double2 nv;
+            nv.x = v.x + (en.x - eo.x);
+            nv.y = v.y + (en.y - eo.y);
+            rn[k] = nv;
+            t += gld(R.coef_s + k) * (nv.x * nv.x + nv.y * nv.y);
+        }
+        if (w < n_long) to = part + w;
+    } else {
+        const int w = blk - n_links - n_update, s = (b0 + w) % M;
+        int m = s - pr.first;
+        if (m < 0) m += M;
+        const bool moved = mode && m < pr.count;
+        if (!(moved && n_update)) {  // (else its update's workgroup has the sum)
+            const int buf = moved && rho_updated ? 1 - R.sel[s] : R.sel[s];
+            const double2* rb = R.rho + ((size_t)buf * M + s) * R.nk;
+            for (int k = tid; k < R.nk; k += kIfaceBlock) {
+                const double2 v = ld2<false>(rb + k);
+                t += gld(R.coef_s + k) * (v.x * v.x + v.y * v.y);
+            }
+            to = part + w;
+        }
     }
-    __shared__ double sh[4];
-    t = block_sum<256>(t, sh);
-    if (threadIdx.x == 0) part[w] = t;
+    t = block_sum<kIfaceBlock>(t, sh);
+    if (tid == 0) {
+        if (to) __hip_atomic_store(to, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_waitcnt(0);  // the term is performed before the workgroup arrives
+        s_last = atomicAdd(arrive, 1u) + 1u == gridDim.x;
+    }
+    __syncthreads();
+    if (!s_last || tid >= kWave) return;
+    double a = 0., l = 0.;
+    for (int j = tid; j < n_links; j += kWave)
+        a += __hip_atomic_load(&R.pair_part[j].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int j = tid; j < n_long; j += kWave) l += __hip_atomic_load(part + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    a = wave_sum(a);
+    l = wave_sum(l);
+    if (tid == 0) {
+        __hip_atomic_store(arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        host_result(out, a + R.long_scale * l);
+    }
 }
 
-// Work items of an interface query: (r, t) for the pair kernel's links
-// (n_chunks == 0), or (r, moved bead << 8 | k chunk) for the rho_k kernel.
-__global__ __launch_bounds__(256) void k_iface_items(uint2* __restrict__ items, int r, int n, int n_chunks) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n) return;
-    items[t] = make_uint2((unsigned)r, n_chunks ? (unsigned)(((t / n_chunks) << 8) | (t % n_chunks)) : (unsigned)t);
-}
-
-// Sums a pair action query: links (mode column) + long-range window partials.
 // PairAction::GetActionLaplacian (pair_action_class.h:336-363) of particle p at
 // level 0: for the window beads b0 <= b < b1, the links (b, b + 1) and
 // (b, b - 1 + M) with every other particle, each through CalcLaplacianU
@@ -1636,10 +1627,9 @@ __global__ __launch_bounds__(256) void k_iface_items(uint2* __restrict__ items, 
 // reference.  NEW mode reads the pending interface proposal's beads.  One
 // workgroup; the thread sums are added in thread order.
 constexpr int kLapBlock = 256;
-__global__ __launch_bounds__(kLapBlock) void k_pair_laplacian(const Rep* __restrict__ reps, int r, int mode, int b0,
-                                                              int b1, int p, double* __restrict__ out) {
+__global__ __launch_bounds__(kLapBlock) void k_pair_laplacian(const Rep* __restrict__ reps, int r, Prop pr, int mode,
+                                                              int b0, int b1, int p, double* __restrict__ out) {
     const Rep& R = reps[r];
-    const Prop pr = *R.prop;
     const int M = R.M, N = R.N, nb = b1 - b0;
     const double eps = 1.e-4;
     __shared__ double red[kLapBlock / kWave];
@@ -1683,25 +1673,13 @@ __global__ __launch_bounds__(kLapBlock) void k_pair_laplacian(const Rep* __restr
     if (threadIdx.x == 0) {
         double t = 0.;
         for (int w = 0; w < kLapBlock / kWave; ++w) t += red[w];
-        *out = t;
+        host_result(out, t);
     }
 }
 
-__global__ void k_action_sum(const Rep* __restrict__ reps, int r, int mode, int n_links, int n_long,
-                             const double* __restrict__ long_part, double* __restrict__ out) {
-    const Rep& R = reps[r];
-    double s = 0., l = 0.;
-    for (int j = threadIdx.x; j < n_links; j += kWave) s += mode ? R.pair_part[j].y : R.pair_part[j].x;
-    for (int j = threadIdx.x; j < n_long; j += kWave) l += long_part[j];
-    s = wave_sum(s);
-    l = wave_sum(l);
-    if (threadIdx.x == 0) *out = s + R.long_scale * l;
-}
-
 // Move::Accept / Reject of an interface proposal.
-__global__ void k_commit(const Rep* __restrict__ reps, int r, int accept, int rho_updated) {
+__global__ void k_commit(const Rep* __restrict__ reps, int r, Prop pr, int accept, int rho_updated) {
     const Rep& R = reps[r];
-    const Prop pr = *R.prop;
     if (accept)
         for (int m = threadIdx.x; m < pr.count; m += blockDim.x) {
             const int s = (pr.first + m) % R.M;
