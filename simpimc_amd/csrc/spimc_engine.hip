@@ -1417,8 +1417,12 @@ int launch_pair_multi(spimc_ctx* c, const Group& G, hipStream_t st) {
 // A permuting bisection round.  One-chain proposals (most of them) run on the
 // Boltzmann bisection's kernels: the LDS pair kernel and the rho_k items;
 // several chains, or a chain whose label changes inside the window, on the
-// label-general pair kernel and k_rho_multi.  rho_k runs beside the pair
-// kernels on the group's second stream.
+// label-general pair kernel and k_rho_multi.  Large rounds run rho_k beside the
+// pair kernels on the group's second stream, small ones both list kernels in one
+// launch.
+// From this much rho_k traffic a round (15 us at the copy rate) it is worth the
+// second stream's events (12 us), with the label-general pair kernel to hide it behind.
+constexpr double kPermForkBytes = 64e6;
 int launch_perm_round(spimc_ctx* c, const Group& G) {
     const int R = G.n;
     Rep* reps = c->d_reps + G.r0;
@@ -1435,39 +1439,56 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
                     c->perm_stage, c->max_N, 0);
     }
     if (rc) return rc;
-    const bool fork = c->any_long && G.side;
+    int max_chunks = 1, max_slots = 1, max_links = 1;
+    double bytes = 0.;
+    // a table of two or more particles proposes two or more chains: nothing for the one-chain kernels
+    bool single = !c->perm_table;
+    for (int r = G.r0; r < G.r0 + G.n; ++r) {
+        const Rep& x = c->reps[r].dev;
+        max_chunks = std::max(max_chunks, x.n_chunks);
+        max_links = std::max(max_links, 1 << x.perm_n_level);
+        bytes += 32. * x.nk * ((1 << x.perm_n_level) - 1);
+        single = single || x.tab_k == 1;
+    }
+    max_slots = max_links - 1;
+    // as many pair workgroups as a full grid: a listed item each, the others return at once
+    const int n_pair = R * kPairMultiBpr, n_rho = 4 * kNumCUs;
+    const int* pair_list = reinterpret_cast<const int*>(G.d_multi + 2);
+    const int* rho_list = pair_list + G.n;
+    const unsigned int* cnt = G.d_multi;
+    const bool fork = c->any_long && G.side && bytes >= kPermForkBytes;
     hipStream_t rst = fork ? G.side : st;
     if (fork) {
         HIPCHK(hipEventRecord(G.ev_fork, st));
         HIPCHK(hipStreamWaitEvent(G.side, G.ev_fork, 0));
     }
-    if (c->any_long) {
-        if (G.n_ritem_bis && (rc = launch_rho(c, rst, G.d_ritem_bis, G.n_ritem_bis, c->fork, nullptr))) return rc;
-        int max_chunks = 1, max_slots = 1;
-        for (int r = G.r0; r < G.r0 + G.n; ++r) {
-            max_chunks = std::max(max_chunks, c->reps[r].dev.n_chunks);
-            max_slots = std::max(max_slots, (1 << c->reps[r].dev.perm_n_level) - 1);
-        }
+    if (c->any_long && single && G.n_ritem_bis &&
+        (rc = launch_rho(c, rst, G.d_ritem_bis, G.n_ritem_bis, fork && c->fork, nullptr)))
+        return rc;
+    if (fork) {
         // a fixed grid over the listed proposals' (replica, slot, chunk) items
         auto fn = c->rho_kpt == 2    ? k_rho_multi_list<2>
                   : c->rho_kpt == 4  ? k_rho_multi_list<4>
                   : c->rho_kpt == 16 ? k_rho_multi_list<16>
                                      : k_rho_multi_list<8>;
-        const int* list = reinterpret_cast<const int*>(G.d_multi + 2) + G.n;
-        if ((rc = launch(c, SPIMC_KERNEL_RHO, fn, 4 * kNumCUs, kRhoBlock, 0, rst, reps, list, G.d_multi, max_slots,
-                         max_chunks)))
+        if ((rc = launch(c, SPIMC_KERNEL_RHO, fn, n_rho, kRhoBlock, 0, rst, reps, rho_list, cnt, max_slots, max_chunks)))
+            return rc;
+        HIPCHK(hipEventRecord(G.ev_join, G.side));
+    }
+    if (tuned && single && (rc = launch_pair_lds(c, st, reps, R, max_links, fork && c->fork, nullptr))) return rc;
+    if (fork || !c->any_long) {
+        if ((rc = launch(c, SPIMC_KERNEL_PAIR, k_pair_multi_list, n_pair, kPairMultiBlock, 0, st, reps, pair_list, cnt,
+                         kPairMultiBpr)))
+            return rc;
+    } else {
+        auto fn = c->rho_kpt == 2    ? k_multi_lists<2>
+                  : c->rho_kpt == 4  ? k_multi_lists<4>
+                  : c->rho_kpt == 16 ? k_multi_lists<16>
+                                     : k_multi_lists<8>;
+        if ((rc = launch(c, SPIMC_KERNEL_PAIR, fn, n_pair + n_rho, kRhoBlock, 0, st, reps, pair_list, rho_list, cnt, n_pair,
+                         kPairMultiBpr, max_slots, max_chunks)))
             return rc;
     }
-    if (fork) HIPCHK(hipEventRecord(G.ev_join, G.side));
-    if (tuned) {
-        int max_links = 1;
-        for (int r = G.r0; r < G.r0 + G.n; ++r) max_links = std::max(max_links, 1 << c->reps[r].dev.perm_n_level);
-        if ((rc = launch_pair_lds(c, st, reps, R, max_links, c->fork, nullptr))) return rc;
-    }
-    // as many workgroups as a full grid: a listed item each, the others return at once
-    if ((rc = launch(c, SPIMC_KERNEL_PAIR, k_pair_multi_list, R * kPairMultiBpr, kPairMultiBlock, 0, st, reps,
-                     reinterpret_cast<const int*>(G.d_multi + 2), (const unsigned int*)G.d_multi, kPairMultiBpr)))
-        return rc;
     if (fork) HIPCHK(hipStreamWaitEvent(st, G.ev_join, 0));
     return launch(c, SPIMC_KERNEL_DECIDE, k_decide_perm, R, 64, 0, st, reps, R, G.d_multi);
 }
@@ -2769,13 +2790,14 @@ int spimc_perm_download(spimc_ctx* c, uint32_t r, uint32_t* sigma) {
     if (rc) return rc;
     if (!sigma) return fail(SPIMC_ERR_ARG, "null argument");
     const Rep& R = c->reps[r].dev;
-    HIPCHK(hipDeviceSynchronize());
     if (!R.perm) {
+        HIPCHK(hipStreamSynchronize(c->stream));
         for (int p = 0; p < R.N; ++p) sigma[p] = (uint32_t)p;
         return SPIMC_OK;
     }
-    std::vector<int> v(R.N);
-    HIPCHK(hipMemcpy(v.data(), R.perm, R.N * sizeof(int), hipMemcpyDeviceToHost));
+    // (an odd N's last word ends in the inverse, which follows)
+    std::vector<int> v(R.N + 1);
+    if ((rc = read_words(c, R.perm, (R.N + 1) / 2, v.data(), nullptr, 0, nullptr))) return rc;
     for (int p = 0; p < R.N; ++p) sigma[p] = (uint32_t)v[p];
     return SPIMC_OK;
 }

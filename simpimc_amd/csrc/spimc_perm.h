@@ -1238,6 +1238,29 @@ __global__ __launch_bounds__(kRhoBlock) void k_rho_multi_list(const Rep* __restr
     }
 }
 
+// Both lists in one launch, for rounds too small to fork: the first n_pair
+// workgroups loop over the pair items, the others over the rho_k items, side by
+// side (16 replicas of N = 32 with the cycle table: a round 112 us on two streams with
+// the one-chain kernels, 96 us so).
+template <int KPT>
+__global__ __launch_bounds__(kRhoBlock) void k_multi_lists(const Rep* __restrict__ reps, const int* __restrict__ pair_list,
+                                                           const int* __restrict__ rho_list,
+                                                           const unsigned int* __restrict__ cnt, int n_pair, int bpr,
+                                                           int slots, int chunks) {
+    static_assert(kRhoBlock == kPairMultiBlock, "one workgroup size");
+    const int blk = blockIdx.x;
+    if (blk < n_pair) {
+        const int n = (int)cnt[0] * bpr;
+        for (int it = blk; it < n; it += n_pair) pair_multi_item(reps, pair_list[it / bpr], it % bpr, bpr);
+    } else {
+        const int per = slots * chunks, n = (int)cnt[1] * per;
+        for (int it = blk - n_pair; it < n; it += (int)gridDim.x - n_pair) {
+            const int q = it % per;
+            rho_multi_item<KPT>(reps, rho_list[it / per], q / chunks, q % chunks);
+        }
+    }
+}
+
 // k_decide for a permuting round, which also empties the group's lists for the
 // next round
 __global__ __launch_bounds__(64) void k_decide_perm(const Rep* __restrict__ reps, int n_reps,
