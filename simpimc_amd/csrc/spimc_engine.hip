@@ -1066,6 +1066,12 @@ int upload_items(const std::vector<uint2>& v, uint2** d, int* n) {
     return SPIMC_OK;
 }
 
+// LDS of k_round beside its static arrays: the tables, or with tables left in
+// global memory room for their axes (more than that is searched where it is).
+size_t round_shmem(const spimc_ctx* c) {
+    return (size_t)(c->lds_doubles_max > 0 ? c->lds_doubles_max : kAxDoubles) * sizeof(double);
+}
+
 int build_work_lists(spimc_ctx* c, Group& G) {
     std::vector<uint2> pb, pd;
     int nb_items = 0, nd_items = 0;
@@ -1106,7 +1112,7 @@ int build_work_lists(spimc_ctx* c, Group& G) {
         G.rho_bytes[0] += 32. * R.nk * ((1 << R.n_level) - 1);
         G.rho_bytes[1] += 32. * R.nk * R.M;
     }
-    if (c->round_fn[0] && c->lds_doubles_max > 0) {
+    if (c->round_fn[0]) {
         // one-launch rounds, per move: pair workgroups per replica (fewer links
         // each when a replica of more than 256 particles splits its links'
         // partners), and as many rho_k items per workgroup as keep the launch
@@ -1119,14 +1125,14 @@ int build_work_lists(spimc_ctx* c, Group& G) {
             const int links = mv == 0 ? G.max_bis_links : G.max_M, n_items = mv == 0 ? ob : od;
             int occ = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)c->round_fn[mv], kRoundBlock,
-                                                             (size_t)c->lds_doubles_max * sizeof(double)) != hipSuccess)
+                                                             round_shmem(c)) != hipSuccess)
                 occ = 1;
             const int cap = std::max(1, occ) * kNumCUs;
             // a link's partners over as many wavefronts as still let every rho_k item
             // have a workgroup of its own (N = 256, M = 128, one
             // replica: 22 us a bisection round with 64 partners each, 26 us with 256)
             for (int qpw : {64, 128, 256}) {
-                const int lpb = waves / pair_split<waves>(max_N, qpw);
+                const int lpb = waves / (c->lds_doubles_max > 0 ? pair_split<waves>(max_N, qpw) : general_split<waves>(max_N, qpw));
                 G.round_qpw[mv] = qpw;
                 G.round_bpr[mv] = std::max(1, std::min((links + lpb - 1) / lpb, (2 * kNumCUs + G.n - 1) / G.n));
                 if (G.n * G.round_bpr[mv] + n_items <= cap) break;
@@ -1298,27 +1304,30 @@ bool pers_eligible(const spimc_ctx* c) {
     return pers_shmem(c) <= kPersLdsBytes;
 }
 
-// One-launch rounds: the LDS pair kernel, the default rho_k chunking, rounds
-// decided in the next proposal's launch, and unpermuted paths.
+// One-launch rounds: the default rho_k chunking, rounds decided in the next
+// proposal's launch, and unpermuted paths.
 bool one_launch_eligible(const spimc_ctx* c) {
-    return c->round_fn[0] && c->round_fn[1] && c->lds_doubles_max > 0 && c->fuse_rounds && !c->perm_on &&
+    return c->round_fn[0] && c->round_fn[1] && c->fuse_rounds && !c->perm_on &&
            c->rho_kpt == kRhoKpt;
 }
 // Whether a stage of this move runs one-launch rounds; not while the device clocks
 // or events time the pair and rho_k kernels (k_round has no separate rho_k kernel
 // to time, so those rounds run as three launches).  By rule: where a rho_k
 // workgroup takes at most two items for the launch to fit what the GPU holds at
-// once, four with tables of more than 48 KB (which three launches stage too).  A
+// once, four with tables of more than 48 KB (which three launches stage too) and
+// with tables in global memory (searched by one wavefront a link there).  A
 // round then, against three launches: N = 32, M = 32, bisection of 1 replica 16
 // and 23 us, of 128 (two items) 22 and 28, of 256 (four) 50 and 33; N = 256,
 // M = 128 with the 96 KB table, bisection of 16 (two items) 27 and 47 us, of 32
 // (four) 30 and 38, of 64 (eight) 84 and 46; displacement of 4 (four) 39 and 38,
-// of 8 (eight) 82 and 45.
+// of 8 (eight) 82 and 45; tabulated Ilkka actions, N = 33, M = 32: bisection of 256
+// (four) 36 and 43, displacement of 64 (four) 35 and 41; N = 200, M = 64,
+// displacement of 16 (four) 53 and 67, of 64 (sixteen) 165 and 124.
 bool one_launch_now(const spimc_ctx* c, int move) {
     if (c->clock || !one_launch_eligible(c)) return false;
     if (!c->auto_one) return c->one_launch && move < c->one_moves;
     if (c->timing) return false;
-    const int most = (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024 ? 4 : 2;
+    const int most = c->lds_doubles_max == 0 || (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024 ? 4 : 2;
     return move < 2 && c->groups[0].round_ipb[move] <= most;
 }
 
@@ -1500,7 +1509,7 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
 // rest; measured slower.)
 int launch_one_round(spimc_ctx* c, const Group& G, int move) {
     const int R = G.n;
-    const size_t shmem = (size_t)c->lds_doubles_max * sizeof(double);
+    const size_t shmem = round_shmem(c);
     return launch(c, SPIMC_KERNEL_PAIR, c->round_fn[move], R * G.round_bpr[move] + G.n_rgrp[move], kRoundBlock, shmem,
                   G.stream, c->d_reps + G.r0, R, G.round_bpr[move], G.round_qpw[move],
                   (const RhoItem*)(move == 0 ? G.d_ritem_bis : G.d_ritem_dis), (const int4*)G.d_rgrp[move],
@@ -2193,21 +2202,20 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
             // one-launch rounds (SPIMC_ONE_LAUNCH or spimc_autotune): the pair type's
             // instantiation with the default rho_k chunking
             using RoundFn = void (*)(const Rep*, int, int, int, const RhoItem*, const int4*, int, unsigned int*);
-            const RoundFn rf[2][2][4] = {
+            const RoundFn rf[2][2][5] = {
                 {{k_round<1, 0, kRhoKpt, false, 0>, k_round<2, 2, kRhoKpt, false, 0>, k_round<2, 0, kRhoKpt, false, 0>,
-                  k_round<0, 0, kRhoKpt, false, 0>},
+                  k_round<0, 0, kRhoKpt, false, 0>, k_round<3, kAxDoubles, kRhoKpt, false, 0>},
                  {k_round<1, 0, kRhoKpt, true, 0>, k_round<2, 2, kRhoKpt, true, 0>, k_round<2, 0, kRhoKpt, true, 0>,
-                  k_round<0, 0, kRhoKpt, true, 0>}},
+                  k_round<0, 0, kRhoKpt, true, 0>, k_round<3, kAxDoubles, kRhoKpt, true, 0>}},
                 {{k_round<1, 0, kRhoKpt, false, 1>, k_round<2, 2, kRhoKpt, false, 1>, k_round<2, 0, kRhoKpt, false, 1>,
-                  k_round<0, 0, kRhoKpt, false, 1>},
+                  k_round<0, 0, kRhoKpt, false, 1>, k_round<3, kAxDoubles, kRhoKpt, false, 1>},
                  {k_round<1, 0, kRhoKpt, true, 1>, k_round<2, 2, kRhoKpt, true, 1>, k_round<2, 0, kRhoKpt, true, 1>,
-                  k_round<0, 0, kRhoKpt, true, 1>}}};
-            for (int mv = 0; mv < 2; ++mv) c->round_fn[mv] = rf[mv][c->rho_nt ? 1 : 0][vi];
-            if (c->lds_doubles_max > 0)
-                for (int mv = 0; mv < 2; ++mv)
-                    if (hipFuncSetAttribute((const void*)c->round_fn[mv], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            c->lds_doubles_max * (int)sizeof(double)) != hipSuccess)
-                        c->round_fn[0] = c->round_fn[1] = nullptr;
+                  k_round<0, 0, kRhoKpt, true, 1>, k_round<3, kAxDoubles, kRhoKpt, true, 1>}}};
+            for (int mv = 0; mv < 2; ++mv) c->round_fn[mv] = rf[mv][c->rho_nt ? 1 : 0][c->lds_doubles_max > 0 ? vi : 4];
+            for (int mv = 0; mv < 2; ++mv)
+                if (hipFuncSetAttribute((const void*)c->round_fn[mv], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)round_shmem(c)) != hipSuccess)
+                    c->round_fn[0] = c->round_fn[1] = nullptr;
             if (const char* fo = std::getenv("SPIMC_ONE_LAUNCH")) {
                 c->auto_one = false;
                 c->one_launch = std::atoi(fo) != 0;

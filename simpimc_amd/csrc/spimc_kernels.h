@@ -801,6 +801,78 @@ __device__ __forceinline__ void pair_links_split(const Rep& R, const double* lds
     }
 }
 
+// The window links of a proposal from the tables in global memory (tabulated
+// Ilkka actions and grids that are not uniform), as pair_links_split: a link's
+// OLD and NEW sums are wavefronts of their own (each is a serial chain of a
+// grid search and loads that depend on it, which a small batch waits for in
+// full), and so are its partner ranges.  An Ilkka table's axes are searched in
+// LDS where the launch has room for them (ax_doubles values).  A range's sum is
+// the one that k_pair forms over the same partners.  A bisection round of 24
+// replicas of N = 33, M = 32: 31.6 us in three launches with k_pair, 20.6 so; of
+// one replica of N = 200, M = 64: 62.7 and 24.0.
+template <int W>
+__host__ __device__ __forceinline__ int general_split(int N, int qpw) {
+    return 2 * pair_split<W / 2>(N, qpw);
+}
+constexpr int kAxDoubles = 1024;
+template <bool COH, int W>
+__device__ __forceinline__ void pair_links_general(const Rep& R, double* lds, int ax_doubles, const Prop& pr, int part,
+                                                   int bpr, int qpw, int w, int lane, double2* wpart) {
+    const int ns = general_split<W>(R.N, qpw), lpb = W / ns, nq = ns / 2;
+    const int q_len = ((R.N + nq - 1) / nq + kWave - 1) / kWave * kWave;
+    const bool axes = R.pair_type == 3 && R.u2.nx + R.u2.ny <= ax_doubles;
+    if (axes) {
+        for (int t = threadIdx.x; t < R.u2.nx; t += W * kWave) lds[t] = R.u2.x[t];
+        for (int t = threadIdx.x; t < R.u2.ny; t += W * kWave) lds[R.u2.nx + t] = R.u2.y[t];
+        __syncthreads();
+    }
+    Spl2 T = R.u2;
+    T.x = lds;
+    T.y = lds + R.u2.nx;
+    const int M = R.M, p = pr.p;
+    for (int jb = part * lpb; jb < pr.n_links; jb += bpr * lpb) {
+        const int j = jb + w / ns, k = w % ns;
+        double u = 0.;
+        if (w < lpb * ns && j < pr.n_links) {
+            const int s0 = (pr.b0 + j) % M, s1 = (s0 + 1) % M, q_lo = (k >> 1) * q_len, q_hi = min(R.N, q_lo + q_len);
+            double p0[3], p1[3];
+            for (int d = 0; d < 3; ++d) {
+                p0[d] = (k & 1) ? pos_new(R, pr, d, s0) : pos_at(R, d, s0, p);
+                p1[d] = (k & 1) ? pos_new(R, pr, d, s1) : pos_at(R, d, s1, p);
+            }
+            for (int q = q_lo + lane; q < q_hi; q += kWave) {
+                if (q == p) continue;
+                double q0[3], q1[3];
+                for (int d = 0; d < 3; ++d) {
+                    q0[d] = pos_at(R, d, s0, q);
+                    q1[d] = pos_at(R, d, s1, q);
+                }
+                LinkGeom g;
+                link_geom(p0, q0, p1, q1, R.L, R.iL, g);
+                u += axes ? ilkka_u(R, T, R.u_long_r, R.r_u_min, R.r_u_max, g.r, g.rp, g.s)
+                          : pair_u(R, g.r, g.rp, g.s);
+            }
+            u = wave_sum(u);
+        }
+        double* part_u = reinterpret_cast<double*>(wpart);
+        if (lane == 0) part_u[w] = u;
+        __syncthreads();
+        if ((int)threadIdx.x < lpb && jb + (int)threadIdx.x < pr.n_links) {
+            const double* f = part_u + threadIdx.x * ns;
+            double so = f[0], sn = f[1];
+            for (int kk = 2; kk < ns; kk += 2) {
+                so += f[kk];
+                sn += f[kk + 1];
+            }
+            if (COH)
+                coh_store2(R.pair_part + jb + threadIdx.x, make_double2(so, sn));
+            else
+                R.pair_part[jb + threadIdx.x] = make_double2(so, sn);
+        }
+        __syncthreads();
+    }
+}
+
 // Copies values [t_lo, n) of the tables a | b (a holds the first na) into lds
 // with nthr threads, 16 values per thread at a time, every load issued before
 // the stores that wait on it (a large table then costs a few load latencies
@@ -1294,6 +1366,7 @@ __global__ __launch_bounds__(kDisBlock) void k_decide_propose_displace(const Rep
 // chains are the same bit for bit.  The last workgroup resets the counter for
 // the next round.
 constexpr int kRoundBlock = kRhoBlock;
+// PT 3: the tables stay in global memory, NORD the doubles of LDS for their axes.
 template <int PT, int NORD, int KPT, bool NT, int MOVE>
 __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ reps, int n_reps, int bpr, int qpw,
                                                        const RhoItem* __restrict__ items,
@@ -1311,26 +1384,33 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
         r = idx / bpr;
         const int part = idx % bpr;
         const Rep R = reps[r];
-        // the tables' first kRoundBlock * 4 values are loaded while the proposal is
-        const int na = R.bt_a.ncoef * R.bt_a.ncomp, nd = R.lds_doubles;
-        double tv[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int t = threadIdx.x + k * kRoundBlock;
-            tv[k] = t < nd ? (t < na ? R.bt_a.c[t] : R.bt_b.c[t - na]) : 0.;
-        }
-        const Prop pr = *R.prop;
-        constexpr int W = kRoundBlock / kWave;
-        if (pr.status == 1 && !pr.generic && part * (W / pair_split<W>(R.N, qpw)) < pr.n_links) {
+        if constexpr (PT == 3) {
+            constexpr int W = kRoundBlock / kWave;
+            const Prop pr = *R.prop;
+            if (pr.status == 1 && !pr.generic && part * (W / general_split<W>(R.N, qpw)) < pr.n_links)
+                pair_links_general<true, W>(R, lds, NORD, pr, part, bpr, qpw, w, lane, wpart);
+        } else {
+            // the tables' first kRoundBlock * 4 values are loaded while the proposal is
+            const int na = R.bt_a.ncoef * R.bt_a.ncomp, nd = R.lds_doubles;
+            double tv[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const int t = threadIdx.x + k * kRoundBlock;
-                if (t < nd) lds[t] = tv[k];
+                tv[k] = t < nd ? (t < na ? R.bt_a.c[t] : R.bt_b.c[t - na]) : 0.;
             }
-            // the rest (large tables: 96 KB for David's)
-            stage_batched(lds, R.bt_a.c, R.bt_b.c, na, nd, 4 * kRoundBlock, kRoundBlock);
-            __syncthreads();
-            pair_links_split<PT, NORD, true, W>(R, lds, pr, part, bpr, qpw, w, lane, wpart);
+            const Prop pr = *R.prop;
+            constexpr int W = kRoundBlock / kWave;
+            if (pr.status == 1 && !pr.generic && part * (W / pair_split<W>(R.N, qpw)) < pr.n_links) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int t = threadIdx.x + k * kRoundBlock;
+                    if (t < nd) lds[t] = tv[k];
+                }
+                // the rest (large tables: 96 KB for David's)
+                stage_batched(lds, R.bt_a.c, R.bt_b.c, na, nd, 4 * kRoundBlock, kRoundBlock);
+                __syncthreads();
+                pair_links_split<PT, NORD, true, W>(R, lds, pr, part, bpr, qpw, w, lane, wpart);
+            }
         }
     } else {
         // a group of up to ipb rho_k items of one replica, one after the other
