@@ -72,7 +72,8 @@ struct Prop {
     double prev;  // action change of the previous (coarser) level
     double u0;    // level-0 uniform
     int p2;       // label of the moved chain after the wrap (bisect; else p)
-    int generic;  // 1: the label-general pair kernel evaluates this proposal
+    short generic;  // 1: the label-general pair kernel evaluates this proposal
+    short buf;    // NEW positions and phases: 0 in prop_new and phase, 1 / 2 in a set made ahead (k_round)
     long long tape_next;  // tape cursor after this attempt
     int n_chain;  // chains of a permuting bisection (0: the cycle walk stopped)
     int e_slice;  // slice after which a permuting bisection relinks the chains
@@ -83,6 +84,16 @@ struct Prop {
     int tab_on;
     double tab_ratio;
     double u_tab;
+};
+// (a batch that streams rho_k finds these in HBM: at 136 bytes
+// k_decide_propose_bisect took 28 us for 512 replicas, at 128 it took 18)
+static_assert(sizeof(Prop) == 128, "one cache line");
+
+// A proposal made ahead, passed between workgroups in 8-byte words.
+struct NextProp {
+    Prop pr;
+    unsigned long long seq;  // its attempt's sequence number
+    unsigned long long has;  // 0: no attempt was left
 };
 
 struct Counters {
@@ -164,6 +175,12 @@ struct Rep {
     int2* rho_rows;        // [M] (slice, committed buffer) of each moved bead, written with the proposal
     Prop* prop;
     double* prop_new;      // [M][3] NEW positions of the moved slices
+    // a bisection made ahead of the decision before it (k_round): two sets of NEW
+    // positions [2^n_level - 1][3] and phases [2^n_level - 1][2][3][max_idx+1], and
+    // the proposal itself
+    double* next_new[2];
+    double2* next_phase[2];
+    NextProp* next;
     double2* pair_part;    // [n_links_max] (old, new)
     double2* rho_part;     // [M][n_chunks] (old, new)
     double2* kin_part;     // interface kinetic (old, new)

@@ -384,6 +384,7 @@ struct Group {
     int round_bpr[2] = {1, 1}, round_ipb[2] = {1, 1}, n_rgrp[2] = {0, 0};  // per move
     double rho_bytes[2] = {0., 0.};  // rho_k read and written by a round, per move
     int4* d_rgrp[2] = {nullptr, nullptr};
+    unsigned char* d_next = nullptr;  // k_round's proposals made ahead
     unsigned int* d_arrive = nullptr;
 };
 
@@ -1127,10 +1128,10 @@ int build_work_lists(spimc_ctx* c, Group& G) {
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)c->round_fn[mv], kRoundBlock,
                                                              round_shmem(c)) != hipSuccess)
                 occ = 1;
-            const int cap = std::max(1, occ) * kNumCUs;
+            // (a bisection's launch holds one more workgroup per replica, for its next proposal)
+            const int held = std::max(1, occ) * kNumCUs, cap = std::max(held / 2, held - (mv == 0 ? G.n : 0));
             // a link's partners over as many wavefronts as still let every rho_k item
-            // have a workgroup of its own (N = 256, M = 128, one
-            // replica: 22 us a bisection round with 64 partners each, 26 us with 256)
+            // have a workgroup of its own
             for (int qpw : {64, 128, 256}) {
                 const int lpb = waves / (c->lds_doubles_max > 0 ? pair_split<waves>(max_N, qpw) : general_split<waves>(max_N, qpw));
                 G.round_qpw[mv] = qpw;
@@ -1157,6 +1158,29 @@ int build_work_lists(spimc_ctx* c, Group& G) {
                 HIPCHK(hipMalloc((void**)&G.d_rgrp[mv], grp.size() * sizeof(int4)));
                 HIPCHK(hipMemcpy(G.d_rgrp[mv], grp.data(), grp.size() * sizeof(int4), hipMemcpyHostToDevice));
             }
+        }
+    }
+    if (c->round_fn[0]) {
+        // the proposals made ahead: a replica's record, then its two sets of positions
+        // and phases
+        size_t bytes = 0;
+        const auto carve = [&](size_t n) {
+            unsigned char* p = G.d_next ? G.d_next + bytes : nullptr;
+            bytes += (n + 255) & ~(size_t)255;
+            return p;
+        };
+        for (int pass = 0; pass < 2; ++pass) {
+            bytes = 0;
+            for (int r = G.r0; r < G.r0 + G.n; ++r) {
+                Rep& R = c->reps[r].dev;
+                const size_t nm = ((size_t)1 << R.n_level) - 1;
+                R.next = (NextProp*)carve(sizeof(NextProp));
+                for (int i = 0; i < 2; ++i) {
+                    R.next_new[i] = (double*)carve(nm * 3 * sizeof(double));
+                    R.next_phase[i] = (double2*)carve(nm * 6 * (R.max_idx + 1) * sizeof(double2));
+                }
+            }
+            if (pass == 0) HIPCHK(hipMalloc((void**)&G.d_next, bytes));
         }
     }
     if (!G.d_arrive) {
@@ -1313,22 +1337,23 @@ bool one_launch_eligible(const spimc_ctx* c) {
 // Whether a stage of this move runs one-launch rounds; not while the device clocks
 // or events time the pair and rho_k kernels (k_round has no separate rho_k kernel
 // to time, so those rounds run as three launches).  By rule: where a rho_k
-// workgroup takes at most two items for the launch to fit what the GPU holds at
-// once, four with tables of more than 48 KB (which three launches stage too) and
-// with tables in global memory (searched by one wavefront a link there).  A
-// round then, against three launches: N = 32, M = 32, bisection of 1 replica 16
-// and 23 us, of 128 (two items) 22 and 28, of 256 (four) 50 and 33; N = 256,
-// M = 128 with the 96 KB table, bisection of 16 (two items) 27 and 47 us, of 32
-// (four) 30 and 38, of 64 (eight) 84 and 46; displacement of 4 (four) 39 and 38,
-// of 8 (eight) 82 and 45; tabulated Ilkka actions, N = 33, M = 32: bisection of 256
-// (four) 36 and 43, displacement of 64 (four) 35 and 41; N = 200, M = 64,
-// displacement of 16 (four) 53 and 67, of 64 (sixteen) 165 and 124.
+// workgroup takes at most three items (displacement: two) for the launch to fit
+// what the GPU holds at once; five and four with tables of more than 48 KB (which
+// three launches stage too) and with tables in global memory (searched by one
+// wavefront a link there).  A round then, against three launches: N = 32, M = 32,
+// bisection of 1 replica 12 and 22 us, of 128 (three items) 23 and 27, of 256
+// (seven) 61 and 33; displacement of 32 (two) 22 and 25, of 64 (six) 49 and 31;
+// N = 256, M = 128 with the 96 KB table, bisection of 1 replica 14.5 and 33, of 24
+// (four) 20.5 and 38, of 32 (five) 27 and 38, of 48 (seven) 58 and 42;
+// displacement of 4 (four) 32 and 38, of 8 (eight) 74 and 45; tabulated Ilkka
+// actions, N = 33, M = 32: bisection of 128 (three) 28 and 35, of 256 (seven) 61
+// and 43, displacement of 64 (four) 34 and 41.
 bool one_launch_now(const spimc_ctx* c, int move) {
     if (c->clock || !one_launch_eligible(c)) return false;
     if (!c->auto_one) return c->one_launch && move < c->one_moves;
     if (c->timing) return false;
-    const int most = c->lds_doubles_max == 0 || (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024 ? 4 : 2;
-    return move < 2 && c->groups[0].round_ipb[move] <= most;
+    const bool large = c->lds_doubles_max == 0 || (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024;
+    return move < 2 && c->groups[0].round_ipb[move] <= (move == 0 ? (large ? 5 : 3) : (large ? 4 : 2));
 }
 
 
@@ -1510,7 +1535,7 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
 int launch_one_round(spimc_ctx* c, const Group& G, int move) {
     const int R = G.n;
     const size_t shmem = round_shmem(c);
-    return launch(c, SPIMC_KERNEL_PAIR, c->round_fn[move], R * G.round_bpr[move] + G.n_rgrp[move], kRoundBlock, shmem,
+    return launch(c, SPIMC_KERNEL_PAIR, c->round_fn[move], (move == 0 ? R : 0) + R * G.round_bpr[move] + G.n_rgrp[move], kRoundBlock, shmem,
                   G.stream, c->d_reps + G.r0, R, G.round_bpr[move], G.round_qpw[move],
                   (const RhoItem*)(move == 0 ? G.d_ritem_bis : G.d_ritem_dis), (const int4*)G.d_rgrp[move],
                   G.round_ipb[move], G.d_arrive);
@@ -2321,7 +2346,7 @@ int spimc_ctx_destroy(spimc_ctx* c) {
             if (g) (void)hipGraphExecDestroy(g);
         for (void* p : {(void*)G.d_pair_bis, (void*)G.d_pair_dis, (void*)G.d_ritem_bis, (void*)G.d_ritem_dis, (void*)G.d_kt,
                         (void*)G.d_multi, (void*)G.d_rgrp[0], (void*)G.d_rgrp[1],
-                        (void*)G.d_arrive})
+                        (void*)G.d_arrive, (void*)G.d_next})
             if (p) (void)hipFree(p);
         if (G.done) (void)hipEventDestroy(G.done);
         if (G.side) {
@@ -2676,7 +2701,7 @@ int spimc_set_bisect_level(spimc_ctx* c, uint32_t r, uint32_t n_level) {
     for (auto& G : c->groups) {
         if ((int)r < G.r0 || (int)r >= G.r0 + G.n) continue;
         for (void** p : {(void**)&G.d_pair_bis, (void**)&G.d_pair_dis, (void**)&G.d_ritem_bis, (void**)&G.d_ritem_dis,
-                         (void**)&G.d_rgrp[0], (void**)&G.d_rgrp[1]})
+                         (void**)&G.d_rgrp[0], (void**)&G.d_rgrp[1], (void**)&G.d_next})
             if (*p) {
                 (void)hipFree(*p);
                 *p = nullptr;

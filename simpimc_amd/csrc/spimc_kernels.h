@@ -95,6 +95,12 @@ __device__ __forceinline__ double pos_at(const Rep& R, int d, int s, int p) {
     return gld(R.pos + ((size_t)d * R.M + s) * R.N + p);
 }
 
+// The NEW positions of a bisection or displacement; only k_round meets those
+// made ahead.
+__device__ __forceinline__ double* prop_beads(const Rep& R, const Prop& pr) {
+    return pr.buf == 0 ? R.prop_new : pr.buf == 1 ? R.next_new[0] : R.next_new[1];
+}
+
 // NEW-mode position of the proposal's particle at slice s
 __device__ __forceinline__ double pos_new(const Rep& R, const Prop& pr, int d, int s) {
     int m = s - pr.first;
@@ -126,7 +132,7 @@ __device__ __forceinline__ void moved_row(const Rep& R, int m, int s) { R.rho_ro
 // slice first + m).  Idle items (no attempt left, rejected at a coarse level,
 // fewer moved beads) are marked invalid.
 __device__ __forceinline__ void rho_items_write(const Rep& R, int move, int status, int count, int first, int lane,
-                                                int nthr = kWave) {
+                                                int nthr = kWave, const double2* phase = nullptr) {
     RhoItem* items = move == 0 ? R.ritems_bis : R.ritems_dis;
     const int n = move == 0 ? R.n_ritems_bis : R.n_ritems_dis;
     if (!items) return;
@@ -138,7 +144,7 @@ __device__ __forceinline__ void rho_items_write(const Rep& R, int move, int stat
             const int s = (first + m) % R.M, cur = R.sel[s];
             d.rc = R.rho + ((size_t)cur * R.M + s) * R.nk;
             d.rn = R.rho + ((size_t)(1 - cur) * R.M + s) * R.nk;
-            d.ph = R.phase + (size_t)m * 6 * stride;
+            d.ph = (phase ? phase : R.phase) + (size_t)m * 6 * stride;
             d.kidx = R.kidx;
             d.coef = R.coef_s;
             d.part = R.rho_part + m * nch + ch;
@@ -221,7 +227,8 @@ struct BisectLds {
     double x_new[(1 << kMaxLevel) + 1][3];
     double z[3 * ((1 << kMaxLevel) - 1) + 1];
     double u[kMaxLevel];
-    int info[4];  // an attempt is left, p, b0, bad draw
+    double sums[4][kMaxLevel];  // bisect_levels: sampling and kinetic sums, OLD then NEW
+    int info[6];  // an attempt is left, p, b0, bad draw; of bisect_levels: status, moved beads
     long long cur;
     unsigned long long seq;
 };
@@ -239,6 +246,21 @@ __device__ __forceinline__ void bisect_take(const Rep& R, BisectLds& S) {
     }
 }
 
+// The normals and level uniforms of attempt seq on the device RNG into S.
+__device__ __forceinline__ void bisect_draws(const Rep& R, int lane, BisectLds& S, unsigned long long seq) {
+    const int n = R.n_level, nb = 1 << n;
+    Rng rng{make_uint2((uint32_t)R.key, (uint32_t)(R.key >> 32)), 1u, seq};
+    // normal g is normal(1 + n + g / 2, g & 1): one call per pair of normals
+    const int n_norm = 3 * (nb - 1);
+    for (int q = lane; 2 * q < n_norm; q += kWave) {
+        double z0, z1;
+        rng.normal2(1 + n + q, &z0, &z1);
+        S.z[2 * q] = z0;
+        S.z[2 * q + 1] = z1;
+    }
+    for (int l = lane; l < n; l += kWave) S.u[l] = rng.unif(1 + l, 0);
+}
+
 // The window's beads of (p, b0) into S, and on the device RNG (draws) the
 // attempt's normals and level uniforms, made while the loads are in flight
 // (the window holds nb + 1 <= 65 beads: two per lane at most).
@@ -253,18 +275,7 @@ __device__ __forceinline__ void bisect_window(const Rep& R, int lane, BisectLds&
         const int lbl = (b0 + j >= M) ? p2 : p;
         for (int d = 0; d < 3; ++d) xw[k][d] = pos_at(R, d, s, lbl);
     }
-    if (draws) {
-        Rng rng{make_uint2((uint32_t)R.key, (uint32_t)(R.key >> 32)), 1u, S.seq};
-        // normal g is normal(1 + n + g / 2, g & 1): one call per pair of normals
-        const int n_norm = 3 * (nb - 1);
-        for (int q = lane; 2 * q < n_norm; q += kWave) {
-            double z0, z1;
-            rng.normal2(1 + n + q, &z0, &z1);
-            S.z[2 * q] = z0;
-            S.z[2 * q + 1] = z1;
-        }
-        for (int l = lane; l < n; l += kWave) S.u[l] = rng.unif(1 + l, 0);
-    }
+    if (draws) bisect_draws(R, lane, S, S.seq);
     for (int k = 0; k < 2; ++k) {
         const int j = lane + k * kWave;
         if (j > nb) break;
@@ -275,41 +286,154 @@ __device__ __forceinline__ void bisect_window(const Rep& R, int lane, BisectLds&
     }
 }
 
-// The start of an attempt on the device RNG, ahead of its proposal and by
-// another wavefront than the one that finishes it (k_round): the counter
-// step, particle and first bead, window, normals and level uniforms into S.
-// The finishing wavefront reloads the window if the decision before it
-// committed moves of the same particle.
-template <class Sync>
-__device__ __forceinline__ void bisect_start_ahead(const Rep& R, int lane, Sync sync, BisectLds& S) {
-    if (lane == 0) bisect_take(R, S);
-    sync();
-    if (!S.info[0]) return;
-    if (lane == 0) {
-        // rng.index(0, 0, N) and rng.index(0, 1, M) from one call
-        Rng rng{make_uint2((uint32_t)R.key, (uint32_t)(R.key >> 32)), 1u, S.seq};
-        const uint4 w = rng.call(0);
-        S.info[1] = (int)(((uint64_t)w.x * (uint32_t)R.N) >> 32);
-        S.info[2] = (int)(((uint64_t)w.y * (uint32_t)R.M) >> 32);
-        S.info[3] = 0;
-        S.cur = 0;
+// Particle and first bead of attempt seq on the device RNG: rng.index(0, 0, N) and
+// rng.index(0, 1, M) from one call.
+__device__ __forceinline__ void bisect_where(const Rep& R, unsigned long long seq, int* p, int* b0) {
+    Rng rng{make_uint2((uint32_t)R.key, (uint32_t)(R.key >> 32)), 1u, seq};
+    const uint4 w = rng.call(0);
+    *p = (int)(((uint64_t)w.x * (uint32_t)R.N) >> 32);
+    *b0 = (int)(((uint64_t)w.y * (uint32_t)R.M) >> 32);
+}
+
+// Bisect::Attempt of the attempt in S (info, window, draws) up to the level-0
+// decision, on the W wavefronts of a workgroup: the same numbers as
+// propose_bisect_impl, whose single wavefront walks levels of sums one after the
+// other.  Only the new midpoints depend on the level above them, so the first
+// wavefront lays all of them down while the others sum the OLD actions (levels in
+// turn); then every wavefront takes levels of the NEW sums; the levels' decisions
+// follow in order.  The proposal goes to pr, its beads and phase chains to the
+// buffers given; after the last barrier S.info holds its status and moved beads.
+template <int W>
+__device__ __forceinline__ void bisect_levels(const Rep& R, BisectLds& S, int w, int lane, Prop* pr, double* beads,
+                                              double2* phase, int buf) {
+    const int n = R.n_level, nb = 1 << n, M = R.M, p = S.info[1], b0 = S.info[2];
+    const int p2 = label_after_wrap(R, p);
+    // (see propose_bisect_impl)
+    const bool wraps = (nb % M) == 0 && p2 == p;
+    if (w == 0) {
+        int g = 3 * lane;
+        for (int level = n - 1; level >= 0; --level) {
+            const int skip = 1 << level, nmid = wraps ? 0 : nb >> (level + 1);
+            const double sigma = sqrt(R.lambda * (R.tau * skip));
+            if (lane < nmid) {
+#pragma clang fp contract(off)
+                const int a = 2 * lane * skip, b = a + skip, c = a + 2 * skip;
+                for (int d = 0; d < 3; ++d) {
+                    const double dn = minimg(sigma * S.z[g + d], R.L, R.iL);
+                    const double t = minimg(S.x_new[c][d] - S.x_new[a][d], R.L, R.iL);
+                    const double rbar = S.x_new[a][d] + 0.5 * t;
+                    S.x_new[b][d] = rbar + dn;
+                }
+            }
+            WaveSync{}();
+            g += 3 * nmid;
+        }
     }
-    sync();
-    const int p = S.info[1];
-    bisect_window(R, lane, S, p, label_after_wrap(R, p), S.info[2], true);
+    for (int half = 0; half < 2; ++half) {
+        // half 0: OLD, beside the midpoints; half 1: NEW
+        const double(*x)[3] = half ? S.x_new : S.x_old;
+        const int first = half ? w : w - 1, step = half ? W : W - 1;
+        for (int level = first < 0 ? n : first; level < n; level += step) {
+            const int skip = 1 << level, nmid = wraps ? 0 : nb >> (level + 1), nlinks = wraps ? 0 : nb >> level;
+            const double level_tau = R.tau * skip;
+            const double i4lt_b = 1. / (4. * R.lambda * (0.5 * R.tau * (double)skip));
+            double lsp = 0., k = 0.;
+            if (lane < nmid) {
+#pragma clang fp contract(off)
+                const int a = 2 * lane * skip, b = a + skip, c = a + 2 * skip;
+                double dd[3];
+                if (half) {
+                    const double sigma = sqrt(R.lambda * level_tau);
+                    // the levels above drew for 1 + 2 + ... + nmid / 2 midpoints
+                    const int g = 3 * (nmid - 1 + lane);
+                    for (int d = 0; d < 3; ++d) dd[d] = minimg(sigma * S.z[g + d], R.L, R.iL);
+                } else {
+                    for (int d = 0; d < 3; ++d) {
+                        const double t = minimg(x[c][d] - x[a][d], R.L, R.iL);
+                        const double rbar = x[a][d] + 0.5 * t;
+                        dd[d] = minimg(x[b][d] - rbar, R.L, R.iL);
+                    }
+                }
+                lsp = -free_neg_log(&R.bis[level], R.bis_images, i4lt_b, dd);
+            }
+            const double i4lt_k = 1. / (4. * R.lambda * level_tau);
+            for (int i = lane; i < nlinks; i += kWave) {
+                const int a = i * skip, b = a + skip;
+                double dd[3];
+                for (int d = 0; d < 3; ++d) dd[d] = minimg(x[a][d] - x[b][d], R.L, R.iL);
+                k += free_neg_log(&R.kin[level], R.kin_images, i4lt_k, dd);
+            }
+            lsp = wave_sum(lsp);
+            k = wave_sum(k);
+            if (lane == 0) {
+                S.sums[2 * half][level] = lsp;
+                S.sums[2 * half + 1][level] = k;
+            }
+        }
+        __syncthreads();
+    }
+    const int nm = wraps ? 0 : nb - 1;
+    if (w == 0) {
+        // the levels' decisions, a log of each level's uniform per lane
+        const double lu = lane < n ? log(S.u[lane]) : 0.;
+        double prev = 0., lsr = 0., ko = 0., kn = 0.;
+        int status = 1;
+        for (int level = n - 1; level >= 0; --level) {
+            lsr = -S.sums[2][level] + S.sums[0][level];
+            ko = S.sums[1][level];
+            kn = S.sums[3][level];
+            if (level == 0) break;
+            const double old_action = 0. + ko, new_action = 0. + kn;
+            const double change = new_action - old_action;
+            const double la = lsr - change + prev;
+            if (la < __shfl(lu, level)) {
+                status = 2;
+                break;
+            }
+            prev = change;
+        }
+        if (lane == 0) {
+            S.info[4] = status;
+            S.info[5] = status == 1 ? nm : 0;
+            pr->status = status;
+            pr->move = 0;
+            pr->p = p;
+            pr->p2 = p2;
+            // (see propose_bisect_impl)
+            pr->generic = status == 1 && (p2 != p) && (b0 + nb > M);
+            pr->buf = buf;
+            pr->b0 = b0;
+            pr->n_links = R.pair_type ? nb : 0;
+            pr->first = (b0 + 1) % M;
+            pr->count = status == 1 ? nm : 0;
+            pr->lsr = lsr;
+            pr->k_old = ko;
+            pr->k_new = kn;
+            pr->prev = prev;
+            pr->u0 = S.u[0];
+            pr->tape_next = 0;
+        }
+    }
+    const int tid = w * kWave + lane;
+    for (int t = tid; t < 3 * nm; t += W * kWave) beads[t] = S.x_new[1 + t / 3][t % 3];
+    if (R.use_long_range) {
+        const int stride = R.max_idx + 1;
+        for (int t = tid; t < 6 * nm; t += W * kWave) {
+            const int m = t / 6, c = t % 6, d = c % 3;
+            phase_chain((c / 3 ? S.x_new[m + 1][d] : S.x_old[m + 1][d]) * R.box, R.max_idx,
+                        phase + ((size_t)m * 6 + c) * stride);
+        }
+    }
+    __syncthreads();
 }
 
 // Bisect::Attempt up to the level-0 decision, one wavefront (lane 0..63) on
-// replica R; items: also write the round's rho_k work items.  ahead: the
-// attempt was started by bisect_start_ahead (device RNG only).
+// replica R; items: also write the round's rho_k work items.
 template <class Sync>
-__device__ __forceinline__ void propose_bisect_impl(const Rep& R, int lane, Sync sync, bool items, BisectLds& S,
-                                                    bool ahead) {
+__device__ __forceinline__ void propose_bisect_impl(const Rep& R, int lane, Sync sync, bool items, BisectLds& S) {
     Prop* pr = R.prop;
-    if (!ahead) {
-        if (lane == 0) bisect_take(R, S);
-        sync();
-    }
+    if (lane == 0) bisect_take(R, S);
+    sync();
     if (!S.info[0]) {
         if (lane == 0) pr->status = 0;
         if (items) rho_items_write(R, 0, 0, 0, 0, lane);
@@ -318,34 +442,28 @@ __device__ __forceinline__ void propose_bisect_impl(const Rep& R, int lane, Sync
     const int n = R.n_level, nb = 1 << n, N = R.N, M = R.M;
     const bool tape = R.tape != nullptr;
     int bad = 0;
-    if (!ahead) {
-        if (lane == 0) {
-            int p, b0;
-            long long cur = 0;
-            if (tape) {
-                cur = *R.tape_cursor;
-                p = (int)tape_get(R, cur, &bad);
-                b0 = (int)tape_get(R, cur + 1, &bad);
-                cur += 2;
-                if (p < 0 || p >= N || b0 < 0 || b0 >= M) {
-                    bad = 1;
-                    p = 0;
-                    b0 = 0;
-                }
-            } else {
-                // rng.index(0, 0, N) and rng.index(0, 1, M) from one call
-                Rng rng{make_uint2((uint32_t)R.key, (uint32_t)(R.key >> 32)), 1u, S.seq};
-                const uint4 w = rng.call(0);
-                p = (int)(((uint64_t)w.x * (uint32_t)N) >> 32);
-                b0 = (int)(((uint64_t)w.y * (uint32_t)M) >> 32);
+    if (lane == 0) {
+        int p, b0;
+        long long cur = 0;
+        if (tape) {
+            cur = *R.tape_cursor;
+            p = (int)tape_get(R, cur, &bad);
+            b0 = (int)tape_get(R, cur + 1, &bad);
+            cur += 2;
+            if (p < 0 || p >= N || b0 < 0 || b0 >= M) {
+                bad = 1;
+                p = 0;
+                b0 = 0;
             }
-            S.info[1] = p;
-            S.info[2] = b0;
-            S.info[3] = bad;
-            S.cur = cur;
+        } else {
+            bisect_where(R, S.seq, &p, &b0);
         }
-        sync();
+        S.info[1] = p;
+        S.info[2] = b0;
+        S.info[3] = bad;
+        S.cur = cur;
     }
+    sync();
     const int p = S.info[1], b0 = S.info[2];
     // the chain walked from (p, b0) carries label p2 after the wrap
     const int p2 = label_after_wrap(R, p);
@@ -353,7 +471,7 @@ __device__ __forceinline__ void propose_bisect_impl(const Rep& R, int lane, Sync
     // its first one, so the reference's bead walks visit no midpoint and no
     // kinetic link (bisect_class.h:51-58,78)
     const bool wraps = (nb % M) == 0 && p2 == p;
-    if (!ahead) bisect_window(R, lane, S, p, p2, b0, !tape);
+    bisect_window(R, lane, S, p, p2, b0, !tape);
     sync();
     long long cur = S.cur;
     double prev = 0.;
@@ -425,6 +543,7 @@ __device__ __forceinline__ void propose_bisect_impl(const Rep& R, int lane, Sync
                     pr->p = p;
                     pr->p2 = p2;
                     pr->generic = 0;
+                    pr->buf = 0;
                     pr->b0 = b0;
                     pr->count = 0;
                     pr->tape_next = cur;
@@ -444,6 +563,7 @@ __device__ __forceinline__ void propose_bisect_impl(const Rep& R, int lane, Sync
                 // moved beads on both sides of the wrap under two labels: the
                 // label-general pair kernel takes the proposal
                 pr->generic = (p2 != p) && (b0 + nb > M);
+                pr->buf = 0;
                 pr->b0 = b0;
                 pr->n_links = R.pair_type ? nb : 0;  // no pair action: no links to evaluate
                 pr->first = (b0 + 1) % M;
@@ -470,7 +590,7 @@ __device__ __forceinline__ void propose_bisect_body(const Rep* __restrict__ reps
     const int r = blockIdx.x;
     if (r >= n_reps) return;
     __shared__ BisectLds S;
-    propose_bisect_impl(reps[r], (int)threadIdx.x, BlockSync{}, true, S, false);
+    propose_bisect_impl(reps[r], (int)threadIdx.x, BlockSync{}, true, S);
 }
 
 // DisplaceParticle::Attempt (displace_particle_class.h:28-72): NEW beads only.
@@ -534,6 +654,7 @@ __device__ __forceinline__ void propose_displace_impl(const Rep& R, int lane, Sy
             pr->p = p;
             pr->p2 = p;
             pr->generic = 0;
+            pr->buf = 0;
             pr->b0 = 0;
             pr->n_links = R.pair_type ? R.M : 0;
             pr->first = 0;
@@ -1029,7 +1150,7 @@ __global__ __launch_bounds__(kRhoBlock) void k_rho_loop(const RhoItem* __restric
 // ---------------------------------------------------------------------------
 template <class Sync>
 __device__ __forceinline__ void commit_impl(const Rep& R, const Prop& pr, int lane, int acc, const double* pre,
-                                            unsigned char pre_sel, Sync sync);
+                                            unsigned char pre_sel, const double* beads, Sync sync);
 // Raises the context's replay-error flag, a word of host memory that the host reads
 // after the stage.
 __device__ __forceinline__ void ctx_error_set(const Rep& R) {
@@ -1120,12 +1241,13 @@ __device__ __forceinline__ int decide_impl(const Rep& R, int lane, Sync sync, in
     }
     const Prop pr = *prp;
     if (pr.status == 0) return -1;
+    const double* beads = COH ? prop_beads(R, pr) : R.prop_new;
     // the commit's loads of a one-particle move, issued before the sums: the
     // lane's first new bead and the selector of its slice
     double pre[3] = {0., 0., 0.};
     unsigned char pre_sel = 0;
     if (pr.status == 1 && pr.move != 3 && lane < pr.count) {
-        for (int d = 0; d < 3; ++d) pre[d] = R.prop_new[3 * lane + d];
+        for (int d = 0; d < 3; ++d) pre[d] = beads[3 * lane + d];
         if (R.use_long_range) pre_sel = R.sel[(pr.first + lane) % R.M];
     }
     if (pr.status == 1) {
@@ -1170,7 +1292,7 @@ __device__ __forceinline__ int decide_impl(const Rep& R, int lane, Sync sync, in
         s_acc = acc;
     }
     sync();
-    commit_impl(R, pr, lane, s_acc, pre, pre_sel, sync);
+    commit_impl(R, pr, lane, s_acc, pre, pre_sel, beads, sync);
     // bookkeeping after the commit's stores are issued
     if (lane == 0) {
         if (R.tape) *R.tape_cursor = tape_next;
@@ -1196,7 +1318,7 @@ __device__ __forceinline__ int decide_impl(const Rep& R, int lane, Sync sync, in
 // selector, loaded before the decision.
 template <class Sync>
 __device__ __forceinline__ void commit_impl(const Rep& R, const Prop& pr, int lane, int acc, const double* pre,
-                                            unsigned char pre_sel, Sync sync) {
+                                            unsigned char pre_sel, const double* beads, Sync sync) {
     const int M = R.M, N = R.N;
     const int s_acc = acc;
     if (s_acc && pr.move == 3) {
@@ -1255,7 +1377,7 @@ __device__ __forceinline__ void commit_impl(const Rep& R, const Prop& pr, int la
             // a bisection chain carries label p2 past the wrap
             const int l = (pr.move == 0 && pr.b0 + m + 1 >= M) ? pr.p2 : pr.p;
             const bool first = m == lane;
-            for (int d = 0; d < 3; ++d) R.pos[((size_t)d * M + s) * N + l] = first ? pre[d] : R.prop_new[3 * m + d];
+            for (int d = 0; d < 3; ++d) R.pos[((size_t)d * M + s) * N + l] = first ? pre[d] : beads[3 * m + d];
             if (R.use_long_range) R.sel[s] = (unsigned char)((first ? pre_sel : R.sel[s]) ^ 1);
         }
     }
@@ -1289,11 +1411,12 @@ __global__ __launch_bounds__(64) void k_decide(const Rep* __restrict__ reps, int
 // K5 of one round and K4 of the next in one launch: a replica's pending
 // proposal is decided and committed (nothing is pending at the first round of
 // a stage), then its next proposal is made.  Saves one dependent launch per
-// round; the stage's last decision is a k_decide of its own.  Two wavefronts
+// round; the stage's last decision is a k_decide of its own.  Four wavefronts
 // per replica: the first decides while, on the device RNG of an unpermuted
-// path, the second starts the next attempt (counter step, draws, window) and
-// afterwards does the decision's bookkeeping, as in k_round.
-constexpr int kBisBlock = 2 * kWave;
+// path, the second and third fetch the next attempt's window and draws; then
+// all four make its levels (bisect_levels): 15 us for 512 replicas of N = 256,
+// M = 128 beside 18 with the levels on one wavefront.
+constexpr int kBisBlock = 4 * kWave;
 __global__ __launch_bounds__(kBisBlock) void k_decide_propose_bisect(const Rep* __restrict__ reps, int n_reps,
                                                                      unsigned long long* __restrict__ kt) {
     __shared__ BisectLds S;
@@ -1306,28 +1429,49 @@ __global__ __launch_bounds__(kBisBlock) void k_decide_propose_bisect(const Rep* 
     // a window that crosses the wrap of a permuted path holds a second label,
     // which the window check after the decision does not follow
     const bool ahead = R.tape == nullptr && R.perm == nullptr;
+    Counters* c = R.cnt;
+    const unsigned int rem = c->remaining;
+    const unsigned long long seq = c->seq;
+    int p = -1, b0 = 0;
+    if (ahead && rem > 0 && w > 0) bisect_where(R, seq, &p, &b0);
     if (w == 0) {
         if (lane == 0) s_out.status = 0;
         const int nb = 1 << R.n_level;
         const int moved = decide_impl(R, lane, WaveSync{}, R.pair_type ? nb : 0,
                                       R.use_long_range ? (nb - 1) * R.n_chunks : 0, &s_out);
         if (lane == 0) s_moved = moved;
-    } else if (ahead) {
-        bisect_start_ahead(R, lane, WaveSync{}, S);
+    } else if (w == 1 && p >= 0) {
+        if (lane == 0) {
+            S.info[1] = p;
+            S.info[2] = b0;
+        }
+        bisect_window(R, lane, S, p, p, b0, false);
+    } else if (w == 2 && p >= 0) {
+        bisect_draws(R, lane, S, seq);
     }
     __syncthreads();
-    if (w == 1) {
-        if (lane == 0 && s_out.status != 0)
-            decide_book(R, s_out.pr, s_out.acc, s_out.status, s_out.po, s_out.pn, s_out.lo, s_out.ln);
+    if (w == 3 && lane == 0 && s_out.status != 0)
+        decide_book(R, s_out.pr, s_out.acc, s_out.status, s_out.po, s_out.pn, s_out.lo, s_out.ln);
+    if (!ahead) {
+        if (w == 0) propose_bisect_impl(R, lane, WaveSync{}, true, S);
         return;
     }
-    if (ahead && S.info[0] && S.info[1] == s_moved) {
-        // the decision just committed beads of the attempt's particle: its window again
-        const int p = S.info[1];
-        bisect_window(R, lane, S, p, p, S.info[2], false);
-        WaveSync{}();
+    if (rem == 0) {
+        if (threadIdx.x == 0) R.prop->status = 0;
+        rho_items_write(R, 0, 0, 0, 0, threadIdx.x, kBisBlock);
+        return;
     }
-    propose_bisect_impl(R, lane, WaveSync{}, true, S, ahead);
+    if (threadIdx.x == 0) {
+        c->remaining = rem - 1;
+        c->seq = seq + 1;
+    }
+    if (S.info[1] == s_moved) {
+        // the decision just committed beads of the attempt's particle: its window again
+        if (w == 0) bisect_window(R, lane, S, s_moved, s_moved, S.info[2], false);
+        __syncthreads();
+    }
+    bisect_levels<kBisBlock / kWave>(R, S, w, lane, R.prop, R.prop_new, R.phase, 0);
+    rho_items_write(R, 0, S.info[4], S.info[5], (S.info[2] + 1) % R.M, threadIdx.x, kBisBlock);
 }
 // Displacement: the decision on the first wavefront, then the proposal, whose
 // M moved slices (positions, phase chains, rho_k items) take all kDisBlock
@@ -1348,24 +1492,73 @@ __global__ __launch_bounds__(kDisBlock) void k_decide_propose_displace(const Rep
 
 // A whole round (MOVE 0 bisection, 1 displacement) in one launch, for batches
 // too small to fill the GPU (a round is then bound by latency, not by
-// throughput).  Workgroups
-// [0, n_reps * bpr) (after the XCD remap) run the window links of the LDS pair
-// kernel, the others a group of up to ipb rho_k items of one replica each
-// (rgrp: first item, items, replica; ipb > 1 only where one item per
+// throughput).  After the XCD remap the first n_reps workgroups (bisection) make
+// the replicas' next proposals, the following n_reps * bpr run the window links
+// of the LDS pair kernel, the others a group of up to ipb rho_k items of one
+// replica each (rgrp: first item, items, replica; ipb > 1 only where one item per
 // workgroup would exceed what the GPU holds at once).  Every workgroup then
-// counts itself in on its replica's arrival counter; the last of the
-// replica's bpr + ceil(n_items / ipb) workgroups decides and commits the replica's
-// proposal (K5) and makes its next one (K4), with its rho_k items, in its
-// first wavefront.  A replica's round thus ends with its own last workgroup:
-// no launch boundary separates the sums from the decision, and nothing waits
-// (the counter is only read by the atomic that increments it).  The sums pass
+// counts itself in on its replica's arrival counter; the replica's last one
+// decides and commits its proposal (K5) and publishes the next, with its rho_k
+// items.  A replica's round thus ends with its own last workgroup: no launch
+// boundary separates the sums from the decision, and nothing waits (the counter
+// is only read by the atomic that increments it).  The sums and the proposal pass
 // between workgroups as agent-scope atomic stores and loads, each waited for
 // before its workgroup arrives; agent-scope fences would instead write back a
 // whole L2 per workgroup, which measured slower than three launches per round.
-// The decision and proposal are the same code as in k_decide_propose_*, so the
-// chains are the same bit for bit.  The last workgroup resets the counter for
-// the next round.
+// The last workgroup resets the counter for the next round.
+//
+// A bisection draws from its sequence number alone and reads only its own
+// particle's beads, so the proposal made beside the pending one is the one that
+// would follow the decision, bit for bit, unless the decision commits beads of
+// the same particle (an acceptance, 1 in N): then the last workgroup makes it
+// again.  What remains after the last arrival is the decision.  A displacement
+// (its M slices' phases) and a replayed tape (its cursor follows the decision)
+// are proposed after the decision.  A bisection round with the proposal in the
+// last workgroup, with it beside the pending one on one wavefront, and on four
+// (bisect_levels): one replica of N = 256, M = 128 23, 18 and 14.5 us; of N = 32,
+// M = 32 16, 15.5 and 12 us.
 constexpr int kRoundBlock = kRhoBlock;
+constexpr int kNextWords = sizeof(NextProp) / 8, kPropWords = sizeof(Prop) / 8;
+static_assert(sizeof(NextProp) % 8 == 0 && sizeof(Prop) % 8 == 0 && kNextWords <= kWave, "one word a lane");
+
+// Workgroup of k_round that makes replica R's next bisection while the others
+// evaluate the pending one: the whole proposal, from the positions before the
+// decision, into the set of buffers the pending one does not use.  It stands
+// unless the decision commits beads of the same particle.
+__device__ __forceinline__ void next_bisect(const Rep& R, BisectLds& S, NextProp& next) {
+    if (R.tape != nullptr) return;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    Counters* c = R.cnt;
+    const unsigned int rem = c->remaining;
+    const unsigned long long seq = c->seq;
+    const int set = R.prop->buf == 1 ? 1 : 0;
+    if (threadIdx.x < kNextWords) ((unsigned long long*)&next)[threadIdx.x] = 0;
+    if (rem > 0) {
+        int p, b0;
+        bisect_where(R, seq, &p, &b0);
+        if (threadIdx.x == 0) {
+            S.info[1] = p;
+            S.info[2] = b0;
+            S.seq = seq;
+        }
+        if (w == 0) bisect_window(R, lane, S, p, label_after_wrap(R, p), b0, false);
+        if (w == 1) bisect_draws(R, lane, S, seq);
+    }
+    __syncthreads();  // every wavefront has read the counters
+    if (rem > 0) {
+        if (threadIdx.x == 0) {
+            c->remaining = rem - 1;
+            c->seq = seq + 1;
+            next.seq = seq;
+            next.has = 1;
+        }
+        bisect_levels<kRoundBlock / kWave>(R, S, w, lane, &next.pr, R.next_new[set], R.next_phase[set], set + 1);
+    }
+    if (threadIdx.x < kNextWords)
+        __hip_atomic_store((unsigned long long*)R.next + threadIdx.x, ((unsigned long long*)&next)[threadIdx.x],
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // PT 3: the tables stay in global memory, NORD the doubles of LDS for their axes.
 template <int PT, int NORD, int KPT, bool NT, int MOVE>
 __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ reps, int n_reps, int bpr, int qpw,
@@ -1378,15 +1571,22 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
     __shared__ double2 wpart[kRoundBlock / kWave];
     __shared__ int s_last;
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    const int n_pair = n_reps * bpr, idx = xcd_remap(blockIdx.x, gridDim.x);
+    __shared__ BisectLds S;
+    __shared__ NextProp s_next;
+    const int n_next = MOVE == 0 ? n_reps : 0;
+    const int n_pair = n_reps * bpr, idx = (int)xcd_remap(blockIdx.x, gridDim.x) - n_next;
     int r;
-    if (idx < n_pair) {
+    if (MOVE == 0 && idx < 0) {
+        r = idx + n_next;
+        next_bisect(reps[r], S, s_next);
+    } else if (idx < n_pair) {
         r = idx / bpr;
         const int part = idx % bpr;
-        const Rep R = reps[r];
+        Rep R = reps[r];
         if constexpr (PT == 3) {
             constexpr int W = kRoundBlock / kWave;
             const Prop pr = *R.prop;
+            R.prop_new = prop_beads(reps[r], pr);
             if (pr.status == 1 && !pr.generic && part * (W / general_split<W>(R.N, qpw)) < pr.n_links)
                 pair_links_general<true, W>(R, lds, NORD, pr, part, bpr, qpw, w, lane, wpart);
         } else {
@@ -1399,6 +1599,7 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
                 tv[k] = t < nd ? (t < na ? R.bt_a.c[t] : R.bt_b.c[t - na]) : 0.;
             }
             const Prop pr = *R.prop;
+            R.prop_new = prop_beads(reps[r], pr);
             constexpr int W = kRoundBlock / kWave;
             if (pr.status == 1 && !pr.generic && part * (W / pair_split<W>(R.N, qpw)) < pr.n_links) {
 #pragma unroll
@@ -1433,15 +1634,13 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
     if (threadIdx.x == 0) {
         const Rep& R = reps[r];
         const int n_items = MOVE == 0 ? R.n_ritems_bis : R.n_ritems_dis;
-        const unsigned int expect = (unsigned int)bpr + (unsigned int)((n_items + ipb - 1) / ipb);
+        const unsigned int expect = (MOVE == 0 ? 1u : 0u) + (unsigned int)bpr + (unsigned int)((n_items + ipb - 1) / ipb);
         s_last = atomicAdd(arrive + r, 1u) + 1u == expect;
     }
     __syncthreads();
     if (!s_last) return;
-    // the replica's last workgroup: its first wavefront decides while, for a
-    // bisection on the device RNG, its second starts the next attempt (the draws
-    // depend on the attempt's sequence number only, not on the decision)
-    __shared__ BisectLds S;
+    // the replica's last workgroup: its first wavefront decides while its second
+    // fetches the proposal made ahead
     __shared__ DecideOut s_out;
     __shared__ int s_moved;
     const Rep& R = reps[r];
@@ -1459,27 +1658,43 @@ __global__ __launch_bounds__(kRoundBlock) void k_round(const Rep* __restrict__ r
                                             R.use_long_range ? nm * R.n_chunks : 0, &s_out);
         if (lane == 0) s_moved = moved;
     } else if (w == 1 && ahead) {
-        bisect_start_ahead(R, lane, WaveSync{}, S);
+        unsigned long long *to = (unsigned long long*)&s_next, *from = (unsigned long long*)R.next;
+        if (lane < kNextWords) to[lane] = __hip_atomic_load(from + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (w == 2) {
+    if (w == 2 && lane == 0 && s_out.status != 0)
         // the decision's counters and flags, off the proposal's path
-        if (lane == 0 && s_out.status != 0)
-            decide_book(R, s_out.pr, s_out.acc, s_out.status, s_out.po, s_out.pn, s_out.lo, s_out.ln);
-        return;
-    }
-    if (w != 0) return;
+        decide_book(R, s_out.pr, s_out.acc, s_out.status, s_out.po, s_out.pn, s_out.lo, s_out.ln);
     if (MOVE == 1) {
-        propose_displace_impl(R, lane, WaveSync{}, true);
+        propose_displace_impl(R, (int)threadIdx.x, BlockSync{}, true, kRoundBlock);
         return;
     }
-    if (ahead && S.info[0] && S.info[1] == s_moved) {
-        // the decision just committed beads of the attempt's particle: its window again
-        const int p = S.info[1];
-        bisect_window(R, lane, S, p, label_after_wrap(R, p), S.info[2], false);
-        WaveSync{}();
+    if (!ahead) {
+        if (w == 0) propose_bisect_impl(R, lane, WaveSync{}, true, S);
+        return;
     }
-    propose_bisect_impl(R, lane, WaveSync{}, true, S, ahead);
+    const int p = s_next.pr.p;
+    if (!(s_next.has && p == s_moved)) {
+        // the decision left the attempt's particle where it was: the proposal made
+        // ahead stands, its rho_k rows are known now
+        if (w == 2) return;
+        const int t = w == 3 ? lane + 2 * kWave : (int)threadIdx.x;
+        if (t < kPropWords) ((unsigned long long*)R.prop)[t] = ((const unsigned long long*)&s_next.pr)[t];
+        rho_items_write(R, 0, s_next.pr.status, s_next.pr.count, s_next.pr.first, t, 3 * kWave,
+                        s_next.pr.buf ? R.next_phase[s_next.pr.buf - 1] : nullptr);
+        return;
+    }
+    // the decision just committed beads of the attempt's particle: the proposal
+    // again, from the same draws
+    if (threadIdx.x == 0) {
+        S.info[1] = p;
+        S.info[2] = s_next.pr.b0;
+    }
+    if (w == 0) bisect_window(R, lane, S, p, label_after_wrap(R, p), s_next.pr.b0, false);
+    if (w == 1) bisect_draws(R, lane, S, s_next.seq);
+    __syncthreads();
+    bisect_levels<kRoundBlock / kWave>(R, S, w, lane, R.prop, R.prop_new, R.phase, 0);
+    rho_items_write(R, 0, S.info[4], S.info[5], (S.info[2] + 1) % R.M, threadIdx.x, kRoundBlock);
 }
 
 // Sums the per-replica work counters into work[WORK_PAIR_LINKS], work[WORK_RHO_SLICEK].
