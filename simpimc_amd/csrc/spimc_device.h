@@ -144,6 +144,7 @@ struct Rep {
     const int4* k_runs;    // [n_runs] runs of consecutive n2 at fixed (n0, n1): {n0, n1, n2 first, +-length}
     const int4* cols;      // [n_cols] the k-vectors of one (n0, n1): {n0 + 128 | (n1 + 128) << 8, |n2| max + 1, first entry}
     const int2* col_k;     // [n_col_k] a column's entries n = 0 ..: the k-vectors at n2 = n and -n, or -1
+    const int2* col_g;     // [n_col_k / 4] each group of four entries: its column's (n0, n1) as in cols, n of the first
     int n_cols, n_col_k;
     const int* k_order;    // [nk] k index of the i-th k-vector in run order
     int n_runs, rho_kpt;   // rho_kpt: k-vectors per thread of the rho_k kernel (sets the k chunks)

@@ -254,7 +254,7 @@ struct RepHost {
     std::vector<int4> k_runs;  // runs of consecutive n2 at fixed (n0, n1), ordered by (n0, n1)
     std::vector<int> k_order;  // k index of each k-vector in run order
     std::vector<int4> cols;    // columns (n0, n1) and their entries (Rep::cols, Rep::col_k)
-    std::vector<int2> col_k;
+    std::vector<int2> col_k, col_g;
     int col_max = 0;           // largest |n2| + 1
     bool col_twice = false;    // a k-vector listed twice
     std::vector<double> kmag, coef_s, coef_b, coef_v;
@@ -726,6 +726,7 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         h.k_order.clear();
         h.cols.clear();
         h.col_k.clear();
+        h.col_g.clear();
         auto emit = [&](int n0, int n1, const std::vector<int>& ks, const std::vector<int>& n2s, int lo, int hi) {
             // ks[lo..hi] have consecutive n2s; split at 0 into an ascending and a descending run
             int z = lo;
@@ -761,6 +762,7 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
             const int len = (top + kAdjColPad) / kAdjColPad * kAdjColPad;
             h.cols.push_back(make_int4((n0 + 128) | (n1 + 128) << 8, len, at, 0));
             h.col_k.resize(at + len, make_int2(-1, -1));
+            for (int q = 0; q < len; q += kAdjColPad) h.col_g.push_back(make_int2((n0 + 128) | (n1 + 128) << 8, q));
             for (size_t i = 0; i < ks.size(); ++i)
                 (n2s[i] >= 0 ? h.col_k[at + n2s[i]].x : h.col_k[at - n2s[i]].y) = ks[i];
             h.col_max = std::max(h.col_max, top + 1);
@@ -853,6 +855,7 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
             R.k_order = cv.take<int>(std::max(nk, 1));
             R.cols = cv.take<int4>(std::max<size_t>(h.cols.size(), 1));
             R.col_k = cv.take<int2>(std::max<size_t>(h.col_k.size(), 1));
+            R.col_g = cv.take<int2>(std::max<size_t>(h.col_g.size(), 1));
             if (h.v_r.n) R.v_r = carve_spline(cv, h.v_r);
             if (h.v_long_r.n) R.v_long_r = carve_spline(cv, h.v_long_r);
             if (h.u.n) R.u = carve_spline(cv, h.u);
@@ -995,6 +998,7 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         R.k_order = O.k_order;
         R.cols = O.cols;
         R.col_k = O.col_k;
+        R.col_g = O.col_g;
         R.v_r = O.v_r;
         R.v_long_r = O.v_long_r;
         R.u = O.u;
@@ -1033,6 +1037,7 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         HIPCHK(hipMemcpy((void*)R.k_order, h.k_order.data(), nk * sizeof(int), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy((void*)R.cols, h.cols.data(), h.cols.size() * sizeof(int4), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy((void*)R.col_k, h.col_k.data(), h.col_k.size() * sizeof(int2), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy((void*)R.col_g, h.col_g.data(), h.col_g.size() * sizeof(int2), hipMemcpyHostToDevice));
     }
     int rc;
     if ((rc = upload_spline(R.v_r, h.v_r)) || (rc = upload_spline(R.v_long_r, h.v_long_r)) ||
@@ -1852,6 +1857,16 @@ int rho_rebuild(spimc_ctx* c, uint32_t r) {
     const Rep& R = c->reps[r].dev;
     if (!R.use_long_range) return SPIMC_OK;
     HIPCHK(hipMemsetAsync(R.sel, 0, R.M, c->stream));
+    // by columns where each k-vector is listed once and the columns' padded entries
+    // (up to two k-vectors each) are not more than the k-vectors, as for every k < k_cut
+    static_assert(kAdjColPad == 4, "k_rho_cols takes four entries a lane");
+    if (!c->reps[r].col_twice && R.n_col_k > 0 && R.n_col_k <= R.nk) {
+        const size_t row = (size_t)3 * (R.max_idx + 1) * sizeof(double2);
+        const int tile = 64 * row <= 48 * 1024 ? 64 : 16;
+        const size_t shmem = std::max(tile * row + 3 * sizeof(double2), (size_t)3 * 16 * 64 * sizeof(double));
+        return launch(c, SPIMC_KERNEL_ESTIMATORS, k_rho_cols, dim3(R.M, (R.n_col_k / 4 + 63) / 64), 256, shmem,
+                      c->stream, c->d_reps, (int)r, tile);
+    }
     const int chunks = (R.nk + 256 * kBuildKpt - 1) / (256 * kBuildKpt);
     dim3 g(R.M, chunks);
     return launch(c, SPIMC_KERNEL_ESTIMATORS, k_rho_build<kBuildKpt>, g, 256, 0, c->stream, c->d_reps, (int)r);

@@ -198,6 +198,68 @@ __global__ __launch_bounds__(256) void k_rho_build(const Rep* __restrict__ reps,
     }
 }
 
+// K3 by columns: the k-vectors (n0, n1, +-n2) of one column share e^{i (n0 phi_0 +
+// n1 phi_1)} = x + iy, and with e^{i n phi_2} = c + is both signs of n take the four
+// sums of xc, ys, xs and yc: rho(+-n) = (xc -+ ys, yc +- xs).  A lane holds four
+// consecutive n of a column (16 sums, 16 multiply-adds a particle for up to eight
+// k-vectors, where k_rho_build spends two complex products and three LDS reads on
+// each), a workgroup 64 such groups of one slice, its wavefronts every fourth
+// particle; the wavefronts' sums are added in order.  Bound by its LDS reads (six
+// of 16 bytes a particle and lane).  One slice array of N = 1024, M = 128 with 4012
+// k-vectors: 306 us by k_rho_build, 88 us so.
+__global__ __launch_bounds__(256) void k_rho_cols(const Rep* __restrict__ reps, int r, int tile) {
+    extern __shared__ double lds[];
+    const Rep& R = reps[r];
+    const int b = blockIdx.x, lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int mx = R.max_idx, stride = mx + 1, N = R.N, ng = R.n_col_k / 4, g = blockIdx.y * kWave + lane;
+    double2* tab = reinterpret_cast<double2*>(lds);  // [tile][3][stride], and three values that a padded group reads
+    const int2 cg = g < ng ? R.col_g[g] : make_int2(128 | 128 << 8, 0);
+    const int n0 = (cg.x & 255) - 128, n1 = (cg.x >> 8) - 128;
+    const int a0 = abs(n0), a1 = stride + abs(n1), a2 = 2 * stride + cg.y;
+    const double g0 = n0 < 0 ? -1. : 1., g1 = n1 < 0 ? -1. : 1.;
+    double s[4][4];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i / 4][i % 4] = 0.;
+    for (int p0 = 0; p0 < N; p0 += tile) {
+        __syncthreads();
+        const int np = min(tile, N - p0);
+        for (int t = threadIdx.x; t < 3 * np; t += 256)
+            phase_chain(pos_at(R, t % 3, b, p0 + t / 3) * R.box, mx, tab + t * stride);
+        __syncthreads();
+        for (int pp = w; pp < np; pp += 256 / kWave) {
+            const double2* f = tab + pp * 3 * stride;
+            double2 e0 = f[a0], e1 = f[a1];
+            e0.y *= g0;
+            e1.y *= g1;
+            const double2 e = cmul(e0, e1);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double2 z = f[a2 + i];
+                s[i][0] = fma(e.x, z.x, s[i][0]);
+                s[i][1] = fma(e.y, z.y, s[i][1]);
+                s[i][2] = fma(e.x, z.y, s[i][2]);
+                s[i][3] = fma(e.y, z.x, s[i][3]);
+            }
+        }
+    }
+    __syncthreads();
+    if (w > 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) lds[((w - 1) * 16 + i) * kWave + lane] = s[i / 4][i % 4];
+    }
+    __syncthreads();
+    if (w > 0 || g >= ng) return;
+    double2* out = R.rho + ((size_t)R.sel[b] * R.M + b) * R.nk;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        for (int v = 0; v < 256 / kWave - 1; ++v)
+            for (int q = 0; q < 4; ++q) s[i][q] += lds[(v * 16 + 4 * i + q) * kWave + lane];
+        const int2 k = R.col_k[4 * g + i];
+        if (k.x >= 0) out[k.x] = make_double2(s[i][0] - s[i][1], s[i][3] + s[i][2]);
+        if (k.y >= 0) out[k.y] = make_double2(s[i][0] + s[i][1], s[i][3] - s[i][2]);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // K4: Bisect::Attempt down to level 0 (bisect_class.h:39-124), one wavefront
 // per replica.  Coarse levels carry only the kinetic action (the pair action
