@@ -421,7 +421,7 @@ int spimc_bead_updates(spimc_ctx* ctx, uint64_t* out);
  * stage kernel that runs a replica's whole stage in one workgroup, with 256,
  * 512 or 1024 threads; and, for at most 256 replicas, rounds of one launch
  * each, for bisection or for both moves, whose last workgroup per replica
- * decides the replica's proposal and makes its next one) it runs one
+ * decides the replica's proposal and publishes its next one) it runs one
  * bisection and one displace attempt per
  * replica untimed, then times n_rounds bisection attempts followed by
  * n_displace displace attempts (the sweep's ratio, N M / 2^l : N, for replica
