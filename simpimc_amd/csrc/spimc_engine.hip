@@ -1957,7 +1957,7 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
             // particles per workgroup: halved until the workgroups number the CUs
             int np = std::min(c->max_N, kCompatBlock);
             while (np > 64 && (long long)c->max_M * nrep * ((c->max_N + np - 1) / np) < kNumCUs) np = (np + 1) / 2;
-            const size_t shmem = ((size_t)c->lds_adj_max + (size_t)kCompatBlock * 3) * sizeof(double);
+            const size_t shmem = (size_t)kCompatBlock * 3 * sizeof(double);
             rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(c->max_M, (c->max_N + np - 1) / np, nrep), kCompatBlock,
                         shmem, c->stream, base, out_est, short_on, np);
         } else {
@@ -2281,12 +2281,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
                                 c->lds_adj_max * (int)sizeof(double)) != hipSuccess)
             c->lds_adj_max = 0;
         if (c->lds_adj_max > 0) {
-            c->compat_fn = vi == 0 ? k_grad_compat_lds<1, 0> : vi == 1 ? k_grad_compat_lds<2, 2>
-                                                     : vi == 2 ? k_grad_compat_lds<2, 0> : k_grad_compat_lds<0, 0>;
-            const size_t b3 = ((size_t)c->lds_adj_max + (size_t)kCompatBlock * 3) * sizeof(double);
-            if (b3 > kPairLdsMaxBytes || hipFuncSetAttribute((const void*)c->compat_fn,
-                                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)b3) != hipSuccess)
-                c->compat_fn = nullptr;
+            c->compat_fn = vi == 0 ? k_grad_compat_split<1> : vi <= 2 ? k_grad_compat_split<2> : k_grad_compat_split<0>;
         }
         {
             // the pair-once kernel adds its waves' partner slots to the tables

@@ -2320,173 +2320,141 @@ __device__ __forceinline__ void stage_tables(const Rep& R, double* lds) {
     __syncthreads();
 }
 
-// The same for the Bare and David actions with the tables in LDS.  Central
-// differences in bead (b, p) of the links (b, b + 1) and (b, b - 1): the bead's
-// own distance r is the same in both links and r' does not move, so the terms of
-// r alone are evaluated once for the two links and those of r' alone not at all:
-// 6 radial terms per pair for Bare (24 with each link action formed whole), 6
-// radial and 12 off-diagonal ones for David.  Where a shifted component crosses
-// half the box the two sides see different images and r' moves with them; those
-// pairs form the whole difference.  The differences are the reference's up to the
-// rounding of the terms that cancel.
-// blockIdx.x: slice; np particles per workgroup (a tile blockIdx.y of the slice's),
-// whose 1024 / np groups of threads share the partners; the groups' sums are added
-// in order.  Bound by FP64 arithmetic and LDS gathers: N = 77, M = 50, 12 replicas
-// 1243 us with a thread per bead on the global tables, 104 us so.
-constexpr int kCompatBlock = 1024;
-// The spline at one point in powers of the fraction f of its interval: two points
-// of one interval share the rounding of the constant term, which then cancels in
-// their difference.  Against extended precision, for differences of at most 2e-4 in
-// r on the Ewald table: 3.6e-17 of the table's largest value, as with the cubics of
-// the global tables; 7.1e-17 in the basis form.  (104 us with that, 102 us so.)
-__device__ __forceinline__ double bt_value(const double* c, const BTab& T, double t) {
-    const double d = t - T.x0, fl = clampd(floor(d * T.ih), 0., (double)(T.knots - 2)), f = fma(d, T.ih, -fl);
-    c += (int)fl;
-    const double c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3];
-    const double a = fma(4., c1, c0 + c2), b1 = 3. * (c2 - c0), b2 = 3. * ((c0 - c1) + (c2 - c1));
-    const double b3 = fma(3., c1 - c2, c3 - c0);
-    return fma(f, fma(f, fma(f, b3, b2), b1), a);
-}
-// radial part of the Bare link action / tau at one distance
-__device__ __forceinline__ double bare_radial_lds(const Rep& R, const double* lds, double r) {
-    r = clampd(r, R.r_v_min, R.r_v_max);
-    double v = R.is_coulomb ? 0.5 / r : 0.5 * bt_value(lds, R.bt_a, r);
-    if (R.use_long_range) {
-        const double* vl = lds + (R.is_coulomb ? 0 : R.bt_a.ncoef);
-        v -= 0.5 * bt_value(vl, R.bt_b, clampd(r, R.r_l_min, R.r_l_max));
+// The same differences for the Bare and David actions, a bead's partners shared by
+// a workgroup.  blockIdx.x: slice; np particles per workgroup (a tile blockIdx.y of
+// the slice's), whose 512 / np groups of threads each take a range of the partners;
+// the groups' sums are added in order.  The bead's own distance is the same in the
+// links (b, b + 1) and (b, b - 1), and r' moves with the bead only where its image
+// does: 6 radial terms at r and 2 at r' per pair instead of 48.  Every link action
+// is added up from its terms in k_grad_compat's order, from the same cubics: a
+// difference over 2 eps magnifies the rounding of a link action 5000 times, and
+// terms left out or in another form (B-splines in LDS: 102 us) come out several
+// times further from 64-bit arithmetic.  Bound by FP64 arithmetic and table
+// gathers: N = 77, M = 50, 12 replicas 1243 us with a thread per bead, 272 us so.
+constexpr int kCompatBlock = 512;  // (1024 spills)
+struct RadialTerms {
+    double a, l;  // the action's own table (or 0.5 / r) and the long-range one
+};
+__device__ __forceinline__ RadialTerms radial_terms(const Rep& R, bool bare, double r) {
+    RadialTerms t{0., 0.};
+    if (bare) {
+        // (clamps as in bare_v: one range after the other)
+        r = clampd(r, R.r_v_min, R.r_v_max);
+        t.a = R.is_coulomb ? 0.5 / r : spl_eval1(R.v_r, r);
+        if (R.use_long_range) {
+            r = clampd(r, R.r_l_min, R.r_l_max);
+            t.l = spl_eval1(R.v_long_r, r);
+        }
+    } else {
+        r = clampd(r, R.g_min, R.g_max);
+        const int i = spl_locate(R.u, r);
+        t.a = spl_val(R.u, i, 1, r - R.u.x[i]);
     }
-    return v;
+    return t;
 }
-__device__ __forceinline__ double david_radial_lds(const Rep& R, const double* lds, double r) {
-    return 0.5 * bt_value(lds, R.bt_a, clampd(r, R.g_min, R.g_max));
-}
-// off-diagonal part of the David link action
-template <int NORD>
-__device__ __forceinline__ double david_off_lds(const Rep& R, const double* lds, double r, double rp, double s2) {
-    const double q = 0.5 * (r + rp), z = r - rp;
-    double u = 0.;
-    if (s2 > 0.0 && q < R.g_max) {
-        const BBasis bq = bt_basis(R.bt_a, q);
-        const double z2 = z * z;
-        double sp[4], zp[4];
-        sp[0] = 1.;
-        zp[0] = 1.;
-#pragma unroll
-        for (int e = 1; e <= (NORD ? NORD : 3); ++e) {
-            sp[e] = sp[e - 1] * s2;
-            zp[e] = zp[e - 1] * z2;
+// pair_u from the radial terms at r and r'
+__device__ __forceinline__ double pair_u_terms(const Rep& R, bool bare, const RadialTerms& t0, const RadialTerms& t1,
+                                               double r0, double r1, double s) {
+    if (bare) {
+        double v = 0.;
+        if (R.is_coulomb) {
+            v += t0.a + t1.a;
+        } else {
+            v += 0.5 * t0.a;
+            v += 0.5 * t1.a;
         }
-        const int n_order = NORD ? NORD : R.n_order;
-#pragma unroll
-        for (int k = 1; k <= (NORD ? NORD : 3); ++k) {
-            if (k > n_order) break;
-#pragma unroll
-            for (int j = 0; j <= k; ++j)
-                u += bt_apply(lds + (size_t)(k * (k + 1) / 2 + j) * R.bt_a.ncoef, bq) * zp[j] * sp[k - j];
+        if (R.use_long_range) {
+            v -= 0.5 * t0.l;
+            v -= 0.5 * t1.l;
         }
+        return R.tau * v;
+    }
+    const double q = 0.5 * (r0 + r1), z = r0 - r1;
+    double u = 0.5 * (t0.a + t1.a);
+    if (s > 0.0 && q < R.g_max) {
+        const int iq = spl_locate(R.u, q);
+        u += david_offdiag(R.u, R.n_order, iq, q - R.u.x[iq], z, s);
     }
     return u;
 }
-template <int PT, int NORD>
-__global__ __launch_bounds__(kCompatBlock) void k_grad_compat_lds(const Rep* __restrict__ reps, int out_est, int short_on,
-                                                                  int np) {
-    extern __shared__ double lds[];
-    const Rep R = reps[blockIdx.z];
+template <int PT>
+__global__ __launch_bounds__(kCompatBlock) void k_grad_compat_split(const Rep* __restrict__ reps, int out_est, int short_on,
+                                                                    int np) {
+    extern __shared__ double lds[];  // [group][np][3]
+    const Rep& R = reps[blockIdx.z];
     const int b = blockIdx.x, p0 = blockIdx.y * np, N = R.N, M = R.M;
     if (b >= M || p0 >= N) return;
     const bool on = short_on && R.pair_type != 0 && N > 1;
-    if (on) stage_tables(R, lds);
-    double* sums = lds + R.lds_doubles;  // [group][np][3]
     const int n = min(np, N - p0), n_grp = kCompatBlock / n;
     const int grp = threadIdx.x / n, lp = threadIdx.x % n, p = p0 + lp;
     const bool bare = PT == 1 || (PT == 0 && R.pair_type == 1);
     const double eps = 1.e-4;
-    double g[3] = {0., 0., 0.};
     if (on && grp < n_grp) {
-        const int bj = b + 1 == M ? 0 : b + 1, bk = b == 0 ? M - 1 : b - 1;
+        double g[3] = {0., 0., 0.};
+        const int b1[2] = {b + 1 == M ? 0 : b + 1, b == 0 ? M - 1 : b - 1};
         const int q_lo = (int)((long long)N * grp / n_grp), q_hi = (int)((long long)N * (grp + 1) / n_grp);
-        double r0[3], pj[3], pk[3];
+        double r0[3], p1[2][3];
         for (int d = 0; d < 3; ++d) {
             r0[d] = pos_at(R, d, b, p);
-            pj[d] = pos_at(R, d, bj, p);
-            pk[d] = pos_at(R, d, bk, p);
+            for (int lk = 0; lk < 2; ++lk) p1[lk][d] = pos_at(R, d, b1[lk], p);
         }
         for (int q = q_lo; q < q_hi; ++q) {
             if (q == p) continue;
-            // r with each component unshifted and shifted by -+eps, and the image each took
-            double rv[3], rs[3][2], vj[3], vk[3];
-            bool wrap[3];
-            double x2[3];
+            double q0[3], q1[2][3], rp[2];
+            RadialTerms tp[2];
+            LinkGeom gg;
             for (int d = 0; d < 3; ++d) {
-                const double qb = pos_at(R, d, b, q), x = qb - r0[d];
-                const double i0 = rint(x * R.iL);
-                rv[d] = x - i0 * R.L;
-                const double xp = qb - (r0[d] + eps), xm = qb - (r0[d] - eps);
-                const double ip = rint(xp * R.iL), im = rint(xm * R.iL);
-                rs[d][0] = xp - ip * R.L;
-                rs[d][1] = xm - im * R.L;
-                x2[d] = rv[d] * rv[d];
-                vj[d] = pos_at(R, d, bj, q) - pj[d];
-                vk[d] = pos_at(R, d, bk, q) - pk[d];
-                // does either side of the difference see another image of r or r'?
-                wrap[d] = ip != im || rint((rs[d][0] - vj[d]) * R.iL) != rint((rs[d][1] - vj[d]) * R.iL) ||
-                          rint((rs[d][0] - vk[d]) * R.iL) != rint((rs[d][1] - vk[d]) * R.iL);
-                vj[d] += rint((rv[d] - vj[d]) * R.iL) * R.L;
-                vk[d] += rint((rv[d] - vk[d]) * R.iL) * R.L;
+                q0[d] = pos_at(R, d, b, q);
+                for (int lk = 0; lk < 2; ++lk) q1[lk][d] = pos_at(R, d, b1[lk], q);
             }
-            const double rj = sqrt_pos(vj[0] * vj[0] + vj[1] * vj[1] + vj[2] * vj[2]);
-            const double rk = sqrt_pos(vk[0] * vk[0] + vk[1] * vk[1] + vk[2] * vk[2]);
+#pragma unroll
+            for (int lk = 0; lk < 2; ++lk) {
+                link_geom(r0, q0, p1[lk], q1[lk], R.L, R.iL, gg);
+                rp[lk] = gg.rp;
+                tp[lk] = radial_terms(R, bare, gg.rp);
+            }
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                double diff = 0.;
+                double f[2][2];
 #pragma unroll
                 for (int sg = 0; sg < 2; ++sg) {
-                    const double x = rs[d][sg];
-                    double r2 = x * x;
-                    for (int e = 0; e < 3; ++e)
-                        if (e != d) r2 += x2[e];
-                    const double r = sqrt_pos(r2);
-                    double f = 2. * (bare ? bare_radial_lds(R, lds, r) : david_radial_lds(R, lds, r));
+                    double a0[3] = {r0[0], r0[1], r0[2]};
+                    a0[d] = sg ? r0[d] - eps : r0[d] + eps;
+                    RadialTerms t;
+#pragma unroll
                     for (int lk = 0; lk < 2; ++lk) {
-                        const double* v = lk ? vk : vj;
-                        double rp = lk ? rk : rj, y = v[d];
-                        if (wrap[d]) {
-                            // r' follows this side's image
-                            y += rint((x - y) * R.iL) * R.L;
-                            double t = y * y;
-                            for (int e = 0; e < 3; ++e)
-                                if (e != d) t += v[e] * v[e];
-                            rp = sqrt_pos(t);
-                            f += bare ? bare_radial_lds(R, lds, rp) : david_radial_lds(R, lds, rp);
-                        }
-                        if (!bare) {
-                            double s2 = (x - y) * (x - y);
-                            for (int e = 0; e < 3; ++e)
-                                if (e != d) {
-                                    const double sv = rv[e] - v[e];
-                                    s2 += sv * sv;
-                                }
-                            f += david_off_lds<NORD>(R, lds, r, rp, s2);
-                        }
+                        link_geom(a0, q0, p1[lk], q1[lk], R.L, R.iL, gg);
+                        if (lk == 0) t = radial_terms(R, bare, gg.r);
+                        RadialTerms t1 = tp[lk];
+                        if (gg.rp != rp[lk]) t1 = radial_terms(R, bare, gg.rp);  // another image of r'
+                        f[lk][sg] = pair_u_terms(R, bare, t, t1, gg.r, gg.rp, gg.s);
                     }
-                    diff += sg ? -f : f;
                 }
-                g[d] += diff;
+                g[d] += (f[0][0] - f[0][1]) + (f[1][0] - f[1][1]);
             }
         }
-        const double c = (bare ? R.tau : 1.) / (2. * eps);
-        for (int d = 0; d < 3; ++d) sums[((size_t)grp * n + lp) * 3 + d] = c * g[d];
+        for (int d = 0; d < 3; ++d) lds[((size_t)grp * n + lp) * 3 + d] = g[d] / (2. * eps);
     }
     __syncthreads();
     double* o = (out_est ? R.grad_est : R.grad) + 3 * ((size_t)b * N + p0);
     for (int t = threadIdx.x; t < 3 * n; t += kCompatBlock) {
         double v = 0.;
         if (on)
-            for (int i = 0; i < n_grp; ++i) v += sums[(size_t)i * 3 * n + t];
+            for (int i = 0; i < n_grp; ++i) v += lds[(size_t)i * 3 * n + t];
         o[t] = v;
     }
 }
 
+// radial part of the Bare link action / tau at one distance
+__device__ __forceinline__ double bare_radial_lds(const Rep& R, const double* lds, double r) {
+    r = clampd(r, R.r_v_min, R.r_v_max);
+    double v = R.is_coulomb ? 0.5 / r : 0.5 * bt_apply(lds, bt_basis(R.bt_a, r));
+    if (R.use_long_range) {
+        const double* vl = lds + (R.is_coulomb ? 0 : R.bt_a.ncoef);
+        v -= 0.5 * bt_apply(vl, bt_basis(R.bt_b, clampd(r, R.r_l_min, R.r_l_max)));
+    }
+    return v;
+}
 // Analytic adjoint, local terms: kinetic links (b-1,b), (b,b+1) and short-range
 // pair links of every other particle.  Writes (overwrites) grad.
 __global__ __launch_bounds__(64) void k_adjoint_local(const Rep* __restrict__ reps, unsigned int terms, int out_est) {

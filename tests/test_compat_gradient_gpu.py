@@ -1,5 +1,6 @@
-"""The reference's finite-difference gradient on the LDS tables against the kernel
-on the global tables, which forms every link action whole.  Both are central
+"""The reference's finite-difference gradient with a bead's partners shared by a
+workgroup against the kernel with a thread per bead, which forms every link action
+whole.  Both are central
 differences of the same actions at the same points; terms that cancel in the
 difference leave rounding of a few 1e-16 of a link action over 2 eps = 2e-4, far
 below 1e-9 of the largest component.  Sizes at the edges of the particle tiles
