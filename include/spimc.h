@@ -274,7 +274,8 @@ int spimc_get_action_noalloc(spimc_ctx* ctx, uint32_t replica, int action, int m
 int spimc_d_action_d_beta(spimc_ctx* ctx, uint32_t replica, int action, double* out);
 /* Action::Potential (action_class.h:52): pair_action_class.h:369-395. */
 int spimc_potential(spimc_ctx* ctx, uint32_t replica, int action, double* out);
-/* Kinetic::VirialEnergy(window) (kinetic_class.h:48-102). */
+/* Kinetic::VirialEnergy(window) (kinetic_class.h:48-102).  Any window: one longer
+ * than n_bead goes on around the path; 0 takes n_bead. */
 int spimc_kinetic_virial_energy(spimc_ctx* ctx, uint32_t replica, uint32_t window, double* out);
 
 /* Per-bead action gradient out[b][p][3] of the committed path.

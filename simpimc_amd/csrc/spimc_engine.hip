@@ -1905,7 +1905,7 @@ int est_pair_whole(spimc_ctx* c, Rep* base, int nrep, int which) {
     dim3 g2((c->max_nk + 63) / 64, nrep);
     return launch(c, SPIMC_KERNEL_ESTIMATORS, k_long_whole, g2, kSumBlock, 0, c->stream, base, which);
 }
-int est_kin_virial(spimc_ctx* c, Rep* base, int nrep, int W) {
+int est_kin_virial(spimc_ctx* c, Rep* base, int nrep, uint32_t W) {
     const int tiles = (c->max_N + 63) / 64;
     int rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_kin_virial, dim3(tiles, nrep), kVirBlock, 0, c->stream, base, W, c->d_vir);
     if (rc) return rc;
@@ -2037,8 +2037,7 @@ int energy_accumulate(spimc_ctx* c, Rep* base, int nrep) {
             return rc;
         return SPIMC_OK;
     }
-    const int W = (int)c->virial_window;
-    rc = est_kin_virial(c, base, nrep, W);
+    rc = est_kin_virial(c, base, nrep, c->virial_window);
     if (rc) return rc;
     int from_sweep = 0;
     if (c->energy_estimator == SPIMC_ENERGY_VIRIAL_COMPAT) {
@@ -2671,8 +2670,7 @@ int spimc_kinetic_virial_energy(spimc_ctx* c, uint32_t r, uint32_t window, doubl
     if (rc) return rc;
     if (!out) return fail(SPIMC_ERR_ARG, "null output");
     const Rep& R = c->reps[r].dev;
-    const int W = window ? (int)window : 0;
-    rc = est_kin_virial(c, c->d_reps + r, 1, W);
+    rc = est_kin_virial(c, c->d_reps + r, 1, window);
     if (rc || (rc = read_words(c, R.scratch + kSlotVirial * R.M, 1, out, nullptr, 0, nullptr))) return rc;
     return sync_and_resolve(c);
 }

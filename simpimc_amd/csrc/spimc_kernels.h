@@ -2168,48 +2168,83 @@ __global__ __launch_bounds__(kSumBlock) void k_long_whole(const Rep* __restrict_
 // Kinetic::VirialEnergy (kinetic_class.h:48-102): -1 / (4 lambda tau W tau) times
 // the sum over the beads of D . d, d the link leaving the bead and D the W links
 // from it, for 64 particles per workgroup; the walks follow the path: past slice
-// M - 1 a bead is followed by slice 0 of the particle perm[label].  A window of the
-// whole closed path has the same D (its winding) at every bead, and a particle's
-// sum is |D|^2: its links are shared by the workgroup's 16 wavefronts.  Otherwise
-// each wavefront takes a share of the beads, adds the first one's W links and then
-// moves the window.  (A thread per particle took two dependent walks of M slices
-// on one workgroup: 493 us for N = 1024, M = 128, 10 us so.)
+// M - 1 a bead is followed by slice 0 of the particle perm[label], however often a
+// window goes round.  A window of whole turns of a path that closes on itself has
+// the same D (its windings) at every bead, and a particle's sum is D . D of one
+// turn: its links are shared by the workgroup's 16 wavefronts.  Otherwise each
+// wavefront takes a share of the beads, adds the first one's W links and then moves
+// the window.  (A thread per particle took two dependent walks of M slices on one
+// workgroup: 493 us for N = 1024, M = 128, 10 us so.)
 constexpr int kVirBlock = 1024;
-__global__ __launch_bounds__(kVirBlock) void k_kin_virial(const Rep* __restrict__ reps, int W_in, double* __restrict__ part) {
+// A walk along the path from slice b of label l.
+struct PathWalk {
+    int b, l;
+    double x[3];
+    __device__ __forceinline__ PathWalk(const Rep& R, int b_, int l_) : b(b_), l(l_) {
+        for (int d = 0; d < 3; ++d) x[d] = pos_at(R, d, b, l);
+    }
+    // the link to the next bead into t
+    __device__ __forceinline__ void step(const Rep& R, double* t) {
+        if (++b == R.M) {
+            b = 0;
+            l = label_after_wrap(R, l);
+        }
+        for (int d = 0; d < 3; ++d) {
+            const double y = pos_at(R, d, b, l);
+            t[d] = minimg(y - x[d], R.L, R.iL);
+            x[d] = y;
+        }
+    }
+};
+__global__ __launch_bounds__(kVirBlock) void k_kin_virial(const Rep* __restrict__ reps, unsigned int W_in,
+                                                          double* __restrict__ part) {
     const Rep& R = reps[blockIdx.y];
-    const int M = R.M, N = R.N, W = W_in > 0 ? W_in : M;
+    const int M = R.M, N = R.N;
+    const unsigned int W = W_in > 0 ? W_in : (unsigned int)M;
     constexpr int G = kVirBlock / kWave;
     __shared__ double sh[kVirBlock * 3];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, p = blockIdx.x * kWave + lane;
     if ((int)blockIdx.x * kWave >= N) return;
     const bool valid = p < N;
-    // link leaving position c of the walk from (p, 0), 0 <= c < 2 M
-    const int pw = valid ? label_after_wrap(R, p) : 0;
-    auto link = [&](int c, double* t) {
-        const int b = c < M ? c : c - M, l = c < M ? p : pw;
-        const int bn = b + 1 == M ? 0 : b + 1, ln = b + 1 == M ? label_after_wrap(R, l) : l;
-        for (int d = 0; d < 3; ++d) t[d] = minimg(pos_at(R, d, bn, ln) - pos_at(R, d, b, l), R.L, R.iL);
-    };
     const int lo = (int)((long long)M * w / G), hi = (int)((long long)M * (w + 1) / G);
-    const bool ring = W == M && R.perm == nullptr;
+    const bool ring = W % (unsigned int)M == 0 && R.perm == nullptr;
     double D[3] = {0., 0., 0.}, t[3], tot = 0.;
-    if (valid && ring) {
-        for (int c = lo; c < hi; ++c) {
-            link(c, t);
-            for (int d = 0; d < 3; ++d) D[d] += t[d];
-        }
-    } else if (valid && lo < hi) {
-        for (int c = lo; c < lo + W; ++c) {
-            link(c, t);
-            for (int d = 0; d < 3; ++d) D[d] += t[d];
-        }
-        for (int c = lo; c < hi; ++c) {
-            double a[3];
-            link(c, a);
-            tot += D[0] * a[0] + D[1] * a[1] + D[2] * a[2];
-            if (c + 1 == hi) break;
-            link(c + W, t);
-            for (int d = 0; d < 3; ++d) D[d] += t[d] - a[d];
+    if (valid && lo < hi) {
+        PathWalk end(R, lo, p);
+        if (ring) {
+            for (int c = lo; c < hi; ++c) {
+                end.step(R, t);
+                for (int d = 0; d < 3; ++d) D[d] += t[d];
+            }
+        } else {
+            unsigned long long left = W;
+            if (W > (unsigned int)M) {
+                // whole turns of the closed path (M slices of every label of its
+                // cycle) are walked once
+                unsigned long long turn = M;
+                for (int l = label_after_wrap(R, p); l != p; l = label_after_wrap(R, l)) turn += M;
+                if (W >= turn) {
+                    for (unsigned long long i = 0; i < turn; ++i) {
+                        end.step(R, t);
+                        for (int d = 0; d < 3; ++d) D[d] += t[d];
+                    }
+                    for (int d = 0; d < 3; ++d) D[d] *= (double)(W / turn);
+                    left = W % turn;
+                }
+            }
+            for (; left > 0; --left) {
+                end.step(R, t);
+                for (int d = 0; d < 3; ++d) D[d] += t[d];
+            }
+            PathWalk start(R, lo, p);
+            for (int c = lo; c < hi; ++c) {
+                double a[3];
+                start.step(R, a);
+                tot += D[0] * a[0] + D[1] * a[1] + D[2] * a[2];
+                if (c + 1 == hi) break;
+                end.step(R, t);
+                for (int d = 0; d < 3; ++d) D[d] += t[d] - a[d];
+            }
         }
     }
     for (int d = 0; d < 3; ++d) sh[threadIdx.x * 3 + d] = ring ? D[d] : d == 0 ? tot : 0.;
@@ -2219,16 +2254,17 @@ __global__ __launch_bounds__(kVirBlock) void k_kin_virial(const Rep* __restrict_
     for (int i = 0; i < G; ++i)
         for (int d = 0; d < 3; ++d) v[d] += sh[(i * kWave + lane) * 3 + d];
     tot = wave_sum(ring ? v[0] * v[0] + v[1] * v[1] + v[2] * v[2] : v[0]);
+    if (ring) tot *= (double)(W / (unsigned int)M);
     if (lane == 0) part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = -tot * R.kin_i4lt / (W * R.tau);
 }
 // its workgroups' sums and the constant into the replica's scratch
-__global__ __launch_bounds__(64) void k_kin_virial_sum(const Rep* __restrict__ reps, int W_in, int n_part, int slot,
+__global__ __launch_bounds__(64) void k_kin_virial_sum(const Rep* __restrict__ reps, unsigned int W_in, int n_part, int slot,
                                                        const double* __restrict__ part) {
     const Rep& R = reps[blockIdx.x];
     double t = 0.;
     for (int i = threadIdx.x; i < (R.N + kWave - 1) / kWave; i += kWave) t += part[(size_t)blockIdx.x * n_part + i];
     t = wave_sum(t);
-    if (threadIdx.x == 0) R.scratch[slot * R.M] = R.kin_dbeta_const / (W_in > 0 ? W_in : R.M) + t;
+    if (threadIdx.x == 0) R.scratch[slot * R.M] = R.kin_dbeta_const / (W_in > 0 ? W_in : (unsigned int)R.M) + t;
 }
 
 // ---------------------------------------------------------------------------
