@@ -21,6 +21,24 @@ constexpr int kMaxKinSplines = 8; // kinetic / bisect image splines at tau * 2^l
 // NEW; long-range pair OLD, NEW; log sample ratio; previous level's change
 constexpr int kTraceWords = 8;
 
+// Wavefronts per window link of a W-wavefront workgroup: a link's partners are
+// split over up to W wavefronts of at least qpw (64, 128 or 256) partners each.
+template <int W>
+__host__ __device__ __forceinline__ int pair_split(int N, int qpw) {
+    const int n = (N + qpw - 1) / qpw;
+    return n < W ? n : W;
+}
+
+// The k-th of a link's ns partner ranges, [first, past the last): 64 partners each,
+// or a multiple of 128, so the last ranges can be short or empty (N = 257 over four:
+// 128, 128, 1 and none).
+__host__ __device__ __forceinline__ int2 pair_range(int N, int ns, int k) {
+    const int q_each = (N + ns - 1) / ns;
+    const int q_len = q_each <= kWave ? kWave : (q_each + 2 * kWave - 1) / (2 * kWave) * (2 * kWave);
+    const int lo = k * q_len, hi = lo + q_len;
+    return make_int2(lo < N ? lo : N, hi < N ? hi : N);
+}
+
 // Natural cubic spline: s(t) = c0 + dt (c1 + dt (c2 + dt c3)), dt = t - x[i].
 struct Spl {
     const double* x;  // [n] knots

@@ -859,7 +859,7 @@ constexpr int kPairLdsBlock = 1024;
 // run over the partners q; the OLD and NEW sums of link j go to pair_part[j]
 // (COH: as agent-scope atomic stores).
 // One lane's OLD and NEW sums of window link j over the partners q_lo + lane,
-// q_lo + lane + 64, ... below q_hi (q_lo a multiple of 128).
+// q_lo + lane + 64, ... below q_hi (at least one: the lanes without one load q_lo).
 // ONE: ranges of at most 64 partners take one each (k_pair_lds has none; the
 // second copy of the evaluation would cost it registers).
 template <int PT, int NORD, bool ONE = false>
@@ -939,31 +939,22 @@ __device__ __forceinline__ void pair_links_lds(const Rep& R, const double* lds, 
     }
 }
 
-// Wavefronts per window link of a W-wavefront workgroup: a link's partners are
-// split over up to W wavefronts of at least qpw (64, 128 or 256) partners each.
-template <int W>
-__host__ __device__ __forceinline__ int pair_split(int N, int qpw) {
-    const int n = (N + qpw - 1) / qpw;
-    return n < W ? n : W;
-}
-
 // The window links of a proposal on a W-wavefront workgroup (part of bpr for
 // the replica), ns = pair_split<W>(N, qpw) wavefronts per link: wavefront w takes
-// link jb + w / ns and partner range w % ns, ranges of q_len partners (64, or a
-// multiple of 128).  A link's sum adds its ranges' wavefront sums in range
+// link jb + w / ns and partner range w % ns (pair_range; an empty one adds nothing).
+// A link's sum adds its ranges' wavefront sums in range
 // order; with ns = 1 it is pair_links_lds's.  Every wavefront of the
 // workgroup calls it (it holds workgroup barriers); wpart: W entries of LDS.
 template <int PT, int NORD, bool COH, int W>
 __device__ __forceinline__ void pair_links_split(const Rep& R, const double* lds, const Prop& pr, int part, int bpr,
                                                  int qpw, int w, int lane, double2* wpart) {
     const int ns = pair_split<W>(R.N, qpw), lpb = W / ns;
-    const int q_each = (R.N + ns - 1) / ns;
-    const int q_len = q_each <= kWave ? kWave : (q_each + 2 * kWave - 1) / (2 * kWave) * (2 * kWave);
+    const int2 qr = pair_range(R.N, ns, w % ns);
     for (int jb = part * lpb; jb < pr.n_links; jb += bpr * lpb) {
-        const int j = jb + w / ns, k = w % ns;
+        const int j = jb + w / ns;
         double uo = 0., un = 0.;
-        if (w < lpb * ns && j < pr.n_links) {
-            pair_link_range<PT, NORD, true>(R, lds, pr, j, k * q_len, min(R.N, (k + 1) * q_len), lane, uo, un);
+        if (w < lpb * ns && j < pr.n_links && qr.x < qr.y) {
+            pair_link_range<PT, NORD, true>(R, lds, pr, j, qr.x, qr.y, lane, uo, un);
             uo = wave_sum(uo);
             un = wave_sum(un);
         }
