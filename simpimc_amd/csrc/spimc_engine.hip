@@ -441,7 +441,8 @@ struct spimc_ctx {
     double* d_adj_part = nullptr;
     size_t adj_part_cap = 0;
     bool perm_table = false;  // the running permuting stage is PermBisectTable's
-    int tab_n = 0;            // largest replica whose cycle table fits in the table proposal's LDS
+    int tab_max_n = 0;        // largest replica with a configured cycle table
+    int tab_n = 0;            // largest of them whose table fits in the table proposal's LDS (0: not set)
     bool adj_pairs_ok = false;  // its tables and slots fit in LDS
     int groups_wanted = 1;
     bool fork = false;  // rho_k beside the pair kernel on a second stream per group
@@ -1469,9 +1470,9 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
     int rc;
     const bool tuned = c->lds_doubles_max > 0;
     if (c->perm_table) {
-        const size_t shmem = tab_lds_head(c->max_N) + (size_t)c->tab_n * c->tab_n * sizeof(double);
+        const size_t shmem = tab_lds_head(c->tab_max_n) + (size_t)c->tab_n * c->tab_n * sizeof(double);
         rc = launch(c, SPIMC_KERNEL_PROPOSE, k_propose_perm<true>, R, kTabBlock, shmem, st, reps, R, (int)tuned,
-                    c->perm_stage, c->max_N, c->tab_n);
+                    c->perm_stage, c->tab_max_n, c->tab_n);
     } else {
         const size_t shmem = (size_t)c->max_N * (sizeof(double) + sizeof(int));
         rc = launch(c, SPIMC_KERNEL_PROPOSE, k_propose_perm<false>, R, kPermBlock, shmem, st, reps, R, (int)tuned,
@@ -1727,17 +1728,24 @@ int ensure_perm(spimc_ctx* c, bool scratch) {
     return upload_reps(c);
 }
 
-// The LDS of the table proposal: what its static arrays, the rows and the
-// binomials leave of the CU's 160 KB holds the cycle table of replicas of up to
-// tab_n particles (about 125); larger ones keep theirs in global memory.
+// The LDS of the table proposal, for the replicas that have a cycle table (at most
+// kTabMaxN particles; larger ones of the context take no attempts): what its static
+// arrays, the rows and the binomials leave of the CU's 160 KB holds the table of
+// replicas of up to tab_n particles (about 125); larger ones keep theirs in global
+// memory.
 int set_tab_lds(spimc_ctx* c) {
     if (c->tab_n) return SPIMC_OK;
     hipFuncAttributes at{};
     HIPCHK(hipFuncGetAttributes(&at, (const void*)k_propose_perm<true>));
-    const size_t used = at.sharedSizeBytes + tab_lds_head(c->max_N), cap = 160 * 1024;
+    c->tab_max_n = 1;
+    for (const auto& h : c->reps)
+        if (h.dev.tab_k > 0) c->tab_max_n = std::max(c->tab_max_n, h.dev.N);
+    const size_t used = at.sharedSizeBytes + tab_lds_head(c->tab_max_n), cap = 160 * 1024;
+    if (used + sizeof(double) > cap)
+        return fail(SPIMC_ERR_UNSUPPORTED, "the table proposal's rows and binomials exceed the workgroup's LDS");
     int n = 1;
     for (const auto& h : c->reps)
-        if (used + (size_t)h.dev.N * h.dev.N * sizeof(double) <= cap) n = std::max(n, h.dev.N);
+        if (h.dev.tab_k > 0 && used + (size_t)h.dev.N * h.dev.N * sizeof(double) <= cap) n = std::max(n, h.dev.N);
     HIPCHK(hipFuncSetAttribute((const void*)k_propose_perm<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)(cap - at.sharedSizeBytes)));
     c->tab_n = n;
@@ -2808,6 +2816,7 @@ int spimc_perm_table_configure(spimc_ctx* c, uint32_t r, uint32_t n_perm_part, u
     if (!h.perm_t) HIPCHK(hipMalloc((void**)&h.perm_t, (size_t)N * N * sizeof(double)));
     h.dev.perm_t = h.perm_t;
     h.dev.tab_k = (int)n_perm_part;
+    c->tab_n = 0;  // set again by the next stage
     h.dev.tab_balance = (int)balance;
     return upload_reps(c);
 }

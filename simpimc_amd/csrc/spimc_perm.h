@@ -38,7 +38,7 @@ __device__ __forceinline__ double chain_new(const Rep& R, int b0, int nb, int n,
 }
 
 // bytes of the table proposal's dynamic LDS before its table: the walk's row and
-// visited map, and the binomials, of the largest replica
+// visited map, and the binomials, of the largest replica that has a cycle table
 __host__ __device__ inline size_t tab_lds_head(int max_n) {
     return ((size_t)max_n * (sizeof(double) + sizeof(int)) + (size_t)7 * (max_n + 1) * sizeof(unsigned int) + 15) &
            ~(size_t)15;
