@@ -244,6 +244,11 @@ BTabHost make_btab(const double* x, int n, const std::vector<const double*>& ys)
 }
 
 constexpr size_t kPairLdsMaxBytes = 150 * 1024;
+// Bounds of the workspaces that the context grows to its largest call and keeps: past
+// them (or where the memory is not to be had) the replicas are taken in turn, or the
+// kernels that need none run.  The weights' holds 59 replicas of N = 256, M = 128 with
+// 1979 k-vectors, the shares' 2600 links of N = 1024: several times what fills the GPU.
+constexpr size_t kWorkCols = 512u << 20, kWorkLinks = 128u << 20, kWorkRows = 32u << 20;
 constexpr size_t kStageBytes = 256 * 1024;  // staging area of small reads (larger ones are plain copies)
 
 struct RepHost {
@@ -467,6 +472,9 @@ struct spimc_ctx {
     int col_max = 0, col_stride = 0;
     double4* d_col_w = nullptr;
     size_t col_w_cap = 0;
+    // what the workspaces may take: the column weights, the links' shares and the rows
+    // of a rho_k download (SPIMC_WORK_BYTES lowers them)
+    size_t work_cols = kWorkCols, work_links = kWorkLinks, work_rows = kWorkRows;
     // timing: per-launch dispatch events (every kernel) and device clocks (pair, rho_k)
     bool timing = false, clock = false;
     double clock_hz = 0.;
@@ -1239,13 +1247,29 @@ int build_groups(spimc_ctx* c, int n_groups) {
     return SPIMC_OK;
 }
 
-int ensure_tmp(spimc_ctx* c, size_t n_doubles) {
-    if (n_doubles > c->tmp_cap) {
-        if (c->d_tmp) (void)hipFree(c->d_tmp);
-        c->d_tmp = nullptr;
-        HIPCHK(hipMalloc((void**)&c->d_tmp, n_doubles * sizeof(double)));
-        c->tmp_cap = n_doubles;
+// Grows a workspace of the context to n entries; false where the memory is not to be
+// had, with the workspace gone: callers that were only faster with it take the
+// kernels that need none.
+bool grow(spimc_ctx* c, void** buf, size_t& cap, size_t n, size_t entry) {
+    if (n <= cap) return true;
+    if (*buf) {
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipFree(*buf);
     }
+    *buf = nullptr;
+    cap = 0;
+    if (hipMalloc(buf, n * entry) != hipSuccess) {
+        *buf = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    cap = n;
+    return true;
+}
+
+int ensure_tmp(spimc_ctx* c, size_t n_doubles) {
+    if (!grow(c, (void**)&c->d_tmp, c->tmp_cap, n_doubles, sizeof(double)))
+        return fail(SPIMC_ERR_NOMEM, "interface partials");
     return SPIMC_OK;
 }
 
@@ -1927,64 +1951,87 @@ int est_finalize(spimc_ctx* c, Rep* base, int nrep, int what, int acc) {
                   c->lds_whole_max > 0 ? (const double*)c->d_whole : (const double*)nullptr, S * Q);
 }
 // The long-range adjoint by columns: the slices' weights, then the particles, as
-// many replicas at a time as keep the weights within kColBytes.
-constexpr size_t kColBytes = 512u << 20;
-int est_long_cols(spimc_ctx* c, Rep* base, int nrep, int out_est, int compat) {
-    const size_t per = (size_t)c->max_M * c->col_stride;
-    const int step = (int)std::max<size_t>(1, std::min<size_t>(nrep, kColBytes / sizeof(double4) / per));
-    if (per * step > c->col_w_cap) {
-        HIPCHK(hipStreamSynchronize(c->stream));
-        if (c->d_col_w) (void)hipFree(c->d_col_w);
-        c->d_col_w = nullptr;
-        c->col_w_cap = 0;
-        HIPCHK(hipMalloc((void**)&c->d_col_w, per * step * sizeof(double4)));
-        c->col_w_cap = per * step;
-    }
+// many replicas at a time as keep the weights within work_cols bytes.  *done: 0 where
+// there is no room for a replica's weights.
+int est_long_cols(spimc_ctx* c, Rep* base, int nrep, int max_M, int max_N, int out_est, int compat, bool* done) {
+    const size_t per = (size_t)max_M * c->col_stride;
+    const int step = (int)std::min<size_t>(nrep, c->work_cols / sizeof(double4) / per);
+    *done = step > 0 && grow(c, (void**)&c->d_col_w, c->col_w_cap, per * step, sizeof(double4));
+    if (!*done) return SPIMC_OK;
     auto fn = c->col_max <= 8 ? k_adjoint_cols<8> : c->col_max <= 12 ? k_adjoint_cols<12> : k_adjoint_cols<kAdjColMax>;
     for (int r = 0; r < nrep; r += step) {
-        const int n = std::min(step, nrep - r), tiles = (c->max_N + 63) / 64;
+        const int n = std::min(step, nrep - r), tiles = (max_N + 63) / 64;
         // segments: enough wavefronts for three per SIMD
-        const long long waves = (long long)tiles * c->max_M * n;
+        const long long waves = (long long)tiles * max_M * n;
         const int seg = (int)std::max<long long>(1, std::min<long long>(8, 12 * kNumCUs / std::max<long long>(1, waves)));
         const int tpb = seg > 1 ? 1 : std::min(4, tiles);
-        int rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_weights, dim3(c->max_M, n), 256, 0, c->stream, base + r,
-                        c->max_M, c->col_stride, c->d_col_w);
+        int rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_weights, dim3(max_M, n), 256, 0, c->stream, base + r, max_M,
+                        c->col_stride, c->d_col_w);
         if (!rc)
-            rc = launch(c, SPIMC_KERNEL_ADJOINT, fn, dim3((tiles + tpb - 1) / tpb, c->max_M, n), 64 * seg * tpb, 0, c->stream,
-                        base + r, seg, c->max_M, c->col_stride, (const double4*)c->d_col_w, out_est, compat);
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, fn, dim3((tiles + tpb - 1) / tpb, max_M, n), 64 * seg * tpb, 0, c->stream,
+                        base + r, seg, max_M, c->col_stride, (const double4*)c->d_col_w, out_est, compat);
+        if (rc) return rc;
+    }
+    return SPIMC_OK;
+}
+// The adjoint's local terms with a workgroup per link (h of them when the links are
+// few), as many replicas at a time as keep the shares within work_links bytes.
+// *done: 0 where there is no room for a replica's shares.
+int est_links(spimc_ctx* c, Rep* base, int nrep, int max_M, int max_N, uint32_t terms, int out_est, size_t shmem, bool* done) {
+    // workgroups per link: as many as give every CU one, at most one per tile pair
+    const int tiles = (max_N + 63) / 64;
+    const int h = std::max(1, std::min(tiles * (tiles + 1) / 2, kNumCUs / std::max(1, max_M * nrep)));
+    const size_t per = (size_t)h * max_M * 6 * max_N;
+    const int step = (int)std::min<size_t>(nrep, c->work_links / sizeof(double) / per);
+    *done = step > 0 && grow(c, (void**)&c->d_adj_part, c->adj_part_cap, per * step, sizeof(double));
+    if (!*done) return SPIMC_OK;
+    for (int r = 0; r < nrep; r += step) {
+        const int n = std::min(step, nrep - r);
+        int rc = SPIMC_OK;
+        if (terms & SPIMC_GRAD_PAIR_SHORT)
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_links_fn, dim3(max_M * h, n), kAdjLdsBlock, shmem, c->stream, base + r,
+                        h, max_M, max_N, c->d_adj_part);
+        if (!rc)
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_gather, dim3(max_M, n), 256, 0, c->stream, base + r, terms, out_est,
+                        h, max_M, max_N, (const double*)c->d_adj_part);
         if (rc) return rc;
     }
     return SPIMC_OK;
 }
 int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, int out_est) {
-    dim3 g((c->max_N + 63) / 64, c->max_M, nrep);
+    // the extent of these replicas (a query's is one of the context's)
+    int max_M = 1, max_N = 1;
+    bool any_long = false, ilkka_long = false;
+    for (int r = 0; r < nrep; ++r) {
+        const Rep& x = c->reps[(base - c->d_reps) + r].dev;
+        max_M = std::max(max_M, x.M);
+        max_N = std::max(max_N, x.N);
+        any_long |= x.use_long_range != 0;
+        ilkka_long |= x.use_long_range && x.pair_type == SPIMC_PAIR_ILKKA;
+    }
+    dim3 g((max_N + 63) / 64, max_M, nrep);
     int rc;
     if (compat) {
         const int short_on = (terms & SPIMC_GRAD_PAIR_SHORT) ? 1 : 0;
         if (c->compat_fn) {
             // particles per workgroup: halved until the workgroups number the CUs
-            int np = std::min(c->max_N, kCompatBlock);
-            while (np > 64 && (long long)c->max_M * nrep * ((c->max_N + np - 1) / np) < kNumCUs) np = (np + 1) / 2;
+            int np = std::min(max_N, kCompatBlock);
+            while (np > 64 && (long long)max_M * nrep * ((max_N + np - 1) / np) < kNumCUs) np = (np + 1) / 2;
             const size_t shmem = (size_t)kCompatBlock * 3 * sizeof(double);
-            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(c->max_M, (c->max_N + np - 1) / np, nrep), kCompatBlock,
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(max_M, (max_N + np - 1) / np, nrep), kCompatBlock,
                         shmem, c->stream, base, out_est, short_on, np);
         } else {
             rc = launch(c, SPIMC_KERNEL_ADJOINT, k_grad_compat, g, 64, 0, c->stream, base, out_est, short_on);
-        }
-        bool ilkka_long = false;
-        for (int r = 0; r < nrep; ++r) {
-            const Rep& Rr = c->reps[(base - c->d_reps) + r].dev;
-            ilkka_long |= Rr.pair_type == SPIMC_PAIR_ILKKA && Rr.use_long_range;
         }
         if (!ilkka_long) return rc;
     } else if (c->lds_adj_max > 0) {
         const size_t shmem = (size_t)c->lds_adj_max * sizeof(double);
         // workgroups per replica: enough to fill the GPU when the replicas are few
-        const int bpr = std::max(1, std::min(c->max_M, (2 * kNumCUs + nrep - 1) / nrep));
+        const int bpr = std::max(1, std::min(max_M, (2 * kNumCUs + nrep - 1) / nrep));
         // pair-once kernel: at most max_M / 2 link ranges of 16 waves' worth per
         // replica; chosen when they give at least kAdjPairsMinWaves waves, else the
         // workgroup-per-link form
-        const int rng_max = std::max(1, c->max_M / 2);
+        const int rng_max = std::max(1, max_M / 2);
         const int bpr2 = std::max(1, std::min((rng_max + kAdjPairWaves - 1) / kAdjPairWaves,
                                               (int)((kAdjPairsMinWaves + kAdjPairWaves * nrep - 1) / (kAdjPairWaves * nrep))));
         const long long waves2 = (long long)nrep * std::min(kAdjPairWaves * bpr2, rng_max);
@@ -1996,37 +2043,24 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
             if (!rc)
                 rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_pairs_fn, dim3(nrep, bpr2), kAdjLdsBlock, shmem2, c->stream,
                             base, terms, out_est, 1);
-        } else if (form == 2) {
-            // workgroups per link: as many as give every CU one, at most one per tile pair
-            const int tiles = (c->max_N + 63) / 64;
-            const int h = std::max(1, std::min(tiles * (tiles + 1) / 2, kNumCUs / std::max(1, c->max_M * nrep)));
-            const size_t need = (size_t)nrep * h * c->max_M * 6 * c->max_N;
-            if (need > c->adj_part_cap) {
-                HIPCHK(hipStreamSynchronize(c->stream));
-                if (c->d_adj_part) (void)hipFree(c->d_adj_part);
-                c->d_adj_part = nullptr;
-                c->adj_part_cap = 0;
-                HIPCHK(hipMalloc((void**)&c->d_adj_part, need * sizeof(double)));
-                c->adj_part_cap = need;
-            }
-            rc = SPIMC_OK;
-            if (terms & SPIMC_GRAD_PAIR_SHORT)
-                rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_links_fn, dim3(c->max_M * h, nrep), kAdjLdsBlock, shmem2,
-                            c->stream, base, h, c->max_M, c->max_N, c->d_adj_part);
-            if (!rc)
-                rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_gather, dim3(c->max_M, nrep), 256, 0, c->stream, base,
-                            terms, out_est, h, c->max_M, c->max_N, (const double*)c->d_adj_part);
         } else {
-            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_lds_fn, dim3(nrep, bpr), kAdjLdsBlock, shmem, c->stream, base,
-                        terms, out_est);
+            bool done = false;
+            rc = form == 2 ? est_links(c, base, nrep, max_M, max_N, terms, out_est, shmem2, &done) : SPIMC_OK;
+            if (!rc && !done)
+                rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_lds_fn, dim3(nrep, bpr), kAdjLdsBlock, shmem, c->stream, base,
+                            terms, out_est);
         }
     } else {
         rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_local, g, 64, 0, c->stream, base, terms, out_est);
     }
-    if (rc || !(terms & SPIMC_GRAD_PAIR_LONG) || !c->any_long) return rc;
-    if (c->col_max > 0) return est_long_cols(c, base, nrep, out_est, compat);
+    if (rc || !(terms & SPIMC_GRAD_PAIR_LONG) || !any_long) return rc;
+    if (c->col_max > 0) {
+        bool done = false;
+        rc = est_long_cols(c, base, nrep, max_M, max_N, out_est, compat, &done);
+        if (rc || done) return rc;
+    }
     if (c->adj_runs_lds > 0) {
-        dim3 gr(c->max_M, nrep);
+        dim3 gr(max_M, nrep);
         return launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_long_runs, gr, kAdjRunBlock, c->adj_runs_lds, c->stream, base,
                       out_est, compat);
     }
@@ -2309,6 +2343,12 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
         for (auto& h : c->reps)
             if (h.dev.use_long_range)
                 c->adj_runs_lds = std::max(c->adj_runs_lds, (size_t)h.dev.nk * sizeof(double2) + (size_t)h.dev.n_runs * sizeof(int4));
+        if (const char* f = std::getenv("SPIMC_WORK_BYTES")) {
+            const size_t v = (size_t)std::max(0ll, std::atoll(f));
+            c->work_cols = std::min(c->work_cols, v);
+            c->work_links = std::min(c->work_links, v);
+            c->work_rows = std::min(c->work_rows, v);
+        }
         // every replica's columns fit the unrolled form (SPIMC_ADJ_RUNS = 0 or 1 asks for the others)
         const char* fr = std::getenv("SPIMC_ADJ_RUNS");
         for (auto& h : c->reps)
@@ -2432,13 +2472,25 @@ int spimc_rho_k_download(spimc_ctx* c, uint32_t r, double* rho) {
     if (!rho) return fail(SPIMC_ERR_ARG, "null output");
     const Rep& R = c->reps[r].dev;
     if (!R.use_long_range) return fail(SPIMC_ERR_STATE, "replica has no long-range action");
-    // the committed rows lie in two buffers: gathered on the device, then one copy
-    // (a copy a row took 1.2 ms for 128 rows)
-    if ((rc = ensure_tmp(c, (size_t)2 * R.M * R.nk))) return rc;
-    k_gather_rho<<<R.M, 256, 0, c->stream>>>(c->d_reps, (int)r, reinterpret_cast<double2*>(c->d_tmp));
-    HIPCHK(hipGetLastError());
+    // the committed rows lie in two buffers: gathered on the device, as many as fit in
+    // work_rows bytes, then one copy (a copy a row took 1.2 ms for 128 rows)
+    const size_t row = (size_t)R.nk * sizeof(double2);
+    const int step = (int)std::min<size_t>(R.M, c->work_rows / std::max<size_t>(row, 1));
+    if (step > 0 && grow(c, (void**)&c->d_tmp, c->tmp_cap, (size_t)2 * step * R.nk, sizeof(double))) {
+        for (int b = 0; b < R.M; b += step) {
+            const int n = std::min(step, R.M - b);
+            k_gather_rho<<<n, 256, 0, c->stream>>>(c->d_reps, (int)r, b, reinterpret_cast<double2*>(c->d_tmp));
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(c->stream));
+            HIPCHK(hipMemcpy(rho + (size_t)2 * b * R.nk, c->d_tmp, n * row, hipMemcpyDeviceToHost));
+        }
+        return SPIMC_OK;
+    }
     HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipMemcpy(rho, c->d_tmp, (size_t)R.M * R.nk * sizeof(double2), hipMemcpyDeviceToHost));
+    std::vector<unsigned char> sel(R.M);
+    HIPCHK(hipMemcpy(sel.data(), R.sel, R.M, hipMemcpyDeviceToHost));
+    for (int b = 0; b < R.M; ++b)
+        HIPCHK(hipMemcpy(rho + (size_t)2 * b * R.nk, R.rho + ((size_t)sel[b] * R.M + b) * R.nk, row, hipMemcpyDeviceToHost));
     return SPIMC_OK;
 }
 

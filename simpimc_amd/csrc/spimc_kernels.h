@@ -1807,12 +1807,12 @@ __global__ __launch_bounds__(256) void k_pack_accepted(const Rep* __restrict__ r
     const unsigned char* a = reps[blockIdx.x].accepted;
     for (unsigned int i = threadIdx.x; i < n; i += 256) out[(size_t)blockIdx.x * mx + i] = a[i];
 }
-// the committed rho_k rows in slice order
-__global__ __launch_bounds__(256) void k_gather_rho(const Rep* __restrict__ reps, int r, double2* __restrict__ out) {
+// the committed rho_k rows of the slices from first in order
+__global__ __launch_bounds__(256) void k_gather_rho(const Rep* __restrict__ reps, int r, int first, double2* __restrict__ out) {
     const Rep& R = reps[r];
-    const int b = blockIdx.x;
+    const int b = first + blockIdx.x;
     const double2* row = R.rho + ((size_t)R.sel[b] * R.M + b) * R.nk;
-    for (int k = threadIdx.x; k < R.nk; k += 256) out[(size_t)b * R.nk + k] = row[k];
+    for (int k = threadIdx.x; k < R.nk; k += 256) out[(size_t)blockIdx.x * R.nk + k] = row[k];
 }
 
 // Stage set-up on the device (kept out of hipMemset so captured graphs stay plain kernels)
