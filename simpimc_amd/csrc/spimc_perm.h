@@ -1238,7 +1238,7 @@ __global__ __launch_bounds__(kRhoBlock) void k_rho_multi_list(const Rep* __restr
     }
 }
 
-// Both lists in one launch, for rounds too small to fork: the first n_pair
+// Both lists in one launch, for rounds with few listed proposals: the first n_pair
 // workgroups loop over the pair items, the others over the rho_k items, side by
 // side (16 replicas of N = 32 with the cycle table: a round 112 us on two streams with
 // the one-chain kernels, 96 us so).
