@@ -416,7 +416,8 @@ int spimc_obs_reset(spimc_ctx* ctx, uint32_t which);
 int spimc_sweep(spimc_ctx* ctx, uint32_t n_sweeps, uint32_t flags);
 /* Bead updates performed so far (Bisect: 2^l - 1 per attempt, Displace: M). */
 int spimc_bead_updates(spimc_ctx* ctx, uint64_t* out);
-/* Launch-shape autotuning.  For each candidate shape (rho_k kernel beside the
+/* Launch-shape autotuning.  For each candidate shape (what the context chooses by
+ * rule for each move and stage, its default; rho_k kernel beside the
  * pair kernel or after it, rho_k workgroups per CU, pair workgroup size; and,
  * when every replica has N M <= 16384 on unpermuted paths, the persistent
  * stage kernel that runs a replica's whole stage in one workgroup, with 256,
@@ -431,7 +432,8 @@ int spimc_bead_updates(spimc_ctx* ctx, uint64_t* out);
  * the shape never changes results beyond rounding.  chosen (optional, 7 ints):
  * fork, rho_k workgroups per CU, pair workgroup size, number of shapes tried,
  * n_displace, persistent stage workgroup size (0: rounds of launches),
- * one-launch rounds for bisection (1), for both moves (2), or none (0).  No
+ * one-launch rounds for bisection (1), for both moves (2), or none (0); where the
+ * rules are kept, what they choose for bisection rounds.  No
  * counterpart in the reference. */
 int spimc_autotune(spimc_ctx* ctx, uint32_t n_rounds, int32_t* chosen);
 

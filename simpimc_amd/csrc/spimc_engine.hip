@@ -401,6 +401,17 @@ struct Group {
     unsigned int* d_arrive = nullptr;
 };
 
+// A launch shape of the move rounds: rho_k beside the pair kernel and its looping
+// workgroups per CU, the pair workgroup size, the persistent stage kernel's, one-launch
+// rounds and for which moves; and which of them the rules choose per stage instead.
+struct LaunchShape {
+    bool fork = false;
+    int bpc = 0, block = kPairLdsBlock, pers = 0;
+    bool one = false;
+    int one_moves = 1;
+    bool auto_fork = true, auto_block = true, auto_one = true;
+};
+
 struct spimc_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -439,6 +450,7 @@ struct spimc_ctx {
     // launch shapes chosen per stage by rule (fork_now, pair_block_now,
     // one_launch_now) until an environment variable or spimc_autotune sets them
     bool auto_fork = true, auto_block = true, auto_one = true;
+    LaunchShape ruled;  // the shape that the context began with
     int pair_variant = 3;  // 0 Bare, 1 David order 2, 2 David other order, 3 mixed
     void (*adj_lds_fn)(const Rep*, unsigned int, int) = nullptr;
     // the pair-once adjoint (two launches), used when its link ranges give the
@@ -1423,6 +1435,22 @@ int set_pers_block(spimc_ctx* c, int bs) {
     c->pers_block = bs;
     c->pers_fn = fn;
     return SPIMC_OK;
+}
+
+LaunchShape get_shape(const spimc_ctx* c) {
+    return {c->fork,      c->rho_bpc,   c->pair_block, c->pers_block, c->one_launch,
+            c->one_moves, c->auto_fork, c->auto_block, c->auto_one};
+}
+int set_shape(spimc_ctx* c, const LaunchShape& s) {
+    c->fork = s.fork;
+    c->rho_bpc = s.bpc;
+    c->one_launch = s.one;
+    c->one_moves = s.one_moves;
+    c->auto_fork = s.auto_fork;
+    c->auto_block = s.auto_block;
+    c->auto_one = s.auto_one;
+    int rc = c->lds_doubles_max > 0 ? set_pair_block(c, s.block) : SPIMC_OK;
+    return rc ? rc : set_pers_block(c, s.pers);
 }
 
 // Drops the captured round and stage graphs (the launch shape changed).
@@ -2411,6 +2439,7 @@ int spimc_ctx_create(const spimc_system_desc* descs, uint32_t n_replicas, uint64
                     (int)c->groups.size(), c->auto_fork ? "by rule" : c->fork ? "yes" : "no");
     }
     if ((rc = spimc_obs_configure(c, SPIMC_ENERGY_THERMAL, 0, 1e300, 0., 0., 100))) return bail(rc);
+    c->ruled = get_shape(c);
     *out = c;
     return SPIMC_OK;
 }
@@ -3102,41 +3131,40 @@ int spimc_autotune(spimc_ctx* c, uint32_t n_rounds, int32_t* chosen) {
     if (!c) return fail(SPIMC_ERR_ARG, "null context");
     if (n_rounds == 0) return fail(SPIMC_ERR_ARG, "n_rounds must be positive");
     if (c->prop_set) return fail(SPIMC_ERR_STATE, "an interface proposal is pending; accept or reject it first");
-    struct Shape {
-        int fork, bpc, bs, pers, one;
+    // launch shapes tried: the one chosen by rule, unless the environment fixes all of
+    // it; rho_k beside the pair kernel with 1-3 looping workgroups per CU and
+    // 256/512-thread pair workgroups, or the two kernels one after the other; for
+    // small replicas also the persistent stage kernel with 256-1024 threads
+    std::vector<LaunchShape> shapes;
+    if (c->ruled.auto_fork || c->ruled.auto_block || c->ruled.auto_one) shapes.push_back(c->ruled);
+    const auto fixed = [](int fork, int bpc, int bs, int pers, int one) {
+        return LaunchShape{fork != 0, bpc, bs, pers, one != 0, one >= 2 ? 2 : 1, false, false, false};
     };
-    // launch shapes tried: rho_k beside the pair kernel with 1-3 looping workgroups
-    // per CU and 256/512-thread pair workgroups, or the two kernels one after the
-    // other; for small replicas also the persistent stage kernel with 256-1024 threads
-    std::vector<Shape> shapes = {{1, 2, 512, 0, 0}, {1, 3, 512, 0, 0}, {1, 1, 512, 0, 0}, {1, 2, 256, 0, 0},
-                                 {1, 3, 256, 0, 0}, {0, 0, 1024, 0, 0}, {0, 2, 512, 0, 0}};
     if (!c->any_long || c->lds_doubles_max == 0)
-        shapes = {{0, 0, 1024, 0, 0}, {0, 0, 512, 0, 0}, {0, 0, 256, 0, 0}};
+        for (int bs : {1024, 512, 256}) shapes.push_back(fixed(0, 0, bs, 0, 0));
+    else
+        for (const LaunchShape& sh : {fixed(1, 2, 512, 0, 0), fixed(1, 3, 512, 0, 0), fixed(1, 1, 512, 0, 0),
+                                      fixed(1, 2, 256, 0, 0), fixed(1, 3, 256, 0, 0), fixed(0, 0, 1024, 0, 0),
+                                      fixed(0, 2, 512, 0, 0)})
+            shapes.push_back(sh);
     if (pers_eligible(c))
-        for (int pb : {256, 512, 1024}) shapes.push_back({c->fork ? 1 : 0, c->rho_bpc, c->pair_block, pb, 0});
+        for (int pb : {256, 512, 1024}) shapes.push_back(fixed(c->fork, c->rho_bpc, c->pair_block, pb, 0));
     // batches of at most one replica per CU: also one-launch bisection rounds,
     // with the displace rounds' rho_k after or beside their pair kernel
     if (one_launch_eligible(c) && (int)c->reps.size() <= kNumCUs) {
-        shapes.push_back({0, 0, c->pair_block, 0, 1});
-        if (c->any_long) shapes.push_back({1, 2, 512, 0, 1});
-        shapes.push_back({0, 0, c->pair_block, 0, 2});
+        shapes.push_back(fixed(0, 0, c->pair_block, 0, 1));
+        if (c->any_long) shapes.push_back(fixed(1, 2, 512, 0, 1));
+        shapes.push_back(fixed(0, 0, c->pair_block, 0, 2));
     }
-    const Shape saved{c->fork ? 1 : 0, c->rho_bpc, c->pair_block, c->pers_block, c->one_launch ? c->one_moves : 0};
+    const LaunchShape saved = get_shape(c);
     // the sweep's mix: N M / 2^l bisection attempts per N displace attempts
     const Rep& R0 = c->reps[0].dev;
     const uint32_t n_dis = std::max<uint32_t>(1, (uint32_t)((uint64_t)n_rounds * (1u << R0.n_level) / R0.M));
-    const bool saved_auto[3] = {c->auto_fork, c->auto_block, c->auto_one};
-    c->auto_fork = c->auto_block = c->auto_one = false;
     double best_t = 1e300;
-    Shape best = saved;
+    LaunchShape best = saved;
     int tried = 0;
-    for (const Shape& sh : shapes) {
-        c->fork = sh.fork != 0;
-        c->rho_bpc = sh.bpc;
-        c->one_launch = sh.one != 0;
-        c->one_moves = sh.one >= 2 ? 2 : 1;
-        int rc = c->lds_doubles_max > 0 ? set_pair_block(c, sh.bs) : SPIMC_OK;
-        if (rc == SPIMC_OK) rc = set_pers_block(c, sh.pers);
+    for (const LaunchShape& sh : shapes) {
+        int rc = set_shape(c, sh);
         if (rc) continue;
         drop_graphs(c);
         // one untimed round of each move under the new shape, then the timed mix
@@ -3146,15 +3174,7 @@ int spimc_autotune(spimc_ctx* c, uint32_t n_rounds, int32_t* chosen) {
         if (rc == SPIMC_OK) rc = run_stage(c, 1, nullptr, n_dis, nullptr, false);
         const double t = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         if (rc) {
-            c->fork = saved.fork != 0;
-            c->rho_bpc = saved.bpc;
-            c->one_launch = saved.one != 0;
-            c->one_moves = saved.one >= 2 ? 2 : 1;
-            if (c->lds_doubles_max > 0) (void)set_pair_block(c, saved.bs);
-            (void)set_pers_block(c, saved.pers);
-            c->auto_fork = saved_auto[0];
-            c->auto_block = saved_auto[1];
-            c->auto_one = saved_auto[2];
+            (void)set_shape(c, saved);
             return rc;
         }
         ++tried;
@@ -3163,24 +3183,19 @@ int spimc_autotune(spimc_ctx* c, uint32_t n_rounds, int32_t* chosen) {
             best = sh;
         }
     }
-    c->fork = best.fork != 0;
-    c->rho_bpc = best.bpc;
-    c->one_launch = best.one != 0;
-    c->one_moves = best.one >= 2 ? 2 : 1;
-    if (c->lds_doubles_max > 0) {
-        int rc = set_pair_block(c, best.bs);
-        if (rc) return rc;
-    }
-    if (int rc = set_pers_block(c, best.pers)) return rc;
+    if (int rc = set_shape(c, best)) return rc;
     drop_graphs(c);
     if (chosen) {
-        chosen[0] = best.fork;
-        chosen[1] = best.bpc;
-        chosen[2] = c->pair_block;
+        // by rule: what it chooses for the first group's bisection rounds
+        const Group& G = c->groups[0];
+        const bool fork = fork_now(c, G, 0);
+        chosen[0] = fork;
+        chosen[1] = c->auto_fork ? (fork ? 2 : 0) : c->rho_bpc;
+        chosen[2] = c->lds_doubles_max > 0 ? pair_block_now(c, G.n, G.max_bis_links, fork) : c->pair_block;
         chosen[3] = tried;
         chosen[4] = (int32_t)n_dis;
         chosen[5] = c->pers_block;
-        chosen[6] = c->one_launch ? c->one_moves : 0;
+        chosen[6] = one_launch_now(c, 0) ? (one_launch_now(c, 1) ? 2 : 1) : 0;
     }
     return SPIMC_OK;
 }
