@@ -366,8 +366,8 @@ class Engine:
 
     # ---- observables ---------------------------------------------------------
     def obs_configure(self, energy=ENERGY_THERMAL, virial_window=0, sk_k_cut=1e300, gr_r_min=0.0, gr_r_max=0.0, gr_n_r=100):
-        self.gr_n_r = gr_n_r
         check(self.lib.spimc_obs_configure(self.h, energy, virial_window, sk_k_cut, gr_r_min, gr_r_max, gr_n_r))
+        self.gr_n_r = gr_n_r  # (a refused call leaves the histogram as it was)
 
     def obs_accumulate(self, which: int):
         check(self.lib.spimc_obs_accumulate(self.h, which))
