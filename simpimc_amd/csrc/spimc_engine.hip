@@ -1354,6 +1354,15 @@ int launch_pair_lds(spimc_ctx* c, hipStream_t st, Rep* reps, int n_reps, int lin
                   st, reps, n_reps, bpr, kt);
 }
 
+// The decision of a bisection round and the next proposal: four wavefronts a replica
+// while the GPU holds all of them at once, else two.
+constexpr int kBisWide = 4 * kNumCUs;
+int launch_decide_bisect(spimc_ctx* c, hipStream_t st, Rep* reps, int n_reps, unsigned long long* kt) {
+    if (n_reps <= kBisWide)
+        return launch(c, SPIMC_KERNEL_PROPOSE, k_decide_propose_bisect<4>, n_reps, 4 * kWave, 0, st, reps, n_reps, kt);
+    return launch(c, SPIMC_KERNEL_PROPOSE, k_decide_propose_bisect<2>, n_reps, 2 * kWave, 0, st, reps, n_reps, kt);
+}
+
 // Dynamic LDS of the persistent kernel: the pair tables (rounded to 16 bytes),
 // then the phase chains of a stage's moved beads (up to M of them).
 constexpr size_t kPersLdsBytes = 160 * 1024 - 24 * 1024;  // the CU's LDS less the kernel's static arrays
@@ -1631,7 +1640,7 @@ int launch_round(spimc_ctx* c, const Group& G, int move) {
     int rc;
     if (c->fuse_rounds) {
         // the previous round's decision and this round's proposal in one launch
-        rc = move == 0 ? launch(c, SPIMC_KERNEL_PROPOSE, k_decide_propose_bisect, R, kBisBlock, 0, st, reps, R, kt)
+        rc = move == 0 ? launch_decide_bisect(c, st, reps, R, kt)
                        : launch(c, SPIMC_KERNEL_PROPOSE, k_decide_propose_displace, R, kDisBlock, 0, st, reps, R, kt);
     } else if (move == 0) {
         rc = launch(c, SPIMC_KERNEL_PROPOSE, k_propose_bisect, R, 64, 0, st, reps, R);
@@ -1872,8 +1881,7 @@ int run_stage(spimc_ctx* c, int move, const uint32_t* counts, uint32_t n_uniform
         for (int g = 0; g < n_groups; ++g) {
             const Group& G = c->groups[g];
             if (!gmx[g]) continue;
-            rc = move == 0 ? launch(c, SPIMC_KERNEL_PROPOSE, k_decide_propose_bisect, G.n, kBisBlock, 0, G.stream,
-                                    c->d_reps + G.r0, G.n, (unsigned long long*)nullptr)
+            rc = move == 0 ? launch_decide_bisect(c, G.stream, c->d_reps + G.r0, G.n, nullptr)
                            : launch(c, SPIMC_KERNEL_PROPOSE, k_decide_propose_displace, G.n, kDisBlock, 0, G.stream,
                                     c->d_reps + G.r0, G.n, (unsigned long long*)nullptr);
             if (rc) return rc;

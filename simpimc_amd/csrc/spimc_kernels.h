@@ -1468,10 +1468,15 @@ __global__ __launch_bounds__(64) void k_decide(const Rep* __restrict__ reps, int
 // per replica: the first decides while, on the device RNG of an unpermuted
 // path, the second and third fetch the next attempt's window and draws; then
 // all four make its levels (bisect_levels): 15 us for 512 replicas of N = 256,
-// M = 128 beside 18 with the levels on one wavefront.
-constexpr int kBisBlock = 4 * kWave;
-__global__ __launch_bounds__(kBisBlock) void k_decide_propose_bisect(const Rep* __restrict__ reps, int n_reps,
-                                                                     unsigned long long* __restrict__ kt) {
+// M = 128 beside 18 with the levels on one wavefront.  At most 128 registers: four
+// workgroups a CU, 1024 replicas at once (with 135, three: a round of 780 replicas of
+// N = 32, M = 32 77.7 us, 72.6 so; of 1024 of N = 12, M = 16 68.4 and 63.0).  Beyond
+// them two wavefronts, the second with the window and the draws (1300 replicas 112
+// and 107 us).
+template <int W>
+__global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(4))) void k_decide_propose_bisect(
+    const Rep* __restrict__ reps, int n_reps, unsigned long long* __restrict__ kt) {
+    constexpr int BS = W * kWave;
     __shared__ BisectLds S;
     __shared__ DecideOut s_out;
     __shared__ int s_moved;
@@ -1499,11 +1504,12 @@ __global__ __launch_bounds__(kBisBlock) void k_decide_propose_bisect(const Rep* 
             S.info[2] = b0;
         }
         bisect_window(R, lane, S, p, p, b0, false);
-    } else if (w == 2 && p >= 0) {
+        if (W == 2) bisect_draws(R, lane, S, seq);
+    } else if (W > 2 && w == 2 && p >= 0) {
         bisect_draws(R, lane, S, seq);
     }
     __syncthreads();
-    if (w == 3 && lane == 0 && s_out.status != 0)
+    if (w == W - 1 && lane == 0 && s_out.status != 0)
         decide_book(R, s_out.pr, s_out.acc, s_out.status, s_out.po, s_out.pn, s_out.lo, s_out.ln);
     if (!ahead) {
         if (w == 0) propose_bisect_impl(R, lane, WaveSync{}, true, S);
@@ -1511,7 +1517,7 @@ __global__ __launch_bounds__(kBisBlock) void k_decide_propose_bisect(const Rep* 
     }
     if (rem == 0) {
         if (threadIdx.x == 0) R.prop->status = 0;
-        rho_items_write(R, 0, 0, 0, 0, threadIdx.x, kBisBlock);
+        rho_items_write(R, 0, 0, 0, 0, threadIdx.x, BS);
         return;
     }
     if (threadIdx.x == 0) {
@@ -1523,8 +1529,8 @@ __global__ __launch_bounds__(kBisBlock) void k_decide_propose_bisect(const Rep* 
         if (w == 0) bisect_window(R, lane, S, s_moved, s_moved, S.info[2], false);
         __syncthreads();
     }
-    bisect_levels<kBisBlock / kWave>(R, S, w, lane, R.prop, R.prop_new, R.phase, 0);
-    rho_items_write(R, 0, S.info[4], S.info[5], (S.info[2] + 1) % R.M, threadIdx.x, kBisBlock);
+    bisect_levels<W>(R, S, w, lane, R.prop, R.prop_new, R.phase, 0);
+    rho_items_write(R, 0, S.info[4], S.info[5], (S.info[2] + 1) % R.M, threadIdx.x, BS);
 }
 // Displacement: the decision on the first wavefront, then the proposal, whose
 // M moved slices (positions, phase chains, rho_k items) take all kDisBlock
