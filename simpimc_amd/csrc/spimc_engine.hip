@@ -395,6 +395,7 @@ struct Group {
     // and the replicas' arrival counters (zero between rounds)
     int round_qpw[2] = {256, 256};  // partners per wavefront of a link
     int round_bpr[2] = {1, 1}, round_ipb[2] = {1, 1}, n_rgrp[2] = {0, 0};  // per move
+    bool round_fits[2] = {false, false};  // the launch's workgroups are about what the GPU holds at once
     double rho_bytes[2] = {0., 0.};  // rho_k read and written by a round, per move
     int4* d_rgrp[2] = {nullptr, nullptr};
     unsigned char* d_next = nullptr;  // k_round's proposals made ahead
@@ -1165,13 +1166,18 @@ int build_work_lists(spimc_ctx* c, Group& G) {
             // (a bisection's launch holds one more workgroup per replica, for its next proposal)
             const int held = std::max(1, occ) * kNumCUs, cap = std::max(held / 2, held - (mv == 0 ? G.n : 0));
             // a link's partners over as many wavefronts as still let every rho_k item
-            // have a workgroup of its own
-            for (int qpw : {64, 128, 256}) {
+            // have a workgroup of its own, else as many as cost no workgroup
+            const auto wgs = [&](int qpw) {
                 const int lpb = waves / (c->lds_doubles_max > 0 ? pair_split<waves>(max_N, qpw) : general_split<waves>(max_N, qpw));
-                G.round_qpw[mv] = qpw;
-                G.round_bpr[mv] = std::max(1, std::min((links + lpb - 1) / lpb, (2 * kNumCUs + G.n - 1) / G.n));
-                if (G.n * G.round_bpr[mv] + n_items <= cap) break;
-            }
+                return std::max(1, (links + lpb - 1) / lpb);
+            };
+            const auto bpr = [&](int qpw) { return std::min(wgs(qpw), (2 * kNumCUs + G.n - 1) / G.n); };
+            G.round_qpw[mv] = 256;
+            for (int qpw : {128, 64})
+                if (wgs(qpw) == wgs(256)) G.round_qpw[mv] = qpw;
+            for (int qpw : {128, 64})
+                if (G.n * bpr(qpw) + n_items <= cap) G.round_qpw[mv] = qpw;
+            G.round_bpr[mv] = bpr(G.round_qpw[mv]);
             // at least half of what the GPU holds goes to rho_k workgroups, also
             // when the pair workgroups alone would fill it
             const int room = std::max(cap / 2, cap - G.n * G.round_bpr[mv]);
@@ -1188,6 +1194,8 @@ int build_work_lists(spimc_ctx* c, Group& G) {
                 o += n;
             }
             G.n_rgrp[mv] = (int)grp.size();
+            const int total = (mv == 0 ? G.n : 0) + G.n * G.round_bpr[mv] + G.n_rgrp[mv];
+            G.round_fits[mv] = total <= (occ > 1 ? held + held / 4 : held);
             if (!grp.empty()) {
                 HIPCHK(hipMalloc((void**)&G.d_rgrp[mv], grp.size() * sizeof(int4)));
                 HIPCHK(hipMemcpy(G.d_rgrp[mv], grp.data(), grp.size() * sizeof(int4), hipMemcpyHostToDevice));
@@ -1395,16 +1403,20 @@ bool one_launch_eligible(const spimc_ctx* c) {
 }
 // Whether a stage of this move runs one-launch rounds; not while the device clocks
 // or events time the pair and rho_k kernels (k_round has no separate rho_k kernel
-// to time, so those rounds run as three launches).  By rule: where a rho_k
-// workgroup takes at most three items (displacement: two) for the launch to fit
-// what the GPU holds at once; five and four with tables of more than 48 KB (which
+// to time, so those rounds run as three launches).  By rule: where the launch's
+// workgroups are about what the GPU holds at once (a quarter more where a CU holds
+// several: a last workgroup of a replica that waits for a slot ends its round late) and a
+// rho_k workgroup takes at most three items (displacement: two) for that; five and four
+// with tables of more than 48 KB (which
 // three launches stage too) and with tables in global memory (searched by one
 // wavefront a link there).  A round then, against three launches: N = 32, M = 32,
 // bisection of 1 replica 12 and 22 us, of 128 (three items) 23 and 27, of 256
 // (seven) 61 and 33; displacement of 32 (two) 22 and 25, of 64 (six) 49 and 31;
 // N = 256, M = 128 with the 96 KB table, bisection of 1 replica 14.5 and 33, of 24
 // (four) 20.5 and 38, of 32 (five) 27 and 38, of 48 (seven) 58 and 42;
-// displacement of 4 (four) 32 and 38, of 8 (eight) 74 and 45; tabulated Ilkka
+// displacement of 4 (four) 32 and 38, of 8 (eight) 74 and 45; two links, N = 12, M = 16
+// with that table, of 96 replicas (240 workgroups) 24 and 25, of 192 (448) 33 and 25;
+// eight, of 32 (208) 18 and 26, of 64 (282, five items) 41 and 27; tabulated Ilkka
 // actions, N = 33, M = 32: bisection of 128 (three) 28 and 35, of 256 (seven) 61
 // and 43, displacement of 64 (four) 34 and 41.
 bool one_launch_now(const spimc_ctx* c, int move) {
@@ -1412,7 +1424,8 @@ bool one_launch_now(const spimc_ctx* c, int move) {
     if (!c->auto_one) return c->one_launch && move < c->one_moves;
     if (c->timing) return false;
     const bool large = c->lds_doubles_max == 0 || (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024;
-    return move < 2 && c->groups[0].round_ipb[move] <= (move == 0 ? (large ? 5 : 3) : (large ? 4 : 2));
+    const Group& G = c->groups[0];
+    return move < 2 && G.round_fits[move] && G.round_ipb[move] <= (move == 0 ? (large ? 5 : 3) : (large ? 4 : 2));
 }
 
 
