@@ -1541,22 +1541,12 @@ int launch_pair_multi(spimc_ctx* c, const Group& G, hipStream_t st) {
 // several chains, or a chain whose label changes inside the window, on the
 // label-general pair kernel and rho_multi_item, over the lists of such proposals.
 // Large rounds run rho_k beside the pair kernels on the group's second stream, the
-// others the two list kernels one after the other or in one launch.
+// others the two list kernels in one launch (k_multi_lists).
 // rho_k beside the pair kernels: from this much rho_k traffic a round, whose time then
 // exceeds what the second stream's events cost.  N = 256, M = 128, 1979 k-vectors, a
 // round of 128 replicas (57 MB) 92 us beside, 87 us in one launch; of 160 (71 MB) 94.5
 // and 93.4; of 192 (85 MB) 96.5 and 97.4; of 256 (114 MB) 103 and 107.
 constexpr double kPermForkBytes = 80e6;
-// Both list kernels in one launch: where few proposals are listed (a path whose
-// one-chain proposals have kernels of their own), and for at most this many replicas
-// also where every proposal is (tables in global memory, cycle tables of two or more).
-// The launch saved is 5-9 us; but every workgroup then holds the LDS of the rho_k items
-// (25 KB), six to a CU, and a long pair list waits for it.  Tabulated Ilkka actions,
-// N = 33, M = 32: 24 replicas 54 us a round in one launch and 58 in two, 64 replicas 72
-// and 65, 512 replicas 288 and 198; cycle table of two, N = 32: 16 replicas 57 and 64,
-// 64 replicas 76 and 69, 256 replicas 171 and 135; one-chain kernels, N = 256, M = 128:
-// 64 replicas 80 and 90.
-constexpr int kPermOneLaunch = 40;
 int launch_perm_round(spimc_ctx* c, const Group& G) {
     const int R = G.n;
     Rep* reps = c->d_reps + G.r0;
@@ -1591,7 +1581,7 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
     const int* rho_list = pair_list + G.n;
     const unsigned int* cnt = G.d_multi;
     const bool fork = c->any_long && G.side && bytes >= kPermForkBytes;
-    const bool one = c->any_long && !fork && ((tuned && single) || R <= kPermOneLaunch);
+    const bool one = c->any_long && !fork;
     hipStream_t rst = fork ? G.side : st;
     if (fork) {
         HIPCHK(hipEventRecord(G.ev_fork, st));
@@ -1600,7 +1590,7 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
     if (c->any_long && single && G.n_ritem_bis &&
         (rc = launch_rho(c, rst, G.d_ritem_bis, G.n_ritem_bis, fork && c->fork, nullptr)))
         return rc;
-    if (c->any_long && !one) {
+    if (fork) {
         // a fixed grid over the listed proposals' (replica, slot, chunk) items
         auto fn = c->rho_kpt == 2    ? k_rho_multi_list<2>
                   : c->rho_kpt == 4  ? k_rho_multi_list<4>
@@ -1608,8 +1598,8 @@ int launch_perm_round(spimc_ctx* c, const Group& G) {
                                      : k_rho_multi_list<8>;
         if ((rc = launch(c, SPIMC_KERNEL_RHO, fn, n_rho, kRhoBlock, 0, rst, reps, rho_list, cnt, max_slots, max_chunks)))
             return rc;
+        HIPCHK(hipEventRecord(G.ev_join, G.side));
     }
-    if (fork) HIPCHK(hipEventRecord(G.ev_join, G.side));
     if (tuned && single && (rc = launch_pair_lds(c, st, reps, R, max_links, fork && c->fork, nullptr))) return rc;
     if (!one) {
         if ((rc = launch(c, SPIMC_KERNEL_PAIR, k_pair_multi_list, n_pair, kPairMultiBlock, 0, st, reps, pair_list, cnt,

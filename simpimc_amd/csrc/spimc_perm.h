@@ -1154,8 +1154,9 @@ __global__ __launch_bounds__(kPairMultiBlock) void k_pair_multi_list(const Rep* 
 // few chains at a time.  Grid (k chunk, slot, replica).
 // ---------------------------------------------------------------------------
 constexpr int kPermPhaseBatch = 4;
-// KPT: k-vectors per thread, the rho_kpt of the replicas' k chunks
-template <int KPT>
+// KPT: k-vectors per thread, the rho_kpt of the replicas' k chunks; KT of them at a
+// time (fewer registers; the sums are the same)
+template <int KPT, int KT = KPT>
 __device__ __forceinline__ void rho_multi_item(const Rep* __restrict__ reps, int r, int m, int chunk) {
     const Rep& R = reps[r];
     const Prop pr = *R.prop;
@@ -1168,53 +1169,60 @@ __device__ __forceinline__ void rho_multi_item(const Rep* __restrict__ reps, int
     const int s = row.x, cur = row.y;
     const double2* rc = R.rho + ((size_t)cur * M + s) * nk;
     double2* rn = R.rho + ((size_t)(1 - cur) * M + s) * nk;
-    const int ck = kRhoBlock * KPT, k_lo = chunk * ck, k_hi = min(nk, k_lo + ck);
-    // this thread's k-vectors: k_lo + threadIdx.x + i * kRhoBlock, i < KPT; the row
-    // and k-table loads are issued before the phase chains are built
-    double dx[KPT], dy[KPT];
-    double2 rv[KPT];
-    int kp[KPT];
+    const int ck = kRhoBlock * KPT, k_end = min(nk, (chunk + 1) * ck);
+    double ao = 0., an = 0.;
+#pragma unroll 1
+    for (int i1 = 0; i1 < KPT; i1 += KT) {
+        // this thread's k-vectors: k_lo + threadIdx.x + i * kRhoBlock, i < KT; the row
+        // and k-table loads are issued before the phase chains are built
+        const int k_lo = chunk * ck + i1 * kRhoBlock, k_hi = min(k_end, k_lo + KT * kRhoBlock);
+        if (i1 > 0 && k_lo >= k_end) break;
+        double dx[KT], dy[KT];
+        double2 rv[KT];
+        int kp[KT];
 #pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        dx[i] = dy[i] = 0.;
-        const int k = k_lo + threadIdx.x + i * kRhoBlock;
-        const bool ok = k < k_hi;
-        rv[i] = ok ? ld2<true>(rc + k) : make_double2(0., 0.);
-        kp[i] = ok ? gld(R.kidx + k) : 0;
-    }
-    for (int i0 = 0; i0 < n; i0 += kPermPhaseBatch) {
-        const int nbat = min(kPermPhaseBatch, n - i0);
-        __syncthreads();
-        for (int c = threadIdx.x; c < nbat * 6; c += kRhoBlock) {
-            const int i = i0 + c / 6, o = (c % 6) / 3, d = c % 3;
-            const double x = o ? chain_new(R, pr.b0, nb, n, m + 1, i, d) : chain_old(R, pr.b0, m + 1, i, d);
-            phase_chain(x * R.box, R.max_idx, tab + (size_t)c * stride);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < KPT; ++i) {
+        for (int i = 0; i < KT; ++i) {
+            dx[i] = dy[i] = 0.;
             const int k = k_lo + threadIdx.x + i * kRhoBlock;
-            if (k >= k_hi) continue;
-            for (int b = 0; b < nbat; ++b) {
-                const double2 en = phase_k(tab + (size_t)(b * 6 + 3) * stride, stride, kp[i]);
-                const double2 eo = phase_k(tab + (size_t)(b * 6) * stride, stride, kp[i]);
-                dx[i] += en.x - eo.x;
-                dy[i] += en.y - eo.y;
+            const bool ok = k < k_hi;
+            rv[i] = ok ? ld2<true>(rc + k) : make_double2(0., 0.);
+            kp[i] = ok ? gld(R.kidx + k) : 0;
+        }
+        for (int i0 = 0; i0 < n; i0 += kPermPhaseBatch) {
+            const int nbat = min(kPermPhaseBatch, n - i0);
+            if (i1 == 0 || n > kPermPhaseBatch) {  // (one batch stays in LDS)
+                __syncthreads();
+                for (int c = threadIdx.x; c < nbat * 6; c += kRhoBlock) {
+                    const int i = i0 + c / 6, o = (c % 6) / 3, d = c % 3;
+                    const double x = o ? chain_new(R, pr.b0, nb, n, m + 1, i, d) : chain_old(R, pr.b0, m + 1, i, d);
+                    phase_chain(x * R.box, R.max_idx, tab + (size_t)c * stride);
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int i = 0; i < KT; ++i) {
+                const int k = k_lo + threadIdx.x + i * kRhoBlock;
+                if (k >= k_hi) continue;
+                for (int b = 0; b < nbat; ++b) {
+                    const double2 en = phase_k(tab + (size_t)(b * 6 + 3) * stride, stride, kp[i]);
+                    const double2 eo = phase_k(tab + (size_t)(b * 6) * stride, stride, kp[i]);
+                    dx[i] += en.x - eo.x;
+                    dy[i] += en.y - eo.y;
+                }
             }
         }
-    }
-    double ao = 0., an = 0.;
 #pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const int k = k_lo + threadIdx.x + i * kRhoBlock;
-        if (k >= k_hi) continue;
-        double2 nv;
-        nv.x = rv[i].x + dx[i];
-        nv.y = rv[i].y + dy[i];
-        st2<true>(rn + k, nv);
-        const double cf = gld(R.coef_s + k);
-        ao += cf * (rv[i].x * rv[i].x + rv[i].y * rv[i].y);
-        an += cf * (nv.x * nv.x + nv.y * nv.y);
+        for (int i = 0; i < KT; ++i) {
+            const int k = k_lo + threadIdx.x + i * kRhoBlock;
+            if (k >= k_hi) continue;
+            double2 nv;
+            nv.x = rv[i].x + dx[i];
+            nv.y = rv[i].y + dy[i];
+            st2<true>(rn + k, nv);
+            const double cf = gld(R.coef_s + k);
+            ao += cf * (rv[i].x * rv[i].x + rv[i].y * rv[i].y);
+            an += cf * (nv.x * nv.x + nv.y * nv.y);
+        }
     }
     ao = block_sum<kRhoBlock>(ao, red);
     an = block_sum<kRhoBlock>(an, red);
@@ -1238,12 +1246,15 @@ __global__ __launch_bounds__(kRhoBlock) void k_rho_multi_list(const Rep* __restr
     }
 }
 
-// Both lists in one launch, for rounds with few listed proposals: the first n_pair
-// workgroups loop over the pair items, the others over the rho_k items, side by
-// side (16 replicas of N = 32 with the cycle table: a round 112 us on two streams with
-// the one-chain kernels, 96 us so).
+// Both lists in one launch, for rounds that do not fork: the first n_pair workgroups
+// loop over the pair items, the others over the rho_k items, side by side.  Its
+// registers are the pair items' (128, four wavefronts a SIMD): the rho_k items take two
+// k-vectors a thread at a time, where eight at once need 215 registers and halve the
+// wavefronts that long pair lists run on.  Tabulated Ilkka actions, N = 33, M = 32, a
+// round of 512 replicas 191 us, 288 us with eight at once, 199 us in two launches; of 24
+// 54, 54 and 58; the cycle table of two, 256 replicas of N = 32 119, 171 and 134 us.
 template <int KPT>
-__global__ __launch_bounds__(kRhoBlock) void k_multi_lists(const Rep* __restrict__ reps, const int* __restrict__ pair_list,
+__global__ __launch_bounds__(kRhoBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_multi_lists(const Rep* __restrict__ reps, const int* __restrict__ pair_list,
                                                            const int* __restrict__ rho_list,
                                                            const unsigned int* __restrict__ cnt, int n_pair, int bpr,
                                                            int slots, int chunks) {
@@ -1256,7 +1267,7 @@ __global__ __launch_bounds__(kRhoBlock) void k_multi_lists(const Rep* __restrict
         const int per = slots * chunks, n = (int)cnt[1] * per;
         for (int it = blk - n_pair; it < n; it += (int)gridDim.x - n_pair) {
             const int q = it % per;
-            rho_multi_item<KPT>(reps, rho_list[it / per], q / chunks, q % chunks);
+            rho_multi_item<KPT, 2>(reps, rho_list[it / per], q / chunks, q % chunks);
         }
     }
 }
