@@ -2077,9 +2077,11 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
             // particles per workgroup: halved until the workgroups number the CUs
             int np = std::min(max_N, kCompatBlock);
             while (np > 64 && (long long)max_M * nrep * ((max_N + np - 1) / np) < kNumCUs) np = (np + 1) / 2;
-            const size_t shmem = (size_t)kCompatBlock * 3 * sizeof(double);
-            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(max_M, (max_N + np - 1) / np, nrep), kCompatBlock,
-                        shmem, c->stream, base, out_est, short_on, np);
+            // a thread for each of a workgroup's pairs, up to kCompatBlock
+            const int bs = (int)std::min<long long>(kCompatBlock, ((long long)np * max_N + 63) / 64 * 64);
+            const size_t shmem = (size_t)bs * 3 * sizeof(double);
+            rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(max_M, (max_N + np - 1) / np, nrep), bs, shmem, c->stream,
+                        base, out_est, short_on, np);
         } else {
             rc = launch(c, SPIMC_KERNEL_ADJOINT, k_grad_compat, g, 64, 0, c->stream, base, out_est, short_on);
         }

@@ -2355,8 +2355,8 @@ __device__ __forceinline__ void stage_tables(const Rep& R, double* lds) {
 
 // The same differences for the Bare and David actions, a bead's partners shared by
 // a workgroup.  blockIdx.x: slice; np particles per workgroup (a tile blockIdx.y of
-// the slice's), whose 512 / np groups of threads each take a range of the partners;
-// the groups' sums are added in order.  The bead's own distance is the same in the
+// the slice's), whose blockDim.x / np groups of threads (at most one a partner) each
+// take a range of the partners; the groups' sums are added in order.  The bead's own distance is the same in the
 // links (b, b + 1) and (b, b - 1), and r' moves with the bead only where its image
 // does: 6 radial terms at r and 2 at r' per pair instead of 48.  Every link action
 // is added up from its terms in k_grad_compat's order, from the same cubics: a
@@ -2418,7 +2418,7 @@ __global__ __launch_bounds__(kCompatBlock) void k_grad_compat_split(const Rep* _
     const int b = blockIdx.x, p0 = blockIdx.y * np, N = R.N, M = R.M;
     if (b >= M || p0 >= N) return;
     const bool on = short_on && R.pair_type != 0 && N > 1;
-    const int n = min(np, N - p0), n_grp = kCompatBlock / n;
+    const int n = min(np, N - p0), n_grp = min((int)blockDim.x / n, N);
     const int grp = threadIdx.x / n, lp = threadIdx.x % n, p = p0 + lp;
     const bool bare = PT == 1 || (PT == 0 && R.pair_type == 1);
     const double eps = 1.e-4;
@@ -2470,7 +2470,7 @@ __global__ __launch_bounds__(kCompatBlock) void k_grad_compat_split(const Rep* _
     }
     __syncthreads();
     double* o = (out_est ? R.grad_est : R.grad) + 3 * ((size_t)b * N + p0);
-    for (int t = threadIdx.x; t < 3 * n; t += kCompatBlock) {
+    for (int t = threadIdx.x; t < 3 * n; t += blockDim.x) {
         double v = 0.;
         if (on)
             for (int i = 0; i < n_grp; ++i) v += lds[(size_t)i * 3 * n + t];
