@@ -1980,6 +1980,17 @@ void whole_split(const spimc_ctx* c, int nrep, int& S, int& Q) {
     const int q_max = (int)std::max<long long>(1, std::min<long long>(W, pairs / kWholeBlock));
     S = std::max(std::min(W, (c->max_M + 7) / 8), std::min(c->max_M, W / q_max));
     Q = std::max(1, std::min(q_max, W / S));
+    // a few workgroups a replica: the split with the least slices (and first slices) a
+    // part, so that none of them is left out (W = 3 as one range of three parts, not two
+    // ranges of one: 68 replicas of N = 249, M = 11)
+    if (8 * S * Q < 7 * W)
+        for (int s = 1; s <= std::min(W, c->max_M); ++s) {
+            const int q = std::min(q_max, W / s);
+            if (((c->max_M + s - 1) / s + 1) * Q < ((c->max_M + S - 1) / S + 1) * q) {
+                S = s;
+                Q = q;
+            }
+        }
 }
 int est_pair_whole(spimc_ctx* c, Rep* base, int nrep, int which) {
     int rc;
