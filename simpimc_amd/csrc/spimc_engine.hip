@@ -2071,12 +2071,13 @@ int est_links(spimc_ctx* c, Rep* base, int nrep, int max_M, int max_N, uint32_t 
 }
 int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, int out_est) {
     // the extent of these replicas (a query's is one of the context's)
-    int max_M = 1, max_N = 1;
+    int max_M = 1, max_N = 1, max_nk = 0;
     bool any_long = false, ilkka_long = false;
     for (int r = 0; r < nrep; ++r) {
         const Rep& x = c->reps[(base - c->d_reps) + r].dev;
         max_M = std::max(max_M, x.M);
         max_N = std::max(max_N, x.N);
+        max_nk = std::max(max_nk, x.nk);
         any_long |= x.use_long_range != 0;
         ilkka_long |= x.use_long_range && x.pair_type == SPIMC_PAIR_ILKKA;
     }
@@ -2127,7 +2128,15 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
         rc = launch(c, SPIMC_KERNEL_ADJOINT, k_adjoint_local, g, 64, 0, c->stream, base, terms, out_est);
     }
     if (rc || !(terms & SPIMC_GRAD_PAIR_LONG) || !any_long) return rc;
-    if (c->col_max > 0) {
+    // by columns, but for many slices of at most one tile of particles and few
+    // k-vectors: the slices' weights, written and read once, then cost more than the
+    // serial chain of the runs, which has other wavefronts to hide behind.  The virial
+    // estimator by columns and by runs: 900 replicas of N = 2, M = 64 with 194 k-vectors
+    // 1184 and 956 us, with 678 2451 and 2229, with 967 3113 and 3621; 512 of N = 33,
+    // M = 32 with 678 (16384 slices) 1030 and 989, 256 523 and 553; 900 of N = 64 2637 and
+    // 2578, of N = 65 4333 and 4424.
+    const bool runs = c->adj_runs_lds > 0 && max_N <= 64 && max_nk <= 800 && (long long)max_M * nrep >= 16384;
+    if (c->col_max > 0 && !runs) {
         bool done = false;
         rc = est_long_cols(c, base, nrep, max_M, max_N, out_est, compat, &done);
         if (rc || done) return rc;
