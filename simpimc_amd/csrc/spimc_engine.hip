@@ -397,6 +397,7 @@ struct Group {
     int round_bpr[2] = {1, 1}, round_ipb[2] = {1, 1}, n_rgrp[2] = {0, 0};  // per move
     bool round_fits[2] = {false, false};  // the launch's workgroups are about what the GPU holds at once
     double rho_bytes[2] = {0., 0.};  // rho_k read and written by a round, per move
+    int max_nk = 0;                  // k-vectors, the largest replica's
     int4* d_rgrp[2] = {nullptr, nullptr};
     unsigned char* d_next = nullptr;  // k_round's proposals made ahead
     unsigned int* d_arrive = nullptr;
@@ -1145,6 +1146,7 @@ int build_work_lists(spimc_ctx* c, Group& G) {
         R.n_ritems_dis = nd;
         ob += nb;
         od += nd;
+        G.max_nk = std::max(G.max_nk, R.nk);
         G.rho_bytes[0] += 32. * R.nk * ((1 << R.n_level) - 1);
         G.rho_bytes[1] += 32. * R.nk * R.M;
     }
@@ -1327,29 +1329,50 @@ int set_pair_block(spimc_ctx* c, int bs) {
     return SPIMC_OK;
 }
 
-// Whether a round's rho_k kernel runs beside its pair kernel.  By rule: from 256 MB
-// of rho_k traffic a round (60 us of it at the copy rate).  The second stream's
-// events cost 12 us a round: N = 256, M = 128, 1979 k-vectors, bisection of 128
-// replicas (121 MB) 69 us beside, 62 us after; displacement of 64 (519 MB) 159 us
-// beside, 176 us after, of 32 (259 MB) 101 and 99; N = 128, M = 64, 257 k-vectors,
-// displacement of 256 replicas (135 MB) 165 us beside, 130 us after.
-constexpr double kForkBytes = 256e6;
+// Tables of this size leave a CU room for one or two workgroups; smaller ones for
+// as many as their registers allow.
+bool large_tables(const spimc_ctx* c) { return (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024; }
+
+// Whether a round's rho_k kernel runs beside its pair kernel.  The second stream's
+// events cost 12 us a round and the pair kernel gives up half of its wavefronts, so by
+// rule it does where large tables leave the pair kernel one workgroup a CU: from 256 MB of
+// rho_k traffic a round (60 us of it at the copy rate), and from 60 MB for 500 replicas or
+// more, whose pair workgroups come in several waves.  With few k-vectors (their items are
+// mostly latency, and two looping workgroups a CU hold less of it) only past four such
+// waves.  After and beside: 1979 k-vectors, N = 256, M = 128, bisection of 128 replicas
+// (122 MB) 60 and 66 us, of 256 (243 MB) 96 and 93, of 512 (486 MB) 174 and 156,
+// displacement of 32 (259 MB) 101 and 99, of 64 (519 MB) 176 and 161; 1847, N = 272,
+// M = 16, bisection of 256 (106 MB) 61 and 64, of 500 (207 MB) 102 and 93; N = 272, M = 4,
+// displacement of 512 (121 MB) 71 and 67; N = 100, M = 16 of 256 (242 MB) 80 and 87, and
+// with 20 KB tables bisection of 500 (207 MB) 76 and 104; 678, N = 64, M = 32, bisection of
+// 1024 (333 MB) 168 and 169, of 1300 (423 MB) 218 and 205, N = 128, M = 32, displacement of
+// 512 (355 MB) 157 and 175; 257, N = 32, M = 32 of 2000 (526 MB, 8 KB tables) 446 and 494;
+// 194, N = 40, M = 16, bisection of 1024 (44 MB) 94 and 94, of 2000 (87 MB) 169 and 156.
 bool fork_now(const spimc_ctx* c, const Group& G, int move) {
-    return c->auto_fork ? G.rho_bytes[move == 1] >= kForkBytes : c->fork;
+    if (!c->auto_fork) return c->fork;
+    if (!large_tables(c)) return false;
+    const double bytes = G.rho_bytes[move == 1];
+    if (G.max_nk >= 1024) return bytes >= 256e6 || (G.n >= 500 && bytes >= 60e6);
+    return G.n > 4 * kNumCUs && bytes >= 80e6;
 }
 
 // Workgroup size of a round's LDS pair kernel, one wavefront a link at a time.  By
 // rule: the smallest whose workgroups still number at most the CUs, so that few
 // replicas spread their links over more of the chip (N = 256, M = 128: bisection
 // of 1 replica 34 us a round with 256 threads, 44 us with 1024; displacement of
-// 16 replicas 63 us with 512, 73 and 72 us with 256 and 1024); beside rho_k 512,
-// which leaves room for its workgroups on every CU.
+// 16 replicas 63 us with 512, 73 and 72 us with 256 and 1024).  Beyond that 1024 with
+// large tables, which every workgroup stages, and with small ones 512, or 256 for up to
+// four links: more wavefronts than links only keep other workgroups out (N = 5, M = 32,
+// two links of 1300 replicas 37 us with 256 threads, 44 with 512, 59 with 1024; N = 32,
+// eight links of 512 replicas 47, 45 and 50; 96 KB tables, eight links of 400 replicas of
+// N = 256 187, 163 and 150).  Beside rho_k 512, which leaves room for its workgroups on
+// every CU.
 int pair_block_now(const spimc_ctx* c, int n_reps, int links, bool beside) {
     if (!c->auto_block) return c->pair_block;
     if (beside) return 512;
     for (int bs : kPairBlocks)
         if ((long long)n_reps * ((links + bs / 64 - 1) / (bs / 64)) <= kNumCUs) return bs;
-    return kPairLdsBlock;
+    return large_tables(c) ? kPairLdsBlock : links <= 4 ? 256 : 512;
 }
 
 int launch_pair_lds(spimc_ctx* c, hipStream_t st, Rep* reps, int n_reps, int links, bool beside, unsigned long long* kt) {
@@ -1423,7 +1446,7 @@ bool one_launch_now(const spimc_ctx* c, int move) {
     if (c->clock || !one_launch_eligible(c)) return false;
     if (!c->auto_one) return c->one_launch && move < c->one_moves;
     if (c->timing) return false;
-    const bool large = c->lds_doubles_max == 0 || (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024;
+    const bool large = c->lds_doubles_max == 0 || large_tables(c);
     const Group& G = c->groups[0];
     return move < 2 && G.round_fits[move] && G.round_ipb[move] <= (move == 0 ? (large ? 5 : 3) : (large ? 4 : 2));
 }
