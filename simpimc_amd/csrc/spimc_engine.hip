@@ -1103,6 +1103,9 @@ int upload_items(const std::vector<uint2>& v, uint2** d, int* n) {
     return SPIMC_OK;
 }
 
+// Room for the proposals made ahead of a group's one-launch rounds: 10000 replicas of
+// N = 256, M = 128 with 1979 k-vectors.
+constexpr size_t kNextBytes = 256u << 20;
 // LDS of k_round beside its static arrays: the tables, or with tables left in
 // global memory room for their axes (more than that is searched where it is).
 size_t round_shmem(const spimc_ctx* c) {
@@ -1224,7 +1227,12 @@ int build_work_lists(spimc_ctx* c, Group& G) {
                     R.next_phase[i] = (double2*)carve(nm * 6 * (R.max_idx + 1) * sizeof(double2));
                 }
             }
-            if (pass == 0) HIPCHK(hipMalloc((void**)&G.d_next, bytes));
+            // (a batch too wide for one-launch rounds by far goes without)
+            if (pass == 0 && (bytes > kNextBytes || hipMalloc((void**)&G.d_next, bytes) != hipSuccess)) {
+                G.d_next = nullptr;
+                (void)hipGetLastError();
+                break;
+            }
         }
     }
     if (!G.d_arrive) {
@@ -1421,6 +1429,8 @@ bool pers_eligible(const spimc_ctx* c) {
 // One-launch rounds: the default rho_k chunking, rounds decided in the next
 // proposal's launch, and unpermuted paths.
 bool one_launch_eligible(const spimc_ctx* c) {
+    for (const Group& G : c->groups)
+        if (!G.d_next) return false;
     return c->round_fn[0] && c->round_fn[1] && c->fuse_rounds && !c->perm_on &&
            c->rho_kpt == kRhoKpt;
 }
