@@ -399,7 +399,10 @@ struct Group {
     double rho_bytes[2] = {0., 0.};  // rho_k read and written by a round, per move
     int max_nk = 0;                  // k-vectors, the largest replica's
     int4* d_rgrp[2] = {nullptr, nullptr};
+    size_t rgrp_cap[2] = {0, 0};
     unsigned char* d_next = nullptr;  // k_round's proposals made ahead
+    size_t next_cap = 0;
+    int round_occ[2] = {0, 0};        // k_round's workgroups on a CU
     unsigned int* d_arrive = nullptr;
 };
 
@@ -1103,6 +1106,26 @@ int upload_items(const std::vector<uint2>& v, uint2** d, int* n) {
     return SPIMC_OK;
 }
 
+// Grows a workspace of the context to n entries; false where the memory is not to be
+// had, with the workspace gone: callers that were only faster with it take the
+// kernels that need none.
+bool grow(spimc_ctx* c, void** buf, size_t& cap, size_t n, size_t entry) {
+    if (n <= cap) return true;
+    if (*buf) {
+        (void)hipStreamSynchronize(c->stream);
+        (void)hipFree(*buf);
+    }
+    *buf = nullptr;
+    cap = 0;
+    if (hipMalloc(buf, n * entry) != hipSuccess) {
+        *buf = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    cap = n;
+    return true;
+}
+
 // Room for the proposals made ahead of a group's one-launch rounds: 10000 replicas of
 // N = 256, M = 128 with 1979 k-vectors.
 constexpr size_t kNextBytes = 256u << 20;
@@ -1164,9 +1187,9 @@ int build_work_lists(spimc_ctx* c, Group& G) {
         for (int r = G.r0; r < G.r0 + G.n; ++r) max_N = std::max(max_N, c->reps[r].dev.N);
         for (int mv = 0; mv < 2; ++mv) {
             const int links = mv == 0 ? G.max_bis_links : G.max_M, n_items = mv == 0 ? ob : od;
-            int occ = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)c->round_fn[mv], kRoundBlock,
-                                                             round_shmem(c)) != hipSuccess)
+            int& occ = G.round_occ[mv];
+            if (!occ && hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)c->round_fn[mv], kRoundBlock,
+                                                                     round_shmem(c)) != hipSuccess)
                 occ = 1;
             // (a bisection's launch holds one more workgroup per replica, for its next proposal)
             const int held = std::max(1, occ) * kNumCUs, cap = std::max(held / 2, held - (mv == 0 ? G.n : 0));
@@ -1202,7 +1225,8 @@ int build_work_lists(spimc_ctx* c, Group& G) {
             const int total = (mv == 0 ? G.n : 0) + G.n * G.round_bpr[mv] + G.n_rgrp[mv];
             G.round_fits[mv] = total <= (occ > 1 ? held + held / 4 : held);
             if (!grp.empty()) {
-                HIPCHK(hipMalloc((void**)&G.d_rgrp[mv], grp.size() * sizeof(int4)));
+                if (!grow(c, (void**)&G.d_rgrp[mv], G.rgrp_cap[mv], grp.size(), sizeof(int4)))
+                    return fail(SPIMC_ERR_NOMEM, "rho_k groups");
                 HIPCHK(hipMemcpy(G.d_rgrp[mv], grp.data(), grp.size() * sizeof(int4), hipMemcpyHostToDevice));
             }
         }
@@ -1228,9 +1252,10 @@ int build_work_lists(spimc_ctx* c, Group& G) {
                 }
             }
             // (a batch too wide for one-launch rounds by far goes without)
-            if (pass == 0 && (bytes > kNextBytes || hipMalloc((void**)&G.d_next, bytes) != hipSuccess)) {
+            if (pass == 0 && (bytes > kNextBytes || !grow(c, (void**)&G.d_next, G.next_cap, bytes, 1))) {
+                if (G.d_next) (void)hipFree(G.d_next);
                 G.d_next = nullptr;
-                (void)hipGetLastError();
+                G.next_cap = 0;
                 break;
             }
         }
@@ -1283,26 +1308,6 @@ int build_groups(spimc_ctx* c, int n_groups) {
     }
     HIPCHK(hipEventCreateWithFlags(&c->stage_ready, hipEventDisableTiming));
     return SPIMC_OK;
-}
-
-// Grows a workspace of the context to n entries; false where the memory is not to be
-// had, with the workspace gone: callers that were only faster with it take the
-// kernels that need none.
-bool grow(spimc_ctx* c, void** buf, size_t& cap, size_t n, size_t entry) {
-    if (n <= cap) return true;
-    if (*buf) {
-        (void)hipStreamSynchronize(c->stream);
-        (void)hipFree(*buf);
-    }
-    *buf = nullptr;
-    cap = 0;
-    if (hipMalloc(buf, n * entry) != hipSuccess) {
-        *buf = nullptr;
-        (void)hipGetLastError();
-        return false;
-    }
-    cap = n;
-    return true;
 }
 
 int ensure_tmp(spimc_ctx* c, size_t n_doubles) {
@@ -2884,8 +2889,7 @@ int spimc_set_bisect_level(spimc_ctx* c, uint32_t r, uint32_t n_level) {
     h.d.bisect_n_level = n_level;
     for (auto& G : c->groups) {
         if ((int)r < G.r0 || (int)r >= G.r0 + G.n) continue;
-        for (void** p : {(void**)&G.d_pair_bis, (void**)&G.d_pair_dis, (void**)&G.d_ritem_bis, (void**)&G.d_ritem_dis,
-                         (void**)&G.d_rgrp[0], (void**)&G.d_rgrp[1], (void**)&G.d_next})
+        for (void** p : {(void**)&G.d_pair_bis, (void**)&G.d_pair_dis, (void**)&G.d_ritem_bis, (void**)&G.d_ritem_dis})
             if (*p) {
                 (void)hipFree(*p);
                 *p = nullptr;
