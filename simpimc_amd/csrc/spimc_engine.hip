@@ -2030,6 +2030,15 @@ void whole_split(const spimc_ctx* c, int nrep, int& S, int& Q) {
             }
         }
 }
+// Threads of the sums over the slices of 64 k-vectors: a wavefront for every four
+// slices, 16 at most (more only hold the slots of other workgroups: S(k) and g(r) of 943
+// replicas of N = 2, M = 12 with 1847 k-vectors 182 us with 16, 129 with a thread per
+// k-vector).
+int sum_block(const spimc_ctx* c) {
+    int waves = 1;
+    while (waves < kSumBlock / kWave && 4 * waves < c->max_M) waves *= 2;
+    return waves * kWave;
+}
 int est_pair_whole(spimc_ctx* c, Rep* base, int nrep, int which) {
     int rc;
     if (c->lds_whole_max > 0) {
@@ -2044,7 +2053,7 @@ int est_pair_whole(spimc_ctx* c, Rep* base, int nrep, int which) {
     }
     if (rc || !c->any_long) return rc;
     dim3 g2((c->max_nk + 63) / 64, nrep);
-    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_long_whole, g2, kSumBlock, 0, c->stream, base, which);
+    return launch(c, SPIMC_KERNEL_ESTIMATORS, k_long_whole, g2, sum_block(c), 0, c->stream, base, which);
 }
 int est_kin_virial(spimc_ctx* c, Rep* base, int nrep, uint32_t W) {
     const int tiles = (c->max_N + 63) / 64;
@@ -2227,7 +2236,7 @@ int obs_accumulate_all(spimc_ctx* c, uint32_t which) {
     if ((which & SPIMC_OBS_SK) && c->any_long) {
         dim3 g((c->max_nk + 63) / 64, R);
         const double kc = c->sk_k_cut;
-        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_sk, g, kSumBlock, 0, c->stream, c->d_reps, kc);
+        rc = launch(c, SPIMC_KERNEL_ESTIMATORS, k_sk, g, sum_block(c), 0, c->stream, c->d_reps, kc);
         if (rc) return rc;
     }
     if (which & SPIMC_OBS_GR) {

@@ -2117,15 +2117,15 @@ __global__ __launch_bounds__(256) void k_pair_whole(const Rep* __restrict__ reps
     if (threadIdx.x == 0) R.scratch[slot * R.M + b] = t;
 }
 
-// sum_b |rho(b,k)|^2 for the 64 k-vectors of a 1024-thread workgroup (k the lane's;
-// valid on the first wavefront): its 16 wavefronts share the slices, four loads in
-// flight each, and are added in order.  (A thread per k-vector that walked the
+// sum_b |rho(b,k)|^2 for the 64 k-vectors of a workgroup (k the lane's; valid on the
+// first wavefront): its wavefronts (16 at most, and no more than have four slices each)
+// share the slices, four loads in flight each, and are added in order.  (A thread per k-vector that walked the
 // slices, each load behind its buffer selector, left 8 workgroups for 1979
 // k-vectors: 73 us for M = 128, 5 us so.)
 constexpr int kSumBlock = 1024;
 __device__ __forceinline__ double sum_rho2(const Rep& R, int k, double* sh) {
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, M = R.M;
-    constexpr int W = kSumBlock / kWave;
+    const int W = blockDim.x / kWave;
     double t = 0.;
     if (k < R.nk)
         for (int b = w; b < M; b += 4 * W) {
