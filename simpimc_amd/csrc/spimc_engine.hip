@@ -68,16 +68,20 @@ constexpr int kRhoKpt = 8;              // k-vectors per thread in k_rho (defaul
 constexpr int kRhoKptMin = 2;     // smallest chunking: bounds the number of k chunks
 constexpr int kPairBlocks[4] = {256, 512, 768, 1024};  // workgroup sizes of the LDS pair kernel
 constexpr int kNumCUs = 256;      // MI355X compute units (for workgroups-per-replica choices)
-// Wavefronts that the pair-once adjoint is given where there are links enough, and the
-// fewest with which it is taken over a workgroup per link: those of its ranges are too
-// few to hide each other's latency below, and a workgroup per link stages the tables
-// once a link, which small replicas do not repay.  The virial estimator, all of its
-// kernels, with ranges and with links: David, N = 32, M = 32 of 64 replicas (1024
-// ranges) 194 and 156 us, of 128 (2048) 240 and 263, of 255 306 and 442; N = 16, M = 8 of
-// 512 (2048) 197 and 238; N = 64, M = 64 of 64 (2048) 405 and 380, of 127 (4064) 557 and
-// 659; N = 256, M = 128 of 32 (2048) 4718 and 3399, of 63 (4032) 6334 and 6818.
+// Wavefronts that the pair-once adjoint is given where there are links enough.
 constexpr long long kAdjPairsWaves = 4096;
-long long adj_pairs_min(int N) { return N <= 32 ? 1536 : 3072; }
+// Whether it is taken over a workgroup per link.  Its workgroups of 16 wavefronts, one
+// to a CU, walk whole ranges of links: full is the share of the chip's wavefronts that
+// have one, with the last wave of workgroups that is partly empty and the ranges that few
+// slices leave out.  A workgroup per link stages the tables and adds up its wavefronts
+// once a link, which costs small replicas more than idle wavefronts and large ones
+// little: the line rises with N.  The virial estimator, all of its kernels, by ranges and
+// by links: N = 16, M = 8, 128 replicas (0.13 full) 93 and 87 us, 512 (0.25) 197 and 238;
+// N = 32, M = 32, 64 (0.25) 176 and 146, 128 (0.5) 225 and 247; N = 48, M = 32, 96 (0.38)
+// 287 and 246, 191 (0.75) 377 and 433; N = 64, M = 64, 64 (0.5) 405 and 377, 96 (0.75)
+// 491 and 541; N = 71, M = 13, 520 (0.25) 1443 and 914; N = 130, M = 33, 260 (0.51) 5214
+// and 3530; N = 256, M = 128, 48 (0.75) 5520 and 5215, 63 (0.98) 6282 and 6803.
+bool adj_ranges(int N, double full) { return full >= std::min(0.8, 0.0105 * N); }
 // PermBisectTable: particles of a replica (an N x N table) and cycle-list entries
 constexpr int kTabMaxN = 1024;
 constexpr double kTabMaxEntries = 268435456.;
@@ -2150,13 +2154,14 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
         // workgroups per replica: enough to fill the GPU when the replicas are few
         const int bpr = std::max(1, std::min(max_M, (2 * kNumCUs + nrep - 1) / nrep));
         // pair-once kernel: at most max_M / 2 link ranges of 16 waves' worth per
-        // replica; chosen when they give at least adj_pairs_min waves, else the
+        // replica; chosen by how full they keep the chip (adj_ranges), else the
         // workgroup-per-link form
         const int rng_max = std::max(1, max_M / 2);
         const int bpr2 = std::max(1, std::min((rng_max + kAdjPairWaves - 1) / kAdjPairWaves,
                                               (int)((kAdjPairsWaves + kAdjPairWaves * nrep - 1) / (kAdjPairWaves * nrep))));
-        const long long waves2 = (long long)nrep * std::min(kAdjPairWaves * bpr2, rng_max);
-        const int form = !c->adj_pairs_ok ? 0 : c->adj_pairs_env >= 0 ? c->adj_pairs_env : waves2 >= adj_pairs_min(max_N) ? 1 : 2;
+        const double wgs = (double)nrep * bpr2, ranges = std::min(kAdjPairWaves * bpr2, rng_max);
+        const double full = wgs / (kNumCUs * std::ceil(wgs / kNumCUs)) * ranges / (kAdjPairWaves * bpr2);
+        const int form = !c->adj_pairs_ok ? 0 : c->adj_pairs_env >= 0 ? c->adj_pairs_env : adj_ranges(max_N, full) ? 1 : 2;
         const size_t shmem2 = shmem + (size_t)kAdjPairWaves * kAdjSlotDoubles * sizeof(double);
         if (form == 1) {
             rc = launch(c, SPIMC_KERNEL_ADJOINT, c->adj_pairs_fn, dim3(nrep, bpr2), kAdjLdsBlock, shmem2, c->stream,
