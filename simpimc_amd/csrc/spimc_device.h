@@ -202,7 +202,6 @@ struct Rep {
     NextProp* next;
     double2* pair_part;    // [n_links_max] (old, new)
     double2* rho_part;     // [M][n_chunks] (old, new)
-    double2* kin_part;     // interface kinetic (old, new)
     Counters* cnt;
     unsigned int* ctx_error;  // shared by all replicas of a context
     unsigned char* accepted; // [accepted_cap]

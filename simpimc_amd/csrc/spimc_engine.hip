@@ -467,7 +467,9 @@ struct spimc_ctx {
     // (1) or a workgroup per link (2)
     void (*adj_pairs_fn)(const Rep*, unsigned int, int, int) = nullptr;
     int adj_pairs_env = -1;
-    // the reference's finite differences on the LDS tables (nullptr: global tables)
+    // the reference's finite differences of the Bare and David actions, a slice's pairs
+    // shared by a workgroup; set where the pair kernels' tables are staged in LDS
+    // (nullptr: a thread per bead, as SPIMC_PAIR_LDS = 0 asks for)
     void (*compat_fn)(const Rep*, int, int, int) = nullptr;
     // the pair-once adjoint with a workgroup per link, for few replicas, and its
     // shares (grown to the largest call)
@@ -921,7 +923,6 @@ int build_replica(spimc_ctx* c, uint32_t r, const spimc_system_desc& s, uint64_t
         R.prop_new = cv.take<double>((size_t)3 * M);
         R.pair_part = cv.take<double2>(M);
         R.rho_part = cv.take<double2>((size_t)M * h.n_chunks);
-        R.kin_part = cv.take<double2>(1);
         R.cnt = cv.take<Counters>(1);
         R.tape_cursor = cv.take<long long>(1);
         R.e_acc = cv.take<double>(2);
@@ -1533,7 +1534,7 @@ void drop_graphs(spimc_ctx* c) {
 }
 
 // A stage in one launch of the persistent kernel, after the stage's counts are
-// set (k_stage_begin reads them from d_counts).
+// set (k_stage_begin reads them from pinned memory).
 int launch_pers_stage(spimc_ctx* c, int move) {
     const int R = (int)c->reps.size();
     int rc = launch(c, SPIMC_KERNEL_DECIDE, k_stage_begin, (R + 63) / 64, 64, 0, c->stream, c->d_reps, R, (const unsigned int*)c->counts);

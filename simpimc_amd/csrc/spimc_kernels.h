@@ -1,17 +1,19 @@
 // spimc_kernels.h -- HIP kernels of the engine (included once, by spimc_engine.hip).
 //
 // Move stages run in rounds: every replica with attempts left performs one
-// attempt per round, through four launches
-//   k_propose_*  one wavefront per replica: draws, bisection sampling of the
-//                coarse levels with their kinetic Metropolis decisions, and the
-//                level-0 NEW beads
-//   k_pair       one wavefront per (replica, link): short-range pair action of
-//                the moved particle against all others, OLD and NEW
-//   k_rho        one workgroup per (replica, moved slice, k chunk): incremental
-//                rho_k update into the spare buffer fused with the long-range
-//                action sums, OLD and NEW
-//   k_decide     one wavefront per replica: level-0 Metropolis decision, commit
-// A single chain (the plain method) is the same launches with one replica.
+// attempt per round.  Its parts:
+//   propose      draws, bisection sampling of the coarse levels with their kinetic
+//                Metropolis decisions, and the level-0 NEW beads
+//   pair links   short-range pair action of the moved particle against all
+//                others on every window link, OLD and NEW
+//   rho_k items  a moved slice's chunk of k-vectors: incremental rho_k update into
+//                the spare buffer fused with the long-range action sums, OLD and NEW
+//   decide       level-0 Metropolis decision and commit
+// In three launches, k_decide_propose_* decides the last round and proposes the next,
+// k_pair_lds (tables in LDS) or k_pair takes the links, k_rho_loop the items.  Batches
+// that fit the GPU at once run them in one, k_round, which for a bisection also makes
+// the next proposal beside the pending one.  A single chain (the plain method) is the
+// same launches with one replica.
 #pragma once
 
 #include "spimc_device.h"

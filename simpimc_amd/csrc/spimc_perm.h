@@ -5,11 +5,13 @@
 //
 //   k_propose_perm  one workgroup per replica: bead0, the iterative cycle walk,
 //                   the bisection of every chain down to level 0
-//   k_pair_multi    workgroups per replica loop over the window links: the
+//   pair_multi_item workgroups per replica loop over the window links: the
 //                   label-based pair action of every label with a moved bead
 //                   on the link, OLD and NEW
-//   k_rho_multi     one workgroup per (replica, moved slice, k chunk): the
+//   rho_multi_item  one workgroup per (replica, moved slice, k chunk): the
 //                   incremental rho_k of a slice with several moved beads
+// over the replicas a round lists, in one launch (k_multi_lists) or beside each other
+// (k_pair_multi_list, k_rho_multi_list).
 // The decision and commit (relabelling included) stay in k_decide.
 #pragma once
 
@@ -1151,7 +1153,7 @@ __global__ __launch_bounds__(kPairMultiBlock) void k_pair_multi_list(const Rep* 
 // slice of moved slot m holds one moved bead per chain; its rho_k row gets the
 // sum of their phase changes, fused with the long-range sums of CalcULong like
 // k_rho.  The beads' phase chains (KSpace::CalcC recurrence) are built in LDS a
-// few chains at a time.  Grid (k chunk, slot, replica).
+// few chains at a time.
 // ---------------------------------------------------------------------------
 constexpr int kPermPhaseBatch = 4;
 // KPT: k-vectors per thread, the rho_kpt of the replicas' k chunks; KT of them at a
@@ -1229,11 +1231,7 @@ __device__ __forceinline__ void rho_multi_item(const Rep* __restrict__ reps, int
     if (threadIdx.x == 0) R.rho_part[m * R.n_chunks + chunk] = make_double2(ao, an);
     __syncthreads();  // the LDS tables and partials are reused by the block's next item
 }
-template <int KPT>
-__global__ __launch_bounds__(kRhoBlock) void k_rho_multi(const Rep* __restrict__ reps) {
-    rho_multi_item<KPT>(reps, blockIdx.z, blockIdx.y, blockIdx.x);
-}
-// The same over the replicas a permuting round listed (cnt[1] of them in
+// The items of the replicas a permuting round listed (cnt[1] of them in
 // list[0..]): a fixed grid loops over their (replica, slot, chunk) items.
 template <int KPT>
 __global__ __launch_bounds__(kRhoBlock) void k_rho_multi_list(const Rep* __restrict__ reps, const int* __restrict__ list,
