@@ -1351,26 +1351,27 @@ int set_pair_block(spimc_ctx* c, int bs) {
 // as many as their registers allow.
 bool large_tables(const spimc_ctx* c) { return (size_t)c->lds_doubles_max * sizeof(double) > 48 * 1024; }
 
-// Whether a round's rho_k kernel runs beside its pair kernel.  The second stream's
-// events cost 12 us a round and the pair kernel gives up half of its wavefronts, so by
-// rule it does where large tables leave the pair kernel one workgroup a CU: from 256 MB of
-// rho_k traffic a round (60 us of it at the copy rate), and from 60 MB for 500 replicas or
-// more, whose pair workgroups come in several waves.  With few k-vectors (their items are
-// mostly latency, and two looping workgroups a CU hold less of it) only past four such
-// waves.  After and beside: 1979 k-vectors, N = 256, M = 128, bisection of 128 replicas
-// (122 MB) 60 and 66 us, of 256 (243 MB) 96 and 93, of 512 (486 MB) 174 and 156,
-// displacement of 32 (259 MB) 101 and 99, of 64 (519 MB) 176 and 161; 1847, N = 272,
-// M = 16, bisection of 256 (106 MB) 61 and 64, of 500 (207 MB) 102 and 93; N = 272, M = 4,
-// displacement of 512 (121 MB) 71 and 67; N = 100, M = 16 of 256 (242 MB) 80 and 87, and
-// with 20 KB tables bisection of 500 (207 MB) 76 and 104; 678, N = 64, M = 32, bisection of
-// 1024 (333 MB) 168 and 169, of 1300 (423 MB) 218 and 205, N = 128, M = 32, displacement of
-// 512 (355 MB) 157 and 175; 257, N = 32, M = 32 of 2000 (526 MB, 8 KB tables) 446 and 494;
-// 194, N = 40, M = 16, bisection of 1024 (44 MB) 94 and 94, of 2000 (87 MB) 169 and 156.
+// Whether a round's rho_k kernel runs beside its pair kernel.  The second stream's events
+// cost 12 us a round and the pair kernel gives up half of its wavefronts, so by rule it
+// does where large tables leave the pair kernel one workgroup a CU: from 256 MB of rho_k
+// traffic a round (60 us of it at the copy rate), from 150 MB where the pair workgroups
+// take a second wave and from 60 MB for 500 replicas or more, where they take several.
+// With few k-vectors (their items are mostly latency, and two looping workgroups a CU hold
+// less of it) only past four such waves.  After and beside: 1979 k-vectors, N = 256, M =
+// 128, bisection of 128 replicas (122 MB) 60 and 66 us, of 256 (243 MB) 96 and 93, of 260
+// (247 MB) 120 and 100, of 512 (486 MB) 174 and 156, displacement of 32 (259 MB) 101 and
+// 99, of 64 (519 MB) 176 and 161; 1847, N = 272, M = 16, bisection of 256 (106 MB) 61 and
+// 64, of 500 (207 MB) 102 and 93; N = 272, M = 4, displacement of 512 (121 MB) 71 and 67;
+// N = 100, M = 16 of 256 (242 MB) 80 and 87, and with 20 KB tables bisection of 500 (207
+// MB) 76 and 104; 678, N = 64, M = 32, bisection of 1024 (333 MB) 168 and 169, of 1300
+// (423 MB) 218 and 205, N = 128, M = 32, displacement of 512 (355 MB) 157 and 175; 257, N
+// = 32, M = 32 of 2000 (526 MB, 8 KB tables) 446 and 494; 194, N = 40, M = 16, bisection
+// of 1024 (44 MB) 94 and 94, of 2000 (87 MB) 169 and 156.
 bool fork_now(const spimc_ctx* c, const Group& G, int move) {
     if (!c->auto_fork) return c->fork;
     if (!large_tables(c)) return false;
     const double bytes = G.rho_bytes[move == 1];
-    if (G.max_nk >= 1024) return bytes >= 256e6 || (G.n >= 500 && bytes >= 60e6);
+    if (G.max_nk >= 1024) return bytes >= (G.n >= 500 ? 60e6 : G.n > kNumCUs ? 150e6 : 256e6);
     return G.n > 4 * kNumCUs && bytes >= 80e6;
 }
 
@@ -1444,24 +1445,22 @@ bool one_launch_eligible(const spimc_ctx* c) {
     return c->round_fn[0] && c->round_fn[1] && c->fuse_rounds && !c->perm_on &&
            c->rho_kpt == kRhoKpt;
 }
-// Whether a stage of this move runs one-launch rounds; not while the device clocks
-// or events time the pair and rho_k kernels (k_round has no separate rho_k kernel
-// to time, so those rounds run as three launches).  By rule: where the launch's
-// workgroups are about what the GPU holds at once (a quarter more where a CU holds
-// several: a last workgroup of a replica that waits for a slot ends its round late) and a
-// rho_k workgroup takes at most three items (displacement: two) for that; five and four
-// with tables of more than 48 KB (which
-// three launches stage too) and with tables in global memory (searched by one
+// Whether a stage of this move runs one-launch rounds; not while the device clocks or
+// events time the pair and rho_k kernels (k_round has no separate rho_k kernel to time, so
+// those rounds run as three launches).  By rule: where the launch's workgroups are about
+// what the GPU holds at once (a quarter more where a CU holds several: a last workgroup of
+// a replica that waits for a slot ends its round late) and a rho_k workgroup takes at most
+// three items (displacement: two) for that; five and four with tables of more than 48 KB
+// (which three launches stage too) and with tables in global memory (searched by one
 // wavefront a link there).  A round then, against three launches: N = 32, M = 32,
-// bisection of 1 replica 12 and 22 us, of 128 (three items) 23 and 27, of 256
-// (seven) 61 and 33; displacement of 32 (two) 22 and 25, of 64 (six) 49 and 31;
-// N = 256, M = 128 with the 96 KB table, bisection of 1 replica 14.5 and 33, of 24
-// (four) 20.5 and 38, of 32 (five) 27 and 38, of 48 (seven) 58 and 42;
-// displacement of 4 (four) 32 and 38, of 8 (eight) 74 and 45; two links, N = 12, M = 16
-// with that table, of 96 replicas (240 workgroups) 24 and 25, of 192 (448) 33 and 25;
-// eight, of 32 (208) 18 and 26, of 64 (282, five items) 41 and 27; tabulated Ilkka
-// actions, N = 33, M = 32: bisection of 128 (three) 28 and 35, of 256 (seven) 61
-// and 43, displacement of 64 (four) 34 and 41.
+// bisection of 1 replica 12 and 22 us, of 128 (three items) 23 and 27, of 256 (seven) 61
+// and 33; displacement of 32 (two) 22 and 25, of 64 (six) 49 and 31; N = 256, M = 128 with
+// the 96 KB table, bisection of 1 replica 14.5 and 33, of 24 (four) 20.5 and 38, of 32
+// (five) 27 and 38, of 48 (seven) 58 and 42; displacement of 4 (four) 32 and 38, of 8
+// (eight) 74 and 45; two links, N = 12, M = 16 with that table, of 96 replicas (240
+// workgroups) 24 and 25, of 192 (448) 33 and 25; eight, of 32 (208) 18 and 26, of 64 (282,
+// five items) 41 and 27; tabulated Ilkka actions, N = 33, M = 32: bisection of 128 (three)
+// 28 and 35, of 256 (seven) 61 and 43, displacement of 64 (four) 34 and 41.
 bool one_launch_now(const spimc_ctx* c, int move) {
     if (c->clock || !one_launch_eligible(c)) return false;
     if (!c->auto_one) return c->one_launch && move < c->one_moves;
