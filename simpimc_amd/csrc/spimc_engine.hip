@@ -1397,8 +1397,13 @@ int pair_block_now(const spimc_ctx* c, int n_reps, int links, bool beside) {
 int launch_pair_lds(spimc_ctx* c, hipStream_t st, Rep* reps, int n_reps, int links, bool beside, unsigned long long* kt) {
     const int bs = pair_block_now(c, n_reps, links, beside), waves = bs / 64;
     // workgroups per replica: one when the replicas fill the GPU, more (up to one
-    // per bs / 64 links) when they are few
-    const int bpr = std::max(1, std::min((links + waves - 1) / waves, (2 * kNumCUs + n_reps - 1) / n_reps));
+    // per bs / 64 links) when they are few; with large tables, where each has a CU to
+    // itself, no more than the CUs: the few of a second wave take as long as the first
+    // (displacement of 132 replicas of N = 213, M = 20, 264 workgroups 78 us a round, 132 61;
+    // 152 of N = 272, M = 17 91 and 66; 64 of N = 256, M = 128 168 and 163)
+    const bool alone = !beside && large_tables(c) && n_reps <= kNumCUs;
+    const int most = alone ? kNumCUs / n_reps : (2 * kNumCUs + n_reps - 1) / n_reps;
+    const int bpr = std::max(1, std::min((links + waves - 1) / waves, most));
     const int i = (int)(std::find(std::begin(kPairBlocks), std::end(kPairBlocks), bs) - std::begin(kPairBlocks));
     return launch(c, SPIMC_KERNEL_PAIR, c->pair_lds_fn[i], n_reps * bpr, bs, (size_t)c->lds_doubles_max * sizeof(double),
                   st, reps, n_reps, bpr, kt);
