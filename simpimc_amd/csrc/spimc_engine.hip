@@ -1228,7 +1228,7 @@ int build_work_lists(spimc_ctx* c, Group& G) {
             }
             G.n_rgrp[mv] = (int)grp.size();
             const int total = (mv == 0 ? G.n : 0) + G.n * G.round_bpr[mv] + G.n_rgrp[mv];
-            G.round_fits[mv] = total <= (occ > 1 ? held + held / 4 : held);
+            G.round_fits[mv] = total <= (mv == 0 && occ > 1 ? held + held / 4 : held);
             if (!grp.empty()) {
                 if (!grow(c, (void**)&G.d_rgrp[mv], G.rgrp_cap[mv], grp.size(), sizeof(int4)))
                     return fail(SPIMC_ERR_NOMEM, "rho_k groups");
@@ -1453,8 +1453,8 @@ bool one_launch_eligible(const spimc_ctx* c) {
 // Whether a stage of this move runs one-launch rounds; not while the device clocks or
 // events time the pair and rho_k kernels (k_round has no separate rho_k kernel to time, so
 // those rounds run as three launches).  By rule: where the launch's workgroups are about
-// what the GPU holds at once (a quarter more where a CU holds several: a last workgroup of
-// a replica that waits for a slot ends its round late) and a rho_k workgroup takes at most
+// what the GPU holds at once (a bisection's a quarter more where a CU holds several: a last
+// workgroup of a replica that waits for a slot ends its round late) and a rho_k workgroup takes at most
 // three items (displacement: two) for that; five and four with tables of more than 48 KB
 // (which three launches stage too) and with tables in global memory (searched by one
 // wavefront a link there).  A round then, against three launches: N = 32, M = 32,
