@@ -2125,6 +2125,33 @@ int est_links(spimc_ctx* c, Rep* base, int nrep, int max_M, int max_N, uint32_t 
     }
     return SPIMC_OK;
 }
+// Workgroups of the finite differences over `slices` slices of N particles: np particles
+// each, and as many groups of threads, each a share of the partners, as make the CUs end
+// first.  A CU holds twelve of the kernel's wavefronts, three a SIMD; kSimd is what a
+// partner costs by the wavefronts of the fullest SIMD, fitted to 36 sizes at three shapes
+// each (latency with one, the FP64 rate with three).  The virial estimator with workgroups
+// of up to 512 threads, halved until they number the CUs, and so: 3 replicas of N = 344,
+// M = 86 (258 such workgroups, two more than the CUs) 15.1 and 8.4 ms; 7 of N = 443,
+// M = 45 23.5 and 16.8 ms; 13 of N = 600, M = 20 36.8 and 26.0 ms.
+void compat_shape(int N, long long slices, int& np, int& bs) {
+    constexpr double kSimd[4] = {0., 1., 1.4, 2.4};
+    double best = 1e300;
+    const int least = (N + kCompatBlock - 1) / kCompatBlock, most = std::max(least, std::min(16, (N + 15) / 16));
+    for (int tiles = least; tiles <= most; ++tiles) {
+        const int n = (N + tiles - 1) / tiles;
+        for (int g = 1; g <= std::min(kCompatBlock / n, N); ++g) {
+            const int waves = (n * g + 63) / 64, held = 12 / waves;  // of a workgroup; workgroups of a CU
+            const long long mine = (slices * tiles + kNumCUs - 1) / kNumCUs;
+            const double cost = ((double)(mine / held) * kSimd[(held * waves + 3) / 4] + kSimd[(mine % held * waves + 3) / 4]) *
+                                ((N + g - 1) / g + 2);
+            if (cost < best) {
+                best = cost;
+                np = n;
+                bs = 64 * waves;
+            }
+        }
+    }
+}
 int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, int out_est) {
     // the extent of these replicas (a query's is one of the context's)
     int max_M = 1, max_N = 1, max_nk = 0;
@@ -2142,11 +2169,8 @@ int est_gradient(spimc_ctx* c, Rep* base, int nrep, uint32_t terms, int compat, 
     if (compat) {
         const int short_on = (terms & SPIMC_GRAD_PAIR_SHORT) ? 1 : 0;
         if (c->compat_fn) {
-            // particles per workgroup: halved until the workgroups number the CUs
-            int np = std::min(max_N, kCompatBlock);
-            while (np > 64 && (long long)max_M * nrep * ((max_N + np - 1) / np) < kNumCUs) np = (np + 1) / 2;
-            // a thread for each of a workgroup's pairs, up to kCompatBlock
-            const int bs = (int)std::min<long long>(kCompatBlock, ((long long)np * max_N + 63) / 64 * 64);
+            int np, bs;
+            compat_shape(max_N, (long long)max_M * nrep, np, bs);
             const size_t shmem = (size_t)bs * 3 * sizeof(double);
             rc = launch(c, SPIMC_KERNEL_ADJOINT, c->compat_fn, dim3(max_M, (max_N + np - 1) / np, nrep), bs, shmem, c->stream,
                         base, out_est, short_on, np);
