@@ -96,7 +96,7 @@ struct Prop {
     int n_chain;  // chains of a permuting bisection (0: the cycle walk stopped)
     int e_slice;  // slice after which a permuting bisection relinks the chains
     int n_level;  // bisection level of a permuting bisection
-    int rho_multi;  // 1: k_rho_multi updates rho_k (several beads per slice); 0: the k_rho items
+    int rho_multi;  // 1: the permuting lists' kernel updates rho_k (several beads per slice); 0: the k_rho items
     // PermBisectTable's final table check, after a level-0 accept (tab_on): reject
     // if tab_ratio < u, u the next tape value or u_tab (device RNG)
     int tab_on;
@@ -243,7 +243,7 @@ struct Rep {
     int perm_n_level;               // bisection level of the permuting move
     int multi_cap;                  // replicas of the group: the second list's offset
     // per group: the proposals of a permuting round that the label-general pair
-    // kernel (cnt[0], list[0..]) and k_rho_multi (cnt[1], list[multi_cap..]) take,
+    // kernel (cnt[0], list[0..]) and k_rho_multi_list (cnt[1], list[multi_cap..]) take,
     // as replica indices within the group
     unsigned int* multi_cnt;
     int* multi_list;

@@ -2365,7 +2365,7 @@ __device__ __forceinline__ void stage_tables(const Rep& R, double* lds) {
 // difference over 2 eps magnifies the rounding of a link action 5000 times, and
 // terms left out or in another form (B-splines in LDS: 102 us) come out several
 // times further from 64-bit arithmetic.  Bound by FP64 arithmetic and table
-// gathers: N = 77, M = 50, 12 replicas 1243 us with a thread per bead, 272 us so.
+// gathers: N = 77, M = 50, 12 replicas 1243 us with a thread per bead, 189 us so.
 constexpr int kCompatBlock = 512;  // (1024 spills)
 struct RadialTerms {
     double a, l;  // the action's own table (or 0.5 / r) and the long-range one

@@ -986,7 +986,7 @@ __global__ __launch_bounds__(TABLE ? kTabBlock : kPermBlock) void k_propose_perm
     // whose label may change at the wrap) goes to the kernels of the Boltzmann
     // bisection: its beads in prop_new, its phase chains and the bisection's
     // rho_k items, and the LDS pair kernel unless its label changes in the
-    // window.  Several chains go to k_pair_multi and k_rho_multi.
+    // window.  Several chains go to the kernels of the two lists.
     const bool single = n == 1 && (!R.use_long_range || (R.ritems_bis && nm * R.n_chunks <= R.n_ritems_bis));
     if (single) {
         const int l1 = R.ch_lbl[0], l2 = R.ch_lbl2[0];
